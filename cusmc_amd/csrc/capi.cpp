@@ -34,9 +34,9 @@ namespace {
 
 // Launch shape for one group of instances.
 struct Plan {
-    int S = 1, C = 1, R = 64, stride = 1;
+    int S = 1, C = 1, R = 64, stride = 1, scratch = 1;
     int occ = 0;  // run-kernel build: 0 registers unrestricted, 3 three waves per SIMD
-    int tab = 0;          // tables staged in LDS: 0 none, 1 all hot tables, 2 all but the locations
+    bool tab = false;     // tables staged in LDS
     int group_waves = 1;  // waves per workgroup
     uint32_t table_bytes = 0, wave_lds = 0;
     size_t lds = 0;
@@ -47,49 +47,70 @@ struct Plan {
 
 constexpr size_t kLdsPerCu = 160 * 1024;
 
-Plan plan_launch(int P, int max_vars, int lanes, int occ, int tables, uint32_t table_bytes, uint32_t small_bytes,
-                 int waves_req,
-                 int waves_per_cu, uint64_t total_runs, uint64_t max_runs_per_inst, bool trace, int cu_count) {
+int tree_levels(int S) {
+    int levels = 0;
+    while ((1 << levels) < S) ++levels;
+    return levels;
+}
+
+// LDS of one wave (sim_body.h): variables of its R runs, scratch, state words
+// and, with digests, locations.
+size_t wave_lds_bytes(int R, int stride, int scratch, int C, bool trace) {
+    return ((size_t)R * stride * 8 + (size_t)scratch * 512 + (size_t)C * 256 * (trace ? 2 : 1) + 15) & ~(size_t)15;
+}
+
+// The most variables a packing may hold: those of the packed runs, a clock
+// time each and two doubles per lane and race-tree level, in 60,000 bytes.
+bool vars_fit(int R, int n_vars, int levels) {
+    return (size_t)R * ((n_vars + 1) | 1) * 8 + (size_t)levels * 1024 <= 60000;
+}
+
+Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs, bool trace) {
     Plan pl;
-    if (occ != 0 && occ != 3) throw std::runtime_error("occupancy must be 0 or 3");
-    if (tables < 0 || tables > 2) throw std::runtime_error("tables must be 0, 1 or 2");
-    pl.occ = occ;
-    int S = lanes ? lanes : (P < 64 ? P : 64);
+    const int P = m->img.n_leaves;
+    const smc_launch want = use ? *use : smc_launch{};
+    if (want.occupancy != 0 && want.occupancy != 3) throw std::runtime_error("occupancy must be 0 or 3");
+    if (want.tables < 0 || want.tables > 2) throw std::runtime_error("tables must be 0, 1 or 2");
+    pl.occ = want.occupancy;
+    int S = want.lanes_per_run ? want.lanes_per_run : (P < 64 ? P : 64);
     if (S <= 0 || S > 64 || (S & (S - 1))) throw std::runtime_error("lanes_per_run must be a power of two <= 64");
     if (S > P) S = P;
     pl.S = S;
     pl.C = P / S;
     if (pl.C > 16) throw std::runtime_error("limit: more than 16 components per lane; use more lanes per run");
     pl.R = 64 / S;
-    pl.stride = (max_vars + 1) | 1;  // clock time, then the variables
-    // per wave: variables of the R packed runs, then two doubles per lane
-    // for each butterfly level of the race tree
-    int levels = 0;
-    while ((1 << levels) < S) ++levels;
-    const size_t wave = ((size_t)pl.R * pl.stride * sizeof(double) + (size_t)2 * levels * 64 * sizeof(double) + 15) & ~(size_t)15;
-    if (wave > 60000) throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
+    pl.stride = m->img.n_vars | 1;
+    const int levels = tree_levels(S);
+    if (!vars_fit(pl.R, m->img.n_vars, levels))
+        throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
+    pl.scratch = std::max(pl.C, levels);
+    const size_t wave = wave_lds_bytes(pl.R, pl.stride, pl.scratch, pl.C, trace);
     pl.wave_lds = (uint32_t)wave;
-    pl.tab = trace ? 0 : tables;  // digest runs (parity checks) read the tables from global memory
-    if (pl.tab) {
-        const uint32_t bytes = pl.tab == 1 ? table_bytes : small_bytes;
-        if (bytes == 0 || bytes % 16) throw std::runtime_error("internal: table size");
-        pl.table_bytes = bytes;
+    if (want.tables) {
+        pl.table_bytes = m->table_bytes;
         pl.group_waves = SMC_MAX_GROUP_WAVES;
-        if (bytes + (size_t)pl.group_waves * wave > kLdsPerCu)
-            throw std::runtime_error("limit: the model tables do not fit in LDS");
+        pl.tab = pl.table_bytes + (size_t)pl.group_waves * wave + 64 <= kLdsPerCu;
+        if (!pl.tab) {
+            // tables that fit at 48 bytes a location are accepted all the
+            // same (they are read from global memory)
+            if (want.tables == 1 && !trace && (size_t)m->dm.n_locs * 48 + (size_t)pl.group_waves * wave > kLdsPerCu)
+                throw std::runtime_error("limit: the model tables do not fit in LDS");
+            pl.table_bytes = 0;
+            pl.group_waves = 1;
+        }
     }
     pl.lds = pl.table_bytes + (size_t)pl.group_waves * wave;
-    int waves = waves_req;
+    int waves = want.waves;
     if (waves <= 0) {
         int blocks = 0;
         hip_check(smc::sim_occupancy(pl.C, trace, pl.occ, pl.tab, pl.group_waves, pl.lds, &blocks), "occupancy query");
         int per_cu = blocks * pl.group_waves;
-        if (waves_per_cu > 0 && waves_per_cu < per_cu) per_cu = waves_per_cu;
+        if (want.waves_per_cu > 0 && want.waves_per_cu < per_cu) per_cu = want.waves_per_cu;
         if (per_cu <= 0) {
             if (pl.tab) throw std::runtime_error("limit: the model tables do not fit in LDS");
             per_cu = 1;
         }
-        waves = cu_count * per_cu;
+        waves = m->cu_count * per_cu;
     }
     waves = (waves + pl.group_waves - 1) / pl.group_waves * pl.group_waves;
     // chunks: enough per wave to balance uneven run lengths, at most 64 rounds of the wave's segments
@@ -98,7 +119,7 @@ Plan plan_launch(int P, int max_vars, int lanes, int occ, int tables, uint32_t t
     if (k < 1) k = 1;
     if (k > 64) k = 64;
     uint64_t chunk = k * pl.R;
-    if (chunk > max_runs_per_inst && max_runs_per_inst > 0) chunk = max_runs_per_inst;
+    if (chunk > total_runs) chunk = total_runs;
     if (chunk < 1) chunk = 1;
     pl.chunk_runs = (uint32_t)chunk;
     pl.waves = waves;
@@ -240,52 +261,61 @@ int smc_model_create(const smc_network *net, int device, smc_model **out) {
             if (im.var_clock[v]) var_start[v] = -var_start[v];
         struct Part { const void *src; size_t bytes; size_t off; };
         std::vector<Part> parts = {
+            {im.hots.data(), im.hots.size() * sizeof(DevHot), 0},
             {im.locs.data(), im.locs.size() * sizeof(DevLoc), 0},
-            {im.invs.data(), im.invs.size() * sizeof(DevInv), 0},
             {im.edges.data(), im.edges.size() * sizeof(DevEdge), 0},
-            {im.guards.data(), im.guards.size() * sizeof(DevGuard), 0},
+            {im.invs.data(), im.invs.size() * sizeof(DevInv), 0},
             {im.upds.data(), im.upds.size() * sizeof(DevUpd), 0},
+            {im.guards.data(), im.guards.size() * sizeof(DevGuard), 0},
             {im.consts.data(), im.consts.size() * sizeof(double), 0},
             {im.code.data(), im.code.size() * sizeof(DevInsn), 0},
             {var_start.data(), var_start.size() * sizeof(double), 0},
+            {im.comp_word.data(), im.comp_word.size() * sizeof(uint32_t), 0},
             {im.comp_init_loc.data(), im.comp_init_loc.size() * sizeof(int32_t), 0},
             {im.var_clock.data(), im.var_clock.size() * sizeof(uint8_t), 0},
             {im.comp_first_loc.data(), im.comp_first_loc.size() * sizeof(int32_t), 0},
             {im.loc_edge0.data(), im.loc_edge0.size() * sizeof(int32_t), 0},
+            {im.loc_rec.data(), im.loc_rec.size() * sizeof(uint32_t), 0},
         };
+        constexpr size_t kStaged = 8;  // hots .. code: what the run kernel reads every step
         size_t total = 0;
-        for (auto &p : parts) { p.off = total; total = align_up(total + p.bytes, 256); }
+        for (size_t i = 0; i < parts.size(); ++i) {
+            // the staged tables lie close together (16-byte records)
+            total = align_up(total, i > 0 && i < kStaged ? 16 : 256);
+            parts[i].off = total;
+            total += parts[i].bytes;
+        }
+        total = align_up(total, 256);
         std::vector<uint8_t> host(total, 0);
         for (auto &p : parts) if (p.bytes) memcpy(host.data() + p.off, p.src, p.bytes);
         hip_check(hipMalloc(&m->arena, total), "hipMalloc model arena");
         hip_check(hipMemcpy(m->arena, host.data(), total, hipMemcpyHostToDevice), "upload model");
         auto at = [&](int i) { return (const void *)((const uint8_t *)m->arena + parts[i].off); };
-        m->table_bytes = (uint32_t)parts[7].off;  // locs .. code: what the run kernel reads every step
-        m->small_off = (uint32_t)parts[1].off;    // invs .. code
-        m->small_bytes = (uint32_t)(parts[7].off - parts[1].off);
+        m->table_bytes = (uint32_t)align_up(parts[kStaged - 1].off + parts[kStaged - 1].bytes, 16);
         DevModel &d = m->dm;
-        d.locs = (decltype(d.locs))at(0);
-        d.invs = (decltype(d.invs))at(1);
+        d.hots = (decltype(d.hots))at(0);
+        d.locs = (decltype(d.locs))at(1);
         d.edges = (decltype(d.edges))at(2);
-        d.guards = (decltype(d.guards))at(3);
+        d.invs = (decltype(d.invs))at(3);
         d.upds = (decltype(d.upds))at(4);
-        d.consts = (decltype(d.consts))at(5);
-        d.code = (decltype(d.code))at(6);
-        d.var_init = (decltype(d.var_init))at(7);
-        d.comp_init_loc = (decltype(d.comp_init_loc))at(8);
-        d.var_clock = (decltype(d.var_clock))at(9);
-        d.comp_first_loc = (decltype(d.comp_first_loc))at(10);
-        d.loc_edge0 = (decltype(d.loc_edge0))at(11);
+        d.guards = (decltype(d.guards))at(5);
+        d.consts = (decltype(d.consts))at(6);
+        d.code = (decltype(d.code))at(7);
+        d.var_init = (decltype(d.var_init))at(8);
+        d.comp_word = (decltype(d.comp_word))at(9);
+        d.comp_init_loc = (decltype(d.comp_init_loc))at(10);
+        d.var_clock = (decltype(d.var_clock))at(11);
+        d.comp_first_loc = (decltype(d.comp_first_loc))at(12);
+        d.loc_edge0 = (decltype(d.loc_edge0))at(13);
+        d.loc_rec = (decltype(d.loc_rec))at(14);
         d.n_comp = im.n_comp;
         d.n_vars = im.n_vars;
-        int nclk = 0;
-        for (int k : im.var_kind) nclk += k == SMC_VAR_CLOCK;
-        d.n_clocks = nclk;
         d.n_leaves = im.n_leaves;
-        d.n_locs = (int)im.locs.size();
-        d.n_edges = net->n_edges;
+        d.n_locs = (int)im.loc_rec.size();
+        d.rec_shift = im.rec_shift;
+        d.base_mask = (1u << im.rec_shift) - 1u;
+        d.tests = im.tests;
         d.freeze = im.freeze ? 1 : 0;
-        d.guarded = im.guarded ? 1 : 0;
         hip_check(hipMalloc(&m->d_inst, sizeof(InstDesc)), "hipMalloc instance");
         hip_check(hipMalloc(&m->d_counter, sizeof(unsigned long long)), "hipMalloc counter");
         hip_check(hipMalloc(&m->d_partials, 1024 * sizeof(ReducePartial)), "hipMalloc partials");
@@ -313,9 +343,7 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
                         launch->tables))
                 ? launch : (m->has_tuned ? &m->tuned : nullptr);
         hip_check(hipSetDevice(m->device), "hipSetDevice");
-        Plan pl = plan_launch(m->img.n_leaves, m->img.n_vars, use ? use->lanes_per_run : 0, use ? use->occupancy : 0,
-                              use ? use->tables : 0, m->table_bytes, m->small_bytes, use ? use->waves : 0,
-                              use ? use->waves_per_cu : 0, n_runs, n_runs, trace, m->cu_count);
+        Plan pl = plan_launch(m, use, n_runs, trace);
         m->runs.ensure(n_runs);
         pl.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
         int waves = pl.waves;
@@ -331,13 +359,11 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         lp.inst = m->d_inst;
         lp.n_inst = 1;
         lp.var_stride = pl.stride;
+        lp.scratch = pl.scratch;
         lp.total_chunks = pl.total_chunks;
         lp.counter = m->d_counter;
         lp.round = nullptr;
-        lp.tables = pl.tab == 1   ? (decltype(lp.tables))m->arena
-                    : pl.tab == 2 ? (decltype(lp.tables))((const uint8_t *)m->arena + m->small_off)
-                                  : nullptr;
-        lp.table_mode = pl.tab;
+        lp.tables = pl.tab ? (decltype(lp.tables))m->arena : nullptr;
         lp.table_bytes = pl.table_bytes;
         lp.wave_lds = pl.wave_lds;
         const uint32_t blocks = reduce_blocks(n_runs);
@@ -392,9 +418,7 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         void *scr = nullptr;
         hip_check(smc::noalloc_scratch(m->device, &scr), "scratch address");
         uint8_t *base = (uint8_t *)scr;
-        Plan pl = plan_launch(m->img.n_leaves, m->img.n_vars, use ? use->lanes_per_run : 0, use ? use->occupancy : 0,
-                              use ? use->tables : 0, m->table_bytes, m->small_bytes, use ? use->waves : 0,
-                              use ? use->waves_per_cu : 0, n_runs, n_runs, false, m->cu_count);
+        Plan pl = plan_launch(m, use, n_runs, false);
         pl.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
         int waves = pl.waves;
         if ((uint64_t)waves > pl.total_chunks)
@@ -423,13 +447,11 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         lp.inst = d_inst;
         lp.n_inst = 1;
         lp.var_stride = pl.stride;
+        lp.scratch = pl.scratch;
         lp.total_chunks = pl.total_chunks;
         lp.counter = d_counter;
         lp.round = nullptr;
-        lp.tables = pl.tab == 1   ? (decltype(lp.tables))m->arena
-                    : pl.tab == 2 ? (decltype(lp.tables))((const uint8_t *)m->arena + m->small_off)
-                                  : nullptr;
-        lp.table_mode = pl.tab;
+        lp.tables = pl.tab ? (decltype(lp.tables))m->arena : nullptr;
         lp.table_bytes = pl.table_bytes;
         lp.wave_lds = pl.wave_lds;
 
@@ -486,9 +508,9 @@ std::string tune_cache_path() {
 uint64_t tune_key(const smc_model *m, const smc_query *q, uint64_t sample_runs) {
     const smc::ModelImage &im = m->img;
     uint64_t h = 1469598103934665603ull;
-    h = fnv_vec(h, im.locs); h = fnv_vec(h, im.invs); h = fnv_vec(h, im.edges); h = fnv_vec(h, im.guards);
+    h = fnv_vec(h, im.hots); h = fnv_vec(h, im.locs); h = fnv_vec(h, im.invs); h = fnv_vec(h, im.edges); h = fnv_vec(h, im.guards);
     h = fnv_vec(h, im.upds); h = fnv_vec(h, im.consts); h = fnv_vec(h, im.code); h = fnv_vec(h, im.var_init);
-    h = fnv_vec(h, im.comp_init_loc);
+    h = fnv_vec(h, im.comp_word);
     const int32_t qi[4] = {q->kind, q->var, q->is_max, q->is_estimate};
     const double qd[2] = {q->threshold, q->time_bound};
     h = fnv1a(h, qi, sizeof qi); h = fnv1a(h, qd, sizeof qd);
@@ -555,12 +577,11 @@ int smc_autotune(smc_model *m, const smc_query *q, uint64_t seed, uint64_t sampl
         for (int S = P < 64 ? P : 64; S >= 1; S >>= 1) {
             if (P / S > 16) break;
             for (int occ : {0, 3})
-                for (int tab : {0, 1, 2}) {
+                for (int tab : {0, 1}) {
                     cands.push_back(smc_launch{S, 0, 0, occ, tab});
                     int blocks = 0;
                     try {
-                        Plan pl = plan_launch(P, m->img.n_vars, S, occ, tab, m->table_bytes, m->small_bytes, 0, 0, sample_runs,
-                                              sample_runs, false, m->cu_count);
+                        Plan pl = plan_launch(m, &cands.back(), sample_runs, false);
                         hip_check(smc::sim_occupancy(pl.C, false, pl.occ, pl.tab, pl.group_waves, pl.lds, &blocks),
                                   "occupancy query");
                         const int per_cu = blocks * pl.group_waves;
@@ -576,8 +597,7 @@ int smc_autotune(smc_model *m, const smc_query *q, uint64_t seed, uint64_t sampl
         for (const smc_launch &c : cands) {
             uint64_t n = sample_runs;
             try {
-                Plan pl = plan_launch(P, m->img.n_vars, c.lanes_per_run, c.occupancy, c.tables, m->table_bytes, m->small_bytes, 0,
-                                      c.waves_per_cu, sample_runs, sample_runs, false, m->cu_count);
+                Plan pl = plan_launch(m, &c, sample_runs, false);
                 n = std::max<uint64_t>(n, 2ull * (uint64_t)pl.waves * (uint64_t)pl.R);
             } catch (const std::exception &) {
                 continue;  // e.g. LDS budget exceeded at this packing
@@ -608,7 +628,7 @@ struct smc_batch {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<smc_batch_item> items;
     std::vector<RunBuffers> bufs;
-    int C = 8, occ = 0, waves = 1, stride = 1;  // the one launch: slots per lane, register policy
+    int C = 8, occ = 0, waves = 1, stride = 1, max_vars = 1;  // the one launch: slots per lane, register policy
     size_t lds = 0;
     InstDesc *d_all = nullptr;
     unsigned long long *d_counter = nullptr;
@@ -642,11 +662,14 @@ namespace {
 struct BatchShape {
     std::vector<InstDesc> inst;
     size_t wave_lds = 0;
+    int scratch = 1;
     uint64_t chunks = 0;
 };
 
 BatchShape batch_shape(smc_batch *b, int C, int waves, uint64_t runs_override) {
     BatchShape sh;
+    bool fits = true;
+    int max_R = 1;
     uint64_t total = 0;
     for (auto &it : b->items) total += runs_override ? std::min<uint64_t>(runs_override, it.n_runs) : it.n_runs;
     const uint64_t per_wave = (total + (uint64_t)waves - 1) / (uint64_t)waves;
@@ -656,10 +679,10 @@ BatchShape batch_shape(smc_batch *b, int C, int waves, uint64_t runs_override) {
         if (P > 64 * C) throw std::runtime_error("internal: instance wider than the launch's packing");
         const int S = P / C >= 1 ? P / C : 1;
         const int R = 64 / S;
-        int levels = 0;
-        while ((1 << levels) < S) ++levels;
-        const size_t wave = ((size_t)R * b->stride * 8 + (size_t)2 * levels * 64 * 8 + 15) & ~(size_t)15;
-        sh.wave_lds = std::max(sh.wave_lds, wave);
+        const int levels = tree_levels(S);
+        fits = fits && vars_fit(R, b->max_vars, levels);
+        sh.scratch = std::max(sh.scratch, std::max(C, levels));
+        max_R = std::max(max_R, R);
         const uint64_t n = runs_override ? std::min<uint64_t>(runs_override, it.n_runs) : it.n_runs;
         uint64_t k = (per_wave + 4ull * R - 1) / (4ull * R);
         k = std::max<uint64_t>(1, std::min<uint64_t>(k, 64));
@@ -673,7 +696,8 @@ BatchShape batch_shape(smc_batch *b, int C, int waves, uint64_t runs_override) {
         sh.chunks += (n + chunk - 1) / chunk;
         sh.inst.push_back(d);
     }
-    if (sh.wave_lds > 60000) throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
+    if (!fits) throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
+    sh.wave_lds = wave_lds_bytes(max_R, b->stride, sh.scratch, C, false);
     return sh;
 }
 
@@ -712,7 +736,8 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
         hip_check(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking), "hipStreamCreate");
         for (hipEvent_t *e : {&b->ev0, &b->ev1}) hip_check(hipEventCreate(e), "hipEventCreate");
         const int cu = items[0].model->cu_count;
-        b->stride = (max_vars + 1) | 1;  // clock time, then the variables
+        b->max_vars = max_vars;
+        b->stride = max_vars | 1;
         b->bufs.resize(n_items);
         uint64_t maxr = 0;
         for (int i = 0; i < n_items; ++i) {
@@ -743,11 +768,11 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
             b->lp.inst = b->d_all;
             b->lp.n_inst = n_items;
             b->lp.var_stride = b->stride;
+            b->lp.scratch = sh.scratch;
             b->lp.total_chunks = sh.chunks;
             b->lp.counter = b->d_counter;
             b->lp.round = b->d_round;
             b->lp.tables = nullptr;
-            b->lp.table_mode = 0;
             b->lp.table_bytes = 0;
             b->lp.wave_lds = (uint32_t)sh.wave_lds;
             hip_check(hipMemcpy(b->d_all, sh.inst.data(), n_items * sizeof(InstDesc), hipMemcpyHostToDevice),

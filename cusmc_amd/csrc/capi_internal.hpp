@@ -82,9 +82,7 @@ struct smc_model {
     smc::ModelImage img;
     DevModel dm{};
     void *arena = nullptr;
-    uint32_t table_bytes = 0;  // arena prefix a run kernel may stage in LDS (the hot tables)
-    uint32_t small_off = 0;    // the hot tables after the location records: offset and bytes
-    uint32_t small_bytes = 0;
+    uint32_t table_bytes = 0;  // arena prefix a run kernel may stage in LDS (what a step reads)
     int cu_count = 0;
     smc::capi::RunBuffers runs;
     InstDesc h_inst{};

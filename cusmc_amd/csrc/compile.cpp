@@ -14,7 +14,14 @@
 //   * guards: only conjuncts on a variable are kept (simulation.cu:209); an
 //     edge with a `!=` conjunct can never be enabled (simulation.cu:249-251)
 //     and is flagged instead.
-//   * locations get a delay class so the kernel does not re-derive it.
+//   * locations get a delay class so the kernel does not re-derive it, and
+//     what every race step reads of them is laid out apart (DevHot).
+//   * comparisons with a constant become interval tests.
+//   * locations with equal records share one record class: the instances of
+//     a template differ only in their private variables, which are named
+//     relative to the component (CSMA/CA with 100 processes: 1,800 locations,
+//     28 classes, and tables of a few kilobytes that every kernel can keep in
+//     LDS).
 #include "compile.hpp"
 
 #include <cstring>
@@ -34,7 +41,19 @@ namespace {
 
 class Lowerer {
 public:
-    Lowerer(const smc_network &n, ModelImage &img) : n_(n), img_(img) {}
+    // base: first private variable of each component (-1: none); owner: the
+    // component a variable is private to (-1: none).  Without them variables
+    // keep their own indices.
+    Lowerer(const smc_network &n, ModelImage &img, const std::vector<int> *owner = nullptr,
+            const std::vector<int> *base = nullptr)
+        : n_(n), img_(img), owner_(owner), base_(base) {}
+
+    // Later references belong to component c.
+    void set_component(int c) { comp_ = c; }
+    bool local(int v) const { return owner_ && (*owner_)[v] == comp_ && comp_ >= 0; }
+    uint32_t index(int v) const { return (uint32_t)(local(v) ? v - (*base_)[comp_] : v); }
+    // Variable operand of a record's 16-bit field.
+    uint16_t field(int v) const { return (uint16_t)(index(v) | (local(v) ? SMC_VAR_LOCAL : 0u)); }
 
     uint32_t ref(int e, double dflt) {
         if (e < 0) return SMC_REF_MAKE(SMC_REF_CONST, const_index(dflt));
@@ -42,7 +61,8 @@ public:
         if (x.op == SMC_E_LIT) return SMC_REF_MAKE(SMC_REF_CONST, const_index(x.value));
         if (x.op == SMC_E_RANDOM) return SMC_REF_MAKE(SMC_REF_CONST, const_index(1.0));
         if (x.op == SMC_E_VAR)
-            return SMC_REF_MAKE(n_.var_kind[x.var] == SMC_VAR_CLOCK ? SMC_REF_CLOCK : SMC_REF_VAR, (uint32_t)x.var);
+            return SMC_REF_MAKE(n_.var_kind[x.var] == SMC_VAR_CLOCK ? SMC_REF_CLOCK : SMC_REF_VAR,
+                                index(x.var) | (local(x.var) ? SMC_REF_LOCAL : 0u));
         std::vector<DevInsn> prog;
         int maxreg = 0;
         uint16_t r = emit(e, 0, prog, &maxreg);
@@ -65,6 +85,8 @@ public:
 private:
     const smc_network &n_;
     ModelImage &img_;
+    const std::vector<int> *owner_, *base_;
+    int comp_ = -1;
     std::unordered_map<uint64_t, uint32_t> const_cache_;
     std::unordered_map<std::string, uint32_t> code_cache_;
 
@@ -106,7 +128,8 @@ private:
         if (x.op == SMC_E_RANDOM) return SMC_OPND(SMC_OPND_CONST, const_index(1.0));
         if (x.op == SMC_E_VAR) {
             if (x.var > SMC_MAX_OPND_INDEX) throw std::runtime_error("limit: variable index above 16383 in an expression");
-            return SMC_OPND(n_.var_kind[x.var] == SMC_VAR_CLOCK ? SMC_OPND_CLOCK : SMC_OPND_VAR, (uint32_t)x.var);
+            return SMC_OPND(n_.var_kind[x.var] == SMC_VAR_CLOCK ? SMC_OPND_CLOCK : SMC_OPND_VAR,
+                            index(x.var) | (local(x.var) ? SMC_OPND_LOCAL : 0u));
         }
         int ar = smc_op_arity(x.op);
         const int kids[3] = {x.a, x.b, x.c};
@@ -134,65 +157,167 @@ private:
     }
 };
 
-// Instances of one template differ in their location numbers only where
-// they read or write local variables; the rest of their records are equal.
-// With edge destinations relative to the source location, equal runs of
-// records (a location's edges, an edge's guards and updates, a location's
-// invariants and blocking test) are stored once: SIR-350's 112 KB of
-// tables shrink to its 34 KB of location records, which fit in LDS.  The
-// network's edge numbering stays available for digests (loc_edge0).
-void share_records(ModelImage &img) {
-    std::vector<DevEdge> edges;
-    std::vector<DevGuard> guards;
-    std::vector<DevUpd> upds;
-    std::vector<DevInv> invs;
-    std::unordered_map<std::string, uint32_t> gmap, umap, emap, imap;
-    auto intern = [](auto &out, auto &map, const auto *first, size_t n) -> uint32_t {
-        if (n == 0) return 0;
-        std::string key((const char *)first, n * sizeof(*first));
-        auto it = map.find(key);
-        if (it != map.end()) return it->second;
-        const uint32_t at = (uint32_t)out.size();
-        out.insert(out.end(), first, first + n);
-        map.emplace(std::move(key), at);
-        return at;
+// The component each variable is private to (read and written by it alone),
+// or -1, and each component's first private variable.
+void private_variables(const smc_network &n, std::vector<int> &owner, std::vector<int> &base) {
+    constexpr int kNone = -1, kShared = -2;
+    owner.assign(n.n_vars, kNone);
+    base.assign(n.n_components, 0);
+    auto use = [&](int v, int c) { owner[v] = owner[v] == kNone || owner[v] == c ? c : kShared; };
+    std::function<void(int, int)> use_expr = [&](int x, int c) {
+        if (x < 0) return;
+        const smc_expr_node &nd = n.exprs[x];
+        if (nd.op == SMC_E_VAR) use(nd.var, c);
+        const int kids[3] = {nd.a, nd.b, nd.c};
+        for (int k = 0; k < smc_op_arity(nd.op); ++k) use_expr(kids[k], c);
     };
-    img.loc_edge0.assign(img.locs.size(), 0);
-    for (size_t l = 0; l < img.locs.size(); ++l) {
-        DevLoc &L = img.locs[l];
-        std::vector<DevEdge> run(img.edges.begin() + L.edge_first, img.edges.begin() + L.edge_first + L.edge_n);
-        for (DevEdge &d : run) {
-            d.dst -= (int32_t)l;
-            d.guard_first = intern(guards, gmap, img.guards.data() + d.guard_first, d.guard_n);
-            d.upd_first = intern(upds, umap, img.upds.data() + d.upd_first, d.upd_n);
+    auto use_constraint = [&](const smc_constraint &C, int c) {
+        if (C.uses_variable) use(C.var, c);
+        use_expr(C.rhs, c);
+    };
+    for (int c = 0; c < n.n_components; ++c)
+        for (int l = n.comp_first_loc[c]; l < n.comp_first_loc[c + 1]; ++l) {
+            const smc_location &L = n.locations[l];
+            use_expr(L.rate, c);
+            for (int k = 0; k < L.inv_count; ++k) use_constraint(n.constraints[L.inv_first + k], c);
+            for (int k = 0; k < L.edge_count; ++k) {
+                const smc_edge &E = n.edges[L.edge_first + k];
+                use_expr(E.weight, c);
+                for (int g = 0; g < E.guard_count; ++g) use_constraint(n.constraints[E.guard_first + g], c);
+                for (int u = 0; u < E.upd_count; ++u) {
+                    use(n.updates[E.upd_first + u].var, c);
+                    use_expr(n.updates[E.upd_first + u].expr, c);
+                }
+            }
         }
-        img.loc_edge0[l] = (int32_t)L.edge_first;
-        L.edge_first = intern(edges, emap, run.data(), run.size());
-        L.inv_first = intern(invs, imap, img.invs.data() + L.inv_first, L.n_inv);
-        if (L.flags & SMC_LF_GUARDED) {
-            size_t k = L.block_first;
-            while (!(img.guards[k].flags & SMC_GF_END_LOC)) ++k;
-            L.block_first = intern(guards, gmap, img.guards.data() + L.block_first, k + 1 - L.block_first);
-        }
+    std::vector<uint8_t> seen(n.n_components, 0);
+    for (int v = 0; v < n.n_vars; ++v) {
+        if (owner[v] < 0) { owner[v] = -1; continue; }
+        if (!seen[owner[v]]) { seen[owner[v]] = 1; base[owner[v]] = v; }
     }
-    img.edges.swap(edges);
-    img.guards.swap(guards);
-    img.upds.swap(upds);
-    img.invs.swap(invs);
 }
 
-}  // namespace
+// Doubles in the order of their values, as integers.
+int64_t order_of(double x) {
+    int64_t b;
+    memcpy(&b, &x, 8);
+    return b < 0 ? (int64_t)0x8000000000000000ull - b : b;
+}
+double double_of(int64_t o) {
+    const int64_t b = o < 0 ? (int64_t)0x8000000000000000ull - o : o;
+    double x;
+    memcpy(&x, &b, 8);
+    return x;
+}
 
-ModelImage compile_model(const smc_network &n) {
-    std::string err = validate(n);
-    if (!err.empty()) throw std::runtime_error(err);
+// The interval of values x for which `x op r` holds (empty: lo > hi).  For
+// `==` the ends are the first and last x with |x - r| <= SMC_TOL in doubles:
+// the rounded difference is monotonic in x, so they are found by bisection.
+void range_of(int op, double r, double *lo, double *hi) {
+    const double INF = HUGE_VAL;
+    *lo = INF;
+    *hi = -INF;
+    if (r != r) return;
+    switch (op) {
+    case SMC_C_LE: *lo = -INF; *hi = r; return;
+    case SMC_C_GE: *lo = r; *hi = INF; return;
+    case SMC_C_LT: if (r > -INF) { *lo = -INF; *hi = std::nextafter(r, -INF); } return;
+    case SMC_C_GT: if (r < INF) { *lo = std::nextafter(r, INF); *hi = INF; } return;
+    case SMC_C_EQ: break;
+    default: return;
+    }
+    if (std::fabs(r) == INF) return;
+    auto end = [&](double outside) {
+        int64_t in = order_of(r), out = order_of(outside);  // the test holds at `in`, fails at `out`
+        while (in - out > 1 || out - in > 1) {
+            const int64_t mid = in / 2 + out / 2 + (in % 2 + out % 2) / 2;
+            if (std::fabs(double_of(mid) - r) <= SMC_TOL) in = mid;
+            else out = mid;
+        }
+        return double_of(in);
+    };
+    *lo = end(-INF);
+    *hi = end(INF);
+}
+
+// Index of the run of n records in `out`, stored once per content.
+template <class T>
+uint32_t intern(std::vector<T> &out, std::unordered_map<std::string, uint32_t> &map, const T *first, size_t n) {
+    if (n == 0) return 0;
+    std::string key((const char *)first, n * sizeof(T));
+    auto it = map.find(key);
+    if (it != map.end()) return it->second;
+    const uint32_t at = (uint32_t)out.size();
+    out.insert(out.end(), first, first + n);
+    map.emplace(std::move(key), at);
+    return at;
+}
+
+// One location before classes are formed.
+struct RawEdge {
+    DevEdge e{};
+    int dst_loc = 0;
+    std::vector<DevGuard> guards;
+    std::vector<DevUpd> upds;
+};
+struct RawLoc {
+    DevHot hot{};
+    DevLoc loc{};
+    std::vector<RawEdge> edges;
+    std::vector<DevInv> invs;
+    std::vector<DevGuard> block;
+};
+
+// Partition of the locations into classes of equal records: first by their
+// own content, then, until nothing splits, by the classes their edges lead
+// to.  Networks whose classes take long to separate (chains of equal
+// locations) keep one class per location.
+std::vector<uint32_t> classes_of(const std::vector<RawLoc> &raw, uint32_t *count) {
+    const size_t n = raw.size();
+    std::vector<uint32_t> cls(n), next(n);
+    auto put = [](std::string &k, const auto &v) {
+        const uint32_t c = (uint32_t)v.size();
+        k.append((const char *)&c, 4);
+        if (c) k.append((const char *)v.data(), c * sizeof(v[0]));
+    };
+    std::unordered_map<std::string, uint32_t> ids;
+    for (size_t l = 0; l < n; ++l) {
+        std::string k((const char *)&raw[l].hot, sizeof(DevHot));
+        k.append((const char *)&raw[l].loc, sizeof(DevLoc));
+        put(k, raw[l].invs);
+        put(k, raw[l].block);
+        for (const RawEdge &e : raw[l].edges) {
+            k.append((const char *)&e.e, sizeof(DevEdge));
+            put(k, e.guards);
+            put(k, e.upds);
+        }
+        cls[l] = ids.emplace(std::move(k), (uint32_t)ids.size()).first->second;
+    }
+    *count = (uint32_t)ids.size();
+    for (int pass = 0; pass < 64; ++pass) {
+        ids.clear();
+        for (size_t l = 0; l < n; ++l) {
+            std::string k((const char *)&cls[l], 4);
+            for (const RawEdge &e : raw[l].edges) k.append((const char *)&cls[e.dst_loc], 4);
+            next[l] = ids.emplace(std::move(k), (uint32_t)ids.size()).first->second;
+        }
+        cls.swap(next);
+        if (ids.size() == *count) return cls;
+        *count = (uint32_t)ids.size();
+    }
+    for (size_t l = 0; l < n; ++l) cls[l] = (uint32_t)l;
+    *count = (uint32_t)n;
+    return cls;
+}
+
+// use_locals: private variables named relative to their component.
+ModelImage lower(const smc_network &n, bool use_locals) {
     ModelImage img;
     img.n_comp = n.n_components;
     img.n_vars = n.n_vars;
     int leaves = 1;
     while (leaves < n.n_components) leaves <<= 1;
     img.n_leaves = leaves;
-    Lowerer lw(n, img);
 
     img.var_init.assign(n.var_init, n.var_init + n.n_vars);
     img.var_kind.assign(n.var_kind, n.var_kind + n.n_vars);
@@ -200,71 +325,60 @@ ModelImage compile_model(const smc_network &n) {
     img.comp_init_loc.assign(n.comp_init_loc, n.comp_init_loc + n.n_components);
     img.comp_first_loc.assign(n.comp_first_loc, n.comp_first_loc + n.n_components + 1);
 
-    for (int l = 0; l < n.n_locations; ++l) {
-        const smc_location &L = n.locations[l];
-        DevLoc d{};
-        d.type = (uint8_t)L.type;
-        d.rate = lw.ref(L.rate, 1.0);
-        d.inv_first = (uint32_t)img.invs.size();
-        for (int k = 0; k < L.inv_count; ++k) {
-            const smc_constraint &C = n.constraints[L.inv_first + k];
-            if (!C.uses_variable) continue;
-            if (n.var_kind[C.var] != SMC_VAR_CLOCK) continue;
-            if (C.op != SMC_C_LE && C.op != SMC_C_LT) continue;
-            DevInv iv{};
-            iv.var = (uint16_t)C.var;
-            iv.strict = C.op == SMC_C_LT;
-            iv.bound = lw.ref(C.rhs, 0.0);
-            if (SMC_REF_KIND(iv.bound) == SMC_REF_CONST) {
-                iv.bound_const = 1;
-                iv.bound_value = img.consts[iv.bound & 0x3FFFFFFFu];
-            }
-            img.invs.push_back(iv);
-        }
-        size_t ninv = img.invs.size() - d.inv_first;
-        if (ninv > 65535) throw std::runtime_error("limit: more than 65535 invariants on a location");
-        d.n_inv = (uint16_t)ninv;
-        if (ninv == 1 && img.invs[d.inv_first].bound_const) {
-            d.flags |= SMC_LF_INL_INV;
-            d.inl_value = img.invs[d.inv_first].bound_value;
-            d.inl_var = img.invs[d.inv_first].var;
-            d.inl_op = img.invs[d.inv_first].strict;
-        }
-        d.klass = L.type > SMC_LOC_GOAL ? SMC_K_ZERO : (ninv > 0 ? SMC_K_BOUNDED : SMC_K_EXP);
-        if (L.edge_count > SMC_MAX_EDGES_PER_LOC)
-            throw std::runtime_error("limit: a location has more than 64 outgoing edges");
-        d.edge_first = (uint32_t)L.edge_first;
-        d.edge_n = (uint16_t)L.edge_count;
-        if (SMC_REF_KIND(d.rate) == SMC_REF_CONST) {
-            d.rate_const = 1;
-            d.rate_value = img.consts[d.rate & 0x3FFFFFFFu];
-        }
-        img.locs.push_back(d);
-    }
-    // Receive edges whose updates commute within one broadcast.  Forms of
-    // an update: ADD (integer variable += integer constant), SET (:= a
-    // constant).  Per variable over all receive edges: all ADD, or all SET
-    // of one value, or written by a single component — then the writes of
-    // one broadcast's receivers give the same result in any order.
+    std::vector<int> owner, base;
+    private_variables(n, owner, base);
+    if (!use_locals) std::fill(base.begin(), base.end(), 0);
+    Lowerer lw(n, img, use_locals ? &owner : nullptr, use_locals ? &base : nullptr);
+    // expression identities across components (rates, for tilt groups)
+    ModelImage plain;
+    Lowerer lw_plain(n, plain);
+
+    std::vector<int8_t> clock_memo(n.n_exprs, -1);
+    std::function<bool(int)> reads_clock = [&](int x) -> bool {
+        if (x < 0) return false;
+        if (clock_memo[x] >= 0) return clock_memo[x] != 0;
+        const smc_expr_node &nd = n.exprs[x];
+        bool r = nd.op == SMC_E_VAR && n.var_kind[nd.var] == SMC_VAR_CLOCK;
+        if (!r && nd.op != SMC_E_LIT && nd.op != SMC_E_VAR)
+            r = reads_clock(nd.a) || reads_clock(nd.b) || reads_clock(nd.c);
+        clock_memo[x] = r ? 1 : 0;
+        return r;
+    };
+    std::function<bool(int)> reads_local = [&](int x) -> bool {
+        if (x < 0) return false;
+        const smc_expr_node &nd = n.exprs[x];
+        if (nd.op == SMC_E_VAR) return lw.local(nd.var);
+        const int kids[3] = {nd.a, nd.b, nd.c};
+        for (int k = 0; k < smc_op_arity(nd.op); ++k)
+            if (reads_local(kids[k])) return true;
+        return false;
+    };
     auto literal = [&](int x, double *v) {
         if (x < 0 || n.exprs[x].op != SMC_E_LIT) return false;
         *v = n.exprs[x].value;
         return true;
     };
     auto is_var = [&](int x, int var) { return x >= 0 && n.exprs[x].op == SMC_E_VAR && n.exprs[x].var == var; };
-    enum { F_OTHER = 0, F_ADD = 1, F_SET = 2 };
+
+    // Forms of an update: ADD (integer variable += constant), SET (:= a
+    // constant).  Subtracting a constant is adding its negative, exactly.
     auto form = [&](const smc_update &U, double *c) -> int {
         const smc_expr_node *x = U.expr >= 0 ? &n.exprs[U.expr] : nullptr;
-        if (!x) return F_OTHER;
+        if (!x) return SMC_U_EXPR;
         if (n.var_kind[U.var] == SMC_VAR_INT &&
             ((x->op == SMC_E_ADD && is_var(x->a, U.var) && literal(x->b, c)) ||
              (x->op == SMC_E_ADD && literal(x->a, c) && is_var(x->b, U.var)) ||
-             (x->op == SMC_E_SUB && is_var(x->a, U.var) && literal(x->b, c) && ((*c = -*c), true))) &&
-            *c == std::floor(*c) && std::fabs(*c) < 2147483648.0)
-            return F_ADD;
-        if (literal(U.expr, c)) return F_SET;
-        return F_OTHER;
+             (x->op == SMC_E_SUB && is_var(x->a, U.var) && literal(x->b, c) && ((*c = -*c), true))))
+            return SMC_U_ADD;
+        if (literal(U.expr, c)) return SMC_U_SET;
+        return SMC_U_EXPR;
     };
+    auto whole = [](double c) { return c == std::floor(c) && std::fabs(c) < 2147483648.0; };
+    // Receive edges whose updates commute within one broadcast: additions
+    // are of integer constants, and per variable over all receive edges all
+    // are ADD, or all SET of one value, or it is written by a single
+    // component — then the writes of one broadcast's receivers give the same
+    // result in any order.
     struct VarUse { int add = 0, set = 0, other = 0, writer = -1; bool one_value = true; double value = 0.0; };
     std::vector<VarUse> use(n.n_vars);
     for (int c = 0; c < n.n_components; ++c)
@@ -277,8 +391,8 @@ ModelImage compile_model(const smc_network &n) {
                     VarUse &vu = use[U.var];
                     double cv = 0.0;
                     const int f = form(U, &cv);
-                    if (f == F_ADD) ++vu.add;
-                    else if (f == F_SET) {
+                    if (f == SMC_U_ADD && whole(cv)) ++vu.add;
+                    else if (f == SMC_U_SET) {
                         if (vu.set && cv != vu.value) vu.one_value = false;
                         vu.value = cv;
                         ++vu.set;
@@ -292,147 +406,263 @@ ModelImage compile_model(const smc_network &n) {
         if (vu.writer >= 0) return true;
         return vu.set == 0 || (vu.add == 0 && vu.one_value);
     };
-    std::vector<uint8_t> fast_edge(n.n_edges, 0);
-    std::vector<int8_t> clock_memo(n.n_exprs, -1);
-    std::function<bool(int)> reads_clock = [&](int x) -> bool {
-        if (x < 0) return false;
-        if (clock_memo[x] >= 0) return clock_memo[x] != 0;
-        const smc_expr_node &nd = n.exprs[x];
-        bool r = nd.op == SMC_E_VAR && n.var_kind[nd.var] == SMC_VAR_CLOCK;
-        if (!r && nd.op != SMC_E_LIT && nd.op != SMC_E_VAR)
-            r = reads_clock(nd.a) || reads_clock(nd.b) || reads_clock(nd.c);
-        clock_memo[x] = r ? 1 : 0;
-        return r;
-    };
 
-    for (int e = 0; e < n.n_edges; ++e) {
-        const smc_edge &E = n.edges[e];
-        DevEdge d{};
-        d.dst = E.dst;
-        d.channel = E.channel;
-        d.weight = lw.ref(E.weight, 1.0);
-        d.dst_goal = n.locations[E.dst].type == SMC_LOC_GOAL;
-        d.guard_first = (uint32_t)img.guards.size();
-        for (int k = 0; k < E.guard_count; ++k) {
-            const smc_constraint &C = n.constraints[E.guard_first + k];
-            if (!C.uses_variable) continue;
-            if (C.op == SMC_C_NE) { d.never = 1; continue; }
-            if (C.var > 65535) throw std::runtime_error("limit: guarded variable index above 65535");
-            DevGuard g{};
-            g.var = (uint16_t)C.var;
-            g.op = (uint8_t)C.op;
-            g.flags = (uint8_t)((n.var_kind[C.var] != SMC_VAR_CLOCK && !reads_clock(C.rhs) ? SMC_GF_CLOCK_FREE : 0) |
-                                (n.var_kind[C.var] == SMC_VAR_CLOCK ? SMC_GF_CLOCK : 0));
-            g.rhs = lw.ref(C.rhs, 0.0);
-            img.guards.push_back(g);
-        }
-        size_t ng = img.guards.size() - d.guard_first;
-        if (ng > 65535) throw std::runtime_error("limit: more than 65535 guards on an edge");
-        d.guard_n = (uint16_t)ng;
-        d.upd_first = (uint32_t)img.upds.size();
-        bool commute = E.channel < 0 && SMC_REF_KIND(d.weight) == SMC_REF_CONST;
-        std::vector<int> seen;
-        for (int k = 0; k < E.upd_count; ++k) {
-            const smc_update &U = n.updates[E.upd_first + k];
-            if (U.var > 65535) throw std::runtime_error("limit: assigned variable index above 65535");
-            DevUpd u{};
-            u.var = (uint16_t)U.var;
-            u.clock = n.var_kind[U.var] == SMC_VAR_CLOCK ? 1 : 0;
-            u.expr = lw.ref(U.expr, 0.0);
-            double cv = 0.0;
-            const int f = E.channel < 0 ? form(U, &cv) : F_OTHER;
-            if (f != F_OTHER && var_commutes(U.var)) {
-                u.kind = f == F_ADD ? SMC_U_ADD : SMC_U_SET;
-                u.value = cv;
-            } else {
-                commute = false;
-            }
-            if (std::find(seen.begin(), seen.end(), U.var) != seen.end()) commute = false;
-            seen.push_back(U.var);
-            img.upds.push_back(u);
-        }
-        fast_edge[e] = commute ? 1 : 0;
-        if (E.upd_count > 65535) throw std::runtime_error("limit: more than 65535 updates on an edge");
-        d.upd_n = (uint16_t)E.upd_count;
-        img.edges.push_back(d);
-    }
-    // time_free: the location's rate and its spontaneous edges' guards read
-    // no clock, so between transitions neither its enabled edges nor its
-    // rate change
     // Null racers leave an all-exponential race only while every rate is
     // constant between transitions (a rate reading a clock changes at each
     // null step of the reference's race).
     bool clock_rate = false;
     for (int l = 0; l < n.n_locations; ++l)
         if (reads_clock(n.locations[l].rate)) clock_rate = true;
-    for (int l = 0; l < n.n_locations; ++l) {
-        const smc_location &L = n.locations[l];
-        bool tf = !reads_clock(L.rate);
-        for (int k = 0; k < L.edge_count && tf; ++k) {
-            const smc_edge &E = n.edges[L.edge_first + k];
-            if (E.channel < 0) continue;
-            for (int g = 0; g < E.guard_count; ++g) {
-                const smc_constraint &G = n.constraints[E.guard_first + g];
-                if (!G.uses_variable) continue;
-                if (n.var_kind[G.var] == SMC_VAR_CLOCK || reads_clock(G.rhs)) tf = false;
+    img.freeze = !clock_rate;
+
+    std::vector<RawLoc> raw(n.n_locations);
+    img.info.resize(n.n_locations);
+    img.loc_edge0.assign(n.n_locations, 0);
+    for (int comp = 0; comp < n.n_components; ++comp) {
+        lw.set_component(comp);
+        for (int l = n.comp_first_loc[comp]; l < n.comp_first_loc[comp + 1]; ++l) {
+            const smc_location &L = n.locations[l];
+            RawLoc &R = raw[l];
+            DevLoc &d = R.loc;
+            LocInfo &info = img.info[l];
+            d.type = (uint8_t)L.type;
+            d.rate = lw.ref(L.rate, 1.0);
+            for (int k = 0; k < L.inv_count; ++k) {
+                const smc_constraint &C = n.constraints[L.inv_first + k];
+                if (!C.uses_variable) continue;
+                if (n.var_kind[C.var] != SMC_VAR_CLOCK) continue;
+                if (C.op != SMC_C_LE && C.op != SMC_C_LT) continue;
+                DevInv iv{};
+                iv.var = lw.field(C.var);
+                iv.strict = C.op == SMC_C_LT;
+                iv.bound = lw.ref(C.rhs, 0.0);
+                if (SMC_REF_KIND(iv.bound) == SMC_REF_CONST) {
+                    iv.bound_const = 1;
+                    iv.bound_value = img.consts[iv.bound & 0x3FFFFFFFu];
+                }
+                R.invs.push_back(iv);
             }
-        }
-        // blocking: always (every spontaneous edge has `!=`, or none), by
-        // the variables (every other spontaneous edge has a clock-free
-        // conjunct that may be false), or never
-        int kind = 1;
-        for (int k = 0; k < L.edge_count && kind != 0; ++k) {
-            const smc_edge &E = n.edges[L.edge_first + k];
-            if (E.channel < 0) continue;
-            bool never = false, clock_free = false;
-            for (int g = 0; g < E.guard_count; ++g) {
-                const smc_constraint &G = n.constraints[E.guard_first + g];
-                if (!G.uses_variable) continue;
-                if (G.op == SMC_C_NE) never = true;
-                else if (n.var_kind[G.var] != SMC_VAR_CLOCK && !reads_clock(G.rhs)) clock_free = true;
+            if (R.invs.size() > 65535) throw std::runtime_error("limit: more than 65535 invariants on a location");
+            d.n_inv = (uint16_t)R.invs.size();
+            d.klass = L.type > SMC_LOC_GOAL ? SMC_K_ZERO : (d.n_inv > 0 ? SMC_K_BOUNDED : SMC_K_EXP);
+            if (L.edge_count > SMC_MAX_EDGES_PER_LOC)
+                throw std::runtime_error("limit: a location has more than 64 outgoing edges");
+            d.edge_n = (uint16_t)L.edge_count;
+            img.loc_edge0[l] = L.edge_first;
+            if (SMC_REF_KIND(d.rate) == SMC_REF_CONST) {
+                d.rate_const = 1;
+                d.rate_value = img.consts[d.rate & 0x3FFFFFFFu];
             }
-            if (never) continue;
-            kind = clock_free ? 2 : 0;
-        }
-        img.locs[l].flags |= (uint8_t)((tf ? SMC_LF_TIME_FREE : 0) | (kind == 1 ? SMC_LF_DEAD : 0) |
-                                       (kind == 2 ? SMC_LF_GUARDED : 0));
-        if (kind == 2 && img.locs[l].klass != SMC_K_ZERO) img.guarded = true;
-        if (kind == 2) {
-            // the blocking test: clock-free conjuncts, edge after edge
-            img.locs[l].block_first = (uint32_t)img.guards.size();
+            info.klass = d.klass;
+            info.type = d.type;
+            info.n_inv = d.n_inv;
+            const uint32_t rate_plain = lw_plain.ref(L.rate, 1.0);
+            if (d.rate_const) memcpy(&info.rate_key, &d.rate_value, 8);
+            else info.rate_key = (int64_t)rate_plain ^ ((int64_t)1 << 62);
+
             for (int k = 0; k < L.edge_count; ++k) {
                 const smc_edge &E = n.edges[L.edge_first + k];
-                if (E.channel < 0) continue;
-                const DevEdge &DE = img.edges[L.edge_first + k];
-                if (DE.never) continue;
-                const size_t first = img.guards.size();
-                for (int g = 0; g < DE.guard_n; ++g) {
-                    const DevGuard G = img.guards[DE.guard_first + g];
-                    if (G.flags & SMC_GF_CLOCK_FREE) img.guards.push_back(G);
+                RawEdge re;
+                DevEdge &e = re.e;
+                e.dst = E.dst - l;
+                re.dst_loc = E.dst;
+                e.channel = E.channel;
+                info.edges.push_back({e.dst, e.channel});
+                e.weight = lw.ref(E.weight, 1.0);
+                if (SMC_REF_KIND(e.weight) == SMC_REF_CONST) {
+                    const int w = smc_to_int(img.consts[e.weight & 0x3FFFFFFFu]);
+                    e.weight = w > 0 ? (uint32_t)w : 0u;
+                    e.flags |= SMC_EF_WEIGHT_CONST;
                 }
-                if (img.guards.size() == first) throw std::runtime_error("internal: guarded edge without a clock-free conjunct");
-                img.guards.back().flags |= SMC_GF_END_EDGE;
+                e.dst_goal = n.locations[E.dst].type == SMC_LOC_GOAL;
+                for (int g = 0; g < E.guard_count; ++g) {
+                    const smc_constraint &C = n.constraints[E.guard_first + g];
+                    if (!C.uses_variable) continue;
+                    if (C.op == SMC_C_NE) { e.never = 1; continue; }
+                    if (C.var > 65535) throw std::runtime_error("limit: guarded variable index above 65535");
+                    DevGuard G{};
+                    G.var = lw.field(C.var);
+                    G.op = (uint8_t)C.op;
+                    G.flags = (uint8_t)((n.var_kind[C.var] != SMC_VAR_CLOCK && !reads_clock(C.rhs) ? SMC_GF_CLOCK_FREE : 0) |
+                                        (n.var_kind[C.var] == SMC_VAR_CLOCK ? SMC_GF_CLOCK : 0));
+                    G.rhs = lw.ref(C.rhs, 0.0);
+                    if (SMC_REF_KIND(G.rhs) == SMC_REF_CONST) {
+                        G.flags |= SMC_GF_RANGE;
+                        range_of(C.op, img.consts[G.rhs & 0x3FFFFFFFu], &G.lo, &G.hi);
+                    }
+                    re.guards.push_back(G);
+                }
+                if (re.guards.size() > 65535) throw std::runtime_error("limit: more than 65535 guards on an edge");
+                e.guard_n = (uint16_t)re.guards.size();
+                for (int k2 = 0; k2 < E.upd_count; ++k2) {
+                    const smc_update &U = n.updates[E.upd_first + k2];
+                    if (U.var > 65535) throw std::runtime_error("limit: assigned variable index above 65535");
+                    DevUpd u{};
+                    u.var = lw.field(U.var);
+                    u.clock = n.var_kind[U.var] == SMC_VAR_CLOCK ? 1 : 0;
+                    u.expr = lw.ref(U.expr, 0.0);
+                    double cv = 0.0;
+                    u.kind = (uint8_t)form(U, &cv);
+                    if (u.kind != SMC_U_EXPR) u.value = cv;
+                    re.upds.push_back(u);
+                }
+                if (E.upd_count > 65535) throw std::runtime_error("limit: more than 65535 updates on an edge");
+                e.upd_n = (uint16_t)E.upd_count;
+                R.edges.push_back(std::move(re));
             }
-            img.guards.back().flags |= SMC_GF_END_LOC;
-            const DevGuard &G = img.guards.back();
-            if (img.locs[l].block_first + 1 == img.guards.size() && SMC_REF_KIND(G.rhs) == SMC_REF_CONST &&
-                !(img.locs[l].flags & SMC_LF_INL_INV)) {
-                img.locs[l].flags |= SMC_LF_INL_BLK;
-                img.locs[l].inl_value = img.consts[G.rhs & 0x3FFFFFFFu];
-                img.locs[l].inl_var = G.var;
-                img.locs[l].inl_op = G.op;
+
+            // time_free: the location's rate and its spontaneous edges'
+            // guards read no clock, so between transitions neither its
+            // enabled edges nor its rate change
+            bool tf = !reads_clock(L.rate);
+            for (int k = 0; k < L.edge_count && tf; ++k) {
+                const smc_edge &E = n.edges[L.edge_first + k];
+                if (E.channel < 0) continue;
+                for (int g = 0; g < E.guard_count; ++g) {
+                    const smc_constraint &G = n.constraints[E.guard_first + g];
+                    if (!G.uses_variable) continue;
+                    if (n.var_kind[G.var] == SMC_VAR_CLOCK || reads_clock(G.rhs)) tf = false;
+                }
             }
+            // blocking: always (every spontaneous edge has `!=`, or none),
+            // by the variables (every other spontaneous edge has a
+            // clock-free conjunct that may be false), or never
+            int kind = 1;
+            for (int k = 0; k < L.edge_count && kind != 0; ++k) {
+                const smc_edge &E = n.edges[L.edge_first + k];
+                if (E.channel < 0) continue;
+                bool never = false, clock_free = false;
+                for (int g = 0; g < E.guard_count; ++g) {
+                    const smc_constraint &G = n.constraints[E.guard_first + g];
+                    if (!G.uses_variable) continue;
+                    if (G.op == SMC_C_NE) never = true;
+                    else if (n.var_kind[G.var] != SMC_VAR_CLOCK && !reads_clock(G.rhs)) clock_free = true;
+                }
+                if (never) continue;
+                kind = clock_free ? 2 : 0;
+            }
+            d.flags = (uint8_t)((tf ? SMC_LF_TIME_FREE : 0) | (kind == 1 ? SMC_LF_DEAD : 0) |
+                                (kind == 2 ? SMC_LF_GUARDED : 0));
+            if (kind == 2) {
+                // the blocking test: clock-free conjuncts, edge after edge
+                for (const RawEdge &re : R.edges) {
+                    if (re.e.channel < 0 || re.e.never) continue;
+                    const size_t first = R.block.size();
+                    for (const DevGuard &G : re.guards)
+                        if (G.flags & SMC_GF_CLOCK_FREE) R.block.push_back(G);
+                    if (R.block.size() == first)
+                        throw std::runtime_error("internal: guarded edge without a clock-free conjunct");
+                    R.block.back().flags |= SMC_GF_END_EDGE;
+                }
+                R.block.back().flags |= SMC_GF_END_LOC;
+            }
+
+            // receive edges
+            bool fast = true, plain_recv = true;
+            int chan = 0, n_recv = 0;
+            int64_t weight = 0;
+            for (int k = 0; k < L.edge_count; ++k) {
+                const smc_edge &E = n.edges[L.edge_first + k];
+                if (E.channel >= 0) continue;
+                const RawEdge &re = R.edges[k];
+                std::vector<int> seen;
+                if (!(re.e.flags & SMC_EF_WEIGHT_CONST)) fast = false;
+                else weight += re.e.weight;
+                for (int k2 = 0; k2 < E.upd_count; ++k2) {
+                    const smc_update &U = n.updates[E.upd_first + k2];
+                    const DevUpd &u = re.upds[k2];
+                    if (u.kind == SMC_U_EXPR || (u.kind == SMC_U_ADD && !whole(u.value)) || !var_commutes(U.var) ||
+                        std::find(seen.begin(), seen.end(), U.var) != seen.end())
+                        fast = false;
+                    seen.push_back(U.var);
+                }
+                if (k >= 32) fast = false;
+                if (re.e.never || re.e.guard_n || (chan && chan != -E.channel)) plain_recv = false;
+                chan = -E.channel;
+                if (k < 32) d.recv_mask |= 1u << k;
+                if (n_recv++ == 0) d.recv_low = re.e.weight;
+            }
+            if (weight >= 2147483648ll) fast = false;
+            if (fast) d.flags |= SMC_LF_RECV_FAST;
+            if (n_recv == 0) d.recv_chan = 0;
+            else if (fast && plain_recv) {
+                d.recv_chan = chan;
+                d.recv_weight = (uint32_t)weight;
+                if (n_recv == 2) d.flags |= SMC_LF_RECV_TWO;
+            } else {
+                d.recv_chan = -1;
+                d.recv_mask = 0;
+            }
+            if (!(d.flags & SMC_LF_RECV_TWO)) d.recv_low = 0;
+
+            // what a race step looks at
+            DevHot &h = R.hot;
+            if (d.klass == SMC_K_ZERO) {
+                h.flags = SMC_HF_ZERO;
+            } else {
+                if (img.freeze && kind == 1) {
+                    h.rate = 0.0;  // out of the race unless bounded
+                } else if (d.rate_const) {
+                    h.rate = d.rate_value > 0.0 ? d.rate_value : 0.0;
+                } else {
+                    h.flags |= SMC_HF_EXPR | (reads_local(L.rate) ? SMC_HF_EXPR_LOCAL : 0);
+                    h.rate_ref = d.rate;
+                }
+                if (d.n_inv == 1 && R.invs[0].bound_const) {
+                    h.flags |= SMC_HF_INV;
+                    h.var = R.invs[0].var;
+                    h.a = R.invs[0].bound_value;
+                    h.b = R.invs[0].strict ? 1e-6 : 0.0;
+                } else if (d.n_inv) {
+                    h.flags |= SMC_HF_XINV;
+                }
+                if (img.freeze && kind == 2) {
+                    if (R.block.size() == 1 && (R.block[0].flags & SMC_GF_RANGE) && !(h.flags & SMC_HF_INV)) {
+                        h.flags |= SMC_HF_GUARD;
+                        h.var = R.block[0].var;
+                        h.a = R.block[0].lo;
+                        h.b = R.block[0].hi;
+                    } else {
+                        h.flags |= SMC_HF_XBLK;
+                    }
+                }
+            }
+            img.tests |= h.flags;
         }
     }
-    img.freeze = !clock_rate;
+
+    // classes of equal locations, and their records; record 0 is a slot
+    // without a component (no edge, rate 0)
+    uint32_t n_cls = 0;
+    const std::vector<uint32_t> cls = classes_of(raw, &n_cls);
+    // a state word holds the class and the base; with more classes than fit
+    // beside a base, the class alone
+    if (use_locals && n_cls >= (1u << 18)) return lower(n, false);
+    img.rec_shift = use_locals ? 13 : 0;
+    img.hots.assign(n_cls + 1, DevHot{});
+    img.locs.assign(n_cls + 1, DevLoc{});
+    std::vector<uint8_t> done(n_cls, 0);
+    std::unordered_map<std::string, uint32_t> gmap, umap, emap, imap;
     for (int l = 0; l < n.n_locations; ++l) {
-        const smc_location &L = n.locations[l];
-        bool fast = true;
-        for (int k = 0; k < L.edge_count; ++k)
-            if (n.edges[L.edge_first + k].channel < 0 && !fast_edge[L.edge_first + k]) fast = false;
-        if (fast) img.locs[l].flags |= SMC_LF_RECV_FAST;
+        img.loc_rec.push_back(cls[l] + 1);
+        if (done[cls[l]]) continue;
+        done[cls[l]] = 1;
+        RawLoc &R = raw[l];
+        std::vector<DevEdge> run;
+        for (RawEdge &re : R.edges) {
+            re.e.guard_first = intern(img.guards, gmap, re.guards.data(), re.guards.size());
+            re.e.upd_first = intern(img.upds, umap, re.upds.data(), re.upds.size());
+            re.e.dst_rec = cls[re.dst_loc] + 1;
+            run.push_back(re.e);
+        }
+        R.loc.edge_first = intern(img.edges, emap, run.data(), run.size());
+        R.loc.inv_first = intern(img.invs, imap, R.invs.data(), R.invs.size());
+        R.loc.block_first = intern(img.guards, gmap, R.block.data(), R.block.size());
+        img.hots[cls[l] + 1] = R.hot;
+        img.locs[cls[l] + 1] = R.loc;
     }
-    share_records(img);
+    for (int c = 0; c < n.n_components; ++c)
+        img.comp_word.push_back((img.loc_rec[n.comp_init_loc[c]] << img.rec_shift) | (uint32_t)base[c]);
     // keep every table non-empty so device pointers are valid
     if (img.invs.empty()) img.invs.push_back(DevInv{});
     if (img.edges.empty()) img.edges.push_back(DevEdge{});
@@ -442,28 +672,17 @@ ModelImage compile_model(const smc_network &n) {
     if (img.code.empty()) img.code.push_back(DevInsn{});
     if (img.var_init.empty()) img.var_init.push_back(0.0);
     if (img.var_clock.empty()) img.var_clock.push_back(0);
-    if (img.loc_edge0.empty()) img.loc_edge0.push_back(0);
     return img;
 }
 
-double eval_ref_host(const ModelImage &m, uint32_t ref, const double *vars) {
-    // vars: values (clocks by value, not as stamps)
-    uint32_t kind = SMC_REF_KIND(ref);
-    if (kind == SMC_REF_CONST) return m.consts[ref & 0x3FFFFFFFu];
-    if (kind == SMC_REF_VAR || kind == SMC_REF_CLOCK) return vars[ref & 0x3FFFFFFFu];
-    uint32_t first = ref & 0xFFFFFFu, count = (ref >> 24) & 0x3Fu;
-    double reg[SMC_NREGS] = {0, 0, 0, 0};
-    auto fetch = [&](uint16_t o) -> double {
-        uint32_t k = o >> 14, i = o & 0x3FFFu;
-        return k == SMC_OPND_REG ? reg[i & 3] : (k == SMC_OPND_VAR || k == SMC_OPND_CLOCK) ? vars[i] : m.consts[i];
-    };
-    for (uint32_t k = 0; k < count; ++k) {
-        const DevInsn &in = m.code[first + k];
-        int ar = smc_op_arity(in.op);
-        double a = ar > 0 ? fetch(in.a) : 0.0, b = ar > 1 ? fetch(in.b) : 0.0, c = ar > 2 ? fetch(in.c) : 0.0;
-        reg[in.dst & 3] = smc_apply_op(in.op, a, b, c);
-    }
-    return reg[0];
+}  // namespace
+
+ModelImage compile_model(const smc_network &n) {
+    std::string err = validate(n);
+    if (!err.empty()) throw std::runtime_error(err);
+    // networks of SMC_MAX_LOCAL_VARS variables or more exceed the run
+    // kernel's LDS budget at every launch shape; they keep plain indices
+    return lower(n, n.n_vars < SMC_MAX_LOCAL_VARS);
 }
 
 }  // namespace smc

@@ -8,8 +8,18 @@
 
 namespace smc {
 
+// A location of the network as written (tilt groups of importance sampling).
+struct LocInfo {
+    uint8_t klass = 0, type = 0;
+    int n_inv = 0;
+    int64_t rate_key = 0;  // the constant's bits, or the identity of the expression
+    struct Edge { int32_t dst, channel; };  // dst relative to the location
+    std::vector<Edge> edges;
+};
+
 struct ModelImage {
-    std::vector<DevLoc> locs;
+    std::vector<DevHot> hots;           // per record class
+    std::vector<DevLoc> locs;           // per record class
     std::vector<DevInv> invs;
     std::vector<DevEdge> edges;
     std::vector<DevGuard> guards;
@@ -17,20 +27,21 @@ struct ModelImage {
     std::vector<double> consts;
     std::vector<DevInsn> code;
     std::vector<double> var_init;
+    std::vector<uint32_t> comp_word;    // initial state word of each component
     std::vector<int32_t> comp_init_loc;
     std::vector<int32_t> comp_first_loc;
     std::vector<uint8_t> var_clock;     // per variable: 1 for a clock
     std::vector<int32_t> var_kind;
     std::vector<int32_t> loc_edge0;     // per location: the network's index of its first edge
+    std::vector<uint32_t> loc_rec;      // per location: its record class
+    std::vector<LocInfo> info;          // per location
     int n_comp = 0, n_vars = 0, n_leaves = 1;
+    int rec_shift = 13;
+    uint32_t tests = 0;   // every SMC_HF_* flag in use
     bool freeze = true;   // no location's rate reads a clock
-    bool guarded = false; // some location is blocked or not by the variables
 };
 
 // Throws std::runtime_error (message prefixed "limit:" for size limits).
 ModelImage compile_model(const smc_network &net);
-
-// Host evaluation of a compiled expression reference (tests, debugging).
-double eval_ref_host(const ModelImage &m, uint32_t ref, const double *vars);
 
 }  // namespace smc

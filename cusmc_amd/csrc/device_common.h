@@ -103,7 +103,8 @@ __device__ __forceinline__ T load_rec(const SMC_GLOBAL T *p) {
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
-// The same from LDS (records 16-byte aligned there too).
+// The same from LDS (16-byte aligned there too); reads of fields there are
+// cheap, so nothing is kept from being narrowed or scheduled.
 template <class T>
 __device__ __forceinline__ T load_rec(const SMC_LDS T *p) {
     static_assert(sizeof(T) % 8 == 0, "record size");
@@ -112,45 +113,29 @@ __device__ __forceinline__ T load_rec(const SMC_LDS T *p) {
         const SMC_LDS uint4 *q = (const SMC_LDS uint4 *)p;
         uint4 v[sizeof(T) / 16];
 #pragma unroll
-        for (int i = 0; i < (int)(sizeof(T) / 16); ++i) {
-            v[i] = q[i];
-            asm("" : "+v"(v[i].x), "+v"(v[i].y), "+v"(v[i].z), "+v"(v[i].w));
-        }
+        for (int i = 0; i < (int)(sizeof(T) / 16); ++i) v[i] = q[i];
         __builtin_memcpy(&r, v, sizeof(T));
     } else {
         const SMC_LDS uint2 *q = (const SMC_LDS uint2 *)p;
         uint2 v[sizeof(T) / 8];
 #pragma unroll
-        for (int i = 0; i < (int)(sizeof(T) / 8); ++i) {
-            v[i] = q[i];
-            asm("" : "+v"(v[i].x), "+v"(v[i].y));
-        }
+        for (int i = 0; i < (int)(sizeof(T) / 8); ++i) v[i] = q[i];
         __builtin_memcpy(&r, v, sizeof(T));
     }
     return r;
 }
 #endif
 
-// A location record.  From the LDS-staged tables: all 48 bytes.  From global
-// memory: the first 32 (one pair of 16-byte loads, as many cache lines as
-// before the inline part existed), with the inline flags cleared, so the
-// general invariant and guard records are used.
-__device__ __forceinline__ DevLoc load_loc(const SMC_GLOBAL DevLoc *p) {
-    const SMC_GLOBAL uint4 *q = (const SMC_GLOBAL uint4 *)p;
-    uint4 v[3];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        v[i] = q[i];
-        asm("" : "+v"(v[i].x), "+v"(v[i].y), "+v"(v[i].z), "+v"(v[i].w));
-    }
-    v[2] = uint4{0u, 0u, 0u, 0u};
-    DevLoc r;
-    __builtin_memcpy(&r, v, sizeof(DevLoc));
-    r.flags &= (uint8_t)~(SMC_LF_INL_INV | SMC_LF_INL_BLK);
-    return r;
+// The first 16 bytes of a record.
+template <class T>
+__device__ __forceinline__ uint4 load_quad(const SMC_GLOBAL T *p) {
+    return load_rec((const SMC_GLOBAL uint4 *)p);
 }
 #if defined(__HIP_DEVICE_COMPILE__)
-__device__ __forceinline__ DevLoc load_loc(const SMC_LDS DevLoc *p) { return load_rec(p); }
+template <class T>
+__device__ __forceinline__ uint4 load_quad(const SMC_LDS T *p) {
+    return load_rec((const SMC_LDS uint4 *)p);
+}
 #endif
 
 // Table pointer of the global arena rebased onto its LDS copy.
@@ -186,41 +171,12 @@ __device__ __forceinline__ void stage_tables(const SMC_GLOBAL uint8_t *src, uint
     __syncthreads();
 }
 
-// The model with every hot table but the location records read from the
-// staged copy, which then starts at the invariants (base: their global
-// address).
-__device__ __forceinline__ DevModelT<SmcMixedTables> lds_model_mixed(const DevModel &mg,
-                                                                     const SMC_GLOBAL uint8_t *base, double *lds) {
-    const SMC_LDS uint8_t *tab = (const SMC_LDS uint8_t *)(SMC_LDS double *)lds;
-    DevModelT<SmcMixedTables> m;
-    m.locs = mg.locs;
-    m.invs = in_lds(mg.invs, base, tab);
-    m.edges = in_lds(mg.edges, base, tab);
-    m.guards = in_lds(mg.guards, base, tab);
-    m.upds = in_lds(mg.upds, base, tab);
-    m.consts = in_lds(mg.consts, base, tab);
-    m.code = in_lds(mg.code, base, tab);
-    m.var_init = mg.var_init;
-    m.comp_init_loc = mg.comp_init_loc;
-    m.var_clock = mg.var_clock;
-    m.comp_first_loc = mg.comp_first_loc;
-    m.loc_edge0 = mg.loc_edge0;
-    m.n_comp = mg.n_comp;
-    m.n_vars = mg.n_vars;
-    m.n_clocks = mg.n_clocks;
-    m.n_leaves = mg.n_leaves;
-    m.n_locs = mg.n_locs;
-    m.n_edges = mg.n_edges;
-    m.freeze = mg.freeze;
-    m.guarded = mg.guarded;
-    return m;
-}
-
 // The model with its hot tables read from the staged copy.
 __device__ __forceinline__ DevModelT<SmcLdsTables> lds_model(const DevModel &mg, const SMC_GLOBAL uint8_t *base,
                                                              double *lds) {
     const SMC_LDS uint8_t *tab = (const SMC_LDS uint8_t *)(SMC_LDS double *)lds;
     DevModelT<SmcLdsTables> m;
+    m.hots = in_lds(mg.hots, base, tab);
     m.locs = in_lds(mg.locs, base, tab);
     m.invs = in_lds(mg.invs, base, tab);
     m.edges = in_lds(mg.edges, base, tab);
@@ -229,41 +185,78 @@ __device__ __forceinline__ DevModelT<SmcLdsTables> lds_model(const DevModel &mg,
     m.consts = in_lds(mg.consts, base, tab);
     m.code = in_lds(mg.code, base, tab);
     m.var_init = mg.var_init;
+    m.comp_word = mg.comp_word;
     m.comp_init_loc = mg.comp_init_loc;
     m.var_clock = mg.var_clock;
     m.comp_first_loc = mg.comp_first_loc;
     m.loc_edge0 = mg.loc_edge0;
+    m.loc_rec = mg.loc_rec;
     m.n_comp = mg.n_comp;
     m.n_vars = mg.n_vars;
-    m.n_clocks = mg.n_clocks;
     m.n_leaves = mg.n_leaves;
     m.n_locs = mg.n_locs;
-    m.n_edges = mg.n_edges;
+    m.rec_shift = mg.rec_shift;
+    m.base_mask = mg.base_mask;
+    m.tests = mg.tests;
     m.freeze = mg.freeze;
-    m.guarded = mg.guarded;
     return m;
 }
 
 // ------------------------------------------------------------ expressions
 
-// Register-bytecode interpreter (expressions.cu:10-119).  Inlined: an
-// out-of-line call costs the whole kernel registers and time even on models
-// that never reach it.
+// What evaluating an expression of one component needs: the run's variables
+// and clock time, and where the component's private variables start.
+struct Ctx {
+    double *vars;
+    double now;
+    uint32_t base;
+};
+
+// Index of a record's variable operand.
+__device__ __forceinline__ uint32_t var_at(uint32_t v, uint32_t base) {
+    return (v & 0x7FFFu) + (base & (uint32_t)((int32_t)(v << 16) >> 31));
+}
+__device__ __forceinline__ uint32_t ref_var(uint32_t ref, uint32_t base) {
+    return (ref & 0x1FFFFFFFu) + ((ref & SMC_REF_LOCAL) ? base : 0u);
+}
+
+// The operators that few models use, out of line: inlined at every
+// expression site they would make up most of the kernels' code.
+__attribute__((noinline)) __device__ double rare_op(int op, double a, double b, double c) {
+    return smc_apply_op(op, a, b, c);
+}
+
+__device__ __forceinline__ double apply_op(int op, double a, double b, double c) {
+    switch (op) {
+    case SMC_E_ADD: return a + b;
+    case SMC_E_SUB: return a - b;
+    case SMC_E_MUL: return a * b;
+    case SMC_E_DIV: return a / b;
+    default: return rare_op(op, a, b, c);
+    }
+}
+
+// Register-bytecode interpreter (expressions.cu:10-119).
 template <class PC, class PI>
-__device__ __forceinline__ double eval_code(uint32_t ref, const double *vars, PC consts, PI code) {
+__device__ __forceinline__ double eval_code(uint32_t ref, const Ctx &x, PC consts, PI code) {
     const uint32_t first = ref & 0xFFFFFFu, count = (ref >> 24) & 0x3Fu;
     double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
+#pragma clang loop unroll(disable)
     for (uint32_t k = 0; k < count; ++k) {
         const DevInsn in = load_rec(code + first + k);
         double o[3];
 #pragma unroll
         for (int s = 0; s < 3; ++s) {
-            const uint16_t x = s == 0 ? in.a : s == 1 ? in.b : in.c;
-            const uint32_t kind = x >> 14, i = x & 0x3FFFu;
-            o[s] = kind == SMC_OPND_REG ? (i == 0 ? r0 : i == 1 ? r1 : i == 2 ? r2 : r3)
-                 : kind == SMC_OPND_VAR ? vars[i] : kind == SMC_OPND_CLOCK ? vars[-1] - vars[i] : consts[i];
+            const uint16_t w = s == 0 ? in.a : s == 1 ? in.b : in.c;
+            const uint32_t kind = w >> 14, i = w & 0x3FFFu;
+            if (kind == SMC_OPND_REG) o[s] = i == 0 ? r0 : i == 1 ? r1 : i == 2 ? r2 : r3;
+            else if (kind == SMC_OPND_CONST) o[s] = consts[i];
+            else {
+                const double v = x.vars[(i & (SMC_OPND_LOCAL - 1u)) + ((i & SMC_OPND_LOCAL) ? x.base : 0u)];
+                o[s] = kind == SMC_OPND_CLOCK ? x.now - v : v;
+            }
         }
-        const double v = smc_apply_op(in.op, o[0], o[1], o[2]);
+        const double v = apply_op(in.op, o[0], o[1], o[2]);
         r0 = in.dst == 0 ? v : r0;
         r1 = in.dst == 1 ? v : r1;
         r2 = in.dst == 2 ? v : r2;
@@ -274,64 +267,30 @@ __device__ __forceinline__ double eval_code(uint32_t ref, const double *vars, PC
 
 // Value of an expression reference: constants and variables inline.
 template <class M>
-__device__ __forceinline__ double eval_ref(uint32_t ref, const double *vars, const M &m) {
+__device__ __forceinline__ double eval_ref(uint32_t ref, const Ctx &x, const M &m) {
     const uint32_t kind = ref >> 30;
+    if (kind == SMC_REF_CODE) return eval_code(ref, x, m.consts, m.code);
     if (kind == SMC_REF_CONST) return m.consts[ref & 0x3FFFFFFFu];
-    if (kind == SMC_REF_VAR) return vars[ref & 0x3FFFFFFFu];
-    if (kind == SMC_REF_CLOCK) return vars[-1] - vars[ref & 0x3FFFFFFFu];
-    return eval_code(ref, vars, m.consts, m.code);
+    const double v = x.vars[ref_var(ref, x.base)];
+    return kind == SMC_REF_CLOCK ? x.now - v : v;
 }
-
-// A location's rate within one race, remembering the last expression this
-// lane evaluated: identical expressions share one reference (the compiler
-// deduplicates bytecode), and variables do not change during a race, so a
-// repeated reference has the same value.  Components of one template in the
-// same location (every susceptible agent of an epidemic, say) then cost one
-// evaluation per lane instead of one per slot.
-struct RateMemo {
-    uint32_t ref = 0xFFFFFFFFu;
-    double value = 0.0;
-};
 
 template <class M>
-__device__ __forceinline__ double location_rate(const DevLoc &L, const double *vars, const M &m, RateMemo &memo) {
-    if (L.rate_const) return L.rate_value;
-    if (L.rate != memo.ref) {
-        memo.value = eval_ref(L.rate, vars, m);
-        memo.ref = L.rate;
-    }
-    return memo.value;
+__device__ __forceinline__ double location_rate(const DevLoc &L, const Ctx &x, const M &m) {
+    const double r = L.rate_const ? L.rate_value : eval_ref(L.rate, x, m);
+    return r > 0.0 ? r : 0.0;
 }
 
-// Rates of the slots in `pend` whose rate is a bytecode expression (refs
-// in ref[]): each pass evaluates, on every lane at once, the expression of
-// the lane's first pending slot and hands the value to all of its pending
-// slots with the same expression.  Evaluating inside the per-slot loop would
-// run the interpreter once per slot index at which any lane of the wave
-// meets a new expression (up to C times per race); here it runs once per
-// distinct expression a lane holds.
-template <int C, class M>
-__device__ __forceinline__ void pending_rates(uint32_t pend, const uint32_t (&ref)[C], double (&leaf)[C],
-                                              const double *vars, const M &m) {
-    while (__ballot(pend != 0)) {
-        uint32_t r = 0xFFFFFFFFu;
-        double v = 0.0;
-        if (pend) {
-            const int j0 = __ffs(pend) - 1;
-            r = ref[0];
-#pragma unroll
-            for (int k = 1; k < C; ++k) r = (j0 == k) ? ref[k] : r;
-            v = eval_ref(r, vars, m);
-            v = v > 0.0 ? v : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < C; ++j)
-            if (((pend >> j) & 1u) && ref[j] == r) {
-                leaf[j] = v;
-                pend &= ~(1u << j);
-            }
-    }
-}
+// ------------------------------------------------------------ slots
+//
+// A lane's component slots are state words in LDS ([slot][lane]: 64 lanes
+// touch 64 consecutive words), so that loops over slots stay rolled where
+// they are cold and any lane can read any slot.  `scr` is 8 bytes per slot
+// and lane of scratch in the same layout.
+template <class M>
+__device__ __forceinline__ uint32_t word_rec(uint32_t w, const M &m) { return w >> m.rec_shift; }
+template <class M>
+__device__ __forceinline__ uint32_t word_base(uint32_t w, const M &m) { return w & m.base_mask; }
 
 // ------------------------------------------------------------ edges
 
@@ -346,97 +305,96 @@ __device__ __forceinline__ bool guard_holds(int op, double x, double r) {
     }
 }
 
-// Enabled edges of location `loc` as a bit mask over its edge list:
-// spontaneous edges (recv_chan == 0) or receive edges on channel recv_chan
-// (check_enabled_edges simulation.cu:268-305, SyncInSerial :363-377).
 template <class M>
-__device__ __forceinline__ uint64_t enabled_mask(int loc, int recv_chan, const double *vars, const M &m) {
-    const DevLoc L = load_loc(m.locs + loc);
-    const int ne = L.edge_n;
+__device__ __forceinline__ bool guard_true(const DevGuard &G, const Ctx &x, const M &m) {
+    double v = x.vars[var_at(G.var, x.base)];
+    if (G.flags & SMC_GF_CLOCK) v = x.now - v;
+    if (G.flags & SMC_GF_RANGE) return G.lo <= v && v <= G.hi;
+    return guard_holds(G.op, v, eval_ref(G.rhs, x, m));
+}
+
+// Whether edge record e is enabled: spontaneous (recv_chan == 0) or a
+// receive edge on channel recv_chan (check_enabled_edges
+// simulation.cu:268-305, SyncInSerial :363-377).
+template <class M>
+__device__ __forceinline__ bool edge_enabled(uint32_t e, int recv_chan, const Ctx &x, const M &m) {
+    const DevEdge E = load_rec(m.edges + e);
+    if (E.never || (recv_chan ? E.channel != -recv_chan : E.channel < 0)) return false;
+    bool ok = true;
+#pragma clang loop unroll(disable)
+    for (int g = 0; g < E.guard_n && ok; ++g) ok = guard_true(load_rec(m.guards + E.guard_first + g), x, m);
+    return ok;
+}
+
+// Enabled edges of a location as a bit mask over its edge list, by one lane.
+template <class M>
+__device__ __forceinline__ uint64_t enabled_mask(uint32_t edge_first, int edge_n, int recv_chan, const Ctx &x,
+                                                 const M &m) {
     uint64_t mask = 0;
-    for (int i = 0; i < ne; ++i) {
-        const DevEdge E = load_rec(m.edges + L.edge_first + i);
-        if (E.never) continue;
-        if (recv_chan ? (E.channel != -recv_chan) : (E.channel < 0)) continue;
-        bool ok = true;
-        for (int g = 0; g < E.guard_n && ok; ++g) {
-            const DevGuard G = load_rec(m.guards + E.guard_first + g);
-            const double x = (G.flags & SMC_GF_CLOCK) ? vars[-1] - vars[G.var] : vars[G.var];
-            ok = guard_holds(G.op, x, eval_ref(G.rhs, vars, m));
-        }
-        if (ok) mask |= 1ull << i;
-    }
+#pragma clang loop unroll(disable)
+    for (int i = 0; i < edge_n; ++i)
+        if (edge_enabled(edge_first + i, recv_chan, x, m)) mask |= 1ull << i;
     return mask;
 }
 
 template <class M>
-__device__ __forceinline__ long long edge_weight(int e, const double *vars, const M &m) {
-    const int w = smc_to_int(eval_ref(m.edges[e].weight, vars, m));
-    return w > 0 ? w : 0;
+__device__ __forceinline__ long long edge_weight(uint32_t e, const Ctx &x, const M &m) {
+    const uint32_t w = m.edges[e].weight;
+    if (m.edges[e].flags & SMC_EF_WEIGHT_CONST) return (long long)w;
+    const int v = smc_to_int(eval_ref(w, x, m));
+    return v > 0 ? v : 0;
 }
 
 // Weighted choice among the edges in mask (two or more) for the uniform u
 // (take_transition simulation.cu:43-79 and get_sum_edge_weight :9-24, with
-// the weights of the enabled edges).
+// the weights of the enabled edges): the sum of the weights first, then from
+// the highest edge down.
 template <class M>
-__device__ __forceinline__ int pick_weighted(uint64_t mask, int edge_first, double u, const double *vars,
-                                             const M &m) {
-    long long W = 0;
-    for (uint64_t r = mask; r; r &= r - 1) W += edge_weight(edge_first + lowest_lane(r), vars, m);
-    const long long rnd = (long long)((double)W * u);
-    long long temp = W;
-    for (uint64_t r = mask; r;) {
+__device__ __forceinline__ int pick_weighted(uint64_t mask, uint32_t edge_first, double u, const Ctx &x, const M &m) {
+    long long W = 0, rnd = 0;
+    int pick = lowest_lane(mask);
+    uint64_t r = mask;
+    bool summed = false;
+    // one loop for the sum and the scan, so the weights' expressions are
+    // expanded once
+#pragma clang loop unroll(disable)
+    for (;;) {
+        if (!r) {
+            if (summed) break;
+            summed = true;
+            rnd = (long long)((double)W * u);
+            r = mask;
+        }
         const int i = 63 - __clzll((long long)r);
         r &= ~(1ull << i);
-        const long long w2 = edge_weight(edge_first + i, vars, m);
-        if (temp - w2 <= rnd) return i;
-        temp -= w2;
+        const long long w = edge_weight(edge_first + i, x, m);
+        if (!summed) W += w;
+        else {
+            W -= w;
+            if (W <= rnd) { pick = i; break; }
+        }
     }
-    return lowest_lane(mask);
+    return pick;
 }
 
 // Weighted choice among the enabled edges in mask; the draw is made only
 // when there is a choice.
 template <class M>
-__device__ __forceinline__ int pick_edge(uint64_t mask, int edge_first, uint64_t seed, uint64_t run,
-                                         uint32_t step, uint32_t purpose, uint32_t comp,
-                                         const double *vars, const M &m) {
+__device__ __forceinline__ int pick_edge(uint64_t mask, uint32_t edge_first, uint64_t seed, uint64_t run,
+                                         uint32_t step, uint32_t comp, const Ctx &x, const M &m) {
     if ((mask & (mask - 1)) == 0) return lowest_lane(mask);
-    const smc_u32x4 w = smc_draw(seed, run, step, purpose, comp);
-    return pick_weighted(mask, edge_first, smc_u01(w.v[0], w.v[1]), vars, m);
+    const smc_u32x4 w = smc_draw(seed, run, step, SMC_P_WINNER, comp);
+    return pick_weighted(mask, edge_first, smc_u01(w.v[0], w.v[1]), x, m);
 }
 
 // The same for component c as a broadcast receiver: its uniform is word
 // c & 3 of the receivers' shared draw c >> 2.
 template <class M>
-__device__ __forceinline__ int pick_receiver(uint64_t mask, int edge_first, uint64_t seed, uint64_t run,
-                                             uint32_t step, uint32_t c, const double *vars, const M &m) {
+__device__ __forceinline__ int pick_receiver(uint64_t mask, uint32_t edge_first, uint64_t seed, uint64_t run,
+                                             uint32_t step, uint32_t c, const Ctx &x, const M &m) {
     if ((mask & (mask - 1)) == 0) return lowest_lane(mask);
     const smc_u32x4 w = smc_draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
-    return pick_weighted(mask, edge_first, smc_receiver_u(w, c), vars, m);
-}
-
-// Rate sum, on the race tree, of the components that cannot fire before
-// the next transition (frozen: blocked, exponential now) in the slots of
-// deadmask.  They leave the race when every racer is exponential; the
-// transition that crosses the time bound still competes with their first
-// null event after the bound, which is drawn from this sum (memoryless
-// races).
-template <int C, class M>
-__device__ __forceinline__ double dead_total(uint32_t deadmask, const int (&loc)[C], const double *vars,
-                                             const M &m, int S) {
-    double dl[C];
-    RateMemo memo;
-#pragma unroll
-    for (int j = 0; j < C; ++j) {
-        dl[j] = 0.0;
-        if ((deadmask >> j) & 1u) {
-            const DevLoc L = load_loc(m.locs + loc[j]);
-            const double r = location_rate(L, vars, m, memo);
-            dl[j] = r > 0.0 ? r : 0.0;
-        }
-    }
-    return tree_total<C>(dl, S);
+    return pick_weighted(mask, edge_first, smc_receiver_u(w, c), x, m);
 }
 
 struct LaneQuery {
@@ -444,43 +402,40 @@ struct LaneQuery {
     double qmax, qmin;
 };
 
-// Fire edge `e` of location `src`: updates in order, query variable
-// tracking, new location (take_transition simulation.cu:88-180).  Returns
-// the destination (edge records hold it relative to the source).
+// The updates of an edge in order, with query variable tracking
+// (take_transition simulation.cu:88-180).  Any number of lanes may run it
+// for the same component at once: they store the same values.
 template <class M>
-__device__ __forceinline__ int fire_edge(int e, int src, double *vars, const M &m, LaneQuery &q,
-                                         bool &goal, int &chan) {
-    const DevEdge E = load_rec(m.edges + e);
+__device__ __forceinline__ void run_updates(const DevEdge &E, const Ctx &x, const M &m, LaneQuery &q) {
+#pragma clang loop unroll(disable)
     for (int k = 0; k < E.upd_n; ++k) {
         const DevUpd U = load_rec(m.upds + E.upd_first + k);
-        const double v = eval_ref(U.expr, vars, m);
-        if ((int)U.var == q.qvar) {
+        const uint32_t at = var_at(U.var, x.base);
+        double v = U.value;
+        if (U.kind == SMC_U_ADD) v = x.vars[at] + v;
+        else if (U.kind == SMC_U_EXPR) v = eval_ref(U.expr, x, m);
+        if ((int)at == q.qvar) {
             if (v > q.qmax) q.qmax = v;
             if (v < q.qmin) q.qmin = v;
         }
-        vars[U.var] = U.clock ? vars[-1] - v : v;
+        x.vars[at] = U.clock ? x.now - v : v;
     }
-    if (E.dst_goal) goal = true;
-    if (E.channel > 0) chan = E.channel;
-    return src + E.dst;
 }
 
-// Slots (bit j) whose component is blocked by the variables: in a
-// location flagged SMC_LF_GUARDED (not zero-delay), every spontaneous edge
-// has a `!=` conjunct or a false conjunct that reads no clock.  A blocked
-// component cannot fire until a transition changes the variables; the
-// kernels recompute the mask after every change of state, on models with
-// such locations (DevModel.guarded).  Locations flagged SMC_LF_DEAD are
-// always blocked and are tested by their flag.
+// ------------------------------------------------------------ blocking
+
 // The blocking test of a location flagged SMC_LF_GUARDED: every edge has a
-// false clock-free conjunct (one pass over its blocking records).
+// false clock-free conjunct (one pass over its blocking records).  A blocked
+// component cannot fire until a transition changes the variables.
+// Locations flagged SMC_LF_DEAD are always blocked and are tested by their
+// flag.
 template <class M>
-__device__ __forceinline__ bool location_blocked(const DevLoc &L, const double *vars, const M &m) {
-    if (L.flags & SMC_LF_INL_BLK) return !guard_holds(L.inl_op, vars[L.inl_var], L.inl_value);
+__device__ __forceinline__ bool location_blocked(uint32_t block_first, const Ctx &x, const M &m) {
     bool e_blk = false;
-    for (uint32_t k = L.block_first;; ++k) {
+#pragma clang loop unroll(disable)
+    for (uint32_t k = block_first;; ++k) {
         const DevGuard G = load_rec(m.guards + k);
-        if (!e_blk) e_blk = !guard_holds(G.op, vars[G.var], eval_ref(G.rhs, vars, m));
+        if (!e_blk) e_blk = !guard_true(G, x, m);
         if (G.flags & SMC_GF_END_EDGE) {
             if (!e_blk) return false;
             e_blk = false;
@@ -489,239 +444,434 @@ __device__ __forceinline__ bool location_blocked(const DevLoc &L, const double *
     }
 }
 
-template <int C, class M>
-__device__ __forceinline__ uint32_t blocked_slots(const int (&loc)[C], const double *vars, const M &m, int sl,
-                                                  int n) {
-    uint32_t b = 0;
-#pragma unroll
-    for (int j = 0; j < C; ++j) {
-        const int c = sl * C + j;
-        if (c >= n) continue;
-        const DevLoc L = load_loc(m.locs + loc[j]);
-        if ((L.flags & SMC_LF_GUARDED) && L.klass != SMC_K_ZERO && location_blocked(L, vars, m)) b |= 1u << j;
+// Delay window of a location's invariants at this time: the least remaining
+// time among the clock bounds still ahead; negative when there is none.
+template <class M>
+__device__ __forceinline__ double window_of(const DevLoc &L, const Ctx &x, const M &m) {
+    double M0 = DBL_MAX;
+    bool bounded = false;
+#pragma clang loop unroll(disable)
+    for (int i = 0; i < L.n_inv; ++i) {
+        const DevInv iv = load_rec(m.invs + L.inv_first + i);
+        const double bound = iv.bound_const ? iv.bound_value : eval_ref(iv.bound, x, m);
+        double ttb = bound - (x.now - x.vars[var_at(iv.var, x.base)]);
+        if (iv.strict) ttb -= 1e-6;
+        if (ttb >= 0.0) { M0 = ttb < M0 ? ttb : M0; bounded = true; }
     }
-    return b;
+    return bounded ? M0 : -1.0;
+}
+
+// The slots whose component cannot fire before the next transition (frozen:
+// blocked, exponential now), their rates in the lane's scratch.  They leave
+// the race; a step raced in full takes them back, and the transition that
+// crosses the time bound still competes with their first null event after
+// the bound, drawn from their sum (memoryless races).
+template <int C, class M>
+__device__ __forceinline__ uint32_t frozen_rates(const uint32_t *words, double *scr, Ctx x, const M &m) {
+    uint32_t frozen = 0;
+#pragma clang loop unroll(disable)
+    for (int j = 0; j < C; ++j) {
+        const uint32_t w = words[64 * j];
+        const DevLoc L = load_rec(m.locs + word_rec(w, m));
+        x.base = word_base(w, m);
+        if (L.klass != SMC_K_ZERO && !(window_of(L, x, m) >= 0.0) &&
+            ((L.flags & SMC_LF_DEAD) || ((L.flags & SMC_LF_GUARDED) && location_blocked(L.block_first, x, m)))) {
+            scr[64 * j] = location_rate(L, x, m);
+            frozen |= 1u << j;
+        }
+    }
+    return frozen;
 }
 
 // Whether no component of the segment's run can fire again before the time
-// bound: each one is blocked (bit of `blk`), or is in a location whose rate
-// and spontaneous guards read no clock and has no enabled spontaneous edge
-// or races at rate 0 (an exponential location).  Zero-delay and
-// clock-bounded locations with an enabled edge can fire.  Nothing but time
-// changes such a state, so the run's outcome is decided; the kernels check
-// it after every change of state.
+// bound: each one is blocked, or is in a location whose rate and spontaneous
+// guards read no clock and has no enabled spontaneous edge or races at rate 0
+// (an exponential location).  Zero-delay and clock-bounded locations with an
+// enabled edge can fire.  Nothing but time changes such a state, so the run's
+// outcome is decided.  For models without frozen racers: there the race
+// itself ends such a run.
 template <int C, class M>
-__device__ __forceinline__ bool absorbed(const int (&loc)[C], const double *vars, const M &m, int sl, int n,
-                                         uint64_t seg_mask, uint32_t blk) {
+__device__ __forceinline__ bool absorbed(const uint32_t *words, Ctx x, const M &m, uint64_t seg_mask) {
     bool can = false;
-    RateMemo memo;
-#pragma unroll
+#pragma clang loop unroll(disable)
     for (int j = 0; j < C; ++j) {
-        const int c = sl * C + j;
-        if (can || c >= n) continue;
-        const DevLoc L = load_loc(m.locs + loc[j]);
+        const uint32_t w = words[64 * j];
+        if (can || !(w >> m.rec_shift)) continue;
+        const DevLoc L = load_rec(m.locs + word_rec(w, m));
+        x.base = word_base(w, m);
         if (L.klass == SMC_K_ZERO) { can = true; continue; }
-        if ((L.flags & SMC_LF_DEAD) || ((blk >> j) & 1u)) continue;
+        if ((L.flags & SMC_LF_DEAD) || ((L.flags & SMC_LF_GUARDED) && location_blocked(L.block_first, x, m))) continue;
         if (!(L.flags & SMC_LF_TIME_FREE)) { can = true; continue; }
-        if (enabled_mask(loc[j], 0, vars, m) == 0) continue;
-        if (L.klass != SMC_K_EXP) { can = true; continue; }
-        const double r = location_rate(L, vars, m, memo);
-        if (r > 0.0) can = true;
+        if (enabled_mask(L.edge_first, L.edge_n, 0, x, m) == 0) continue;
+        if (L.klass != SMC_K_EXP || location_rate(L, x, m) > 0.0) can = true;
     }
     return (__ballot(can) & seg_mask) == 0;
 }
 
-template <int C, class T>
-__device__ __forceinline__ T slot_get(const T (&a)[C], int j);
-template <int C, class T>
-__device__ __forceinline__ void slot_set(T (&a)[C], int j, T v);
+// ------------------------------------------------------------ race
 
-// Receivers of one broadcast fired in parallel (SyncInSerial
-// simulation.cu:378-404 fires them one by one in component order).  Valid
-// when every receive edge of the segment's receivers commutes (SMC_LF_RECV_FAST):
-// constant weights make each receiver's pick independent of the others'
-// updates, and integer additions and private constants give the same
-// variables in any order.  The query variable's running max/min needs the
-// values in component order: they are v0 plus the prefix sums of the
-// additions, an exclusive scan over the segment (blocked layout: lane order
-// then slot order is component order).  TRACE mixes the fired edges into
-// the digest in component order.  Returns false, having changed nothing,
-// when some enabled edge does not commute.
+// What each slot does in the coming step.
+template <int C>
+struct RaceSlots {
+    double leaf[C];         // rate in the exponential race, 0 if not in it
+    uint32_t bounded;       // slots with a clock-bounded delay (window in the lane's scratch)
+    uint32_t zero;          // slots with delay 0
+};
+
+// Classify the lane's slots and evaluate their rates.  Nearly everything is
+// one straight line per slot over its class's 32-byte DevHot record (three
+// LDS reads, a handful of compares; no branch depends on a lane), because
+// the lanes of a wave hold components in every kind of location: as
+// branches, every slot would run every kind's code.  Invariants and blocking
+// tests beyond one record take a rolled loop beforehand, on models that have
+// them; xblk keeps those blocking results until the next change of state.
 template <int C, class M>
-__device__ __forceinline__ bool fire_receivers_fast(const uint64_t (&mk)[C], int (&loc)[C], double *vars,
-                                                    const M &m, LaneQuery &q, bool &goal, uint64_t seed,
-                                                    uint64_t run, uint32_t step, int sl, int S, int seg_base,
-                                                    uint64_t seg_mask, uint32_t &trans, bool trace,
-                                                    uint64_t &digest) {
-    bool slow = false;
-#pragma unroll
-    for (int j = 0; j < C; ++j)
-        if (mk[j] && !(m.locs[loc[j]].flags & SMC_LF_RECV_FAST)) slow = true;
-    if (__ballot(slow) & seg_mask) return false;
-
-    int ej[C], eg[C];  // fired edge per slot: record index, and the network's index (digests)
-    int fired = 0;
-    bool any_fired = false;
-    double qsum = 0.0, qhi = -DBL_MAX, qlo = DBL_MAX;  // prefix sums of this lane's query additions
-    bool qany = false;
-    // Receivers 4g .. 4g+3 share draw g: the lane's slots of one draw are
-    // G consecutive slots (C is a power of two), drawn once at the first of
-    // them when any of them has a choice to make.
-    constexpr int G = C < 4 ? C : 4;
-    smc_u32x4 rw = {{0u, 0u, 0u, 0u}};
+__device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *words, double *scr, Ctx x, const M &m,
+                                           bool changed, uint32_t &xblk) {
+    const uint32_t tests = m.tests;
+    uint32_t bounded = 0, zero = 0, out = 0, expr = 0, own = 0;
+    if (tests & (SMC_HF_XINV | SMC_HF_XBLK)) {
+        if (changed) xblk = 0;
+#pragma clang loop unroll(disable)
+        for (int j = 0; j < C; ++j) {
+            const uint32_t w = words[64 * j];
+            const uint32_t f = m.hots[word_rec(w, m)].flags;
+            if (f & (SMC_HF_XINV | SMC_HF_XBLK)) {
+                const DevLoc L = load_rec(m.locs + word_rec(w, m));
+                x.base = word_base(w, m);
+                const uint32_t bit = 1u << j;
+                if (f & SMC_HF_XINV) {
+                    const double M0 = window_of(L, x, m);
+                    if (M0 >= 0.0) {
+                        if (M0 == 0.0) zero |= bit;
+                        else bounded |= bit;
+                        scr[64 * j] = M0;
+                    }
+                }
+                if ((f & SMC_HF_XBLK) && changed && location_blocked(L.block_first, x, m)) xblk |= bit;
+            }
+        }
+        out = bounded | zero | xblk;
+    }
+    uint32_t ref[C];
 #pragma unroll
     for (int j = 0; j < C; ++j) {
-        ej[j] = -1;
-        eg[j] = -1;
-        const uint32_t c = (uint32_t)(sl * C + j);
-        if (j % G == 0) {
-            bool choice = false;
-#pragma unroll
-            for (int k = j; k < j + G; ++k) choice |= (mk[k] & (mk[k] - 1)) != 0;
-            if (choice) rw = smc_draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
+        const uint32_t w = words[64 * j], bit = 1u << j;
+        const DevHot h = load_rec(m.hots + word_rec(w, m));
+        double leaf = h.rate;
+        bool in = !(out & bit);
+        if (tests & (SMC_HF_INV | SMC_HF_GUARD)) {
+            const double v = x.vars[var_at(h.var, word_base(w, m))];
+            const bool guard_out = (h.flags & SMC_HF_GUARD) && !(h.a <= v && v <= h.b);
+            const double left = h.a - (x.now - v) - h.b;
+            const bool bnd = (h.flags & SMC_HF_INV) && left >= 0.0;
+            if (bnd) {
+                scr[64 * j] = left;
+                if (left == 0.0) zero |= bit;
+                else bounded |= bit;
+            }
+            in = in && !guard_out && !bnd;
         }
-        if (mk[j]) {
-            const int first = (int)m.locs[loc[j]].edge_first;
-            const int i = (mk[j] & (mk[j] - 1)) ? pick_weighted(mk[j], first, smc_receiver_u(rw, c), vars, m)
-                                                : lowest_lane(mk[j]);
-            const int e = first + i;
-            ej[j] = e;
-            if (trace) eg[j] = m.loc_edge0[loc[j]] + i;
-            ++fired;
-            any_fired = true;
-            const DevEdge E = load_rec(m.edges + e);
-            for (int k = 0; k < E.upd_n; ++k) {
-                const DevUpd U = load_rec(m.upds + E.upd_first + k);
-                if ((int)U.var != q.qvar) continue;
-                if (U.kind == SMC_U_ADD) {
-                    qsum += U.value;
-                    qhi = fmax(qhi, qsum);
-                    qlo = fmin(qlo, qsum);
-                    qany = true;
-                } else {
-                    q.qmax = fmax(q.qmax, U.value);
-                    q.qmin = fmin(q.qmin, U.value);
+        if (!in) leaf = 0.0;
+        rs.leaf[j] = leaf;
+        if (h.flags & SMC_HF_ZERO) zero |= bit;
+        if (tests & SMC_HF_EXPR) {
+            ref[j] = h.rate_ref;
+            if (in && (h.flags & SMC_HF_EXPR)) expr |= bit;
+            if (h.flags & SMC_HF_EXPR_LOCAL) own |= bit;
+        }
+    }
+    rs.bounded = bounded;
+    rs.zero = zero;
+    // Rates that are expressions: each pass evaluates, on every lane at once,
+    // the expression of the lane's first pending slot and hands the value to
+    // all of its pending slots with the same expression (unless it reads the
+    // component's own variables).  Evaluated slot by slot, the interpreter
+    // would run up to C times per race; here once per distinct expression a
+    // lane holds.
+    if (tests & SMC_HF_EXPR) {
+        while (__ballot(expr != 0)) {
+            double v = 0.0;
+            uint32_t r = 0xFFFFFFFFu, first = 0;
+            if (expr) {
+                first = expr & -expr;
+                const uint32_t w = words[64 * (__ffs(first) - 1)];
+                r = m.hots[word_rec(w, m)].rate_ref;
+                x.base = word_base(w, m);
+                v = eval_ref(r, x, m);
+                v = v > 0.0 ? v : 0.0;
+            }
+#pragma unroll
+            for (int j = 0; j < C; ++j) {
+                const uint32_t bit = 1u << j;
+                if ((expr & bit) && (first == bit || (ref[j] == r && !(own & bit)))) {
+                    rs.leaf[j] = v;
+                    expr &= ~bit;
                 }
             }
         }
     }
-    if (q.qvar >= 0 && (__ballot(qany) & seg_mask)) {
-        double incl = qsum;
-        for (int k = 1; k < S; k <<= 1) {
-            const double y = __shfl_up(incl, k, S);
-            if (sl >= k) incl += y;
-        }
-        const double v0 = vars[q.qvar] + (incl - qsum);  // value before this lane's additions
-        if (qany) {
-            q.qmax = fmax(q.qmax, v0 + qhi);
-            q.qmin = fmin(q.qmin, v0 + qlo);
+}
+
+// The exponential race over the segment: a fixed pairwise tree over the
+// leaves (in-lane levels, then a butterfly).  `level` keeps each level's own
+// partial sum per lane in LDS (level-major) from the sum to the descent; the
+// sibling's is exchanged again.  Returns the total.
+template <int C>
+__device__ __forceinline__ double race_total(const double (&leaf)[C], double *level, int S) {
+    double tr[2 * C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) tr[C + j] = leaf[j];
+#pragma unroll
+    for (int i = C - 1; i >= 1; --i) tr[i] = tr[2 * i] + tr[2 * i + 1];
+    double s = (C == 1) ? leaf[0] : tr[1];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        if ((1 << k) < S) {
+            level[64 * k] = s;
+            s = s + seg_xchg(s, k);
         }
     }
-    wave_sync();  // every lane has read the variables before they change
+    return s;
+}
+
+// The component reached by descending the tree with v in [0, total): left
+// while v is below the left sum (or the right one is 0).  Every lane of the
+// segment gets it.
+template <int C>
+__device__ __forceinline__ int race_pick(const double (&leaf)[C], const double *level, double v, int S, int sl,
+                                         int seg_base, uint64_t seg_mask) {
+    int b = 0;
+#pragma unroll
+    for (int k = 5; k >= 0; --k) {
+        if ((1 << k) < S) {
+            const bool in_left = ((sl >> k) & 1) == 0;
+            const double own = level[64 * k], sib = seg_xchg(own, k);
+            const double left = in_left ? own : sib;
+            const double right = in_left ? sib : own;
+            if (!(v < left || right == 0.0)) { v = v - left; b += 1 << k; }
+        }
+    }
+    // the lane's tree again, from the same leaves (same sums), halved at
+    // each level: cur holds the leaves under the current node
+    int node = 0;
+    if constexpr (C > 1) {
+        double cur[C];
+#pragma unroll
+        for (int j = 0; j < C; ++j) cur[j] = leaf[j];
+#pragma unroll
+        for (int half = C / 2; half >= 1; half >>= 1) {
+            double l[C / 2 > 0 ? C / 2 : 1], r[C / 2 > 0 ? C / 2 : 1];
+#pragma unroll
+            for (int j = 0; j < half; ++j) { l[j] = cur[j]; r[j] = cur[half + j]; }
+#pragma unroll
+            for (int w = half; w > 1; w >>= 1)
+#pragma unroll
+                for (int j = 0; j < w / 2; ++j) { l[j] = l[2 * j] + l[2 * j + 1]; r[j] = r[2 * j] + r[2 * j + 1]; }
+            const bool go_left = v < l[0] || r[0] == 0.0;
+            if (!go_left) { v = v - l[0]; node += half; }
+#pragma unroll
+            for (int j = 0; j < half; ++j) cur[j] = go_left ? cur[j] : cur[half + j];
+        }
+    }
+    const int Lw = lowest_lane(__ballot(sl == b) & seg_mask);
+    return (Lw - seg_base) * C + __shfl(node, Lw);
+}
+
+// ------------------------------------------------------------ receivers
+
+// Receivers of the broadcast `chan` sent by component `sender`
+// (SyncInSerial simulation.cu:357-407): the enabled receive edges of every
+// other component, then one edge fired per component that has any.
+//
+// Nearly always every receive edge commutes (SMC_LF_RECV_FAST): constant
+// weights make each receiver's pick independent of the others' updates, and
+// integer additions and private constants give the same variables in any
+// order, so all fire at once.  The query variable's running max/min needs
+// the values in component order: they are v0 plus the prefix sums of the
+// additions, an exclusive scan over the segment (blocked layout: lane order
+// then slot order is component order).  Otherwise they fire one at a time in
+// component order, the enabled sets computed before any of them fires.
+// TRACE mixes the fired edges into the digest in component order; LOCS keeps
+// the network's locations beside the state words; `trans` counts this
+// lane's.
+template <int C, bool TRACE, bool LOCS, class M>
+__device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int32_t *locs, Ctx x, const M &m, int chan,
+                                               int sender, LaneQuery &q, bool &goal, uint64_t seed, uint64_t run,
+                                               uint32_t step, int lane, int sl, int S, int seg_base, uint64_t seg_mask,
+                                               uint32_t &trans, uint64_t &digest) {
+    uint32_t mk[C];
+    uint32_t other = 0;  // slots whose receive edges are not all unguarded on one channel
 #pragma unroll
     for (int j = 0; j < C; ++j) {
-        if (ej[j] >= 0) {
-            const DevEdge &E = m.edges[ej[j]];
-            for (int k = 0; k < E.upd_n; ++k) {
-                const DevUpd U = load_rec(m.upds + E.upd_first + k);
-                if (U.kind == SMC_U_ADD) atomicAdd(&vars[U.var], U.value);
-                else vars[U.var] = U.clock ? vars[-1] - U.value : U.value;
+        const uint32_t w = words[64 * j];
+        const uint4 rv = load_quad(m.locs + word_rec(w, m));  // recv_chan, recv_mask, ...
+        const bool me = sl * C + j == sender;
+        mk[j] = ((int)rv.x == chan && !me) ? rv.y : 0u;
+        if ((int)rv.x == -1 && !me) other |= 1u << j;
+    }
+    uint64_t slow = 0;
+    if (__ballot(other != 0)) {
+        // enabled sets by edge, kept in the scratch (64 bits per slot)
+        uint64_t *set = (uint64_t *)scr;
+        bool serial = false;
+#pragma clang loop unroll(disable)
+        for (int j = 0; j < C; ++j) {
+            uint64_t e = 0;
+            if ((other >> j) & 1u) {
+                const uint32_t w = words[64 * j];
+                const DevLoc L = load_rec(m.locs + word_rec(w, m));
+                x.base = word_base(w, m);
+                e = enabled_mask(L.edge_first, L.edge_n, chan, x, m);
+                if (e && !(L.flags & SMC_LF_RECV_FAST)) serial = true;
             }
-            if (E.dst_goal) goal = true;
-            loc[j] = loc[j] + E.dst;
+            set[64 * j] = e;
+        }
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            if ((other >> j) & 1u) mk[j] = (uint32_t)set[64 * j];
+            else set[64 * j] = mk[j];
+        }
+        slow = __ballot(serial) & seg_mask;
+    }
+    if (!slow) {
+        int fired[TRACE ? C : 1];  // the network's index of each slot's edge (digests)
+        bool any = false;
+        double qsum = 0.0, qhi = -DBL_MAX, qlo = DBL_MAX;  // prefix sums of this lane's query additions
+        bool qany = false;
+        const double v0 = q.qvar >= 0 ? x.vars[q.qvar] : 0.0;
+        wave_sync();  // read before any receiver's additions
+        // Receivers 4g .. 4g+3 share draw g: the lane's slots of one draw are
+        // G consecutive slots (C is a power of two), drawn once at the first
+        // of them when any of them has a choice to make.
+        constexpr int G = C < 4 ? C : 4;
+        smc_u32x4 rw = {{0u, 0u, 0u, 0u}};
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            if (TRACE) fired[j] = -1;
+            const uint32_t c = (uint32_t)(sl * C + j);
+            if (j % G == 0) {
+                bool choice = false;
+#pragma unroll
+                for (int k = j; k < j + G; ++k) choice |= (mk[k] & (mk[k] - 1)) != 0;
+                if (choice) rw = smc_draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
+            }
+            if (mk[j]) {
+                const uint32_t w = words[64 * j];
+                const DevLoc L = load_rec(m.locs + word_rec(w, m));
+                int i = 31 - __clz((int)mk[j]);
+                if (mk[j] & (mk[j] - 1)) {
+                    // weighted choice from the highest edge down; weights are
+                    // constants summing below 2^31
+                    const double u = smc_receiver_u(rw, c);
+                    if ((L.flags & SMC_LF_RECV_TWO) && mk[j] == L.recv_mask) {
+                        const int rnd = (int)((double)L.recv_weight * u);
+                        if (!((int)L.recv_low <= rnd)) i = __ffs(mk[j]) - 1;
+                    } else {
+                        int W = 0;
+                        for (uint32_t r = mk[j]; r; r &= r - 1) W += (int)m.edges[L.edge_first + __ffs(r) - 1].weight;
+                        const int rnd = (int)((double)W * u);
+                        i = __ffs(mk[j]) - 1;
+                        for (uint32_t r = mk[j]; r;) {
+                            const int k = 31 - __clz((int)r);
+                            r &= ~(1u << k);
+                            W -= (int)m.edges[L.edge_first + k].weight;
+                            if (W <= rnd) { i = k; break; }
+                        }
+                    }
+                }
+                const DevEdge E = load_rec(m.edges + L.edge_first + i);
+                ++trans;
+                any = true;
+                const uint32_t base = word_base(w, m);
+#pragma clang loop unroll(disable)
+                for (int k = 0; k < E.upd_n; ++k) {
+                    const DevUpd U = load_rec(m.upds + E.upd_first + k);
+                    const uint32_t at = var_at(U.var, base);
+                    if (U.kind == SMC_U_ADD) {
+                        if ((int)at == q.qvar) {
+                            qsum += U.value;
+                            qhi = fmax(qhi, qsum);
+                            qlo = fmin(qlo, qsum);
+                            qany = true;
+                        }
+                        atomicAdd(&x.vars[at], U.value);
+                    } else {
+                        if ((int)at == q.qvar) {
+                            q.qmax = fmax(q.qmax, U.value);
+                            q.qmin = fmin(q.qmin, U.value);
+                        }
+                        x.vars[at] = U.clock ? x.now - U.value : U.value;
+                    }
+                }
+                if (E.dst_goal) goal = true;
+                words[64 * j] = (E.dst_rec << m.rec_shift) | base;
+                if (TRACE) fired[j] = m.loc_edge0[locs[64 * j]] + i;
+                if (LOCS) locs[64 * j] += E.dst;
+            }
+        }
+        if (q.qvar >= 0 && (__ballot(qany) & seg_mask)) {
+            double incl = qsum;
+            for (int k = 1; k < S; k <<= 1) {
+                const double y = __shfl_up(incl, k, S);
+                if (sl >= k) incl += y;
+            }
+            const double at = v0 + (incl - qsum);  // value before this lane's additions
+            if (qany) {
+                q.qmax = fmax(q.qmax, at + qhi);
+                q.qmin = fmin(q.qmin, at + qlo);
+            }
+        }
+        if (TRACE) {
+            for (uint64_t lanes_with = __ballot(any) & seg_mask; lanes_with; lanes_with &= lanes_with - 1) {
+                const int L = lowest_lane(lanes_with);
+#pragma unroll
+                for (int j = 0; j < C; ++j) {
+                    const int e = __shfl(fired[j], L);
+                    if (e >= 0)
+                        digest = smc_mix(digest, ((uint64_t)step << 40) |
+                                                     ((uint64_t)((L - seg_base) * C + j) << 20) | (uint64_t)e);
+                }
+            }
+        }
+    } else {
+        // one at a time: the lanes holding enabled receivers in lane order,
+        // their slots in slot order; each picks with its own stream
+        const uint64_t *set = (const uint64_t *)scr;
+        bool any = false;
+#pragma clang loop unroll(disable)
+        for (int j = 0; j < C; ++j) any |= set[64 * j] != 0;
+        for (uint64_t lanes_with = __ballot(any) & seg_mask; lanes_with; lanes_with &= lanes_with - 1) {
+            const int L = lowest_lane(lanes_with);
+#pragma clang loop unroll(disable)
+            for (int j = 0; j < C; ++j) {
+                const uint64_t mask = set[64 * j];
+                if ((__ballot(mask != 0) >> L) & 1ull) {
+                    const int c = (L - seg_base) * C + j;
+                    int e_fired = -1;  // the network's index of the fired edge (digests)
+                    if (lane == L) {
+                        const uint32_t w = words[64 * j];
+                        const uint32_t first = m.locs[word_rec(w, m)].edge_first;
+                        x.base = word_base(w, m);
+                        const int i = pick_receiver(mask, first, seed, run, step, (uint32_t)c, x, m);
+                        const DevEdge E = load_rec(m.edges + first + i);
+                        run_updates(E, x, m, q);
+                        if (E.dst_goal) goal = true;
+                        words[64 * j] = (E.dst_rec << m.rec_shift) | x.base;
+                        ++trans;
+                        if (TRACE) e_fired = m.loc_edge0[locs[64 * j]] + i;
+                        if (LOCS) locs[64 * j] += E.dst;
+                    }
+                    wave_sync();
+                    if (TRACE) {
+                        const int e = __shfl(e_fired, L);
+                        digest = smc_mix(digest, ((uint64_t)step << 40) | ((uint64_t)c << 20) | (uint64_t)e);
+                    }
+                }
+            }
         }
     }
     wave_sync();
-    // the segment's total, bit by bit (fired <= C <= 16): independent ballots
-    // instead of a chain of shuffles
-    uint32_t total = 0;
-#pragma unroll
-    for (int b = 0; b < 5; ++b) total += (uint32_t)__popcll(__ballot((fired >> b) & 1) & seg_mask) << b;
-    trans += total;
-    if (trace) {
-        for (uint64_t lanes_with = __ballot(any_fired) & seg_mask; lanes_with; lanes_with &= lanes_with - 1) {
-            const int L = lowest_lane(lanes_with);
-#pragma unroll
-            for (int j = 0; j < C; ++j) {
-                const int e = __shfl(eg[j], L);
-                if (e >= 0)
-                    digest = smc_mix(digest, ((uint64_t)step << 40) | ((uint64_t)((L - seg_base) * C + j) << 20) |
-                                                 (uint64_t)e);
-            }
-        }
-    }
-    return true;
-}
-
-// Rotate slot arrays by one (slot 1 to the front): a rolled loop over the
-// slots then touches slot 0 only, a constant index, so the arrays stay in
-// registers rather than being spilled for dynamic indexing.
-template <int C, class T>
-__device__ __forceinline__ void rotate_slots(T (&a)[C]) {
-    const T f = a[0];
-#pragma unroll
-    for (int k = 0; k < C - 1; ++k) a[k] = a[k + 1];
-    a[C - 1] = f;
-}
-
-// Receivers of one broadcast fired one at a time in component order
-// (SyncInSerial simulation.cu:378-404): the lanes holding enabled receivers
-// in lane order, their slots in slot order.  Enabled sets mk were computed
-// before any of them fires; each picks with its own stream.
-template <int C, class M>
-__device__ __forceinline__ void fire_receivers_serial(uint64_t (&mk)[C], int (&loc)[C], bool any, double *vars,
-                                                      const M &m, LaneQuery &q, bool &goal, uint64_t seed,
-                                                      uint64_t run, uint32_t step, int lane, int seg_base,
-                                                      uint64_t seg_mask, uint32_t &trans, bool trace,
-                                                      uint64_t &digest) {
-    int dummy_chan = 0;
-    for (uint64_t lanes_with = __ballot(any) & seg_mask; lanes_with; lanes_with &= lanes_with - 1) {
-        const int L = lowest_lane(lanes_with);
-        // slot j is at the front of the rotated slot arrays
-#pragma clang loop unroll(disable)
-        for (int j = 0; j < C; ++j) {
-            if ((__ballot(mk[0] != 0) >> L) & 1ull) {
-                const int c = (L - seg_base) * C + j;
-                int e_fired = -1;  // the network's index of the fired edge (digests)
-                if (lane == L) {
-                    const int first = (int)m.locs[loc[0]].edge_first;
-                    const int i = pick_receiver(mk[0], first, seed, run, step, (uint32_t)c, vars, m);
-                    if (trace) e_fired = m.loc_edge0[loc[0]] + i;
-                    loc[0] = fire_edge(first + i, loc[0], vars, m, q, goal, dummy_chan);
-                }
-                wave_sync();
-                ++trans;
-                if (trace) {
-                    const int e = __shfl(e_fired, L);
-                    digest = smc_mix(digest, ((uint64_t)step << 40) | ((uint64_t)c << 20) | (uint64_t)e);
-                }
-            }
-            rotate_slots<C>(mk);
-            rotate_slots<C>(loc);
-        }
-    }
-}
-
-// Register-resident slot arrays read at a run-time slot index.  Each element
-// passes through an empty asm so the select chain stays a chain of register
-// selects: without it the optimiser folds select(load a[k], load a[j]) into
-// a load through a selected address, which pins the array in scratch.
-template <class T>
-__device__ __forceinline__ T in_register(T v) {
-    asm("" : "+v"(v));
-    return v;
-}
-template <int C, class T>
-__device__ __forceinline__ T slot_get(const T (&a)[C], int j) {
-    T r = in_register(a[0]);
-#pragma unroll
-    for (int k = 1; k < C; ++k) r = (j == k) ? in_register(a[k]) : r;
-    return r;
-}
-template <int C, class T>
-__device__ __forceinline__ void slot_set(T (&a)[C], int j, T v) {
-#pragma unroll
-    for (int k = 0; k < C; ++k) a[k] = (j == k) ? v : a[k];
 }
 
 }  // namespace

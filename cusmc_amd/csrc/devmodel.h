@@ -9,9 +9,9 @@
 //
 //   expression reference (uint32):  bits 31..30 kind
 //       SMC_REF_CONST  index into consts[]
-//       SMC_REF_VAR    variable id (an integer variable)
+//       SMC_REF_VAR    variable operand (an integer variable)
 //       SMC_REF_CODE   bits 0..23 first instruction, bits 24..29 count
-//       SMC_REF_CLOCK  variable id of a clock
+//       SMC_REF_CLOCK  variable operand of a clock
 //
 //   instruction (8 bytes): op, dst register, up to three operands; an
 //   operand (uint16) is a register r0..r3, a variable, a constant or a
@@ -19,11 +19,17 @@
 //   index.  The value of an expression is register r0 after its last
 //   instruction.
 //
+// Variables private to one component are named relative to that component's
+// first private variable (the `local` bit of a variable operand), so that the
+// instances of one template have the same records: the network's locations
+// fall into classes of equal records (DevHot + DevLoc; equal edges, guards,
+// updates, and destinations of equal class), and a component's state is one
+// word: the class of its location and its private variables' base.
+//
 // Clocks are stored as reset stamps: a run's variable array holds, for a
 // clock x, the time s at which x would have been 0, and its value is t - s
-// with t the run's clock time, kept just before the variables (vars[-1]).
-// Time then advances with one store, however many clocks the network has;
-// assigning x := v stores s = t - v.
+// with t the run's clock time.  Time then advances without a store, however
+// many clocks the network has; assigning x := v stores s = t - v.
 #pragma once
 
 #include <stdint.h>
@@ -42,6 +48,12 @@
 #define SMC_OPND_CONST 2u
 #define SMC_OPND_CLOCK 3u
 #define SMC_OPND(kind, idx) ((uint16_t)(((kind) << 14) | (idx)))
+
+// A variable operand: index, and whether it counts from the component's base.
+#define SMC_VAR_LOCAL 0x8000u                  // in the records' 16-bit fields
+#define SMC_OPND_LOCAL 0x2000u                 // in an instruction's operand
+#define SMC_REF_LOCAL 0x20000000u              // in an expression reference
+#define SMC_MAX_LOCAL_VARS 8192                // networks with fewer variables use local operands
 
 #define SMC_NREGS 4
 #define SMC_MAX_CODE_LEN 63
@@ -63,9 +75,19 @@ enum {
                             // there is none): always blocked
     SMC_LF_GUARDED = 4,     // blocked or not by the variables: every spontaneous edge without
                             // `!=` has a conjunct that reads no clock (DevLoc.block_first)
-    SMC_LF_RECV_FAST = 8,   // every receive edge commutes (see DevUpd)
-    SMC_LF_INL_INV = 16,    // one invariant with a constant bound, inline in DevLoc.inl_*
-    SMC_LF_INL_BLK = 32     // the blocking test is one conjunct `var op constant`, inline
+    SMC_LF_RECV_FAST = 8,   // every receive edge commutes (see DevUpd), constant weights below 2^31 in all
+    SMC_LF_RECV_TWO = 16    // exactly two receive edges (recv_low: the lower one's weight)
+};
+
+// What a race step has to look at in a location (DevHot.flags).
+enum {
+    SMC_HF_ZERO = 1,        // zero delay
+    SMC_HF_INV = 2,         // one invariant with a constant bound: a = bound, b = 1e-6 if strict
+    SMC_HF_GUARD = 4,       // leaves the race while its variable is outside [a, b]
+    SMC_HF_EXPR = 8,        // the rate is the expression rate_ref
+    SMC_HF_EXPR_LOCAL = 16, // ... which reads private variables
+    SMC_HF_XINV = 32,       // other invariants: DevInv records
+    SMC_HF_XBLK = 64        // other blocking tests: guard records from block_first
 };
 
 struct DevInsn {
@@ -74,28 +96,36 @@ struct DevInsn {
     uint16_t a, b, c;
 };
 
-struct DevLoc {             // 48 bytes: 32 of location, 16 of inline data
-    uint8_t klass;
-    uint8_t type;
-    uint16_t n_inv;         // clock upper-bound invariants
-    uint32_t rate;          // expression reference
-    uint32_t inv_first;
+// The part of a location that every race step reads for every component, 32
+// bytes: two 16-byte LDS reads.  `rate` is what the component races at if
+// nothing else holds (0 for a zero-delay location, for one that can never
+// fire, and for a rate that is not positive).
+struct DevHot {
+    double rate;
+    double a, b;
+    uint32_t rate_ref;
+    uint16_t var;           // variable operand of the invariant or guard
+    uint16_t flags;         // SMC_HF_*
+};
+
+// The rest, 48 bytes: receive edges, then edge range, invariants, blocking
+// test, rate.
+struct DevLoc {
+    int32_t recv_chan;      // every receive edge is unguarded, on this channel; 0 none; -1 other
+    uint32_t recv_mask;     // the receive edges, as bits of the edge list
+    uint32_t recv_weight;   // sum of their weights
+    uint32_t recv_low;      // SMC_LF_RECV_TWO
     uint32_t edge_first;    // edges [edge_first, edge_first + edge_n)
-    double rate_value;      // the rate when it is a constant (rate_const)
     uint16_t edge_n;
-    uint8_t rate_const;
+    uint8_t klass;
     uint8_t flags;          // SMC_LF_*
+    uint32_t inv_first;     // clock upper-bound invariants
     uint32_t block_first;   // SMC_LF_GUARDED: the blocking test, guard records from here on
-    // The commonest invariant (one, constant bound) or blocking test (one
-    // conjunct `var op constant`) as plain values, read with the location
-    // from the LDS-staged tables (one dependent trip less in the race's slot
-    // loop).  Kernels reading the tables from global memory load the first
-    // 32 bytes only and take the general records (load_loc).
-    double inl_value;       // SMC_LF_INL_INV: the bound; SMC_LF_INL_BLK: the constant
-    uint16_t inl_var;       // the clock bounded, or the variable compared
-    uint8_t inl_op;         // SMC_LF_INL_INV: 1 if strict; SMC_LF_INL_BLK: smc_cons_op
-    uint8_t inl_pad0;
-    uint32_t inl_pad1;
+    double rate_value;      // the rate when it is a constant (rate_const)
+    uint32_t rate;          // expression reference
+    uint16_t n_inv;
+    uint8_t rate_const;
+    uint8_t type;
 };
 
 struct DevInv {             // x <= bound  (strict: x < bound), 16 bytes
@@ -105,6 +135,9 @@ struct DevInv {             // x <= bound  (strict: x < bound), 16 bytes
     uint32_t bound;         // expression reference
     double bound_value;
 };
+
+// DevEdge.flags
+enum { SMC_EF_WEIGHT_CONST = 1 };  // weight is the constant itself (0 if negative), else a reference
 
 struct DevEdge {            // 32 bytes
     int32_t dst;            // destination relative to the source location
@@ -116,8 +149,8 @@ struct DevEdge {            // 32 bytes
     uint16_t upd_n;
     uint8_t dst_goal;       // destination is a goal location
     uint8_t never;          // has a `!=` guard: never enabled (simulation.cu:249-251)
-    uint16_t pad0;
-    uint32_t pad1;
+    uint16_t flags;         // SMC_EF_*
+    uint32_t dst_rec;       // record class of the destination
 };
 
 // DevGuard.flags
@@ -125,7 +158,8 @@ enum {
     SMC_GF_CLOCK_FREE = 1,  // neither var nor rhs reads a clock: fixed between transitions
     SMC_GF_CLOCK = 2,       // var is a clock
     SMC_GF_END_EDGE = 4,    // blocking test: last conjunct of its edge
-    SMC_GF_END_LOC = 8      // blocking test: last record of the location
+    SMC_GF_END_LOC = 8,     // blocking test: last record of the location
+    SMC_GF_RANGE = 16       // constant right side: holds for values in [lo, hi]
 };
 
 // A guard-blocked location's blocking test is a run of guard records (from
@@ -133,17 +167,22 @@ enum {
 // without `!=`, edge after edge.  The location is blocked when every edge
 // has a false conjunct among them.
 
-struct DevGuard {           // variables[var] op rhs
+// variables[var] op rhs, 24 bytes.  With a constant right side every
+// operator is the test of an interval of doubles (the tolerance of `==`
+// included: the interval's ends are the last values that pass it).
+struct DevGuard {
+    double lo, hi;
     uint16_t var;
     uint8_t op;             // smc_cons_op, never SMC_C_NE
     uint8_t flags;          // SMC_GF_*
     uint32_t rhs;
 };
 
-// Update kinds: a commuting receive edge has only SMC_U_ADD updates
-// (integer variable += integer constant) and SMC_U_SET updates (a variable
-// written by one component only := constant), so the receivers of one
-// broadcast can fire in any order with the same result.
+// Update kinds: integer variable plus a constant, a constant, or anything
+// else.  A commuting receive edge has only ADD updates of an integer constant
+// and SET updates of a variable written by one component only (or by all
+// with the same value), so the receivers of one broadcast can fire in any
+// order with the same result.
 enum { SMC_U_EXPR = 0, SMC_U_ADD = 1, SMC_U_SET = 2 };
 
 struct DevUpd {             // 16 bytes
@@ -174,20 +213,12 @@ struct SmcGlobalTables {
 struct SmcLdsTables {
     template <class T> using ptr = const SMC_LDS T *;
 };
-// Location records from global memory, every other hot table from the LDS
-// copy: for networks whose many location records would crowd LDS while
-// their edge, guard, update and expression records (shared by template
-// instances) are few.
-struct SmcMixedTables {
-    template <class T>
-    using ptr = typename std::conditional<std::is_same<T, DevLoc>::value, const SMC_GLOBAL T *,
-                                          const SMC_LDS T *>::type;
-};
 
 // Everything the run kernel needs to know about one model; passed by value.
 template <class A>
 struct DevModelT {
-    typename A::template ptr<DevLoc> locs;
+    typename A::template ptr<DevHot> hots;     // [n_recs] record 0: no component
+    typename A::template ptr<DevLoc> locs;     // [n_recs]
     typename A::template ptr<DevInv> invs;
     typename A::template ptr<DevEdge> edges;
     typename A::template ptr<DevGuard> guards;
@@ -195,18 +226,20 @@ struct DevModelT {
     typename A::template ptr<double> consts;
     typename A::template ptr<DevInsn> code;
     const SMC_GLOBAL double *var_init;     // stored form at time 0: initial value, -initial value for a clock
-    const SMC_GLOBAL int32_t *comp_init_loc;
+    const SMC_GLOBAL uint32_t *comp_word;      // [n_comp] initial state word (class << rec_shift | base)
+    const SMC_GLOBAL int32_t *comp_init_loc;   // [n_comp]
     const SMC_GLOBAL uint8_t *var_clock;   // [n_vars] 1: the variable is a clock
     const SMC_GLOBAL int32_t *comp_first_loc;  // [n_comp + 1] location range of each component
     const SMC_GLOBAL int32_t *loc_edge0;       // [n_locs] the network's index of each location's first edge
                                                // (edge records are shared: digests name network edges)
+    const SMC_GLOBAL uint32_t *loc_rec;        // [n_locs] record class of each location
     int32_t n_comp;
     int32_t n_vars;
-    int32_t n_clocks;
     int32_t n_leaves;           // next power of two >= n_comp
     int32_t n_locs;
-    int32_t n_edges;
+    int32_t rec_shift;          // state word: class << rec_shift | base of the private variables
+    uint32_t base_mask;         // (1 << rec_shift) - 1
+    uint32_t tests;             // every SMC_HF_* flag some location has
     int32_t freeze;             // no rate reads a clock: blocked components may leave the race
-    int32_t guarded;            // some location is flagged SMC_LF_GUARDED
 };
 using DevModel = DevModelT<SmcGlobalTables>;

@@ -567,9 +567,9 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         s->C = P / s->S;
         if (s->C > 8) throw std::runtime_error("internal: more than 8 slots per lane");
         s->R = 64 / s->S;
-        s->stride = (img.n_vars + 1) | 1;  // clock time, then the variables
+        s->stride = img.n_vars | 1;
 
-        s->n_locs = (int)img.locs.size();
+        s->n_locs = (int)img.info.size();
         s->n_vars = img.n_vars;
         s->n_comp = img.n_comp;
         s->F = s->n_locs + s->n_vars + 1;
@@ -592,15 +592,12 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
                 const int l0 = img.comp_first_loc[cpt], l1 = img.comp_first_loc[cpt + 1];
                 std::vector<int64_t> sig{l1 - l0};
                 for (int l = l0; l < l1; ++l) {
-                    const DevLoc &Lc = img.locs[l];
-                    int64_t rate_key;
-                    if (Lc.rate_const) memcpy(&rate_key, &Lc.rate_value, 8);
-                    else rate_key = (int64_t)Lc.rate ^ ((int64_t)1 << 62);
-                    sig.insert(sig.end(), {(int64_t)Lc.klass, (int64_t)Lc.type, (int64_t)Lc.n_inv, rate_key,
-                                           (int64_t)Lc.edge_n});
-                    for (int e = (int)Lc.edge_first; e < (int)Lc.edge_first + Lc.edge_n; ++e) {
-                        sig.push_back((int64_t)l + img.edges[e].dst - l0);  // destinations are relative
-                        sig.push_back((int64_t)img.edges[e].channel);
+                    const smc::LocInfo &Lc = img.info[l];
+                    sig.insert(sig.end(), {(int64_t)Lc.klass, (int64_t)Lc.type, (int64_t)Lc.n_inv, Lc.rate_key,
+                                           (int64_t)Lc.edges.size()});
+                    for (const auto &e : Lc.edges) {
+                        sig.push_back((int64_t)l + e.dst - l0);  // destinations are relative
+                        sig.push_back((int64_t)e.channel);
                     }
                 }
                 auto it = base_of.find(sig);
@@ -619,14 +616,18 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         s->Gpad = (int)rup((size_t)std::max(s->n_groups, 1), 64);
         s->G16 = (int)rup((size_t)std::max(s->n_groups, 1), 16);
         // advance kernel LDS: per wave the variables of its 64/S rows, their
-        // tilt tables (theta and 2^theta, up to Gpad entries) and the race
-        // tree's levels (2 log2(S) doubles per lane), after a shared part
-        // (tilt index and a shared 2^theta vector, Lpad each)
+        // tilt tables (theta and 2^theta, up to Gpad entries), slot scratch,
+        // race-tree levels, state words and locations (is_advance.h), after a
+        // shared part (tilt index and a shared 2^theta vector, Lpad each)
         int levels = 0;
         while ((1 << levels) < s->S) ++levels;
-        s->wave_lds = (uint32_t)rup((size_t)s->R * s->stride * sizeof(double) + (size_t)s->R * s->Gpad * 12 +
-                                        (size_t)2 * levels * 64 * sizeof(double), 16);
-        if (s->wave_lds > 60000) throw std::runtime_error("limit: variables exceed the LDS budget");
+        const size_t tilts = (size_t)s->R * s->Gpad * 12;
+        // the most variables and tilts a packing may hold: with a clock time
+        // per row and two doubles per lane and level, 60,000 bytes
+        if ((size_t)s->R * ((img.n_vars + 1) | 1) * 8 + tilts + (size_t)levels * 1024 > 60000)
+            throw std::runtime_error("limit: variables exceed the LDS budget");
+        s->wave_lds = (uint32_t)rup((size_t)s->R * s->stride * sizeof(double) + tilts +
+                                        (size_t)(s->C + levels) * 64 * sizeof(double) + (size_t)s->C * 512, 16);
         {
             const size_t shared = (size_t)s->Lpad * 12;
             // hot tables staged in LDS when the model's tuned launch does so
@@ -662,7 +663,7 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
 
         // tiltable locations: every location that is not zero-delay
         s->h_tiltable.assign(L, 0);
-        for (int l = 0; l < s->n_locs; ++l) s->h_tiltable[l] = img.locs[l].klass != SMC_K_ZERO;
+        for (int l = 0; l < s->n_locs; ++l) s->h_tiltable[l] = img.info[l].klass != SMC_K_ZERO;
         // feature scales: clocks by the time bound, other variables by the
         // largest initial magnitude or the component count
         std::vector<float> scale(std::max(s->n_vars, 1), 1.f);
