@@ -597,6 +597,10 @@ ModelImage lower(const smc_network &n, bool use_locals) {
 
             // what a race step looks at
             DevHot &h = R.hot;
+            auto hot_var = [&](uint16_t v) {
+                h.var = (uint16_t)((v & ~SMC_VAR_LOCAL) * 8u);
+                if (v & SMC_VAR_LOCAL) h.flags |= 8;
+            };
             if (d.klass == SMC_K_ZERO) {
                 h.flags = SMC_HF_ZERO;
             } else {
@@ -610,7 +614,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                 }
                 if (d.n_inv == 1 && R.invs[0].bound_const) {
                     h.flags |= SMC_HF_INV;
-                    h.var = R.invs[0].var;
+                    hot_var(R.invs[0].var);
                     h.a = R.invs[0].bound_value;
                     h.b = R.invs[0].strict ? 1e-6 : 0.0;
                 } else if (d.n_inv) {
@@ -619,7 +623,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                 if (img.freeze && kind == 2) {
                     if (R.block.size() == 1 && (R.block[0].flags & SMC_GF_RANGE) && !(h.flags & SMC_HF_INV)) {
                         h.flags |= SMC_HF_GUARD;
-                        h.var = R.block[0].var;
+                        hot_var(R.block[0].var);
                         h.a = R.block[0].lo;
                         h.b = R.block[0].hi;
                     } else {
@@ -627,7 +631,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                     }
                 }
             }
-            img.tests |= h.flags;
+            img.tests |= h.flags & ~(uint32_t)SMC_HF_LOCAL;
         }
     }
 

@@ -20,6 +20,31 @@ __device__ __forceinline__ void wave_sync() {
 
 __device__ __forceinline__ int lowest_lane(uint64_t m) { return __ffsll((unsigned long long)m) - 1; }
 
+// A wave-uniform value, opaque to the optimiser from here on.  What is
+// computed from it inside a loop (the round keys of a draw, the levels a
+// segment has) stays there: hoisted, these invariants take some sixty scalar
+// registers that no kernel here has left, and come back as lane reads of
+// spilled registers, one vector instruction each.
+__device__ __forceinline__ int scalar_here(int v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ uint64_t scalar_here(uint64_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ int lane_here(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// smc_draw with the key schedule computed at the draw (scalar adds beside
+// the rounds).
+__device__ __forceinline__ smc_u32x4 draw(uint64_t seed, uint64_t run, uint32_t step, uint32_t purpose,
+                                          uint32_t comp) {
+    return smc_draw(scalar_here(seed), run, step, purpose, comp);
+}
+
 // ------------------------------------------------------------ segment exchange
 //
 // Level k of a butterfly over an aligned segment: each lane receives the
@@ -383,7 +408,7 @@ template <class M>
 __device__ __forceinline__ int pick_edge(uint64_t mask, uint32_t edge_first, uint64_t seed, uint64_t run,
                                          uint32_t step, uint32_t comp, const Ctx &x, const M &m) {
     if ((mask & (mask - 1)) == 0) return lowest_lane(mask);
-    const smc_u32x4 w = smc_draw(seed, run, step, SMC_P_WINNER, comp);
+    const smc_u32x4 w = draw(seed, run, step, SMC_P_WINNER, comp);
     return pick_weighted(mask, edge_first, smc_u01(w.v[0], w.v[1]), x, m);
 }
 
@@ -393,7 +418,7 @@ template <class M>
 __device__ __forceinline__ int pick_receiver(uint64_t mask, uint32_t edge_first, uint64_t seed, uint64_t run,
                                              uint32_t step, uint32_t c, const Ctx &x, const M &m) {
     if ((mask & (mask - 1)) == 0) return lowest_lane(mask);
-    const smc_u32x4 w = smc_draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
+    const smc_u32x4 w = draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
     return pick_weighted(mask, edge_first, smc_receiver_u(w, c), x, m);
 }
 
@@ -514,72 +539,94 @@ __device__ __forceinline__ bool absorbed(const uint32_t *words, Ctx x, const M &
 template <int C>
 struct RaceSlots {
     double leaf[C];         // rate in the exponential race, 0 if not in it
-    uint32_t bounded;       // slots with a clock-bounded delay (window in the lane's scratch)
+    uint32_t bounded;       // slots with a clock-bounded delay (window in the lane's scratch; 0: also in zero)
     uint32_t zero;          // slots with delay 0
 };
 
-// Classify the lane's slots and evaluate their rates.  Nearly everything is
-// one straight line per slot over its class's 32-byte DevHot record (three
-// LDS reads, a handful of compares; no branch depends on a lane), because
-// the lanes of a wave hold components in every kind of location: as
-// branches, every slot would run every kind's code.  Invariants and blocking
-// tests beyond one record take a rolled loop beforehand, on models that have
-// them; xblk keeps those blocking results until the next change of state.
+// Classify the lane's slots and evaluate their rates: one straight line over
+// the lane's slots, each reading its class's 32-byte DevHot record and its
+// variable.  No branch depends on a lane or a slot: the lanes of a wave hold
+// components in every kind of location, so branches would run every kind's
+// code for every slot, and they would keep the slots' reads, a chain of three
+// each, from overlapping.  Invariants and blocking tests beyond one record
+// take a rolled loop afterwards, on models that have them; xblk keeps those
+// blocking results until the next change of state.
 template <int C, class M>
 __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *words, double *scr, Ctx x, const M &m,
                                            bool changed, uint32_t &xblk) {
     const uint32_t tests = m.tests;
-    uint32_t bounded = 0, zero = 0, out = 0, expr = 0, own = 0;
-    if (tests & (SMC_HF_XINV | SMC_HF_XBLK)) {
-        if (changed) xblk = 0;
-#pragma clang loop unroll(disable)
+    uint32_t bounded = 0, zero = 0, expr = 0, own = 0;
+    uint32_t ref[C];
+    auto flag = [](uint32_t d, uint32_t f, uint32_t bit) { return (d & (f << 16)) ? bit : 0u; };
+    if (tests & (SMC_HF_INV | SMC_HF_GUARD)) {
+        DevHot h[C];
+        uint32_t base[C];
+        double v[C];
+#pragma unroll
         for (int j = 0; j < C; ++j) {
             const uint32_t w = words[64 * j];
+            base[j] = word_base(w, m);
+            h[j] = load_rec(m.hots + word_rec(w, m));
+        }
+#pragma unroll
+        for (int j = 0; j < C; ++j)
+            v[j] = *(const double *)((const char *)x.vars + h[j].var + base[j] * (h[j].flags & SMC_HF_LOCAL));
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            const uint32_t bit = 1u << j, d = (uint32_t)h[j].flags << 16;
+            const double left = h[j].a - (x.now - v[j]) - h[j].b;
+            const bool bnd = ((int32_t)d < 0) & (left >= 0.0);
+            const bool out = ((d & (SMC_HF_GUARD << 16)) != 0) & !((h[j].a <= v[j]) & (v[j] <= h[j].b));
+            const bool in = !(bnd | out);
+            scr[64 * j] = left;  // read only if bounded
+            bounded |= bnd ? bit : 0u;
+            zero |= (bnd & (left == 0.0)) ? bit : 0u;
+            zero |= flag(d, SMC_HF_ZERO, bit);
+            rs.leaf[j] = in ? h[j].rate : 0.0;
+            ref[j] = h[j].rate_ref;
+            expr |= in ? flag(d, SMC_HF_EXPR, bit) : 0u;
+            own |= flag(d, SMC_HF_EXPR_LOCAL, bit);
+        }
+    } else {
+        DevHot h[C];
+#pragma unroll
+        for (int j = 0; j < C; ++j) h[j] = load_rec(m.hots + word_rec(words[64 * j], m));
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            const uint32_t bit = 1u << j, d = (uint32_t)h[j].flags << 16;
+            zero |= flag(d, SMC_HF_ZERO, bit);
+            rs.leaf[j] = h[j].rate;
+            ref[j] = h[j].rate_ref;
+            expr |= flag(d, SMC_HF_EXPR, bit);
+            own |= flag(d, SMC_HF_EXPR_LOCAL, bit);
+        }
+    }
+    if (tests & (SMC_HF_XINV | SMC_HF_XBLK)) {
+        if (changed) xblk = 0;
+        uint32_t out = 0;
+#pragma clang loop unroll(disable)
+        for (int j = 0; j < C; ++j) {
+            const uint32_t w = words[64 * j], bit = 1u << j;
             const uint32_t f = m.hots[word_rec(w, m)].flags;
             if (f & (SMC_HF_XINV | SMC_HF_XBLK)) {
                 const DevLoc L = load_rec(m.locs + word_rec(w, m));
                 x.base = word_base(w, m);
-                const uint32_t bit = 1u << j;
                 if (f & SMC_HF_XINV) {
                     const double M0 = window_of(L, x, m);
                     if (M0 >= 0.0) {
                         if (M0 == 0.0) zero |= bit;
-                        else bounded |= bit;
+                        bounded |= bit;
                         scr[64 * j] = M0;
+                        out |= bit;
                     }
                 }
                 if ((f & SMC_HF_XBLK) && changed && location_blocked(L.block_first, x, m)) xblk |= bit;
             }
         }
-        out = bounded | zero | xblk;
-    }
-    uint32_t ref[C];
+        out |= xblk;
+        expr &= ~out;
 #pragma unroll
-    for (int j = 0; j < C; ++j) {
-        const uint32_t w = words[64 * j], bit = 1u << j;
-        const DevHot h = load_rec(m.hots + word_rec(w, m));
-        double leaf = h.rate;
-        bool in = !(out & bit);
-        if (tests & (SMC_HF_INV | SMC_HF_GUARD)) {
-            const double v = x.vars[var_at(h.var, word_base(w, m))];
-            const bool guard_out = (h.flags & SMC_HF_GUARD) && !(h.a <= v && v <= h.b);
-            const double left = h.a - (x.now - v) - h.b;
-            const bool bnd = (h.flags & SMC_HF_INV) && left >= 0.0;
-            if (bnd) {
-                scr[64 * j] = left;
-                if (left == 0.0) zero |= bit;
-                else bounded |= bit;
-            }
-            in = in && !guard_out && !bnd;
-        }
-        if (!in) leaf = 0.0;
-        rs.leaf[j] = leaf;
-        if (h.flags & SMC_HF_ZERO) zero |= bit;
-        if (tests & SMC_HF_EXPR) {
-            ref[j] = h.rate_ref;
-            if (in && (h.flags & SMC_HF_EXPR)) expr |= bit;
-            if (h.flags & SMC_HF_EXPR_LOCAL) own |= bit;
-        }
+        for (int j = 0; j < C; ++j) rs.leaf[j] = ((out >> j) & 1u) ? 0.0 : rs.leaf[j];
     }
     rs.bounded = bounded;
     rs.zero = zero;
@@ -642,10 +689,11 @@ template <int C>
 __device__ __forceinline__ int race_pick(const double (&leaf)[C], const double *level, double v, int S, int sl,
                                          int seg_base, uint64_t seg_mask) {
     int b = 0;
+    const int at = lane_here(sl);
 #pragma unroll
     for (int k = 5; k >= 0; --k) {
         if ((1 << k) < S) {
-            const bool in_left = ((sl >> k) & 1) == 0;
+            const bool in_left = ((at >> k) & 1) == 0;
             const double own = level[64 * k], sib = seg_xchg(own, k);
             const double left = in_left ? own : sib;
             const double right = in_left ? sib : own;
@@ -754,7 +802,7 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int
                 bool choice = false;
 #pragma unroll
                 for (int k = j; k < j + G; ++k) choice |= (mk[k] & (mk[k] - 1)) != 0;
-                if (choice) rw = smc_draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
+                if (choice) rw = draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
             }
             if (mk[j]) {
                 const uint32_t w = words[64 * j];

@@ -81,13 +81,14 @@ enum {
 
 // What a race step has to look at in a location (DevHot.flags).
 enum {
-    SMC_HF_ZERO = 1,        // zero delay
-    SMC_HF_INV = 2,         // one invariant with a constant bound: a = bound, b = 1e-6 if strict
-    SMC_HF_GUARD = 4,       // leaves the race while its variable is outside [a, b]
-    SMC_HF_EXPR = 8,        // the rate is the expression rate_ref
-    SMC_HF_EXPR_LOCAL = 16, // ... which reads private variables
-    SMC_HF_XINV = 32,       // other invariants: DevInv records
-    SMC_HF_XBLK = 64        // other blocking tests: guard records from block_first
+    SMC_HF_LOCAL = 0xFF,    // the variable counts from the component's base: 8 (bytes) or 0
+    SMC_HF_ZERO = 0x100,    // zero delay
+    SMC_HF_EXPR = 0x200,    // the rate is the expression rate_ref
+    SMC_HF_EXPR_LOCAL = 0x400,  // ... which reads private variables
+    SMC_HF_XINV = 0x800,    // other invariants: DevInv records
+    SMC_HF_XBLK = 0x1000,   // other blocking tests: guard records from block_first
+    SMC_HF_GUARD = 0x4000,  // leaves the race while its variable is outside [a, b]
+    SMC_HF_INV = 0x8000     // one invariant with a constant bound: a = bound, b = 1e-6 if strict
 };
 
 struct DevInsn {
@@ -104,7 +105,7 @@ struct DevHot {
     double rate;
     double a, b;
     uint32_t rate_ref;
-    uint16_t var;           // variable operand of the invariant or guard
+    uint16_t var;           // byte offset of the invariant's or guard's variable
     uint16_t flags;         // SMC_HF_*
 };
 
@@ -196,15 +197,18 @@ struct DevUpd {             // 16 bytes
 // The tables live in device global memory.  Device code sees their pointers
 // in the global address space, so reads compile to global loads (their own
 // wait counter) rather than flat loads, which the compiler must also order
-// against LDS traffic; host code sees plain pointers of the same size.  A
-// run kernel may stage the tables in LDS and read them through a second
+// against LDS traffic; host code sees plain pointers of the same size.
+// Launch records that no kernel writes are read through the constant address
+// space (scalar loads).  A run kernel may stage the tables in LDS and read them through a second
 // instance of the same record (DevModelT<SmcLdsTables>).
 #if defined(__HIP_DEVICE_COMPILE__)
 #define SMC_GLOBAL __attribute__((address_space(1)))
 #define SMC_LDS __attribute__((address_space(3)))
+#define SMC_CONSTANT __attribute__((address_space(4)))
 #else
 #define SMC_GLOBAL
 #define SMC_LDS
+#define SMC_CONSTANT
 #endif
 
 struct SmcGlobalTables {

@@ -271,7 +271,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
             for (uint32_t b = rs.bounded; b;) {
                 const int j = __ffs(b) - 1;
                 const uint32_t c = (uint32_t)(sl * C + j);
-                const smc_u32x4 rw = smc_draw(P.seed, run, step, SMC_P_UNIFORM, smc_uniform_draw(c));
+                const smc_u32x4 rw = draw(P.seed, run, step, SMC_P_UNIFORM, smc_uniform_draw(c));
                 // slot j, then slot j + 1 when it shares the draw
                 const int nj = (C > 1 && !(c & 1u) && ((b >> (j + 1)) & 1u)) ? 2 : 1;
 #pragma clang loop unroll(disable)
@@ -293,7 +293,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
             double dexp = INF;
             int wexp = 0x7FFFFFFF;
             if (Rt > 0.0) {
-                const smc_u32x4 rw = smc_draw(P.seed, run, step, SMC_P_RACE, 0);
+                const smc_u32x4 rw = draw(P.seed, run, step, SMC_P_RACE, 0);
                 dexp = -smc_log2(smc_u01(rw.v[0], rw.v[1])) / Rt;
                 wexp = race_pick<C>(leaft, lvl, smc_u01(rw.v[2], rw.v[3]) * Rt, S, sl, seg_base, seg_mask);
             }
@@ -321,7 +321,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                 for (int j = 0; j < C; ++j) dl[j] = ((fz >> j) & 1u) ? scr[64 * j] : 0.0;
                 const double Rd = tree_total<C>(dl, S);
                 if (Rd > 0.0) {
-                    const smc_u32x4 rw = smc_draw(P.seed, run, step, SMC_P_DEAD, 0);
+                    const smc_u32x4 rw = draw(P.seed, run, step, SMC_P_DEAD, 0);
                     const double td = P.bound + (-smc_log2(smc_u01(rw.v[0], rw.v[1])) / Rd);
                     if (td < t + d) { d = td - t; w = -1; exp_won = false; u_won = false; }
                 }

@@ -53,6 +53,11 @@ namespace {
 
 // ------------------------------------------------------------ run kernel
 
+// The same pointer, as far as the optimiser knows another one.
+__device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTANT InstDesc *p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
 
 // One wave at a time takes a chunk of runs of one instance from the launch's
 // queue, so the instance (its tables, query and outputs) is uniform across
@@ -70,8 +75,9 @@ namespace {
 // wait for, and a step's code has to stay in the 64 KB instruction cache
 // (with per-slot copies of the general code in every branch it was 320 KB).
 // Fischer-32, 1e6 runs at 4 lanes a run: 76.2 ms in that form, 51.0 ms with
-// record classes, one straight slot loop and rolled cold paths; SIR-350,
-// 2e5 runs at 64 lanes: 355 ms and 117 ms.
+// record classes and rolled cold paths, 44.2 ms with the slot loop free of
+// branches and its invariants out of spilled registers; SIR-350, 2e5 runs at
+// 64 lanes: 355, 117 and 97 ms.
 //
 // LDS: [tables: lp.table_bytes, TAB only] then per wave [variables of the
 // wave's 64/S runs: var_stride doubles each][scratch: 8 bytes per slot and
@@ -106,32 +112,62 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
         if (lp.inst[mid].chunk_first <= g) lo = mid;
         else hi = mid - 1;
     }
-    const DevModel mg = lp.inst[lo].m;
+    // What every step needs of the instance stays in registers; what only a
+    // run's start or end needs is read again there (through `inst` made
+    // opaque, or it would be loaded here and spilled).
+    const SMC_CONSTANT InstDesc *inst = (const SMC_CONSTANT InstDesc *)(uintptr_t)lp.inst + lo;
     DevModelT<Tables> m;
-    if constexpr (TAB) m = lds_model(mg, lp.tables, lds);
-    else m = mg;
-    const SimParams p = lp.inst[lo].p;
+    if constexpr (TAB) {
+        const SMC_LDS uint8_t *copy = (const SMC_LDS uint8_t *)(SMC_LDS double *)lds;
+        m.hots = in_lds(inst->m.hots, lp.tables, copy);
+        m.locs = in_lds(inst->m.locs, lp.tables, copy);
+        m.invs = in_lds(inst->m.invs, lp.tables, copy);
+        m.edges = in_lds(inst->m.edges, lp.tables, copy);
+        m.guards = in_lds(inst->m.guards, lp.tables, copy);
+        m.upds = in_lds(inst->m.upds, lp.tables, copy);
+        m.consts = in_lds(inst->m.consts, lp.tables, copy);
+        m.code = in_lds(inst->m.code, lp.tables, copy);
+    } else {
+        m.hots = inst->m.hots;
+        m.locs = inst->m.locs;
+        m.invs = inst->m.invs;
+        m.edges = inst->m.edges;
+        m.guards = inst->m.guards;
+        m.upds = inst->m.upds;
+        m.consts = inst->m.consts;
+        m.code = inst->m.code;
+    }
+    m.loc_edge0 = inst->m.loc_edge0;
+    m.rec_shift = inst->m.rec_shift;
+    m.base_mask = inst->m.base_mask;
+    m.tests = inst->m.tests;
+    m.freeze = inst->m.freeze;
+    const uint64_t seed = inst->p.seed;
+    const double bound = inst->p.bound;
+    const bool reach = inst->p.reach != 0;
+    const uint32_t max_steps = inst->p.max_steps;
     // the instance's packing: S lanes per run, 64 / S runs per wave
-    const int S = lp.inst[lo].lanes;
-    const int sl = lane & (S - 1);
+    const int S0 = inst->lanes;
+    const int sl = lane & (S0 - 1);
     const int seg_base = lane - sl;
-    const uint64_t seg_ones = (S == 64) ? ~0ull : ((1ull << S) - 1ull);
+    const uint64_t seg_ones = (S0 == 64) ? ~0ull : ((1ull << S0) - 1ull);
     const uint64_t seg_mask = seg_ones << seg_base;
-    double *vars = wbase + (size_t)(lane / S) * lp.var_stride;
-    double *scr = wbase + (size_t)(64 / S) * lp.var_stride + lane;
-    uint32_t *words_of = (uint32_t *)(wbase + (size_t)(64 / S) * lp.var_stride + 64 * lp.scratch);
+    double *vars = wbase + (size_t)(lane / S0) * lp.var_stride;
+    double *scr = wbase + (size_t)(64 / S0) * lp.var_stride + lane;
+    uint32_t *words_of = (uint32_t *)(wbase + (size_t)(64 / S0) * lp.var_stride + 64 * lp.scratch);
     uint32_t *words = words_of + lane;
     int32_t *locs = (int32_t *)words_of + 64 * C + lane;  // TRACE only
-    const uint32_t chunk_runs = lp.inst[lo].chunk_runs;
-    const uint64_t chunk = g - lp.inst[lo].chunk_first;
+    const uint32_t chunk_runs = inst->chunk_runs;
+    const uint64_t chunk = g - inst->chunk_first;
     const uint32_t r_first = (uint32_t)(chunk * chunk_runs);
-    const uint32_t r_end = (uint32_t)((uint64_t)r_first + chunk_runs < p.n_runs ? r_first + chunk_runs : p.n_runs);
+    const uint32_t r_end = (uint32_t)((uint64_t)r_first + chunk_runs < inst->p.n_runs ? r_first + chunk_runs
+                                                                               : inst->p.n_runs);
     if (lane == 0) chunk_next = r_first;
     wave_sync();
-    const int n = m.n_comp;
 
     bool active = false, done = false;
-    uint64_t run = 0, ridx = 0;
+    uint64_t run = 0;
+    uint32_t ridx = 0;
     double t = 0.0;
     uint32_t step = 0, trans = 0;  // trans: edges fired by this lane (the winner's count on lane 0)
     int chan = 0, sender = -1;
@@ -139,9 +175,10 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     bool changed = true;  // state changed since the last blocking tests
     uint32_t xblk = 0;    // blocked slots at the last change of state (tests of several records)
     uint64_t digest = 0;
-    LaneQuery q{p.qvar, p.qinit, p.qinit};
+    LaneQuery q{inst->p.qvar, 0.0, 0.0};
 
     for (;;) {
+        const int S = scalar_here(S0);
         if (!active && !done) {
             unsigned int r = 0;
             if (sl == 0) r = atomicAdd(&chunk_next, 1u);
@@ -149,19 +186,20 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
             if (r >= r_end) {
                 done = true;
             } else {
+                const SMC_CONSTANT InstDesc *I = opaque(inst);
                 ridx = r;
-                run = p.run_begin + round * p.n_runs + r;
+                run = I->p.run_begin + round * I->p.n_runs + r;
                 active = true;
                 t = 0.0; step = 0; trans = 0; chan = 0; sender = -1;
                 goal = false; changed = true;
-                q.qmax = p.qinit; q.qmin = p.qinit;
+                q.qmax = I->p.qinit; q.qmin = I->p.qinit;
                 digest = TRACE ? smc_mix(0, run) : 0;
-                for (int v = sl; v < m.n_vars; v += S) vars[v] = m.var_init[v];
+                for (int v = sl; v < I->m.n_vars; v += S) vars[v] = I->m.var_init[v];
 #pragma clang loop unroll(disable)
                 for (int j = 0; j < C; ++j) {
                     const int c = sl * C + j;
-                    words[64 * j] = c < n ? m.comp_word[c] : 0u;
-                    if (TRACE) locs[64 * j] = c < n ? m.comp_init_loc[c] : -1;
+                    words[64 * j] = c < I->m.n_comp ? I->m.comp_word[c] : 0u;
+                    if (TRACE) locs[64 * j] = c < I->m.n_comp ? I->m.comp_init_loc[c] : -1;
                 }
                 wave_sync();
             }
@@ -171,14 +209,14 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
 
         // ---- loop test (simulation.cu:835-849)
         bool hit = false, end = false;
-        if (!(t < p.bound)) end = true;
-        else if (p.reach && goal) { end = true; hit = true; }
-        else if (step >= p.max_steps) end = true;
+        if (!(t < bound)) end = true;
+        else if (reach && goal) { end = true; hit = true; }
+        else if (step >= max_steps) end = true;
 
         if (!end && chan > 0) {
             // pending broadcast receivers (SyncInSerial simulation.cu:357-407)
             bool entered = false;
-            fire_receivers<C, TRACE, TRACE>(words, scr, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, p.seed, run,
+            fire_receivers<C, TRACE, TRACE>(words, scr, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, seed, run,
                                             step, lane, sl, S, seg_base, seg_mask, trans, digest);
             changed = true;
             chan = 0;
@@ -191,7 +229,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
         // by this iteration's receivers counts only if this step, raced by
         // every component, keeps t < bound (simulation.cu:409-415, 835-849):
         // no absorption exit and no left-out null racers then.
-        const bool full = p.reach && goal;
+        const bool full = reach && goal;
         // with frozen racers the race itself ends a run that nothing can
         // leave (no event: blocked racers are out, the rest race at rate 0),
         // so the scan is needed only without them
@@ -228,7 +266,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                 for (uint32_t b = rs.bounded; b;) {
                     const int j = __ffs(b) - 1;
                     const uint32_t c = (uint32_t)(sl * C + j);
-                    const smc_u32x4 rw = smc_draw(p.seed, run, step, SMC_P_UNIFORM, smc_uniform_draw(c));
+                    const smc_u32x4 rw = draw(seed, run, step, SMC_P_UNIFORM, smc_uniform_draw(c));
                     const double du = scr[64 * j] * smc_uniform_u(rw, c);
                     if (du < umin) { umin = du; unif_j = j; }
                     b &= b - 1;
@@ -242,7 +280,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                 double dexp = INF;
                 int wexp = 0x7FFFFFFF;
                 if (R > 0.0) {
-                    const smc_u32x4 rw = smc_draw(p.seed, run, step, SMC_P_RACE, 0);
+                    const smc_u32x4 rw = draw(seed, run, step, SMC_P_RACE, 0);
                     dexp = -smc_log2(smc_u01(rw.v[0], rw.v[1])) / R;
                     wexp = race_pick<C>(rs.leaf, scr, smc_u01(rw.v[2], rw.v[3]) * R, S, sl, seg_base, seg_mask);
                 }
@@ -262,15 +300,15 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                 else d = INF;  // no racer: no event
                 // the step that crosses the bound: the left-out null racers'
                 // first event after the bound may come first
-                if (m.freeze && !full && d < INF && !(t + d < p.bound)) {
+                if (m.freeze && !full && d < INF && !(t + d < bound)) {
                     const uint32_t fz = frozen_rates<C>(words, scr, Ctx{vars, t, 0}, m);
                     double dl[C];
 #pragma unroll
                     for (int j = 0; j < C; ++j) dl[j] = ((fz >> j) & 1u) ? scr[64 * j] : 0.0;
                     const double Rd = tree_total<C>(dl, S);
                     if (Rd > 0.0) {
-                        const smc_u32x4 rw = smc_draw(p.seed, run, step, SMC_P_DEAD, 0);
-                        const double td = p.bound + (-smc_log2(smc_u01(rw.v[0], rw.v[1])) / Rd);
+                        const smc_u32x4 rw = draw(seed, run, step, SMC_P_DEAD, 0);
+                        const double td = bound + (-smc_log2(smc_u01(rw.v[0], rw.v[1])) / Rd);
                         if (td < t + d) { d = td - t; w = -1; }
                     }
                 }
@@ -297,7 +335,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                         mask |= ((__ballot(en) >> seg_base) & seg_ones) << i0;
                     }
                     if (mask) {
-                        const int i = pick_edge(mask, first, p.seed, run, step, (uint32_t)w, x, m);
+                        const int i = pick_edge(mask, first, seed, run, step, (uint32_t)w, x, m);
                         const DevEdge E = load_rec(m.edges + first + i);
                         run_updates(E, x, m, q);
                         *slot = (E.dst_rec << m.rec_shift) | x.base;
@@ -331,26 +369,27 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                     qmin = fmin(qmin, seg_xchg(qmin, k));
                     fired += (uint32_t)__shfl_xor((int)fired, 1 << k);
                 }
-            const double value = p.is_max ? qmax : qmin;
+            const SMC_CONSTANT InstDesc *I = opaque(inst);
+            const double value = I->p.is_max ? qmax : qmin;
             if (TRACE) {
                 digest = smc_mix(digest, smc_digest_bits(t));
-                for (int v = 0; v < m.n_vars; ++v)
-                    digest = smc_mix(digest, smc_digest_bits(m.var_clock[v] ? t - vars[v] : vars[v]));
-                for (int c = 0; c < n; ++c) {
+                for (int v = 0; v < I->m.n_vars; ++v)
+                    digest = smc_mix(digest, smc_digest_bits(I->m.var_clock[v] ? t - vars[v] : vars[v]));
+                for (int c = 0; c < I->m.n_comp; ++c) {
                     const int lv = ((int32_t *)words_of)[64 * C + (c % C) * 64 + seg_base + c / C];
                     digest = smc_mix(digest, (uint64_t)(uint32_t)lv);
                 }
             }
             if (sl == 0) {
                 uint8_t flag;
-                if (p.reach) flag = hit ? 1 : 0;
-                else flag = p.is_max ? (value > p.threshold) : (value < p.threshold);
-                p.flag[ridx] = flag;
-                p.value[ridx] = value;
-                p.steps[ridx] = step;
-                p.trans[ridx] = fired;
-                if (p.time) p.time[ridx] = t;
-                if (TRACE && p.digest) p.digest[ridx] = digest;
+                if (reach) flag = hit ? 1 : 0;
+                else flag = I->p.is_max ? (value > I->p.threshold) : (value < I->p.threshold);
+                I->p.flag[ridx] = flag;
+                I->p.value[ridx] = value;
+                I->p.steps[ridx] = step;
+                I->p.trans[ridx] = fired;
+                if (I->p.time) I->p.time[ridx] = t;
+                if (TRACE && I->p.digest) I->p.digest[ridx] = digest;
             }
             wave_sync();
             active = false;
