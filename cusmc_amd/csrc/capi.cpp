@@ -315,6 +315,7 @@ int smc_model_create(const smc_network *net, int device, smc_model **out) {
         d.rec_shift = im.rec_shift;
         d.base_mask = (1u << im.rec_shift) - 1u;
         d.tests = im.tests;
+        d.one_rate = im.one_rate;
         d.freeze = im.freeze ? 1 : 0;
         hip_check(hipMalloc(&m->d_inst, sizeof(InstDesc)), "hipMalloc instance");
         hip_check(hipMalloc(&m->d_counter, sizeof(unsigned long long)), "hipMalloc counter");

@@ -268,6 +268,41 @@ struct RawLoc {
     std::vector<DevGuard> block;
 };
 
+// A record's variable operand as a byte offset and its local factor.
+void inline_var(uint16_t v, uint16_t *offset, uint16_t *flags) {
+    *offset = (uint16_t)((v & ~SMC_VAR_LOCAL) * 8u);
+    *flags = (uint16_t)(*flags | ((v & SMC_VAR_LOCAL) ? 8 : 0));
+}
+
+// Move an edge's first constant guard and its leading plain updates (at most
+// two) into its record.
+void inline_edge(RawEdge &re) {
+    DevEdge &e = re.e;
+    e.flags |= SMC_EF_NO_GUARD;
+    for (size_t k = 0; k < re.guards.size(); ++k) {
+        const DevGuard G = re.guards[k];
+        if (!(G.flags & SMC_GF_RANGE)) continue;
+        e.flags &= ~(uint32_t)SMC_EF_NO_GUARD;
+        e.lo = G.lo;
+        e.hi = G.hi;
+        if (G.flags & SMC_GF_CLOCK) e.g_flags |= SMC_EG_CLOCK;
+        inline_var(G.var, &e.g_var, &e.g_flags);
+        re.guards.erase(re.guards.begin() + k);
+        break;
+    }
+    size_t u = 0;
+    for (; u < 2 && u < re.upds.size() && re.upds[u].kind != SMC_U_EXPR; ++u) {
+        const DevUpd &U = re.upds[u];
+        uint16_t &var = u ? e.u1_var : e.u0_var, &flags = u ? e.u1_flags : e.u0_flags;
+        (u ? e.u1_value : e.u0_value) = U.value;
+        flags |= (uint16_t)((U.kind == SMC_U_ADD ? SMC_EU_ADD : SMC_EU_SET) | (U.clock ? SMC_EU_CLOCK : 0));
+        inline_var(U.var, &var, &flags);
+    }
+    re.upds.erase(re.upds.begin(), re.upds.begin() + u);
+    e.guard_n = (uint16_t)re.guards.size();
+    e.upd_n = (uint16_t)re.upds.size();
+}
+
 // Partition of the locations into classes of equal records: first by their
 // own content, then, until nothing splits, by the classes their edges lead
 // to.  Networks whose classes take long to separate (chains of equal
@@ -415,6 +450,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
         if (reads_clock(n.locations[l].rate)) clock_rate = true;
     img.freeze = !clock_rate;
 
+    int n_rates = 0;  // distinct rate expressions (2: several, or one that reads private variables)
     std::vector<RawLoc> raw(n.n_locations);
     img.info.resize(n.n_locations);
     img.loc_edge0.assign(n.n_locations, 0);
@@ -474,11 +510,11 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                     e.weight = w > 0 ? (uint32_t)w : 0u;
                     e.flags |= SMC_EF_WEIGHT_CONST;
                 }
-                e.dst_goal = n.locations[E.dst].type == SMC_LOC_GOAL;
+                if (n.locations[E.dst].type == SMC_LOC_GOAL) e.flags |= SMC_EF_GOAL;
                 for (int g = 0; g < E.guard_count; ++g) {
                     const smc_constraint &C = n.constraints[E.guard_first + g];
                     if (!C.uses_variable) continue;
-                    if (C.op == SMC_C_NE) { e.never = 1; continue; }
+                    if (C.op == SMC_C_NE) { e.flags |= SMC_EF_NEVER; continue; }
                     if (C.var > 65535) throw std::runtime_error("limit: guarded variable index above 65535");
                     DevGuard G{};
                     G.var = lw.field(C.var);
@@ -493,7 +529,6 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                     re.guards.push_back(G);
                 }
                 if (re.guards.size() > 65535) throw std::runtime_error("limit: more than 65535 guards on an edge");
-                e.guard_n = (uint16_t)re.guards.size();
                 for (int k2 = 0; k2 < E.upd_count; ++k2) {
                     const smc_update &U = n.updates[E.upd_first + k2];
                     if (U.var > 65535) throw std::runtime_error("limit: assigned variable index above 65535");
@@ -507,7 +542,6 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                     re.upds.push_back(u);
                 }
                 if (E.upd_count > 65535) throw std::runtime_error("limit: more than 65535 updates on an edge");
-                e.upd_n = (uint16_t)E.upd_count;
                 R.edges.push_back(std::move(re));
             }
 
@@ -546,7 +580,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
             if (kind == 2) {
                 // the blocking test: clock-free conjuncts, edge after edge
                 for (const RawEdge &re : R.edges) {
-                    if (re.e.channel < 0 || re.e.never) continue;
+                    if (re.e.channel < 0 || (re.e.flags & SMC_EF_NEVER)) continue;
                     const size_t first = R.block.size();
                     for (const DevGuard &G : re.guards)
                         if (G.flags & SMC_GF_CLOCK_FREE) R.block.push_back(G);
@@ -577,7 +611,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                     seen.push_back(U.var);
                 }
                 if (k >= 32) fast = false;
-                if (re.e.never || re.e.guard_n || (chan && chan != -E.channel)) plain_recv = false;
+                if ((re.e.flags & SMC_EF_NEVER) || !re.guards.empty() || (chan && chan != -E.channel)) plain_recv = false;
                 chan = -E.channel;
                 if (k < 32) d.recv_mask |= 1u << k;
                 if (n_recv++ == 0) d.recv_low = re.e.weight;
@@ -593,14 +627,24 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                 d.recv_chan = -1;
                 d.recv_mask = 0;
             }
-            if (!(d.flags & SMC_LF_RECV_TWO)) d.recv_low = 0;
+            if (!(d.flags & SMC_LF_RECV_TWO)) d.recv_low = 0xFFFFFFFFu;
+
+            // spontaneous edges with constant weights
+            int64_t pick_sum = 0;
+            bool pick = true;
+            for (int k = 0; k < L.edge_count; ++k) {
+                const RawEdge &re = R.edges[k];
+                if (re.e.channel < 0) continue;
+                if (k >= 32 || !(re.e.flags & SMC_EF_WEIGHT_CONST)) { pick = false; break; }
+                d.pick_mask |= 1u << k;
+                pick_sum += re.e.weight;
+            }
+            if (!pick || pick_sum >= 2147483648ll) d.pick_mask = 0;
+            if (d.pick_mask) d.pick_weight = (uint32_t)pick_sum;
 
             // what a race step looks at
             DevHot &h = R.hot;
-            auto hot_var = [&](uint16_t v) {
-                h.var = (uint16_t)((v & ~SMC_VAR_LOCAL) * 8u);
-                if (v & SMC_VAR_LOCAL) h.flags |= 8;
-            };
+            auto hot_var = [&](uint16_t v) { inline_var(v, &h.var, &h.flags); };
             if (d.klass == SMC_K_ZERO) {
                 h.flags = SMC_HF_ZERO;
             } else {
@@ -611,6 +655,9 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                 } else {
                     h.flags |= SMC_HF_EXPR | (reads_local(L.rate) ? SMC_HF_EXPR_LOCAL : 0);
                     h.rate_ref = d.rate;
+                    if ((h.flags & SMC_HF_EXPR_LOCAL) || (n_rates && img.one_rate != d.rate)) n_rates = 2;
+                    else n_rates = std::max(n_rates, 1);
+                    img.one_rate = d.rate;
                 }
                 if (d.n_inv == 1 && R.invs[0].bound_const) {
                     h.flags |= SMC_HF_INV;
@@ -631,9 +678,12 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                     }
                 }
             }
+            for (RawEdge &re : R.edges) inline_edge(re);
             img.tests |= h.flags & ~(uint32_t)SMC_HF_LOCAL;
         }
     }
+
+    if (n_rates != 1) img.one_rate = SMC_NO_REF;
 
     // classes of equal locations, and their records; record 0 is a slot
     // without a component (no edge, rate 0)

@@ -38,6 +38,7 @@ struct ModelImage {
     int n_comp = 0, n_vars = 0, n_leaves = 1;
     int rec_shift = 13;
     uint32_t tests = 0;   // every SMC_HF_* flag in use
+    uint32_t one_rate = SMC_NO_REF;  // the one rate expression, if there is just one
     bool freeze = true;   // no location's rate reads a clock
 };
 

@@ -38,11 +38,67 @@ __device__ __forceinline__ int lane_here(int v) {
     return v;
 }
 
+// Whether any active lane has c: a wave-uniform condition, so what it guards
+// is branched around as a whole, and with `unlikely` laid out away from the
+// straight path.  A branch on a lane's own condition is taken whenever no
+// lane needs the code, and with few waves on a SIMD the taken branches, not
+// the instructions, are a step's latency (a step of the race took 336 of
+// them).
+__device__ __forceinline__ bool any_lane(bool c) { return __ballot(c) != 0; }
+#define unlikely(c) __builtin_expect(!!(c), 0)
+
+__device__ __forceinline__ double scalar_here(double v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+// smc_log2 (the same operations in the same order) with its coefficients in
+// scalar registers, where the compiler would move each into vector registers
+// beside every multiply-add, and with the quotient's refinement written out:
+// numerator and denominator are far from the ranges that the full division
+// sequence scales and fixes up, and without those the steps are its own.
+__device__ __forceinline__ double device_log2(double x) {
+    const uint64_t b = smc_bits(x);
+    int e = (int)((b >> 52) & 0x7FF) - 1023;
+    double m = smc_from_bits((b & 0x000FFFFFFFFFFFFFull) | 0x3FF0000000000000ull);
+    const bool high = m > 1.4142135623730951;
+    m = high ? m * 0.5 : m;
+    e += high ? 1 : 0;
+    const double n = m - 1.0, d = m + 1.0;
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(r, fma(-d, r, 1.0), r);
+    r = fma(r, fma(-d, r, 1.0), r);
+    const double q = n * r;
+    const double s = fma(fma(-d, q, n), r, q);
+    const double z = s * s;
+    double p = scalar_here(1.0 / 23.0);
+    p = fma(p, z, scalar_here(1.0 / 21.0));
+    p = fma(p, z, scalar_here(1.0 / 19.0));
+    p = fma(p, z, scalar_here(1.0 / 17.0));
+    p = fma(p, z, scalar_here(1.0 / 15.0));
+    p = fma(p, z, scalar_here(1.0 / 13.0));
+    p = fma(p, z, scalar_here(1.0 / 11.0));
+    p = fma(p, z, scalar_here(1.0 / 9.0));
+    p = fma(p, z, scalar_here(1.0 / 7.0));
+    p = fma(p, z, scalar_here(1.0 / 5.0));
+    p = fma(p, z, scalar_here(1.0 / 3.0));
+    p = fma(p, z, 1.0);
+    const double ln_m = (2.0 * s) * p;
+    return fma(ln_m, scalar_here(1.4426950408889634074), (double)e);
+}
+
 // smc_draw with the key schedule computed at the draw (scalar adds beside
 // the rounds).
 __device__ __forceinline__ smc_u32x4 draw(uint64_t seed, uint64_t run, uint32_t step, uint32_t purpose,
                                           uint32_t comp) {
     return smc_draw(scalar_here(seed), run, step, purpose, comp);
+}
+
+// The same addressed by the counter's second word, (purpose << 24) | index.
+__device__ __forceinline__ smc_u32x4 draw_at(uint64_t seed, uint64_t run, uint32_t step, uint32_t where) {
+    seed = scalar_here(seed);
+    const smc_u32x4 ctr = {{step, where, (uint32_t)run, (uint32_t)(run >> 32)}};
+    return smc_philox4x32_10(ctr, (uint32_t)seed, (uint32_t)(seed >> 32));
 }
 
 // ------------------------------------------------------------ segment exchange
@@ -151,17 +207,37 @@ __device__ __forceinline__ T load_rec(const SMC_LDS T *p) {
 }
 #endif
 
-// The first 16 bytes of a record.
+// 16 bytes of a record, and an edge's guard interval.
 template <class T>
-__device__ __forceinline__ uint4 load_quad(const SMC_GLOBAL T *p) {
-    return load_rec((const SMC_GLOBAL uint4 *)p);
+__device__ __forceinline__ uint4 load_quad(const SMC_GLOBAL T *p, int i) {
+    return load_rec((const SMC_GLOBAL uint4 *)p + i);
+}
+struct DevRange { double lo, hi; };
+__device__ __forceinline__ DevRange load_range(const SMC_GLOBAL DevEdge *p) {
+    return load_rec((const SMC_GLOBAL DevRange *)p + 1);
 }
 #if defined(__HIP_DEVICE_COMPILE__)
 template <class T>
-__device__ __forceinline__ uint4 load_quad(const SMC_LDS T *p) {
-    return load_rec((const SMC_LDS uint4 *)p);
+__device__ __forceinline__ uint4 load_quad(const SMC_LDS T *p, int i) {
+    return load_rec((const SMC_LDS uint4 *)p + i);
+}
+__device__ __forceinline__ DevRange load_range(const SMC_LDS DevEdge *p) {
+    return load_rec((const SMC_LDS DevRange *)p + 1);
 }
 #endif
+// Record i of a table.  24-bit products: a full-rate instruction, where the
+// 32-bit multiply of an index is a quarter-rate one.
+template <class T>
+__device__ __forceinline__ const SMC_GLOBAL T *rec_at(const SMC_GLOBAL T *p, uint32_t i) {
+    return (const SMC_GLOBAL T *)((const SMC_GLOBAL char *)p + __umul24(i, (uint32_t)sizeof(T)));
+}
+#if defined(__HIP_DEVICE_COMPILE__)
+template <class T>
+__device__ __forceinline__ const SMC_LDS T *rec_at(const SMC_LDS T *p, uint32_t i) {
+    return (const SMC_LDS T *)((const SMC_LDS char *)p + __umul24(i, (uint32_t)sizeof(T)));
+}
+#endif
+__device__ __forceinline__ double quad_f64(const uint4 &q) { return __hiloint2double((int)q.y, (int)q.x); }
 
 // Table pointer of the global arena rebased onto its LDS copy.
 template <class T>
@@ -223,6 +299,7 @@ __device__ __forceinline__ DevModelT<SmcLdsTables> lds_model(const DevModel &mg,
     m.rec_shift = mg.rec_shift;
     m.base_mask = mg.base_mask;
     m.tests = mg.tests;
+    m.one_rate = mg.one_rate;
     m.freeze = mg.freeze;
     return m;
 }
@@ -306,6 +383,45 @@ __device__ __forceinline__ double location_rate(const DevLoc &L, const Ctx &x, c
     return r > 0.0 ? r : 0.0;
 }
 
+// The value of a reference that is the same for every lane and reads no
+// private variable: the instructions are decoded in scalar registers.
+template <class M>
+__device__ __forceinline__ double eval_uniform(uint32_t ref, const Ctx &x, const M &m) {
+    if ((ref >> 30) != SMC_REF_CODE) return eval_ref(ref, x, m);
+    const uint32_t first = ref & 0xFFFFFFu, count = (ref >> 24) & 0x3Fu;
+    double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0;
+#pragma clang loop unroll(disable)
+    for (uint32_t k = 0; k < count; ++k) {
+        const DevInsn in = load_rec(m.code + first + k);
+        uint32_t lo, hi;
+        __builtin_memcpy(&lo, &in, 4);
+        __builtin_memcpy(&hi, (const char *)&in + 4, 4);
+        lo = __builtin_amdgcn_readfirstlane(lo);
+        hi = __builtin_amdgcn_readfirstlane(hi);
+        auto operand = [&](uint32_t w) {
+            const uint32_t kind = w >> 14, i = w & 0x3FFFu;
+            if (kind == SMC_OPND_REG) return i == 0 ? r0 : i == 1 ? r1 : i == 2 ? r2 : r3;
+            if (kind == SMC_OPND_CONST) return (double)m.consts[i];
+            const double v = x.vars[i];
+            return kind == SMC_OPND_CLOCK ? x.now - v : v;
+        };
+        const int op = (int)(lo & 0xFFu);
+        const uint32_t dst = (lo >> 8) & 0xFFu;
+        const double a = operand(lo >> 16), b = operand(hi & 0xFFFFu);
+        double v;
+        if (op == SMC_E_ADD) v = a + b;
+        else if (op == SMC_E_SUB) v = a - b;
+        else if (op == SMC_E_MUL) v = a * b;
+        else if (op == SMC_E_DIV) v = a / b;
+        else v = rare_op(op, a, b, operand(hi >> 16));
+        if (dst == 0) r0 = v;
+        else if (dst == 1) r1 = v;
+        else if (dst == 2) r2 = v;
+        else r3 = v;
+    }
+    return r0;
+}
+
 // ------------------------------------------------------------ slots
 //
 // A lane's component slots are state words in LDS ([slot][lane]: 64 lanes
@@ -334,20 +450,38 @@ template <class M>
 __device__ __forceinline__ bool guard_true(const DevGuard &G, const Ctx &x, const M &m) {
     double v = x.vars[var_at(G.var, x.base)];
     if (G.flags & SMC_GF_CLOCK) v = x.now - v;
-    if (G.flags & SMC_GF_RANGE) return G.lo <= v && v <= G.hi;
-    return guard_holds(G.op, v, eval_ref(G.rhs, x, m));
+    bool ok = G.lo <= v && v <= G.hi;
+    const bool general = !(G.flags & SMC_GF_RANGE);
+    if (unlikely(any_lane(general))) {
+        if (general) ok = guard_holds(G.op, v, eval_ref(G.rhs, x, m));
+    }
+    return ok;
+}
+
+// A variable named by a byte offset and a factor (8 or 0) of the base.
+__device__ __forceinline__ double *var_ptr(const Ctx &x, uint32_t offset, uint32_t flags) {
+    return (double *)((char *)x.vars + offset + __umul24(x.base, flags & 0xFFu));
 }
 
 // Whether edge record e is enabled: spontaneous (recv_chan == 0) or a
 // receive edge on channel recv_chan (check_enabled_edges
-// simulation.cu:268-305, SyncInSerial :363-377).
+// simulation.cu:268-305, SyncInSerial :363-377).  `here`: the lane has an
+// edge to test (others read a valid record all the same).
 template <class M>
-__device__ __forceinline__ bool edge_enabled(uint32_t e, int recv_chan, const Ctx &x, const M &m) {
-    const DevEdge E = load_rec(m.edges + e);
-    if (E.never || (recv_chan ? E.channel != -recv_chan : E.channel < 0)) return false;
-    bool ok = true;
+__device__ __forceinline__ bool edge_enabled(bool here, uint32_t e, int recv_chan, const Ctx &x, const M &m) {
+    const uint4 head = load_quad(rec_at(m.edges, e), 0), tail = load_quad(rec_at(m.edges, e), 2);
+    const DevRange range = load_range(rec_at(m.edges, e));
+    const int channel = (int)head.w;
+    double v = *var_ptr(x, tail.x & 0xFFFFu, tail.x >> 16);
+    v = (tail.x & (SMC_EG_CLOCK << 16)) ? x.now - v : v;
+    bool ok = here & !(head.y & SMC_EF_NEVER) & (recv_chan ? channel == -recv_chan : channel >= 0) &
+              (((head.y & SMC_EF_NO_GUARD) != 0) | ((range.lo <= v) & (v <= range.hi)));
+    const int more = (int)(tail.z & 0xFFFFu);  // guard_n
+    if (any_lane(ok && more)) {
 #pragma clang loop unroll(disable)
-    for (int g = 0; g < E.guard_n && ok; ++g) ok = guard_true(load_rec(m.guards + E.guard_first + g), x, m);
+        for (int g = 0; any_lane(ok && g < more); ++g)
+            if (ok && g < more) ok = guard_true(load_rec(rec_at(m.guards, tail.y + g)), x, m);
+    }
     return ok;
 }
 
@@ -358,16 +492,39 @@ __device__ __forceinline__ uint64_t enabled_mask(uint32_t edge_first, int edge_n
     uint64_t mask = 0;
 #pragma clang loop unroll(disable)
     for (int i = 0; i < edge_n; ++i)
-        if (edge_enabled(edge_first + i, recv_chan, x, m)) mask |= 1ull << i;
+        if (edge_enabled(true, edge_first + i, recv_chan, x, m)) mask |= 1ull << i;
+    return mask;
+}
+
+// The same for spontaneous edges by all S lanes of a segment, each testing
+// one edge at a time.
+template <class M>
+__device__ __forceinline__ uint64_t enabled_mask_by_lanes(uint32_t edge_first, int edge_n, const Ctx &x, const M &m,
+                                                          int S, int sl, int seg_base, uint64_t seg_ones) {
+    uint64_t mask = 0;
+    int i0 = 0;
+#pragma clang loop unroll(disable)
+    do {
+        const bool here = i0 + sl < edge_n;
+        const bool ok = edge_enabled(here, edge_first + (here ? i0 + sl : 0), 0, x, m);
+        mask |= ((__ballot(ok) >> seg_base) & seg_ones) << (i0 & 63);
+        i0 += S;
+    } while (any_lane(i0 < edge_n));
     return mask;
 }
 
 template <class M>
 __device__ __forceinline__ long long edge_weight(uint32_t e, const Ctx &x, const M &m) {
-    const uint32_t w = m.edges[e].weight;
-    if (m.edges[e].flags & SMC_EF_WEIGHT_CONST) return (long long)w;
-    const int v = smc_to_int(eval_ref(w, x, m));
-    return v > 0 ? v : 0;
+    const uint4 head = load_quad(rec_at(m.edges, e), 0);
+    long long w = (long long)head.z;
+    const bool general = !(head.y & SMC_EF_WEIGHT_CONST);
+    if (unlikely(any_lane(general))) {
+        if (general) {
+            const int v = smc_to_int(eval_ref(head.z, x, m));
+            w = v > 0 ? v : 0;
+        }
+    }
+    return w;
 }
 
 // Weighted choice among the edges in mask (two or more) for the uniform u
@@ -403,13 +560,39 @@ __device__ __forceinline__ int pick_weighted(uint64_t mask, uint32_t edge_first,
 }
 
 // Weighted choice among the enabled edges in mask; the draw is made only
-// when there is a choice.
+// when there is a choice.  With all of the location's spontaneous edges
+// enabled and their weights constant (full, total: DevLoc.pick_*), the sum is
+// known and one upward pass over the edges finds the last whose lower
+// neighbours' weights do not exceed the draw.
 template <class M>
-__device__ __forceinline__ int pick_edge(uint64_t mask, uint32_t edge_first, uint64_t seed, uint64_t run,
-                                         uint32_t step, uint32_t comp, const Ctx &x, const M &m) {
-    if ((mask & (mask - 1)) == 0) return lowest_lane(mask);
-    const smc_u32x4 w = draw(seed, run, step, SMC_P_WINNER, comp);
-    return pick_weighted(mask, edge_first, smc_u01(w.v[0], w.v[1]), x, m);
+__device__ __forceinline__ int pick_edge(uint64_t mask, uint32_t edge_first, uint32_t full, uint32_t total,
+                                         uint64_t seed, uint64_t run, uint32_t step, uint32_t comp, const Ctx &x,
+                                         const M &m) {
+    int i = lowest_lane(mask);
+    const bool choice = (mask & (mask - 1)) != 0;
+    if (any_lane(choice)) {
+        const smc_u32x4 w = draw(seed, run, step, SMC_P_WINNER, comp);
+        const double u = smc_u01(w.v[0], w.v[1]);
+        const bool quick = choice & (mask == (uint64_t)full);
+        if (any_lane(quick)) {
+            const int rnd = (int)((double)total * u);
+            uint32_t r = quick ? full : 0u;
+            int below = 0;
+#pragma clang loop unroll(disable)
+            do {
+                const int k = r ? __ffs(r) - 1 : 0;
+                const int wk = (int)rec_at(m.edges, edge_first + k)->weight;
+                i = (r && below <= rnd) ? k : i;
+                below += wk;
+                r &= r - 1;
+            } while (any_lane(r != 0));
+        }
+        const bool slow = choice & !quick;
+        if (any_lane(slow)) {
+            if (slow) i = pick_weighted(mask, edge_first, u, x, m);
+        }
+    }
+    return i;
 }
 
 // The same for component c as a broadcast receiver: its uniform is word
@@ -427,24 +610,54 @@ struct LaneQuery {
     double qmax, qmin;
 };
 
-// The updates of an edge in order, with query variable tracking
-// (take_transition simulation.cu:88-180).  Any number of lanes may run it
-// for the same component at once: they store the same values.
-template <class M>
-__device__ __forceinline__ void run_updates(const DevEdge &E, const Ctx &x, const M &m, LaneQuery &q) {
-#pragma clang loop unroll(disable)
-    for (int k = 0; k < E.upd_n; ++k) {
-        const DevUpd U = load_rec(m.upds + E.upd_first + k);
-        const uint32_t at = var_at(U.var, x.base);
-        double v = U.value;
-        if (U.kind == SMC_U_ADD) v = x.vars[at] + v;
-        else if (U.kind == SMC_U_EXPR) v = eval_ref(U.expr, x, m);
-        if ((int)at == q.qvar) {
-            if (v > q.qmax) q.qmax = v;
-            if (v < q.qmin) q.qmin = v;
+// One plain update (value, variable and flags as in DevEdge), with query
+// variable tracking.
+__device__ __forceinline__ void plain_update(double value, uint32_t var_flags, const Ctx &x, LaneQuery &q) {
+    const uint32_t flags = var_flags >> 16;
+    double *at = var_ptr(x, var_flags & 0xFFFFu, flags);
+    double v = value;
+    if (flags & SMC_EU_ADD) v = *at + v;
+    if (flags & (SMC_EU_ADD | SMC_EU_SET)) {
+        if (at == x.vars + q.qvar) {
+            q.qmax = v > q.qmax ? v : q.qmax;
+            q.qmin = v < q.qmin ? v : q.qmin;
         }
-        x.vars[at] = U.clock ? x.now - v : v;
+        *at = (flags & SMC_EU_CLOCK) ? x.now - v : v;
     }
+}
+
+// The updates of edge record e in order (take_transition
+// simulation.cu:88-180).  Any number of lanes may run it for the same
+// component at once: they store the same values.  Returns the record's first
+// 16 bytes.
+template <class M>
+__device__ __forceinline__ uint4 fire_updates(uint32_t e, const Ctx &x, const M &m, LaneQuery &q) {
+    const uint4 head = load_quad(rec_at(m.edges, e), 0), more = load_quad(rec_at(m.edges, e), 2);
+    const uint4 u0 = load_quad(rec_at(m.edges, e), 3), u1 = load_quad(rec_at(m.edges, e), 4);
+    plain_update(quad_f64(u0), u0.z, x, q);
+    plain_update(quad_f64(u1), u1.z, x, q);
+    const int n = (int)(more.z >> 16);  // upd_n
+    if (any_lane(n != 0)) {
+#pragma clang loop unroll(disable)
+        for (int k = 0; any_lane(k < n); ++k) {
+            if (k < n) {
+                const DevUpd U = load_rec(m.upds + more.w + k);
+                const uint32_t at = var_at(U.var, x.base);
+                double v = U.value;
+                if (U.kind == SMC_U_ADD) v = x.vars[at] + v;
+                const bool general = U.kind == SMC_U_EXPR;
+                if (any_lane(general)) {
+                    if (general) v = eval_ref(U.expr, x, m);
+                }
+                if ((int)at == q.qvar) {
+                    if (v > q.qmax) q.qmax = v;
+                    if (v < q.qmin) q.qmin = v;
+                }
+                x.vars[at] = U.clock ? x.now - v : v;
+            }
+        }
+    }
+    return head;
 }
 
 // ------------------------------------------------------------ blocking
@@ -459,7 +672,7 @@ __device__ __forceinline__ bool location_blocked(uint32_t block_first, const Ctx
     bool e_blk = false;
 #pragma clang loop unroll(disable)
     for (uint32_t k = block_first;; ++k) {
-        const DevGuard G = load_rec(m.guards + k);
+        const DevGuard G = load_rec(rec_at(m.guards, k));
         if (!e_blk) e_blk = !guard_true(G, x, m);
         if (G.flags & SMC_GF_END_EDGE) {
             if (!e_blk) return false;
@@ -555,8 +768,17 @@ template <int C, class M>
 __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *words, double *scr, Ctx x, const M &m,
                                            bool changed, uint32_t &xblk) {
     const uint32_t tests = m.tests;
-    uint32_t bounded = 0, zero = 0, expr = 0, own = 0;
+    uint32_t bounded = 0, zero = 0;
+    uint32_t expr = 0;     // slots whose rate is still to be evaluated
+    uint32_t own = 0;
     uint32_t ref[C];
+    // a network with one rate expression: evaluated once, for every slot
+    const bool one = m.one_rate != SMC_NO_REF;
+    double shared = 0.0;
+    if (one) {
+        shared = eval_uniform(m.one_rate, x, m);
+        shared = shared > 0.0 ? shared : 0.0;
+    }
     auto flag = [](uint32_t d, uint32_t f, uint32_t bit) { return (d & (f << 16)) ? bit : 0u; };
     if (tests & (SMC_HF_INV | SMC_HF_GUARD)) {
         DevHot h[C];
@@ -570,7 +792,7 @@ __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *wor
         }
 #pragma unroll
         for (int j = 0; j < C; ++j)
-            v[j] = *(const double *)((const char *)x.vars + h[j].var + base[j] * (h[j].flags & SMC_HF_LOCAL));
+            v[j] = *(const double *)((const char *)x.vars + h[j].var + __umul24(base[j], h[j].flags & SMC_HF_LOCAL));
 #pragma unroll
         for (int j = 0; j < C; ++j) {
             const uint32_t bit = 1u << j, d = (uint32_t)h[j].flags << 16;
@@ -582,7 +804,8 @@ __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *wor
             bounded |= bnd ? bit : 0u;
             zero |= (bnd & (left == 0.0)) ? bit : 0u;
             zero |= flag(d, SMC_HF_ZERO, bit);
-            rs.leaf[j] = in ? h[j].rate : 0.0;
+            const double rate = (d & (SMC_HF_EXPR << 16)) ? shared : h[j].rate;
+            rs.leaf[j] = in ? rate : 0.0;
             ref[j] = h[j].rate_ref;
             expr |= in ? flag(d, SMC_HF_EXPR, bit) : 0u;
             own |= flag(d, SMC_HF_EXPR_LOCAL, bit);
@@ -595,7 +818,7 @@ __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *wor
         for (int j = 0; j < C; ++j) {
             const uint32_t bit = 1u << j, d = (uint32_t)h[j].flags << 16;
             zero |= flag(d, SMC_HF_ZERO, bit);
-            rs.leaf[j] = h[j].rate;
+            rs.leaf[j] = (d & (SMC_HF_EXPR << 16)) ? shared : h[j].rate;
             ref[j] = h[j].rate_ref;
             expr |= flag(d, SMC_HF_EXPR, bit);
             own |= flag(d, SMC_HF_EXPR_LOCAL, bit);
@@ -636,7 +859,7 @@ __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *wor
     // component's own variables).  Evaluated slot by slot, the interpreter
     // would run up to C times per race; here once per distinct expression a
     // lane holds.
-    if (tests & SMC_HF_EXPR) {
+    if ((tests & SMC_HF_EXPR) && !one) {
         while (__ballot(expr != 0)) {
             double v = 0.0;
             uint32_t r = 0xFFFFFFFFu, first = 0;
@@ -672,12 +895,12 @@ __device__ __forceinline__ double race_total(const double (&leaf)[C], double *le
 #pragma unroll
     for (int i = C - 1; i >= 1; --i) tr[i] = tr[2 * i] + tr[2 * i + 1];
     double s = (C == 1) ? leaf[0] : tr[1];
+    // one way out of the levels, taken once
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-        if ((1 << k) < S) {
-            level[64 * k] = s;
-            s = s + seg_xchg(s, k);
-        }
+        if ((1 << k) >= S) break;
+        level[64 * k] = s;
+        s = s + seg_xchg(s, k);
     }
     return s;
 }
@@ -748,18 +971,24 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int
                                                int sender, LaneQuery &q, bool &goal, uint64_t seed, uint64_t run,
                                                uint32_t step, int lane, int sl, int S, int seg_base, uint64_t seg_mask,
                                                uint32_t &trans, uint64_t &digest) {
+    // the enabled receive edges of every slot but the sender's: one bit set
+    // each, from its location's record where they are all unguarded on one
+    // channel
     uint32_t mk[C];
-    uint32_t other = 0;  // slots whose receive edges are not all unguarded on one channel
+    uint32_t other = 0;
+    {
+        uint4 rv[C];  // recv_chan, recv_mask, ...
 #pragma unroll
-    for (int j = 0; j < C; ++j) {
-        const uint32_t w = words[64 * j];
-        const uint4 rv = load_quad(m.locs + word_rec(w, m));  // recv_chan, recv_mask, ...
-        const bool me = sl * C + j == sender;
-        mk[j] = ((int)rv.x == chan && !me) ? rv.y : 0u;
-        if ((int)rv.x == -1 && !me) other |= 1u << j;
+        for (int j = 0; j < C; ++j) rv[j] = load_quad(m.locs + word_rec(words[64 * j], m), 0);
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            const bool me = sl * C + j == sender;
+            mk[j] = (((int)rv[j].x == chan) & !me) ? rv[j].y : 0u;
+            other |= (((int)rv[j].x == -1) & !me) ? 1u << j : 0u;
+        }
     }
     uint64_t slow = 0;
-    if (__ballot(other != 0)) {
+    if (any_lane(other != 0)) {
         // enabled sets by edge, kept in the scratch (64 bits per slot)
         uint64_t *set = (uint64_t *)scr;
         bool serial = false;
@@ -796,69 +1025,90 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int
         smc_u32x4 rw = {{0u, 0u, 0u, 0u}};
 #pragma unroll
         for (int j = 0; j < C; ++j) {
-            if (TRACE) fired[j] = -1;
             const uint32_t c = (uint32_t)(sl * C + j);
             if (j % G == 0) {
                 bool choice = false;
 #pragma unroll
                 for (int k = j; k < j + G; ++k) choice |= (mk[k] & (mk[k] - 1)) != 0;
-                if (choice) rw = draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
+                if (any_lane(choice)) rw = draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c));
             }
-            if (mk[j]) {
+            if (any_lane(mk[j] != 0)) {
                 const uint32_t w = words[64 * j];
-                const DevLoc L = load_rec(m.locs + word_rec(w, m));
-                int i = 31 - __clz((int)mk[j]);
-                if (mk[j] & (mk[j] - 1)) {
-                    // weighted choice from the highest edge down; weights are
-                    // constants summing below 2^31
+                const bool on = mk[j] != 0, choice = (mk[j] & (mk[j] - 1)) != 0;
+                const uint4 rv = load_quad(m.locs + word_rec(w, m), 0);
+                const uint32_t ef = m.locs[word_rec(w, m)].edge_first;
+                int i = on ? __ffs(mk[j]) - 1 : 0;
+                if (any_lane(choice)) {
+                    // weighted choice; weights are constants summing below
+                    // 2^31.  Two edges: the higher one unless the draw falls
+                    // below the lower one's weight.
                     const double u = smc_receiver_u(rw, c);
-                    if ((L.flags & SMC_LF_RECV_TWO) && mk[j] == L.recv_mask) {
-                        const int rnd = (int)((double)L.recv_weight * u);
-                        if (!((int)L.recv_low <= rnd)) i = __ffs(mk[j]) - 1;
-                    } else {
-                        int W = 0;
-                        for (uint32_t r = mk[j]; r; r &= r - 1) W += (int)m.edges[L.edge_first + __ffs(r) - 1].weight;
-                        const int rnd = (int)((double)W * u);
-                        i = __ffs(mk[j]) - 1;
-                        for (uint32_t r = mk[j]; r;) {
-                            const int k = 31 - __clz((int)r);
-                            r &= ~(1u << k);
-                            W -= (int)m.edges[L.edge_first + k].weight;
-                            if (W <= rnd) { i = k; break; }
+                    const bool two = choice & (rv.w != 0xFFFFFFFFu) & (mk[j] == rv.y);
+                    const int rnd2 = (int)((double)rv.z * u);
+                    if (two & ((int)rv.w <= rnd2)) i = 31 - __clz((int)mk[j]);
+                    const bool several = choice & !two;
+                    if (unlikely(any_lane(several))) {
+                        if (several) {
+                            int W = 0;
+                            for (uint32_t r = mk[j]; r; r &= r - 1) W += (int)rec_at(m.edges, ef + __ffs(r) - 1)->weight;
+                            const int rnd = (int)((double)W * u);
+                            for (uint32_t r = mk[j]; r;) {
+                                const int k = 31 - __clz((int)r);
+                                r &= ~(1u << k);
+                                W -= (int)rec_at(m.edges, ef + k)->weight;
+                                if (W <= rnd) { i = k; break; }
+                            }
                         }
                     }
                 }
-                const DevEdge E = load_rec(m.edges + L.edge_first + i);
-                ++trans;
-                any = true;
+                const uint32_t e = ef + i;
+                const uint4 head = load_quad(rec_at(m.edges, e), 0), tail = load_quad(rec_at(m.edges, e), 2);
                 const uint32_t base = word_base(w, m);
-#pragma clang loop unroll(disable)
-                for (int k = 0; k < E.upd_n; ++k) {
-                    const DevUpd U = load_rec(m.upds + E.upd_first + k);
-                    const uint32_t at = var_at(U.var, base);
-                    if (U.kind == SMC_U_ADD) {
-                        if ((int)at == q.qvar) {
-                            qsum += U.value;
+                any |= on;
+                trans += on ? 1u : 0u;
+                goal |= on & ((head.y & SMC_EF_GOAL) != 0);
+                if (on) words[64 * j] = (head.x << m.rec_shift) | base;
+                if (TRACE) fired[j] = on ? m.loc_edge0[on ? locs[64 * j] : 0] + i : -1;
+                if (LOCS && on) locs[64 * j] += rec_at(m.edges, e)->dst;
+                // updates: additions and constants
+                auto update = [&](double value, double *at, bool add, bool clock) {
+                    if (add) {
+                        if (at == x.vars + q.qvar) {
+                            qsum += value;
                             qhi = fmax(qhi, qsum);
                             qlo = fmin(qlo, qsum);
                             qany = true;
                         }
-                        atomicAdd(&x.vars[at], U.value);
+                        atomicAdd(at, value);
                     } else {
-                        if ((int)at == q.qvar) {
-                            q.qmax = fmax(q.qmax, U.value);
-                            q.qmin = fmin(q.qmin, U.value);
+                        if (at == x.vars + q.qvar) {
+                            q.qmax = fmax(q.qmax, value);
+                            q.qmin = fmin(q.qmin, value);
                         }
-                        x.vars[at] = U.clock ? x.now - U.value : U.value;
+                        *at = clock ? x.now - value : value;
+                    }
+                };
+                x.base = base;
+                const uint4 u0 = load_quad(rec_at(m.edges, e), 3);
+                if (any_lane(on && (u0.z >> 16) >= SMC_EU_ADD)) {
+                    const uint4 u1 = load_quad(rec_at(m.edges, e), 4);
+                    if (on && (u0.z >> 16) >= SMC_EU_ADD)
+                        update(quad_f64(u0), var_ptr(x, u0.z & 0xFFFFu, u0.z >> 16), (u0.z & (SMC_EU_ADD << 16)) != 0,
+                               (u0.z & (SMC_EU_CLOCK << 16)) != 0);
+                    if (on && (u1.z >> 16) >= SMC_EU_ADD)
+                        update(quad_f64(u1), var_ptr(x, u1.z & 0xFFFFu, u1.z >> 16), (u1.z & (SMC_EU_ADD << 16)) != 0,
+                               (u1.z & (SMC_EU_CLOCK << 16)) != 0);
+                    const int n = on ? (int)(tail.z >> 16) : 0;
+                    if (any_lane(n != 0)) {
+                        for (int k = 0; k < n; ++k) {
+                            const DevUpd U = load_rec(m.upds + tail.w + k);
+                            update(U.value, x.vars + var_at(U.var, base), U.kind == SMC_U_ADD, U.clock != 0);
+                        }
                     }
                 }
-                if (E.dst_goal) goal = true;
-                words[64 * j] = (E.dst_rec << m.rec_shift) | base;
-                if (TRACE) fired[j] = m.loc_edge0[locs[64 * j]] + i;
-                if (LOCS) locs[64 * j] += E.dst;
-            }
+            } else if (TRACE) fired[j] = -1;
         }
-        if (q.qvar >= 0 && (__ballot(qany) & seg_mask)) {
+        if (q.qvar >= 0 && any_lane(qany)) {
             double incl = qsum;
             for (int k = 1; k < S; k <<= 1) {
                 const double y = __shfl_up(incl, k, S);
@@ -902,13 +1152,12 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int
                         const uint32_t first = m.locs[word_rec(w, m)].edge_first;
                         x.base = word_base(w, m);
                         const int i = pick_receiver(mask, first, seed, run, step, (uint32_t)c, x, m);
-                        const DevEdge E = load_rec(m.edges + first + i);
-                        run_updates(E, x, m, q);
-                        if (E.dst_goal) goal = true;
-                        words[64 * j] = (E.dst_rec << m.rec_shift) | x.base;
+                        const uint4 head = fire_updates(first + i, x, m, q);
+                        if (head.y & SMC_EF_GOAL) goal = true;
+                        words[64 * j] = (head.x << m.rec_shift) | x.base;
                         ++trans;
                         if (TRACE) e_fired = m.loc_edge0[locs[64 * j]] + i;
-                        if (LOCS) locs[64 * j] += E.dst;
+                        if (LOCS) locs[64 * j] += rec_at(m.edges, first + i)->dst;
                     }
                     wave_sync();
                     if (TRACE) {

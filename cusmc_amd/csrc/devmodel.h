@@ -39,6 +39,7 @@
 #define SMC_REF_VAR 1u
 #define SMC_REF_CODE 2u
 #define SMC_REF_CLOCK 3u
+#define SMC_NO_REF 0xFFFFFFFFu
 #define SMC_REF_KIND(r) ((r) >> 30)
 #define SMC_REF_MAKE(kind, payload) (((uint32_t)(kind) << 30) | (uint32_t)(payload))
 #define SMC_REF_CODE_MAKE(first, count) (((uint32_t)SMC_REF_CODE << 30) | ((uint32_t)(count) << 24) | (uint32_t)(first))
@@ -76,7 +77,7 @@ enum {
     SMC_LF_GUARDED = 4,     // blocked or not by the variables: every spontaneous edge without
                             // `!=` has a conjunct that reads no clock (DevLoc.block_first)
     SMC_LF_RECV_FAST = 8,   // every receive edge commutes (see DevUpd), constant weights below 2^31 in all
-    SMC_LF_RECV_TWO = 16    // exactly two receive edges (recv_low: the lower one's weight)
+    SMC_LF_RECV_TWO = 16    // recv_chan > 0 and exactly two receive edges
 };
 
 // What a race step has to look at in a location (DevHot.flags).
@@ -109,24 +110,27 @@ struct DevHot {
     uint16_t flags;         // SMC_HF_*
 };
 
-// The rest, 48 bytes: receive edges, then edge range, invariants, blocking
-// test, rate.
+// The rest, 64 bytes: receive edges; spontaneous edges; invariants, blocking
+// test and rate.
 struct DevLoc {
     int32_t recv_chan;      // every receive edge is unguarded, on this channel; 0 none; -1 other
     uint32_t recv_mask;     // the receive edges, as bits of the edge list
     uint32_t recv_weight;   // sum of their weights
-    uint32_t recv_low;      // SMC_LF_RECV_TWO
+    uint32_t recv_low;      // of two receive edges, the lower one's weight; else 0xFFFFFFFF
     uint32_t edge_first;    // edges [edge_first, edge_first + edge_n)
     uint16_t edge_n;
     uint8_t klass;
     uint8_t flags;          // SMC_LF_*
+    uint32_t pick_mask;     // the spontaneous edges, and the sum of their weights, if these
+    uint32_t pick_weight;   // are constants below 2^31 in all (else mask 0)
     uint32_t inv_first;     // clock upper-bound invariants
     uint32_t block_first;   // SMC_LF_GUARDED: the blocking test, guard records from here on
-    double rate_value;      // the rate when it is a constant (rate_const)
     uint32_t rate;          // expression reference
     uint16_t n_inv;
     uint8_t rate_const;
     uint8_t type;
+    double rate_value;      // the rate when it is a constant (rate_const)
+    uint64_t pad;
 };
 
 struct DevInv {             // x <= bound  (strict: x < bound), 16 bytes
@@ -138,20 +142,37 @@ struct DevInv {             // x <= bound  (strict: x < bound), 16 bytes
 };
 
 // DevEdge.flags
-enum { SMC_EF_WEIGHT_CONST = 1 };  // weight is the constant itself (0 if negative), else a reference
+enum {
+    SMC_EF_GOAL = 1,          // destination is a goal location
+    SMC_EF_NEVER = 2,         // has a `!=` guard: never enabled (simulation.cu:249-251)
+    SMC_EF_WEIGHT_CONST = 4,  // weight is the constant itself (0 if negative), else a reference
+    SMC_EF_NO_GUARD = 8       // no guard in the record
+};
+// DevEdge.g_flags, u0_flags, u1_flags: low byte 8 if the variable counts from
+// the component's base, else 0
+enum { SMC_EG_CLOCK = 0x100, SMC_EU_ADD = 0x100, SMC_EU_SET = 0x200, SMC_EU_CLOCK = 0x400 };
 
-struct DevEdge {            // 32 bytes
-    int32_t dst;            // destination relative to the source location
-    int32_t channel;
-    uint32_t weight;
-    uint32_t guard_first;
-    uint32_t upd_first;
-    uint16_t guard_n;
-    uint16_t upd_n;
-    uint8_t dst_goal;       // destination is a goal location
-    uint8_t never;          // has a `!=` guard: never enabled (simulation.cu:249-251)
-    uint16_t flags;         // SMC_EF_*
+// An edge, 80 bytes: with its first guard against a constant and its first
+// two plain updates (add or set a constant), which is all that most edges
+// have, so that firing one is a straight line of three dependent reads.
+// Variables are byte offsets.
+struct DevEdge {
     uint32_t dst_rec;       // record class of the destination
+    uint32_t flags;         // SMC_EF_*
+    uint32_t weight;
+    int32_t channel;
+    double lo, hi;          // the guard holds for values in [lo, hi]
+    uint16_t g_var, g_flags;
+    uint32_t guard_first;   // other guards
+    uint16_t guard_n;
+    uint16_t upd_n;         // other updates, after u0 and u1
+    uint32_t upd_first;
+    double u0_value;
+    uint16_t u0_var, u0_flags;  // neither ADD nor SET: no update
+    int32_t dst;            // destination relative to the source location
+    double u1_value;
+    uint16_t u1_var, u1_flags;
+    uint32_t pad;
 };
 
 // DevGuard.flags
@@ -244,6 +265,8 @@ struct DevModelT {
     int32_t rec_shift;          // state word: class << rec_shift | base of the private variables
     uint32_t base_mask;         // (1 << rec_shift) - 1
     uint32_t tests;             // every SMC_HF_* flag some location has
+    uint32_t one_rate;          // the one rate expression of the network (reading no private
+                                // variable), or SMC_NO_REF
     int32_t freeze;             // no rate reads a clock: blocked components may leave the race
 };
 using DevModel = DevModelT<SmcGlobalTables>;

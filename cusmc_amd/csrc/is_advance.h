@@ -281,7 +281,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                     const double M = scr[64 * jk];
                     const int ti = theta ? tl.tix[locs[64 * jk]] : -1;
                     const bool tilted = ti >= 0 && theta[ti] != 0.0f;
-                    const double du = tilted ? M * (1.0 - smc_exp2(smc_log2(1.0 - u) / tex[ti])) : M * u;
+                    const double du = tilted ? M * (1.0 - smc_exp2(device_log2(1.0 - u) / tex[ti])) : M * u;
                     if (du < umin) { umin = du; unif_j = jk; }
                     b &= b - 1;
                 }
@@ -294,7 +294,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
             int wexp = 0x7FFFFFFF;
             if (Rt > 0.0) {
                 const smc_u32x4 rw = draw(P.seed, run, step, SMC_P_RACE, 0);
-                dexp = -smc_log2(smc_u01(rw.v[0], rw.v[1])) / Rt;
+                dexp = -device_log2(smc_u01(rw.v[0], rw.v[1])) / Rt;
                 wexp = race_pick<C>(leaft, lvl, smc_u01(rw.v[2], rw.v[3]) * Rt, S, sl, seg_base, seg_mask);
             }
             double gu = umin;
@@ -322,7 +322,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                 const double Rd = tree_total<C>(dl, S);
                 if (Rd > 0.0) {
                     const smc_u32x4 rw = draw(P.seed, run, step, SMC_P_DEAD, 0);
-                    const double td = P.bound + (-smc_log2(smc_u01(rw.v[0], rw.v[1])) / Rd);
+                    const double td = P.bound + (-device_log2(smc_u01(rw.v[0], rw.v[1])) / Rd);
                     if (td < t + d) { d = td - t; w = -1; exp_won = false; u_won = false; }
                 }
             }
@@ -344,7 +344,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                         if ((rs.bounded >> j) & 1u) {
                             const int ti = tl.tix[locs[64 * j]];
                             if (ti >= 0 && theta[ti] != 0.0f)
-                                ut[j] = (1.0 - tex[ti]) * smc_log2(1.0 - d / scr[64 * j]);
+                                ut[j] = (1.0 - tex[ti]) * device_log2(1.0 - d / scr[64 * j]);
                         }
                     }
                     log2lr = log2lr + tree_total<C>(ut, S);
@@ -359,7 +359,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
 #pragma unroll
                 for (int j = 0; j < C; ++j) {
                     if (rs.leaf[j] > 0.0) hz[64 * j] = hz[64 * j] + LN2 * rs.leaf[j] * d;
-                    else if ((rs.bounded >> j) & 1u) hz[64 * j] = hz[64 * j] + -LN2 * smc_log2(1.0 - d / scr[64 * j]);
+                    else if ((rs.bounded >> j) & 1u) hz[64 * j] = hz[64 * j] + -LN2 * device_log2(1.0 - d / scr[64 * j]);
                 }
             }
         }
@@ -371,30 +371,25 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
             const int at = (w % C) * 64 + seg_base + w / C;
             const uint32_t ww = tl.words[at];
             const Ctx x{vars, t, word_base(ww, m)};
-            const uint32_t first = m.locs[word_rec(ww, m)].edge_first;
-            const int ne = m.locs[word_rec(ww, m)].edge_n;
-            uint64_t mask = 0;
-#pragma clang loop unroll(disable)
-            for (int i0 = 0; i0 < ne; i0 += S) {
-                const bool en = i0 + sl < ne && edge_enabled(first + i0 + sl, 0, x, m);
-                mask |= ((__ballot(en) >> seg_base) & seg_ones) << i0;
-            }
+            const uint4 L1 = load_quad(m.locs + word_rec(ww, m), 1);
+            const uint32_t first = L1.x;            // edge_first
+            const int ne = (int)(L1.y & 0xFFFFu);   // edge_n
+            const uint64_t mask = enabled_mask_by_lanes(first, ne, x, m, S, sl, seg_base, seg_ones);
             if (mask) {
-                const int i = pick_edge(mask, first, P.seed, run, step, (uint32_t)w, x, m);
-                const DevEdge E = load_rec(m.edges + first + i);
-                run_updates(E, x, m, q);
-                tl.words[at] = (E.dst_rec << m.rec_shift) | x.base;
+                const int i = pick_edge(mask, first, L1.z, L1.w, P.seed, run, step, (uint32_t)w, x, m);
+                const uint4 head = fire_updates(first + i, x, m, q);
+                tl.words[at] = (head.x << m.rec_shift) | x.base;
                 const int32_t lw = tl.locs[at];
                 // the network's edge index (digests name it; records are shared)
                 if (P.trace)
                     digest = smc_mix(digest, ((uint64_t)step << 40) | ((uint64_t)w << 20) |
                                                  (uint64_t)(m.loc_edge0[lw] + i));
                 wave_sync();  // every lane has read the location
-                tl.locs[at] = lw + E.dst;
-                if (E.dst_goal) goal = true;
+                tl.locs[at] = lw + rec_at(m.edges, first + i)->dst;
+                goal |= (head.y & SMC_EF_GOAL) != 0;
                 if (sl == 0) ++trans;
                 changed = true;
-                chan = E.channel > 0 ? E.channel : 0;
+                chan = (int)head.w > 0 ? (int)head.w : 0;
                 sender = chan > 0 ? w : -1;
                 fired_any = true;
             }

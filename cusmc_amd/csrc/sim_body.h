@@ -76,8 +76,9 @@ __device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTAN
 // (with per-slot copies of the general code in every branch it was 320 KB).
 // Fischer-32, 1e6 runs at 4 lanes a run: 76.2 ms in that form, 51.0 ms with
 // record classes and rolled cold paths, 44.2 ms with the slot loop free of
-// branches and its invariants out of spilled registers; SIR-350, 2e5 runs at
-// 64 lanes: 355, 117 and 97 ms.
+// branches and its invariants out of spilled registers, 40.7 ms with the
+// step's rare parts behind branches the whole wave takes or leaves; SIR-350,
+// 2e5 runs at 64 lanes: 355, 117, 97 and 81.8 ms.
 //
 // LDS: [tables: lp.table_bytes, TAB only] then per wave [variables of the
 // wave's 64/S runs: var_stride doubles each][scratch: 8 bytes per slot and
@@ -141,6 +142,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     m.rec_shift = inst->m.rec_shift;
     m.base_mask = inst->m.base_mask;
     m.tests = inst->m.tests;
+    m.one_rate = inst->m.one_rate;
     m.freeze = inst->m.freeze;
     const uint64_t seed = inst->p.seed;
     const double bound = inst->p.bound;
@@ -172,56 +174,97 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     uint32_t step = 0, trans = 0;  // trans: edges fired by this lane (the winner's count on lane 0)
     int chan = 0, sender = -1;
     bool goal = false;
+    bool over = false;    // no event can follow: the run ends at its clock
     bool changed = true;  // state changed since the last blocking tests
     uint32_t xblk = 0;    // blocked slots at the last change of state (tests of several records)
     uint64_t digest = 0;
     LaneQuery q{inst->p.qvar, 0.0, 0.0};
 
+    // The loop's straight path is one step of every run of the wave; the rest
+    // is behind wave-uniform conditions.
     for (;;) {
         const int S = scalar_here(S0);
-        if (!active && !done) {
-            unsigned int r = 0;
-            if (sl == 0) r = atomicAdd(&chunk_next, 1u);
-            r = __shfl(r, seg_base);
-            if (r >= r_end) {
-                done = true;
-            } else {
-                const SMC_CONSTANT InstDesc *I = opaque(inst);
-                ridx = r;
-                run = I->p.run_begin + round * I->p.n_runs + r;
-                active = true;
-                t = 0.0; step = 0; trans = 0; chan = 0; sender = -1;
-                goal = false; changed = true;
-                q.qmax = I->p.qinit; q.qmin = I->p.qinit;
-                digest = TRACE ? smc_mix(0, run) : 0;
-                for (int v = sl; v < I->m.n_vars; v += S) vars[v] = I->m.var_init[v];
-#pragma clang loop unroll(disable)
-                for (int j = 0; j < C; ++j) {
-                    const int c = sl * C + j;
-                    words[64 * j] = c < I->m.n_comp ? I->m.comp_word[c] : 0u;
-                    if (TRACE) locs[64 * j] = c < I->m.n_comp ? I->m.comp_init_loc[c] : -1;
+        // ---- loop test (simulation.cu:835-849)
+        const bool in_time = t < bound;
+        const bool at_goal = reach & goal & in_time & !over;
+        const bool end = active & (!in_time | over | at_goal | (step >= max_steps));
+        if (unlikely(any_lane(end | (!active & !done)))) {
+            const SMC_CONSTANT InstDesc *I = opaque(inst);
+            if (end) {
+                // per-run result (simulation.cu:887-893, statistics.cuh:126-163)
+                double qmax = q.qmax, qmin = q.qmin;
+                uint32_t fired = trans;
+#pragma unroll
+                for (int k = 0; k < 6; ++k)
+                    if ((1 << k) < S) {
+                        qmax = fmax(qmax, seg_xchg(qmax, k));
+                        qmin = fmin(qmin, seg_xchg(qmin, k));
+                        fired += (uint32_t)__shfl_xor((int)fired, 1 << k);
+                    }
+                const double value = I->p.is_max ? qmax : qmin;
+                if (TRACE) {
+                    digest = smc_mix(digest, smc_digest_bits(t));
+                    for (int v = 0; v < I->m.n_vars; ++v)
+                        digest = smc_mix(digest, smc_digest_bits(I->m.var_clock[v] ? t - vars[v] : vars[v]));
+                    for (int c = 0; c < I->m.n_comp; ++c) {
+                        const int lv = ((int32_t *)words_of)[64 * C + (c % C) * 64 + seg_base + c / C];
+                        digest = smc_mix(digest, (uint64_t)(uint32_t)lv);
+                    }
+                }
+                if (sl == 0) {
+                    uint8_t flag;
+                    if (reach) flag = at_goal ? 1 : 0;
+                    else flag = I->p.is_max ? (value > I->p.threshold) : (value < I->p.threshold);
+                    I->p.flag[ridx] = flag;
+                    I->p.value[ridx] = value;
+                    I->p.steps[ridx] = step;
+                    I->p.trans[ridx] = fired;
+                    if (I->p.time) I->p.time[ridx] = t;
+                    if (TRACE && I->p.digest) I->p.digest[ridx] = digest;
                 }
                 wave_sync();
+                active = false;
             }
+            if (!active && !done) {
+                unsigned int r = 0;
+                if (sl == 0) r = atomicAdd(&chunk_next, 1u);
+                r = __shfl(r, seg_base);
+                if (r >= r_end) {
+                    done = true;
+                } else {
+                    ridx = r;
+                    run = I->p.run_begin + round * I->p.n_runs + r;
+                    active = true;
+                    t = 0.0; step = 0; trans = 0; chan = 0; sender = -1;
+                    goal = false; over = false; changed = true;
+                    q.qmax = I->p.qinit; q.qmin = I->p.qinit;
+                    digest = TRACE ? smc_mix(0, run) : 0;
+                    for (int v = sl; v < I->m.n_vars; v += S) vars[v] = I->m.var_init[v];
+#pragma clang loop unroll(disable)
+                    for (int j = 0; j < C; ++j) {
+                        const int c = sl * C + j;
+                        words[64 * j] = c < I->m.n_comp ? I->m.comp_word[c] : 0u;
+                        if (TRACE) locs[64 * j] = c < I->m.n_comp ? I->m.comp_init_loc[c] : -1;
+                    }
+                    wave_sync();
+                }
+            }
+            if (!any_lane(active)) break;
+            continue;  // a new run passes the loop test first
         }
-        if (__ballot(!done) == 0) break;
-        if (done) continue;
+        if (!active) continue;
 
-        // ---- loop test (simulation.cu:835-849)
-        bool hit = false, end = false;
-        if (!(t < bound)) end = true;
-        else if (reach && goal) { end = true; hit = true; }
-        else if (step >= max_steps) end = true;
-
-        if (!end && chan > 0) {
+        if (any_lane(chan > 0)) {
             // pending broadcast receivers (SyncInSerial simulation.cu:357-407)
-            bool entered = false;
-            fire_receivers<C, TRACE, TRACE>(words, scr, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, seed, run,
-                                            step, lane, sl, S, seg_base, seg_mask, trans, digest);
-            changed = true;
-            chan = 0;
-            sender = -1;
-            goal = goal || (__ballot(entered) & seg_mask) != 0;
+            if (chan > 0) {
+                bool entered = false;
+                fire_receivers<C, TRACE, TRACE>(words, scr, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, seed,
+                                                run, step, lane, sl, S, seg_base, seg_mask, trans, digest);
+                changed = true;
+                chan = 0;
+                sender = -1;
+                goal = goal || (__ballot(entered) & seg_mask) != 0;
+            }
         }
 
         // ---- race (compute_possible_delay :409-541, find_minimum_delay
@@ -229,171 +272,157 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
         // by this iteration's receivers counts only if this step, raced by
         // every component, keeps t < bound (simulation.cu:409-415, 835-849):
         // no absorption exit and no left-out null racers then.
-        const bool full = reach && goal;
-        // with frozen racers the race itself ends a run that nothing can
-        // leave (no event: blocked racers are out, the rest race at rate 0),
-        // so the scan is needed only without them
-        if (!end && !m.freeze && changed && !full && absorbed<C>(words, Ctx{vars, t, 0}, m, seg_mask)) end = true;
-        if (!end) {
-            double d = 0.0;
-            int w = -1;
-            RaceSlots<C> rs;
-            race_slots<C>(rs, words, scr, Ctx{vars, t, 0}, m, changed, xblk);
-            if (!full) changed = false;
-            // A frozen component (blocked, exponential) only makes null steps
-            // until the next transition.  Leaving it out of the race keeps
-            // the law of everything else: exponential racers are memoryless
-            // (rates constant between transitions), and a uniform racer
-            // redrawn at every step has hazard 1/(W - tau), a function of the
-            // absolute time alone (W: the end of its window).  It races as in
-            // the reference when the step decides the outcome (full).
+        const bool full = reach & goal;
+        if (unlikely(!m.freeze)) {
+            // with frozen racers the race itself ends a run that nothing can
+            // leave (no event: blocked racers are out, the rest race at rate
+            // 0), so the scan is needed only without them
+            if (changed && !full && absorbed<C>(words, Ctx{vars, t, 0}, m, seg_mask)) over = true;
+            if (over) continue;
+        }
+        RaceSlots<C> rs;
+        race_slots<C>(rs, words, scr, Ctx{vars, t, 0}, m, changed, xblk);
+        changed = full;
+        // A frozen component (blocked, exponential) only makes null steps
+        // until the next transition.  Leaving it out of the race keeps the
+        // law of everything else: exponential racers are memoryless (rates
+        // constant between transitions), and a uniform racer redrawn at every
+        // step has hazard 1/(W - tau), a function of the absolute time alone
+        // (W: the end of its window).  It races as in the reference when the
+        // step decides the outcome (full).
+        if (unlikely(any_lane(full))) {
             if (m.freeze && full) {
                 const uint32_t fz = frozen_rates<C>(words, scr, Ctx{vars, t, 0}, m);
 #pragma unroll
                 for (int j = 0; j < C; ++j)
                     if ((fz >> j) & 1u) rs.leaf[j] = scr[64 * j];
             }
-            const uint64_t zb = __ballot(rs.zero != 0) & seg_mask;
-            if (zb) {
-                const int Lz = lowest_lane(zb);
-                w = (Lz - seg_base) * C + __shfl(__ffs(rs.zero) - 1, Lz);
-            } else {
-                // uniform delays under clock bounds, lowest slot first on ties;
-                // slots 2i and 2i+1 of a lane share one draw
-                double umin = INF;
-                int unif_j = -1;
+        }
+        double d = 0.0;
+        int w = -1;
+        const uint64_t zb = __ballot(rs.zero != 0) & seg_mask;
+        if (any_lane(zb == 0)) {
+            // some run races (the others' result is replaced below)
+            double umin = INF;
+            int unif_j = -1;
+            // Draws: one for the race, and the uniform delays under clock
+            // bounds (slots 2i and 2i+1 of a lane share one; lowest slot
+            // first on ties).  The lanes of a run make them side by side: a
+            // lane without delays left to draw makes the race's, and its
+            // words are handed to the others afterwards.
+            smc_u32x4 race{};
+            uint64_t got = 0;  // lanes of the run that made the race's draw
+            {
+                uint32_t b = rs.bounded;
 #pragma clang loop unroll(disable)
-                for (uint32_t b = rs.bounded; b;) {
-                    const int j = __ffs(b) - 1;
+                do {
+                    const bool delay = b != 0;
+                    const int j = delay ? __ffs(b) - 1 : 0;
                     const uint32_t c = (uint32_t)(sl * C + j);
-                    const smc_u32x4 rw = draw(seed, run, step, SMC_P_UNIFORM, smc_uniform_draw(c));
+                    const smc_u32x4 rw = draw_at(seed, run, step,
+                                                 delay ? ((uint32_t)SMC_P_UNIFORM << 24) | smc_uniform_draw(c)
+                                                       : (uint32_t)SMC_P_RACE << 24);
                     const double du = scr[64 * j] * smc_uniform_u(rw, c);
-                    if (du < umin) { umin = du; unif_j = j; }
+                    if (delay && du < umin) { umin = du; unif_j = j; }
                     b &= b - 1;
-                    if (C > 1 && !(c & 1u) && ((b >> (j + 1)) & 1u)) {
-                        const double du1 = scr[64 * (j + 1)] * smc_uniform_u(rw, c + 1);
-                        if (du1 < umin) { umin = du1; unif_j = j + 1; }
-                        b &= b - 1;
+                    if (C > 1) {
+                        const int j1 = j + 1 < C ? j + 1 : j;
+                        const bool pair = !(c & 1u) && ((b >> j1) & 1u);
+                        const double du1 = scr[64 * j1] * smc_uniform_u(rw, c + 1);
+                        if (pair && du1 < umin) { umin = du1; unif_j = j1; }
+                        b = pair ? b & (b - 1) : b;
                     }
-                }
-                const double R = race_total<C>(rs.leaf, scr, S);
-                double dexp = INF;
-                int wexp = 0x7FFFFFFF;
-                if (R > 0.0) {
-                    const smc_u32x4 rw = draw(seed, run, step, SMC_P_RACE, 0);
-                    dexp = -smc_log2(smc_u01(rw.v[0], rw.v[1])) / R;
-                    wexp = race_pick<C>(rs.leaf, scr, smc_u01(rw.v[2], rw.v[3]) * R, S, sl, seg_base, seg_mask);
-                }
-                double gu = umin;
-                int wu = 0x7FFFFFFF;
-                if (__ballot(unif_j >= 0) & seg_mask) {  // some slot of the run drew a delay
+                    // every draw of the race is the same: keep the last
+                    race.v[0] = delay ? race.v[0] : rw.v[0];
+                    race.v[1] = delay ? race.v[1] : rw.v[1];
+                    race.v[2] = delay ? race.v[2] : rw.v[2];
+                    race.v[3] = delay ? race.v[3] : rw.v[3];
+                    got |= __ballot(!delay) & seg_mask;
+                } while (any_lane(b != 0 || got == 0));
+                const int from = lowest_lane(got);
 #pragma unroll
-                    for (int k = 0; k < 6; ++k)
-                        if ((1 << k) < S) gu = fmin(gu, seg_xchg(gu, k));
-                    if (gu < INF) {
-                        const int Lu = lowest_lane(__ballot(unif_j >= 0 && umin == gu) & seg_mask);
-                        wu = (Lu - seg_base) * C + __shfl(unif_j, Lu);
-                    }
+                for (int k = 0; k < 4; ++k) race.v[k] = (uint32_t)__shfl((int)race.v[k], from);
+            }
+            const double R = race_total<C>(rs.leaf, scr, S);
+            const double e = -device_log2(smc_u01(race.v[0], race.v[1])) / R;
+            w = race_pick<C>(rs.leaf, scr, smc_u01(race.v[2], race.v[3]) * R, S, sl, seg_base, seg_mask);
+            const double dexp = R > 0.0 ? e : INF;
+            d = dexp;
+            if (any_lane(unif_j >= 0)) {
+                double gu = umin;
+#pragma unroll
+                for (int k = 0; k < 6; ++k) {
+                    if ((1 << k) >= S) break;
+                    gu = fmin(gu, seg_xchg(gu, k));
                 }
-                if (gu < dexp || (gu == dexp && wu < wexp)) { d = gu; w = wu; }
-                else if (dexp < INF) { d = dexp; w = wexp; }
-                else d = INF;  // no racer: no event
-                // the step that crosses the bound: the left-out null racers'
-                // first event after the bound may come first
-                if (m.freeze && !full && d < INF && !(t + d < bound)) {
+                // the lowest lane holding the least delay (any lane of a run
+                // without one: gu is infinite and loses)
+                const uint64_t at = __ballot(unif_j >= 0 && umin == gu) & seg_mask;
+                const int Lu = at ? lowest_lane(at) : seg_base;
+                const int wu = (Lu - seg_base) * C + __shfl(unif_j, Lu);
+                if (gu < dexp || (gu == dexp && gu < INF && wu < w)) { d = gu; w = wu; }
+            }
+            // the step that crosses the bound: the left-out null racers'
+            // first event after the bound may come first
+            const bool cross = m.freeze && !full && zb == 0 && d < INF && !(t + d < bound);
+            if (unlikely(any_lane(cross))) {
+                if (cross) {
                     const uint32_t fz = frozen_rates<C>(words, scr, Ctx{vars, t, 0}, m);
                     double dl[C];
 #pragma unroll
                     for (int j = 0; j < C; ++j) dl[j] = ((fz >> j) & 1u) ? scr[64 * j] : 0.0;
                     const double Rd = tree_total<C>(dl, S);
                     if (Rd > 0.0) {
-                        const smc_u32x4 rw = draw(seed, run, step, SMC_P_DEAD, 0);
-                        const double td = bound + (-smc_log2(smc_u01(rw.v[0], rw.v[1])) / Rd);
+                        const smc_u32x4 dw = draw(seed, run, step, SMC_P_DEAD, 0);
+                        const double td = bound + (-device_log2(smc_u01(dw.v[0], dw.v[1])) / Rd);
                         if (td < t + d) { d = td - t; w = -1; }
                     }
                 }
             }
-            if (!(d < INF)) {
-                end = true;  // no event: the run ends at its clock
-            } else {
-                // clocks advance (find_minimum_delay :632-651)
-                t = t + d;
-                if (w >= 0) {
-                    // the winner's transition (check_enabled_edges :268-305,
-                    // take_transition :27-181) by every lane of its segment:
-                    // each tests one of the location's edges; the pick and
-                    // the updates are the same on all of them
-                    uint32_t *slot = words_of + (w % C) * 64 + seg_base + w / C;
-                    const uint32_t ww = *slot;
-                    const Ctx x{vars, t, word_base(ww, m)};
-                    const uint32_t first = m.locs[word_rec(ww, m)].edge_first;
-                    const int ne = m.locs[word_rec(ww, m)].edge_n;
-                    uint64_t mask = 0;
-#pragma clang loop unroll(disable)
-                    for (int i0 = 0; i0 < ne; i0 += S) {
-                        const bool en = i0 + sl < ne && edge_enabled(first + i0 + sl, 0, x, m);
-                        mask |= ((__ballot(en) >> seg_base) & seg_ones) << i0;
-                    }
-                    if (mask) {
-                        const int i = pick_edge(mask, first, seed, run, step, (uint32_t)w, x, m);
-                        const DevEdge E = load_rec(m.edges + first + i);
-                        run_updates(E, x, m, q);
-                        *slot = (E.dst_rec << m.rec_shift) | x.base;
-                        if (TRACE) {
-                            int32_t *wloc = (int32_t *)words_of + 64 * C + (w % C) * 64 + seg_base + w / C;
-                            const int32_t lw = *wloc;
-                            digest = smc_mix(digest, ((uint64_t)step << 40) | ((uint64_t)w << 20) |
-                                                         (uint64_t)(m.loc_edge0[lw] + i));
-                            *wloc = lw + E.dst;
-                        }
-                        if (E.dst_goal) goal = true;
-                        if (sl == 0) ++trans;
-                        changed = true;
-                        chan = E.channel > 0 ? E.channel : 0;
-                        sender = chan > 0 ? w : -1;
-                    }
-                    wave_sync();
-                }
-                ++step;
-            }
         }
-
-        if (end) {
-            // per-run result (simulation.cu:887-893, statistics.cuh:126-163)
-            double qmax = q.qmax, qmin = q.qmin;
-            uint32_t fired = trans;
-#pragma unroll
-            for (int k = 0; k < 6; ++k)
-                if ((1 << k) < S) {
-                    qmax = fmax(qmax, seg_xchg(qmax, k));
-                    qmin = fmin(qmin, seg_xchg(qmin, k));
-                    fired += (uint32_t)__shfl_xor((int)fired, 1 << k);
+        if (any_lane(zb != 0)) {
+            // a zero delay wins, the lowest component first
+            const int Lz = zb ? lowest_lane(zb) : seg_base;
+            const int wz = (Lz - seg_base) * C + __shfl(__ffs(rs.zero) - 1, Lz);
+            if (zb) { d = 0.0; w = wz; }
+        }
+        over = !(d < INF);  // no racer: no event
+        if (over) continue;
+        // clocks advance (find_minimum_delay :632-651)
+        t = t + d;
+        if (w >= 0) {
+            // the winner's transition (check_enabled_edges :268-305,
+            // take_transition :27-181) by every lane of its segment: each
+            // tests one of the location's edges; the pick and the updates are
+            // the same on all of them
+            uint32_t *slot = words_of + (w % C) * 64 + seg_base + w / C;
+            const uint32_t ww = *slot;
+            const Ctx x{vars, t, word_base(ww, m)};
+            const uint4 L1 = load_quad(m.locs + word_rec(ww, m), 1);
+            const uint32_t first = L1.x;            // edge_first
+            const int ne = (int)(L1.y & 0xFFFFu);   // edge_n
+            const uint64_t mask = enabled_mask_by_lanes(first, ne, x, m, S, sl, seg_base, seg_ones);
+            if (mask) {
+                const int i = pick_edge(mask, first, L1.z, L1.w, seed, run, step, (uint32_t)w, x, m);
+                const uint4 head = fire_updates(first + i, x, m, q);
+                *slot = (head.x << m.rec_shift) | x.base;
+                if (TRACE) {
+                    int32_t *wloc = (int32_t *)words_of + 64 * C + (w % C) * 64 + seg_base + w / C;
+                    const int32_t lw = *wloc;
+                    digest = smc_mix(digest, ((uint64_t)step << 40) | ((uint64_t)w << 20) |
+                                                 (uint64_t)(m.loc_edge0[lw] + i));
+                    wave_sync();  // every lane has read the location
+                    *wloc = lw + rec_at(m.edges, first + i)->dst;
                 }
-            const SMC_CONSTANT InstDesc *I = opaque(inst);
-            const double value = I->p.is_max ? qmax : qmin;
-            if (TRACE) {
-                digest = smc_mix(digest, smc_digest_bits(t));
-                for (int v = 0; v < I->m.n_vars; ++v)
-                    digest = smc_mix(digest, smc_digest_bits(I->m.var_clock[v] ? t - vars[v] : vars[v]));
-                for (int c = 0; c < I->m.n_comp; ++c) {
-                    const int lv = ((int32_t *)words_of)[64 * C + (c % C) * 64 + seg_base + c / C];
-                    digest = smc_mix(digest, (uint64_t)(uint32_t)lv);
-                }
-            }
-            if (sl == 0) {
-                uint8_t flag;
-                if (reach) flag = hit ? 1 : 0;
-                else flag = I->p.is_max ? (value > I->p.threshold) : (value < I->p.threshold);
-                I->p.flag[ridx] = flag;
-                I->p.value[ridx] = value;
-                I->p.steps[ridx] = step;
-                I->p.trans[ridx] = fired;
-                if (I->p.time) I->p.time[ridx] = t;
-                if (TRACE && I->p.digest) I->p.digest[ridx] = digest;
+                goal |= (head.y & SMC_EF_GOAL) != 0;
+                trans += sl == 0 ? 1u : 0u;
+                changed = true;
+                chan = (int)head.w > 0 ? (int)head.w : 0;
+                sender = chan > 0 ? w : -1;
             }
             wave_sync();
-            active = false;
         }
+        ++step;
     }
   }
 }

@@ -100,8 +100,15 @@ SMC_HD smc_u32x4 smc_draw(uint64_t seed, uint64_t run, uint32_t step,
     return smc_philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
 }
 
-/* Uniform double on (0, 1]: 53 random bits k, u = (k + 1) * 2^-53 (exact). */
+/* Uniform double on (0, 1]: 53 random bits k = hi * 2^21 + (lo >> 11),
+ * u = (k + 1) * 2^-53 (exact).  On the GPU the two halves are converted apart
+ * (there is no 64-bit conversion): both products and their sum are exact, so
+ * it is the same value. */
 SMC_HD double smc_u01(uint32_t hi, uint32_t lo) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return fma((double)hi, 2.3283064365386962890625e-10,
+               (double)((lo >> 11) + 1u) * 1.1102230246251565404236316680908203125e-16);
+#endif
     uint64_t k = ((uint64_t)hi << 21) | (uint64_t)(lo >> 11);
     return (double)(k + 1u) * 1.1102230246251565404236316680908203125e-16;
 }
