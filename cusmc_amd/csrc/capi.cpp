@@ -34,7 +34,7 @@ namespace {
 
 // Launch shape for one group of instances.
 struct Plan {
-    int S = 1, C = 1, R = 64, stride = 1, scratch = 1;
+    int S = 1, C = 1, R = 64, stride = 1;
     int occ = 0;  // run-kernel build: 0 registers unrestricted, 3 three waves per SIMD
     bool tab = false;     // tables staged in LDS
     int group_waves = 1;  // waves per workgroup
@@ -53,10 +53,10 @@ int tree_levels(int S) {
     return levels;
 }
 
-// LDS of one wave (sim_body.h): variables of its R runs, scratch, state words
-// and, with digests, locations.
-size_t wave_lds_bytes(int R, int stride, int scratch, int C, bool trace) {
-    return ((size_t)R * stride * 8 + (size_t)scratch * 512 + (size_t)C * 256 * (trace ? 2 : 1) + 15) & ~(size_t)15;
+// LDS of one wave (sim_body.h): variables of its R runs, state words and,
+// with digests, locations.
+size_t wave_lds_bytes(int R, int stride, int C, bool trace) {
+    return ((size_t)R * stride * 8 + (size_t)C * 256 * (trace ? 2 : 1) + 15) & ~(size_t)15;
 }
 
 // The most variables a packing may hold: those of the packed runs, a clock
@@ -79,12 +79,11 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
     pl.C = P / S;
     if (pl.C > 16) throw std::runtime_error("limit: more than 16 components per lane; use more lanes per run");
     pl.R = 64 / S;
-    pl.stride = m->img.n_vars | 1;
+    pl.stride = (m->img.n_vars + 1) | 1;  // the variables and a constant 0
     const int levels = tree_levels(S);
     if (!vars_fit(pl.R, m->img.n_vars, levels))
         throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
-    pl.scratch = std::max(pl.C, levels);
-    const size_t wave = wave_lds_bytes(pl.R, pl.stride, pl.scratch, pl.C, trace);
+    const size_t wave = wave_lds_bytes(pl.R, pl.stride, pl.C, trace);
     pl.wave_lds = (uint32_t)wave;
     if (want.tables) {
         pl.table_bytes = m->table_bytes;
@@ -360,7 +359,6 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         lp.inst = m->d_inst;
         lp.n_inst = 1;
         lp.var_stride = pl.stride;
-        lp.scratch = pl.scratch;
         lp.total_chunks = pl.total_chunks;
         lp.counter = m->d_counter;
         lp.round = nullptr;
@@ -448,7 +446,6 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         lp.inst = d_inst;
         lp.n_inst = 1;
         lp.var_stride = pl.stride;
-        lp.scratch = pl.scratch;
         lp.total_chunks = pl.total_chunks;
         lp.counter = d_counter;
         lp.round = nullptr;
@@ -663,7 +660,7 @@ namespace {
 struct BatchShape {
     std::vector<InstDesc> inst;
     size_t wave_lds = 0;
-    int scratch = 1;
+    int levels = 0;
     uint64_t chunks = 0;
 };
 
@@ -682,7 +679,6 @@ BatchShape batch_shape(smc_batch *b, int C, int waves, uint64_t runs_override) {
         const int R = 64 / S;
         const int levels = tree_levels(S);
         fits = fits && vars_fit(R, b->max_vars, levels);
-        sh.scratch = std::max(sh.scratch, std::max(C, levels));
         max_R = std::max(max_R, R);
         const uint64_t n = runs_override ? std::min<uint64_t>(runs_override, it.n_runs) : it.n_runs;
         uint64_t k = (per_wave + 4ull * R - 1) / (4ull * R);
@@ -698,7 +694,7 @@ BatchShape batch_shape(smc_batch *b, int C, int waves, uint64_t runs_override) {
         sh.inst.push_back(d);
     }
     if (!fits) throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
-    sh.wave_lds = wave_lds_bytes(max_R, b->stride, sh.scratch, C, false);
+    sh.wave_lds = wave_lds_bytes(max_R, b->stride, C, false);
     return sh;
 }
 
@@ -738,7 +734,7 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
         for (hipEvent_t *e : {&b->ev0, &b->ev1}) hip_check(hipEventCreate(e), "hipEventCreate");
         const int cu = items[0].model->cu_count;
         b->max_vars = max_vars;
-        b->stride = max_vars | 1;
+        b->stride = (max_vars + 1) | 1;  // the variables and a constant 0
         b->bufs.resize(n_items);
         uint64_t maxr = 0;
         for (int i = 0; i < n_items; ++i) {
@@ -769,7 +765,6 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
             b->lp.inst = b->d_all;
             b->lp.n_inst = n_items;
             b->lp.var_stride = b->stride;
-            b->lp.scratch = sh.scratch;
             b->lp.total_chunks = sh.chunks;
             b->lp.counter = b->d_counter;
             b->lp.round = b->d_round;

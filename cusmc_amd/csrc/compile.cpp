@@ -644,42 +644,48 @@ ModelImage lower(const smc_network &n, bool use_locals) {
 
             // what a race step looks at
             DevHot &h = R.hot;
-            auto hot_var = [&](uint16_t v) { inline_var(v, &h.var, &h.flags); };
+            uint32_t hf = 0;
+            uint16_t hot_at = (uint16_t)(n.n_vars * 8u), hot_local = 0;  // the constant 0
+            h.a = -HUGE_VAL;
+            h.b = HUGE_VAL;
             if (d.klass == SMC_K_ZERO) {
-                h.flags = SMC_HF_ZERO;
+                hf = SMC_HF_ZERO;
+                h.rate = -0.0;
             } else {
                 if (img.freeze && kind == 1) {
-                    h.rate = 0.0;  // out of the race unless bounded
+                    hf |= SMC_HF_DEAD;
                 } else if (d.rate_const) {
                     h.rate = d.rate_value > 0.0 ? d.rate_value : 0.0;
                 } else {
-                    h.flags |= SMC_HF_EXPR | (reads_local(L.rate) ? SMC_HF_EXPR_LOCAL : 0);
-                    h.rate_ref = d.rate;
-                    if ((h.flags & SMC_HF_EXPR_LOCAL) || (n_rates && img.one_rate != d.rate)) n_rates = 2;
+                    const bool own = reads_local(L.rate);
+                    hf |= SMC_HF_EXPR | (own ? SMC_HF_EXPR_LOCAL : 0);
+                    if (own || (n_rates && img.one_rate != d.rate)) n_rates = 2;
                     else n_rates = std::max(n_rates, 1);
                     img.one_rate = d.rate;
                 }
                 if (d.n_inv == 1 && R.invs[0].bound_const) {
-                    h.flags |= SMC_HF_INV;
-                    hot_var(R.invs[0].var);
+                    hf |= SMC_HF_INV;
+                    inline_var(R.invs[0].var, &hot_at, &hot_local);
                     h.a = R.invs[0].bound_value;
                     h.b = R.invs[0].strict ? 1e-6 : 0.0;
                 } else if (d.n_inv) {
-                    h.flags |= SMC_HF_XINV;
+                    hf |= SMC_HF_XINV;
                 }
                 if (img.freeze && kind == 2) {
-                    if (R.block.size() == 1 && (R.block[0].flags & SMC_GF_RANGE) && !(h.flags & SMC_HF_INV)) {
-                        h.flags |= SMC_HF_GUARD;
-                        hot_var(R.block[0].var);
+                    if (R.block.size() == 1 && (R.block[0].flags & SMC_GF_RANGE) && !(hf & SMC_HF_INV)) {
+                        hf |= SMC_HF_GUARD;
+                        inline_var(R.block[0].var, &hot_at, &hot_local);
                         h.a = R.block[0].lo;
                         h.b = R.block[0].hi;
                     } else {
-                        h.flags |= SMC_HF_XBLK;
+                        hf |= SMC_HF_XBLK;
                     }
                 }
             }
+            h.what = (uint32_t)hot_at | (hf << 16);
+            h.base = hot_local ? 0x1FFFu : 0u;
             for (RawEdge &re : R.edges) inline_edge(re);
-            img.tests |= h.flags & ~(uint32_t)SMC_HF_LOCAL;
+            img.tests |= hf;
         }
     }
 
@@ -694,6 +700,9 @@ ModelImage lower(const smc_network &n, bool use_locals) {
     if (use_locals && n_cls >= (1u << 18)) return lower(n, false);
     img.rec_shift = use_locals ? 13 : 0;
     img.hots.assign(n_cls + 1, DevHot{});
+    img.hots[0].a = -HUGE_VAL;
+    img.hots[0].b = HUGE_VAL;
+    img.hots[0].what = (uint16_t)(n.n_vars * 8u);
     img.locs.assign(n_cls + 1, DevLoc{});
     std::vector<uint8_t> done(n_cls, 0);
     std::unordered_map<std::string, uint32_t> gmap, umap, emap, imap;

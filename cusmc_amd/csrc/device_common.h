@@ -134,6 +134,56 @@ __device__ __forceinline__ double seg_xchg(double x, int k) {
     }
 }
 
+// The lower and the upper half's value at level k of such a reduction, on
+// every lane of the two halves: quad permutes, row shifts into one half of
+// the banks, and swaps of rows; none goes through LDS.
+__device__ __forceinline__ void seg_halves(double x, int k, double &lower, double &upper) {
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    switch (k) {
+    case 0:
+        lower = dpp_f64<0xA0>(x);  // quad_perm [0,0,2,2]
+        upper = dpp_f64<0xF5>(x);  // quad_perm [1,1,3,3]
+        return;
+    case 1:
+        lower = dpp_f64<0x44>(x);  // quad_perm [0,1,0,1]
+        upper = dpp_f64<0xEE>(x);  // quad_perm [2,3,2,3]
+        return;
+    case 2:  // row_shr:4 into banks 1 and 3, row_shl:4 into banks 0 and 2
+        lower = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x114, 0xF, 0xA, false),
+                                 __builtin_amdgcn_update_dpp(lo, lo, 0x114, 0xF, 0xA, false));
+        upper = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x104, 0xF, 0x5, false),
+                                 __builtin_amdgcn_update_dpp(lo, lo, 0x104, 0xF, 0x5, false));
+        return;
+    case 3:  // row_shr:8 into banks 2 and 3, row_shl:8 into banks 0 and 1
+        lower = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x118, 0xF, 0xC, false),
+                                 __builtin_amdgcn_update_dpp(lo, lo, 0x118, 0xF, 0xC, false));
+        upper = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x108, 0xF, 0x3, false),
+                                 __builtin_amdgcn_update_dpp(lo, lo, 0x108, 0xF, 0x3, false));
+        return;
+    case 4: {
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        lower = __hiloint2double((int)h[0], (int)l[0]);
+        upper = __hiloint2double((int)h[1], (int)l[1]);
+        return;
+    }
+    default: {
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        lower = __hiloint2double((int)h[0], (int)l[0]);
+        upper = __hiloint2double((int)h[1], (int)l[1]);
+        return;
+    }
+    }
+}
+
+// Lanes of the upper halves at level k.
+__device__ __forceinline__ uint64_t upper_lanes(int k) {
+    constexpr uint64_t m[6] = {0xAAAAAAAAAAAAAAAAull, 0xCCCCCCCCCCCCCCCCull, 0xF0F0F0F0F0F0F0F0ull,
+                               0xFF00FF00FF00FF00ull, 0xFFFF0000FFFF0000ull, 0xFFFFFFFF00000000ull};
+    return m[k];
+}
+
 
 // Pairwise tree sum over the segment, as in the run kernel (in-lane levels,
 // then the butterfly); every lane gets the total.
@@ -422,12 +472,22 @@ __device__ __forceinline__ double eval_uniform(uint32_t ref, const Ctx &x, const
     return r0;
 }
 
+// Rotate slot arrays by one (slot 1 to the front): a rolled loop over the
+// slots then touches slot 0 only, a constant index, so the arrays stay in
+// registers.
+template <int C, class T>
+__device__ __forceinline__ void rotate_slots(T (&a)[C]) {
+    const T f = a[0];
+#pragma unroll
+    for (int k = 0; k < C - 1; ++k) a[k] = a[k + 1];
+    a[C - 1] = f;
+}
+
 // ------------------------------------------------------------ slots
 //
 // A lane's component slots are state words in LDS ([slot][lane]: 64 lanes
 // touch 64 consecutive words), so that loops over slots stay rolled where
-// they are cold and any lane can read any slot.  `scr` is 8 bytes per slot
-// and lane of scratch in the same layout.
+// they are cold and any lane can read any slot.
 template <class M>
 __device__ __forceinline__ uint32_t word_rec(uint32_t w, const M &m) { return w >> m.rec_shift; }
 template <class M>
@@ -699,28 +759,6 @@ __device__ __forceinline__ double window_of(const DevLoc &L, const Ctx &x, const
     return bounded ? M0 : -1.0;
 }
 
-// The slots whose component cannot fire before the next transition (frozen:
-// blocked, exponential now), their rates in the lane's scratch.  They leave
-// the race; a step raced in full takes them back, and the transition that
-// crosses the time bound still competes with their first null event after
-// the bound, drawn from their sum (memoryless races).
-template <int C, class M>
-__device__ __forceinline__ uint32_t frozen_rates(const uint32_t *words, double *scr, Ctx x, const M &m) {
-    uint32_t frozen = 0;
-#pragma clang loop unroll(disable)
-    for (int j = 0; j < C; ++j) {
-        const uint32_t w = words[64 * j];
-        const DevLoc L = load_rec(m.locs + word_rec(w, m));
-        x.base = word_base(w, m);
-        if (L.klass != SMC_K_ZERO && !(window_of(L, x, m) >= 0.0) &&
-            ((L.flags & SMC_LF_DEAD) || ((L.flags & SMC_LF_GUARDED) && location_blocked(L.block_first, x, m)))) {
-            scr[64 * j] = location_rate(L, x, m);
-            frozen |= 1u << j;
-        }
-    }
-    return frozen;
-}
-
 // Whether no component of the segment's run can fire again before the time
 // bound: each one is blocked, or is in a location whose rate and spontaneous
 // guards read no clock and has no enabled spontaneous edge or races at rate 0
@@ -752,77 +790,126 @@ __device__ __forceinline__ bool absorbed(const uint32_t *words, Ctx x, const M &
 template <int C>
 struct RaceSlots {
     double leaf[C];         // rate in the exponential race, 0 if not in it
-    uint32_t bounded;       // slots with a clock-bounded delay (window in the lane's scratch; 0: also in zero)
-    uint32_t zero;          // slots with delay 0
+    double left[C];         // window of a bounded slot (kept for up to two slots, else see slot_window)
+    uint32_t bounded;       // slots with a clock-bounded delay
+    uint32_t zero;          // slots that fire at once: zero-delay locations, bounds reached
 };
 
-// Classify the lane's slots and evaluate their rates: one straight line over
-// the lane's slots, each reading its class's 32-byte DevHot record and its
-// variable.  No branch depends on a lane or a slot: the lanes of a wave hold
-// components in every kind of location, so branches would run every kind's
-// code for every slot, and they would keep the slots' reads, a chain of three
-// each, from overlapping.  Invariants and blocking tests beyond one record
-// take a rolled loop afterwards, on models that have them; xblk keeps those
-// blocking results until the next change of state.
-template <int C, class M>
-__device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *words, double *scr, Ctx x, const M &m,
-                                           bool changed, uint32_t &xblk) {
-    const uint32_t tests = m.tests;
-    uint32_t bounded = 0, zero = 0;
-    uint32_t expr = 0;     // slots whose rate is still to be evaluated
-    uint32_t own = 0;
-    uint32_t ref[C];
-    // a network with one rate expression: evaluated once, for every slot
-    const bool one = m.one_rate != SMC_NO_REF;
-    double shared = 0.0;
-    if (one) {
-        shared = eval_uniform(m.one_rate, x, m);
-        shared = shared > 0.0 ? shared : 0.0;
+// A record's variable, given the component's state word.
+__device__ __forceinline__ double hot_value(const DevHot &h, uint32_t word, const double *vars) {
+    return *(const double *)((const char *)vars + ((word & h.base) << 3) + (h.what & 0xFFFFu));
+}
+
+// The delay window of slot j, which is bounded.
+template <class M>
+__device__ __forceinline__ double slot_window(const uint32_t *words, int j, Ctx x, const M &m) {
+    const uint32_t w = words[64 * j];
+    const DevHot h = load_rec(m.hots + word_rec(w, m));
+    double left = h.a - (x.now - hot_value(h, w, x.vars)) - h.b;
+    const bool other = (h.what & (SMC_HF_XINV << 16)) != 0;
+    if (unlikely(any_lane(other))) {
+        if (other) {
+            x.base = word_base(w, m);
+            left = window_of(load_rec(m.locs + word_rec(w, m)), x, m);
+        }
     }
-    auto flag = [](uint32_t d, uint32_t f, uint32_t bit) { return (d & (f << 16)) ? bit : 0u; };
-    if (tests & (SMC_HF_INV | SMC_HF_GUARD)) {
-        DevHot h[C];
-        uint32_t base[C];
-        double v[C];
+    return left;
+}
+
+// Classify the lane's slots: one straight line over them, each reading its
+// class's 32-byte record and its variable.  No branch depends on a lane or a
+// slot: the lanes of a wave hold components in every kind of location, so
+// branches would run every kind's code for every slot, and they would keep
+// the slots' reads, a chain of three each, from overlapping.  What only some
+// slots of a step need (the length of a bounded delay, rates that are
+// expressions) is left to later passes over those.  17 vector instructions a
+// slot; with delays, expressions and zero tests in line it was 40.
+// TESTS: some location has an invariant or a guard; RATE: 0 all rates are
+// constant, 1 one expression of the value `shared`, 2 several (bits expr).
+//
+// Slot masks collect one bit a slot by shifting: bit 31 of a word (the sign
+// of a zero delay's rate), or the lane's bit of a comparison's result as the
+// carry of an addition, the last slot first.
+__device__ __forceinline__ uint32_t shift_in_sign(uint32_t mask, uint32_t word) {
+    return __builtin_amdgcn_alignbit(mask, word, 31);
+}
+__device__ __forceinline__ uint32_t shift_in(uint32_t mask, bool c) {
+    const uint64_t lanes = __ballot(c);
+    asm("v_addc_co_u32 %0, vcc, %0, %0, %1" : "+v"(mask) : "s"(lanes) : "vcc");
+    return mask;
+}
+
+template <int C, bool TESTS, int RATE, class M>
+__device__ __forceinline__ void classify(RaceSlots<C> &rs, const uint32_t *words, const Ctx &x, const M &m,
+                                         double shared, uint32_t &expr, uint32_t &own) {
+    // slots read at a time: registers for their records
+    constexpr int G = C > 8 ? 8 : C;
+    uint32_t bounded = 0, ahead = 0, zero = 0;
 #pragma unroll
-        for (int j = 0; j < C; ++j) {
-            const uint32_t w = words[64 * j];
-            base[j] = word_base(w, m);
-            h[j] = load_rec(m.hots + word_rec(w, m));
+    for (int j0 = C - G; j0 >= 0; j0 -= G) {
+        uint32_t w[G];
+        DevHot h[G];
+        double v[G];
+#pragma unroll
+        for (int j = 0; j < G; ++j) w[j] = words[64 * (j0 + j)];
+#pragma unroll
+        for (int j = 0; j < G; ++j) h[j] = load_rec(m.hots + word_rec(w[j], m));
+        if (TESTS) {
+#pragma unroll
+            for (int j = 0; j < G; ++j) v[j] = hot_value(h[j], w[j], x.vars);
         }
 #pragma unroll
-        for (int j = 0; j < C; ++j)
-            v[j] = *(const double *)((const char *)x.vars + h[j].var + __umul24(base[j], h[j].flags & SMC_HF_LOCAL));
-#pragma unroll
-        for (int j = 0; j < C; ++j) {
-            const uint32_t bit = 1u << j, d = (uint32_t)h[j].flags << 16;
-            const double left = h[j].a - (x.now - v[j]) - h[j].b;
-            const bool bnd = ((int32_t)d < 0) & (left >= 0.0);
-            const bool out = ((d & (SMC_HF_GUARD << 16)) != 0) & !((h[j].a <= v[j]) & (v[j] <= h[j].b));
-            const bool in = !(bnd | out);
-            scr[64 * j] = left;  // read only if bounded
-            bounded |= bnd ? bit : 0u;
-            zero |= (bnd & (left == 0.0)) ? bit : 0u;
-            zero |= flag(d, SMC_HF_ZERO, bit);
-            const double rate = (d & (SMC_HF_EXPR << 16)) ? shared : h[j].rate;
-            rs.leaf[j] = in ? rate : 0.0;
-            ref[j] = h[j].rate_ref;
-            expr |= in ? flag(d, SMC_HF_EXPR, bit) : 0u;
-            own |= flag(d, SMC_HF_EXPR_LOCAL, bit);
+        for (int j = G - 1; j >= 0; --j) {
+            const uint32_t bit = 1u << (j0 + j), d = h[j].what;
+            double rate = h[j].rate;
+            zero = shift_in_sign(zero, (uint32_t)__double2hiint(rate));
+            if (RATE == 1) rate = (d & (SMC_HF_EXPR << 16)) ? shared : rate;
+            bool in = true;
+            if (TESTS) {
+                // an invariant x <= a holds the delay to a - x - b while that
+                // is not negative (a - x >= b), and at 0 makes it a zero delay
+                const double ax = h[j].a - (x.now - v[j]);
+                const bool inv = (int32_t)d < 0;
+                const bool bnd = inv & (ax >= h[j].b);
+                const bool inside = (h[j].a <= v[j]) & (v[j] <= h[j].b);
+                in = inv ? !bnd : inside;
+                bounded = shift_in(bounded, bnd);
+                ahead = shift_in(ahead, ax > h[j].b);
+                if (C <= 2) rs.left[j] = ax - h[j].b;
+            }
+            rs.leaf[j0 + j] = in ? rate : 0.0;
+            if (RATE == 2) {
+                expr |= (in & ((d & (SMC_HF_EXPR << 16)) != 0)) ? bit : 0u;
+                own |= (d & (SMC_HF_EXPR_LOCAL << 16)) ? bit : 0u;
+            }
         }
+        if (j0) __builtin_amdgcn_sched_barrier(0);
+    }
+    rs.bounded = bounded;
+    rs.zero = zero | (bounded & ~ahead);
+}
+
+// The same, with the invariants, blocking tests and rates that take more than
+// a record, on models that have them.  xblk keeps the blocking results until
+// the next change of state.
+template <int C, class M>
+__device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *words, Ctx x, const M &m, bool changed,
+                                           uint32_t &xblk) {
+    const uint32_t tests = m.tests;
+    uint32_t expr = 0;     // slots whose rate is still to be evaluated
+    uint32_t own = 0;      // ... from private variables
+    const bool with_tests = (tests & (SMC_HF_INV | SMC_HF_GUARD)) != 0;
+    if (!(tests & SMC_HF_EXPR)) {
+        if (with_tests) classify<C, true, 0>(rs, words, x, m, 0.0, expr, own);
+        else classify<C, false, 0>(rs, words, x, m, 0.0, expr, own);
+    } else if (m.one_rate != SMC_NO_REF) {
+        // one rate expression: evaluated once, for every slot
+        double shared = eval_uniform(m.one_rate, x, m);
+        shared = shared > 0.0 ? shared : 0.0;
+        if (with_tests) classify<C, true, 1>(rs, words, x, m, shared, expr, own);
+        else classify<C, false, 1>(rs, words, x, m, shared, expr, own);
     } else {
-        DevHot h[C];
-#pragma unroll
-        for (int j = 0; j < C; ++j) h[j] = load_rec(m.hots + word_rec(words[64 * j], m));
-#pragma unroll
-        for (int j = 0; j < C; ++j) {
-            const uint32_t bit = 1u << j, d = (uint32_t)h[j].flags << 16;
-            zero |= flag(d, SMC_HF_ZERO, bit);
-            rs.leaf[j] = (d & (SMC_HF_EXPR << 16)) ? shared : h[j].rate;
-            ref[j] = h[j].rate_ref;
-            expr |= flag(d, SMC_HF_EXPR, bit);
-            own |= flag(d, SMC_HF_EXPR_LOCAL, bit);
-        }
+        classify<C, true, 2>(rs, words, x, m, 0.0, expr, own);
     }
     if (tests & (SMC_HF_XINV | SMC_HF_XBLK)) {
         if (changed) xblk = 0;
@@ -830,17 +917,18 @@ __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *wor
 #pragma clang loop unroll(disable)
         for (int j = 0; j < C; ++j) {
             const uint32_t w = words[64 * j], bit = 1u << j;
-            const uint32_t f = m.hots[word_rec(w, m)].flags;
+            const uint32_t f = m.hots[word_rec(w, m)].what >> 16;
             if (f & (SMC_HF_XINV | SMC_HF_XBLK)) {
                 const DevLoc L = load_rec(m.locs + word_rec(w, m));
                 x.base = word_base(w, m);
                 if (f & SMC_HF_XINV) {
-                    const double M0 = window_of(L, x, m);
-                    if (M0 >= 0.0) {
-                        if (M0 == 0.0) zero |= bit;
-                        bounded |= bit;
-                        scr[64 * j] = M0;
+                    const double left = window_of(L, x, m);
+                    if (left >= 0.0) {
+                        rs.bounded |= bit;
+                        if (left == 0.0) rs.zero |= bit;
                         out |= bit;
+                        if (j == 0) rs.left[0] = left;  // (constant indices: the array stays in registers)
+                        else if (C == 2) rs.left[C - 1] = left;
                     }
                 }
                 if ((f & SMC_HF_XBLK) && changed && location_blocked(L.block_first, x, m)) xblk |= bit;
@@ -851,22 +939,23 @@ __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *wor
 #pragma unroll
         for (int j = 0; j < C; ++j) rs.leaf[j] = ((out >> j) & 1u) ? 0.0 : rs.leaf[j];
     }
-    rs.bounded = bounded;
-    rs.zero = zero;
     // Rates that are expressions: each pass evaluates, on every lane at once,
     // the expression of the lane's first pending slot and hands the value to
     // all of its pending slots with the same expression (unless it reads the
     // component's own variables).  Evaluated slot by slot, the interpreter
     // would run up to C times per race; here once per distinct expression a
     // lane holds.
-    if ((tests & SMC_HF_EXPR) && !one) {
-        while (__ballot(expr != 0)) {
+    if ((tests & SMC_HF_EXPR) && m.one_rate == SMC_NO_REF) {
+        uint32_t ref[C];
+#pragma unroll
+        for (int j = 0; j < C; ++j) ref[j] = m.locs[word_rec(words[64 * j], m)].rate;
+        while (any_lane(expr != 0)) {
             double v = 0.0;
-            uint32_t r = 0xFFFFFFFFu, first = 0;
+            uint32_t r = SMC_NO_REF, first = 0;
             if (expr) {
                 first = expr & -expr;
                 const uint32_t w = words[64 * (__ffs(first) - 1)];
-                r = m.hots[word_rec(w, m)].rate_ref;
+                r = m.locs[word_rec(w, m)].rate;
                 x.base = word_base(w, m);
                 v = eval_ref(r, x, m);
                 v = v > 0.0 ? v : 0.0;
@@ -883,12 +972,80 @@ __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *wor
     }
 }
 
+// The rate of slot j if its component is frozen: exponential now and unable
+// to fire before the next transition (dead, or blocked by the variables).
+// Frozen components leave the race; a step raced in full takes them back,
+// and the transition that crosses the time bound still competes with their
+// first null event after the bound, drawn from their sum (memoryless races).
+template <class M>
+__device__ __forceinline__ bool frozen_slot(const uint32_t *words, int j, Ctx x, const M &m, double *rate) {
+    const uint32_t w = words[64 * j];
+    const DevHot h = load_rec(m.hots + word_rec(w, m));
+    const uint32_t d = h.what >> 16;
+    const double v = hot_value(h, w, x.vars);
+    const bool bnd = (d & SMC_HF_INV) && h.a - (x.now - v) >= h.b;
+    bool frozen = (d & SMC_HF_DEAD) || ((d & SMC_HF_GUARD) && !(h.a <= v && v <= h.b));
+    frozen = frozen && !bnd;
+    *rate = h.rate;
+    const bool other = (d & (SMC_HF_XINV | SMC_HF_XBLK)) || (frozen && (d & (SMC_HF_DEAD | SMC_HF_EXPR)));
+    if (any_lane(other)) {
+        if (other) {
+            const DevLoc L = load_rec(m.locs + word_rec(w, m));
+            x.base = word_base(w, m);
+            if (d & (SMC_HF_XINV | SMC_HF_XBLK))
+                frozen = !bnd && !((d & SMC_HF_XINV) && window_of(L, x, m) >= 0.0) &&
+                         (frozen || ((d & SMC_HF_XBLK) && location_blocked(L.block_first, x, m)));
+            if (frozen) *rate = location_rate(L, x, m);
+        }
+    }
+    return frozen;
+}
+
+// Their sum on the race tree (every lane of the segment gets it): leaves in
+// order, each completed pair added up at once.
+template <int C, class M>
+__device__ __forceinline__ double frozen_total(const uint32_t *words, const Ctx &x, const M &m, int S) {
+    double half[4] = {0.0, 0.0, 0.0, 0.0}, s = 0.0;
+#pragma clang loop unroll(disable)
+    for (int j = 0; j < C; ++j) {
+        double r;
+        const bool frozen = frozen_slot(words, j, x, m, &r);
+        s = frozen ? r : 0.0;
+#pragma unroll
+        for (int k = 0; (1 << k) < C; ++k) {
+            if (!((j >> k) & 1)) {
+                half[k] = s;
+                break;
+            }
+            s = half[k] + s;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        if ((1 << k) >= S) break;
+        s = s + seg_xchg(s, k);
+    }
+    return s;
+}
+
+// Frozen slots back into the race (their leaves are 0).
+template <int C, class M>
+__device__ __forceinline__ void race_frozen(RaceSlots<C> &rs, const uint32_t *words, const Ctx &x, const M &m) {
+#pragma clang loop unroll(disable)
+    for (int j = 0; j < C; ++j) {
+        double r;
+        if (frozen_slot(words, j, x, m, &r)) rs.leaf[0] = r;
+        rotate_slots<C>(rs.leaf);
+    }
+}
+
 // The exponential race over the segment: a fixed pairwise tree over the
 // leaves (in-lane levels, then a butterfly).  `level` keeps each level's own
-// partial sum per lane in LDS (level-major) from the sum to the descent; the
-// sibling's is exchanged again.  Returns the total.
+// partial sum from the sum to the descent (12 registers; in LDS, read back
+// and exchanged through it again, the two took 40 instructions and several
+// hundred cycles more on a full segment).  Returns the total.
 template <int C>
-__device__ __forceinline__ double race_total(const double (&leaf)[C], double *level, int S) {
+__device__ __forceinline__ double race_total(const double (&leaf)[C], double (&level)[6], int S) {
     double tr[2 * C];
 #pragma unroll
     for (int j = 0; j < C; ++j) tr[C + j] = leaf[j];
@@ -899,28 +1056,34 @@ __device__ __forceinline__ double race_total(const double (&leaf)[C], double *le
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
         if ((1 << k) >= S) break;
-        level[64 * k] = s;
-        s = s + seg_xchg(s, k);
+        level[k] = s;
+        if (k < 4) {
+            s = s + seg_xchg(s, k);
+        } else {
+            double lower, upper;
+            seg_halves(s, k, lower, upper);
+            s = lower + upper;
+        }
     }
     return s;
 }
 
 // The component reached by descending the tree with v in [0, total): left
-// while v is below the left sum (or the right one is 0).  Every lane of the
-// segment gets it.
+// while v is below the left sum (or the right one is 0).  Each lane follows
+// the path to itself; the one whose path the descent takes at every level
+// (`on`) has it.  Every lane of the segment gets the component.
 template <int C>
-__device__ __forceinline__ int race_pick(const double (&leaf)[C], const double *level, double v, int S, int sl,
+__device__ __forceinline__ int race_pick(const double (&leaf)[C], const double (&level)[6], double v, int S,
                                          int seg_base, uint64_t seg_mask) {
-    int b = 0;
-    const int at = lane_here(sl);
+    uint64_t on = seg_mask;
 #pragma unroll
     for (int k = 5; k >= 0; --k) {
         if ((1 << k) < S) {
-            const bool in_left = ((at >> k) & 1) == 0;
-            const double own = level[64 * k], sib = seg_xchg(own, k);
-            const double left = in_left ? own : sib;
-            const double right = in_left ? sib : own;
-            if (!(v < left || right == 0.0)) { v = v - left; b += 1 << k; }
+            double left, right;
+            seg_halves(level[k], k, left, right);
+            const bool upper = __builtin_amdgcn_inverse_ballot_w64(upper_lanes(k));
+            on &= __ballot((v < left) | (right == 0.0)) ^ upper_lanes(k);
+            v = v - (upper ? left : 0.0);
         }
     }
     // the lane's tree again, from the same leaves (same sums), halved at
@@ -945,7 +1108,7 @@ __device__ __forceinline__ int race_pick(const double (&leaf)[C], const double *
             for (int j = 0; j < half; ++j) cur[j] = go_left ? cur[j] : cur[half + j];
         }
     }
-    const int Lw = lowest_lane(__ballot(sl == b) & seg_mask);
+    const int Lw = on ? lowest_lane(on) : seg_base;
     return (Lw - seg_base) * C + __shfl(node, Lw);
 }
 
@@ -967,7 +1130,7 @@ __device__ __forceinline__ int race_pick(const double (&leaf)[C], const double *
 // the network's locations beside the state words; `trans` counts this
 // lane's.
 template <int C, bool TRACE, bool LOCS, class M>
-__device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int32_t *locs, Ctx x, const M &m, int chan,
+__device__ __forceinline__ void fire_receivers(uint32_t *words, int32_t *locs, Ctx x, const M &m, int chan,
                                                int sender, LaneQuery &q, bool &goal, uint64_t seed, uint64_t run,
                                                uint32_t step, int lane, int sl, int S, int seg_base, uint64_t seg_mask,
                                                uint32_t &trans, uint64_t &digest) {
@@ -988,26 +1151,24 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int
         }
     }
     uint64_t slow = 0;
+    uint32_t mk_hi[C];  // edges past the 32nd (only where receivers fire one at a time)
+#pragma unroll
+    for (int j = 0; j < C; ++j) mk_hi[j] = 0;
     if (any_lane(other != 0)) {
-        // enabled sets by edge, kept in the scratch (64 bits per slot)
-        uint64_t *set = (uint64_t *)scr;
         bool serial = false;
 #pragma clang loop unroll(disable)
         for (int j = 0; j < C; ++j) {
-            uint64_t e = 0;
             if ((other >> j) & 1u) {
                 const uint32_t w = words[64 * j];
                 const DevLoc L = load_rec(m.locs + word_rec(w, m));
                 x.base = word_base(w, m);
-                e = enabled_mask(L.edge_first, L.edge_n, chan, x, m);
+                const uint64_t e = enabled_mask(L.edge_first, L.edge_n, chan, x, m);
                 if (e && !(L.flags & SMC_LF_RECV_FAST)) serial = true;
+                mk[0] = (uint32_t)e;
+                mk_hi[0] = (uint32_t)(e >> 32);
             }
-            set[64 * j] = e;
-        }
-#pragma unroll
-        for (int j = 0; j < C; ++j) {
-            if ((other >> j) & 1u) mk[j] = (uint32_t)set[64 * j];
-            else set[64 * j] = mk[j];
+            rotate_slots<C>(mk);
+            rotate_slots<C>(mk_hi);
         }
         slow = __ballot(serial) & seg_mask;
     }
@@ -1135,15 +1296,14 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int
     } else {
         // one at a time: the lanes holding enabled receivers in lane order,
         // their slots in slot order; each picks with its own stream
-        const uint64_t *set = (const uint64_t *)scr;
         bool any = false;
-#pragma clang loop unroll(disable)
-        for (int j = 0; j < C; ++j) any |= set[64 * j] != 0;
+#pragma unroll
+        for (int j = 0; j < C; ++j) any |= (mk[j] | mk_hi[j]) != 0;
         for (uint64_t lanes_with = __ballot(any) & seg_mask; lanes_with; lanes_with &= lanes_with - 1) {
             const int L = lowest_lane(lanes_with);
 #pragma clang loop unroll(disable)
             for (int j = 0; j < C; ++j) {
-                const uint64_t mask = set[64 * j];
+                const uint64_t mask = ((uint64_t)mk_hi[0] << 32) | mk[0];
                 if ((__ballot(mask != 0) >> L) & 1ull) {
                     const int c = (L - seg_base) * C + j;
                     int e_fired = -1;  // the network's index of the fired edge (digests)
@@ -1165,6 +1325,8 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, double *scr, int
                         digest = smc_mix(digest, ((uint64_t)step << 40) | ((uint64_t)c << 20) | (uint64_t)e);
                     }
                 }
+                rotate_slots<C>(mk);
+                rotate_slots<C>(mk_hi);
             }
         }
     }

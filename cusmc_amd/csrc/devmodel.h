@@ -80,14 +80,14 @@ enum {
     SMC_LF_RECV_TWO = 16    // recv_chan > 0 and exactly two receive edges
 };
 
-// What a race step has to look at in a location (DevHot.flags).
+// What a race step has to look at in a location (high half of DevHot.what).
 enum {
-    SMC_HF_LOCAL = 0xFF,    // the variable counts from the component's base: 8 (bytes) or 0
     SMC_HF_ZERO = 0x100,    // zero delay
-    SMC_HF_EXPR = 0x200,    // the rate is the expression rate_ref
+    SMC_HF_EXPR = 0x200,    // the rate is an expression (DevLoc.rate)
     SMC_HF_EXPR_LOCAL = 0x400,  // ... which reads private variables
     SMC_HF_XINV = 0x800,    // other invariants: DevInv records
     SMC_HF_XBLK = 0x1000,   // other blocking tests: guard records from block_first
+    SMC_HF_DEAD = 0x2000,   // out of the race unless bounded
     SMC_HF_GUARD = 0x4000,  // leaves the race while its variable is outside [a, b]
     SMC_HF_INV = 0x8000     // one invariant with a constant bound: a = bound, b = 1e-6 if strict
 };
@@ -100,14 +100,16 @@ struct DevInsn {
 
 // The part of a location that every race step reads for every component, 32
 // bytes: two 16-byte LDS reads.  `rate` is what the component races at if
-// nothing else holds (0 for a zero-delay location, for one that can never
-// fire, and for a rate that is not positive).
+// nothing else holds (-0, with its sign bit, for a zero-delay location and
+// only there; 0 for one that can never fire and for a rate that is not
+// positive).  A location with neither
+// invariant nor guard tests a constant 0 (kept behind the run's variables)
+// against [-inf, inf], so that all take the same steps.
 struct DevHot {
     double rate;
     double a, b;
-    uint32_t rate_ref;
-    uint16_t var;           // byte offset of the invariant's or guard's variable
-    uint16_t flags;         // SMC_HF_*
+    uint32_t what;          // low half: the variable's byte offset; high half: SMC_HF_*
+    uint32_t base;          // mask of the state word's base: all ones if the variable is private, else 0
 };
 
 // The rest, 64 bytes: receive edges; spontaneous edges; invariants, blocking

@@ -567,7 +567,7 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         s->C = P / s->S;
         if (s->C > 8) throw std::runtime_error("internal: more than 8 slots per lane");
         s->R = 64 / s->S;
-        s->stride = img.n_vars | 1;
+        s->stride = (img.n_vars + 1) | 1;  // the variables and a constant 0
 
         s->n_locs = (int)img.info.size();
         s->n_vars = img.n_vars;
@@ -617,8 +617,8 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         s->G16 = (int)rup((size_t)std::max(s->n_groups, 1), 16);
         // advance kernel LDS: per wave the variables of its 64/S rows, their
         // tilt tables (theta and 2^theta, up to Gpad entries), slot scratch,
-        // race-tree levels, state words and locations (is_advance.h), after a
-        // shared part (tilt index and a shared 2^theta vector, Lpad each)
+        // state words and locations (is_advance.h), after a shared part (tilt
+        // index and a shared 2^theta vector, Lpad each)
         int levels = 0;
         while ((1 << levels) < s->S) ++levels;
         const size_t tilts = (size_t)s->R * s->Gpad * 12;
@@ -627,7 +627,7 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         if ((size_t)s->R * ((img.n_vars + 1) | 1) * 8 + tilts + (size_t)levels * 1024 > 60000)
             throw std::runtime_error("limit: variables exceed the LDS budget");
         s->wave_lds = (uint32_t)rup((size_t)s->R * s->stride * sizeof(double) + tilts +
-                                        (size_t)(s->C + levels) * 64 * sizeof(double) + (size_t)s->C * 512, 16);
+                                        (size_t)s->C * 64 * sizeof(double) + (size_t)s->C * 512, 16);
         {
             const size_t shared = (size_t)s->Lpad * 12;
             // hot tables staged in LDS when the model's tuned launch does so

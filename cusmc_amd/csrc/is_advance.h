@@ -97,7 +97,6 @@ struct TiltLds {
     double *row_ex;       // the wave's rows: [64/S][theta_cap] 2^theta
     float *row_th;        // [64/S][theta_cap] theta
     double *scr;          // the wave's slot scratch [C][64] (windows of bounded slots)
-    double *lvl;          // the wave's race-tree levels [log2(S)][64]
     uint32_t *words;      // state words [C][64]
     int32_t *locs;        // locations [C][64]
     double *rec;          // recording build: [C][64] rates, [C][64] int32 locations, [C][64] uint32 wins
@@ -138,6 +137,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
     LaneQuery q{P.qvar, st.qmax[row], st.qmin[row]};
     uint64_t digest = st.digest[row];
     for (int v = sl; v < m.n_vars; v += S) vars[v] = st.vars[(size_t)row * m.n_vars + v];
+    if (sl == 0) vars[m.n_vars] = 0.0;
     // recording build: per slot the starting location, the base cumulative
     // hazard over the macro-step's races and the wins, in LDS ([slot][lane])
     double *hz = tl.rec + lane;
@@ -194,10 +194,10 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
     auto receivers = [&]() {
         bool entered = false;
         if (P.trace)
-            fire_receivers<C, true, true>(words, scr, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, P.seed, run,
+            fire_receivers<C, true, true>(words, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, P.seed, run,
                                           step, lane, sl, S, seg_base, seg_mask, trans, digest);
         else
-            fire_receivers<C, false, true>(words, scr, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, P.seed, run,
+            fire_receivers<C, false, true>(words, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, P.seed, run,
                                            step, lane, sl, S, seg_base, seg_mask, trans, digest);
         chan = 0;
         sender = -1;
@@ -239,15 +239,15 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
         int w = -1;
         bool exp_won = false;
         RaceSlots<C> rs;
-        race_slots<C>(rs, words, scr, Ctx{vars, t, 0}, m, changed, xblk);
+        race_slots<C>(rs, words, Ctx{vars, t, 0}, m, changed, xblk);
+        // windows of the bounded slots
+        for (uint32_t b = rs.bounded; b; b &= b - 1) {
+            const int j = __ffs(b) - 1;
+            scr[64 * j] = slot_window(words, j, Ctx{vars, t, 0}, m);
+        }
         if (!full) changed = false;
         // frozen components race only in a full race (as in the run kernel)
-        if (m.freeze && full) {
-            const uint32_t fz = frozen_rates<C>(words, scr, Ctx{vars, t, 0}, m);
-#pragma unroll
-            for (int j = 0; j < C; ++j)
-                if ((fz >> j) & 1u) rs.leaf[j] = scr[64 * j];
-        }
+        if (m.freeze && full) race_frozen<C>(rs, words, Ctx{vars, t, 0}, m);
         // tilted rates
         double leaft[C];
 #pragma unroll
@@ -287,7 +287,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                 }
             }
             // tilted race: the run kernel's tree over the tilted rates
-            double *lvl = tl.lvl + lane;
+            double lvl[6] = {};
             const double Rt = race_total<C>(leaft, lvl, S);
             const double R = theta ? tree_total<C>(rs.leaf, S) : Rt;
             double dexp = INF;
@@ -295,7 +295,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
             if (Rt > 0.0) {
                 const smc_u32x4 rw = draw(P.seed, run, step, SMC_P_RACE, 0);
                 dexp = -device_log2(smc_u01(rw.v[0], rw.v[1])) / Rt;
-                wexp = race_pick<C>(leaft, lvl, smc_u01(rw.v[2], rw.v[3]) * Rt, S, sl, seg_base, seg_mask);
+                wexp = race_pick<C>(leaft, lvl, smc_u01(rw.v[2], rw.v[3]) * Rt, S, seg_base, seg_mask);
             }
             double gu = umin;
             int wu = 0x7FFFFFFF;
@@ -315,11 +315,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
             // the step that crosses the bound: the left-out null racers'
             // first event after it (base rates, no tilt)
             if (m.freeze && !full && d < INF && !(t + d < P.bound)) {
-                const uint32_t fz = frozen_rates<C>(words, scr, Ctx{vars, t, 0}, m);
-                double dl[C];
-#pragma unroll
-                for (int j = 0; j < C; ++j) dl[j] = ((fz >> j) & 1u) ? scr[64 * j] : 0.0;
-                const double Rd = tree_total<C>(dl, S);
+                const double Rd = frozen_total<C>(words, Ctx{vars, t, 0}, m, S);
                 if (Rd > 0.0) {
                     const smc_u32x4 rw = draw(P.seed, run, step, SMC_P_DEAD, 0);
                     const double td = P.bound + (-device_log2(smc_u01(rw.v[0], rw.v[1])) / Rd);
@@ -478,8 +474,7 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     const int wv = threadIdx.x >> 6, W = blockDim.x >> 6;
     // LDS: [tables: TAB only][tilt index: lpad int32][2^theta: lpad doubles]
     //      then per wave [variables][rows' 2^theta][rows' theta][scratch: C
-    //      doubles per lane][race-tree levels: log2(S) doubles per lane]
-    //      [state words, locations: 4 C bytes per lane each][recording
+    //      doubles per lane][state words, locations: 4 C bytes per lane each][recording
     //      build: 16 C bytes per lane]
     double *shared = lds + (TAB ? P.table_bytes / 8 : 0);
     int32_t *tix = (int32_t *)shared;
@@ -492,10 +487,7 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     tl.row_ex = wlds + (size_t)R * P.var_stride;
     tl.row_th = (float *)(tl.row_ex + (size_t)R * P.theta_cap);
     tl.scr = (double *)(tl.row_th + (size_t)R * P.theta_cap);
-    tl.lvl = tl.scr + 64 * C;
-    int levels = 0;
-    while ((1 << levels) < P.lanes) ++levels;
-    tl.words = (uint32_t *)(tl.lvl + (size_t)levels * 64);
+    tl.words = (uint32_t *)(tl.scr + 64 * C);
     tl.locs = (int32_t *)tl.words + 64 * C;
     tl.rec = (double *)(tl.locs + 64 * C);
     for (int i = threadIdx.x; i < P.lpad; i += blockDim.x) tix[i] = P.tilt_index[i];

@@ -39,8 +39,7 @@ struct InstDesc {
 struct LaunchParams {
     const InstDesc *inst;       // sorted by chunk_first
     int32_t n_inst;
-    int32_t var_stride;         // doubles of LDS per segment (>= every n_vars)
-    int32_t scratch;            // 8-byte scratch words per lane (>= slots per lane, >= race-tree levels)
+    int32_t var_stride;         // doubles of LDS per segment (> every n_vars)
     uint64_t total_chunks;
     unsigned long long *counter;  // chunks handed out (cleared by launch_prep)
     const uint64_t *round;      // optional: runs of round r start at run_begin + r * n_runs

@@ -77,14 +77,14 @@ __device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTAN
 // Fischer-32, 1e6 runs at 4 lanes a run: 76.2 ms in that form, 51.0 ms with
 // record classes and rolled cold paths, 44.2 ms with the slot loop free of
 // branches and its invariants out of spilled registers, 40.7 ms with the
-// step's rare parts behind branches the whole wave takes or leaves; SIR-350,
-// 2e5 runs at 64 lanes: 355, 117, 97 and 81.8 ms.
+// step's rare parts behind branches the whole wave takes or leaves, 36.3 ms
+// with the race's sums and windows kept out of LDS; SIR-350, 2e5 runs at 64
+// lanes: 355, 117, 97, 81.8 and 76.8 ms.
 //
 // LDS: [tables: lp.table_bytes, TAB only] then per wave [variables of the
-// wave's 64/S runs: var_stride doubles each][scratch: 8 bytes per slot and
-// lane, at least 8 per level of the race tree and lane][state words: 4 bytes
-// per slot and lane][TRACE: locations, the same]; lp.wave_lds covers the
-// largest of these over the launch's instances.
+// wave's 64/S runs and a constant 0: var_stride doubles each][state words: 4
+// bytes per slot and lane][TRACE: locations, the same]; lp.wave_lds covers
+// the largest of these over the launch's instances.
 template <int C, bool TRACE, bool TAB>
 __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     extern __shared__ __attribute__((aligned(16))) double lds[];
@@ -155,8 +155,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     const uint64_t seg_ones = (S0 == 64) ? ~0ull : ((1ull << S0) - 1ull);
     const uint64_t seg_mask = seg_ones << seg_base;
     double *vars = wbase + (size_t)(lane / S0) * lp.var_stride;
-    double *scr = wbase + (size_t)(64 / S0) * lp.var_stride + lane;
-    uint32_t *words_of = (uint32_t *)(wbase + (size_t)(64 / S0) * lp.var_stride + 64 * lp.scratch);
+    uint32_t *words_of = (uint32_t *)(wbase + (size_t)(64 / S0) * lp.var_stride);
     uint32_t *words = words_of + lane;
     int32_t *locs = (int32_t *)words_of + 64 * C + lane;  // TRACE only
     const uint32_t chunk_runs = inst->chunk_runs;
@@ -240,6 +239,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                     q.qmax = I->p.qinit; q.qmin = I->p.qinit;
                     digest = TRACE ? smc_mix(0, run) : 0;
                     for (int v = sl; v < I->m.n_vars; v += S) vars[v] = I->m.var_init[v];
+                    if (sl == 0) vars[I->m.n_vars] = 0.0;
 #pragma clang loop unroll(disable)
                     for (int j = 0; j < C; ++j) {
                         const int c = sl * C + j;
@@ -258,7 +258,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
             // pending broadcast receivers (SyncInSerial simulation.cu:357-407)
             if (chan > 0) {
                 bool entered = false;
-                fire_receivers<C, TRACE, TRACE>(words, scr, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, seed,
+                fire_receivers<C, TRACE, TRACE>(words, locs, Ctx{vars, t, 0}, m, chan, sender, q, entered, seed,
                                                 run, step, lane, sl, S, seg_base, seg_mask, trans, digest);
                 changed = true;
                 chan = 0;
@@ -281,7 +281,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
             if (over) continue;
         }
         RaceSlots<C> rs;
-        race_slots<C>(rs, words, scr, Ctx{vars, t, 0}, m, changed, xblk);
+        race_slots<C>(rs, words, Ctx{vars, t, 0}, m, changed, xblk);
         changed = full;
         // A frozen component (blocked, exponential) only makes null steps
         // until the next transition.  Leaving it out of the race keeps the
@@ -291,12 +291,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
         // (W: the end of its window).  It races as in the reference when the
         // step decides the outcome (full).
         if (unlikely(any_lane(full))) {
-            if (m.freeze && full) {
-                const uint32_t fz = frozen_rates<C>(words, scr, Ctx{vars, t, 0}, m);
-#pragma unroll
-                for (int j = 0; j < C; ++j)
-                    if ((fz >> j) & 1u) rs.leaf[j] = scr[64 * j];
-            }
+            if (m.freeze && full) race_frozen<C>(rs, words, Ctx{vars, t, 0}, m);
         }
         double d = 0.0;
         int w = -1;
@@ -322,15 +317,20 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                     const smc_u32x4 rw = draw_at(seed, run, step,
                                                  delay ? ((uint32_t)SMC_P_UNIFORM << 24) | smc_uniform_draw(c)
                                                        : (uint32_t)SMC_P_RACE << 24);
-                    const double du = scr[64 * j] * smc_uniform_u(rw, c);
+                    const double M0 = C > 2 ? slot_window(words, j, Ctx{vars, t, 0}, m)
+                                            : (C == 2 && j ? rs.left[C - 1] : rs.left[0]);
+                    const double du = M0 * smc_uniform_u(rw, c);
                     if (delay && du < umin) { umin = du; unif_j = j; }
                     b &= b - 1;
                     if (C > 1) {
                         const int j1 = j + 1 < C ? j + 1 : j;
                         const bool pair = !(c & 1u) && ((b >> j1) & 1u);
-                        const double du1 = scr[64 * j1] * smc_uniform_u(rw, c + 1);
-                        if (pair && du1 < umin) { umin = du1; unif_j = j1; }
-                        b = pair ? b & (b - 1) : b;
+                        if (any_lane(pair)) {
+                            const double M1 = C > 2 ? slot_window(words, j1, Ctx{vars, t, 0}, m) : rs.left[C - 1];
+                            const double du1 = M1 * smc_uniform_u(rw, c + 1);
+                            if (pair && du1 < umin) { umin = du1; unif_j = j1; }
+                            b = pair ? b & (b - 1) : b;
+                        }
                     }
                     // every draw of the race is the same: keep the last
                     race.v[0] = delay ? race.v[0] : rw.v[0];
@@ -343,9 +343,10 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) race.v[k] = (uint32_t)__shfl((int)race.v[k], from);
             }
-            const double R = race_total<C>(rs.leaf, scr, S);
+            double level[6] = {};
+            const double R = race_total<C>(rs.leaf, level, S);
             const double e = -device_log2(smc_u01(race.v[0], race.v[1])) / R;
-            w = race_pick<C>(rs.leaf, scr, smc_u01(race.v[2], race.v[3]) * R, S, sl, seg_base, seg_mask);
+            w = race_pick<C>(rs.leaf, level, smc_u01(race.v[2], race.v[3]) * R, S, seg_base, seg_mask);
             const double dexp = R > 0.0 ? e : INF;
             d = dexp;
             if (any_lane(unif_j >= 0)) {
@@ -367,11 +368,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
             const bool cross = m.freeze && !full && zb == 0 && d < INF && !(t + d < bound);
             if (unlikely(any_lane(cross))) {
                 if (cross) {
-                    const uint32_t fz = frozen_rates<C>(words, scr, Ctx{vars, t, 0}, m);
-                    double dl[C];
-#pragma unroll
-                    for (int j = 0; j < C; ++j) dl[j] = ((fz >> j) & 1u) ? scr[64 * j] : 0.0;
-                    const double Rd = tree_total<C>(dl, S);
+                    const double Rd = frozen_total<C>(words, Ctx{vars, t, 0}, m, S);
                     if (Rd > 0.0) {
                         const smc_u32x4 dw = draw(seed, run, step, SMC_P_DEAD, 0);
                         const double td = bound + (-device_log2(smc_u01(dw.v[0], dw.v[1])) / Rd);
