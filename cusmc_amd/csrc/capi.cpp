@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -40,12 +41,13 @@ struct Plan {
     int group_waves = 1;  // waves per workgroup
     uint32_t table_bytes = 0, wave_lds = 0;
     size_t lds = 0;
-    int waves = 1;
-    uint32_t chunk_runs = 64;
-    uint64_t total_chunks = 0;
+    int waves = 1, per_cu = 1;
+    uint32_t chunk_runs = 1;
+    int segments = 64;  // segments of a wave that take runs
 };
 
 constexpr size_t kLdsPerCu = 160 * 1024;
+constexpr size_t kLdsStatic = 64;  // the run kernel's own
 
 int tree_levels(int S) {
     int levels = 0;
@@ -63,6 +65,23 @@ size_t wave_lds_bytes(int R, int stride, int C, bool trace) {
 // time each and two doubles per lane and race-tree level, in 60,000 bytes.
 bool vars_fit(int R, int n_vars, int levels) {
     return (size_t)R * ((n_vars + 1) | 1) * 8 + (size_t)levels * 1024 <= 60000;
+}
+
+// Waves per CU that the registers of a run-kernel build allow (a property of
+// the built code, asked for once per build).
+int register_waves(int C, bool trace, int occ, bool tab) {
+    static std::atomic<int> known[5][2][2][2];
+    int c = 0;
+    while ((1 << c) < C) ++c;
+    std::atomic<int> &k = known[c][trace][occ == 3][tab];
+    int v = k.load(std::memory_order_relaxed);
+    if (!v) {
+        int blocks = 0;
+        hip_check(smc::sim_occupancy(C, trace, occ, tab, 1, 0, &blocks), "occupancy query");
+        v = std::max(1, blocks);
+        k.store(v, std::memory_order_relaxed);
+    }
+    return v;
 }
 
 Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs, bool trace) {
@@ -85,43 +104,48 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
         throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
     const size_t wave = wave_lds_bytes(pl.R, pl.stride, pl.C, trace);
     pl.wave_lds = (uint32_t)wave;
+    // what the registers allow per CU, and for staged tables the waves per
+    // workgroup (one copy of the tables each) that put most waves on a CU
+    int per_cu = register_waves(pl.C, trace, pl.occ, want.tables != 0);
     if (want.tables) {
-        pl.table_bytes = m->table_bytes;
-        pl.group_waves = SMC_MAX_GROUP_WAVES;
-        pl.tab = pl.table_bytes + (size_t)pl.group_waves * wave + 64 <= kLdsPerCu;
-        if (!pl.tab) {
-            // tables that fit at 48 bytes a location are accepted all the
-            // same (they are read from global memory)
-            if (want.tables == 1 && !trace && (size_t)m->dm.n_locs * 48 + (size_t)pl.group_waves * wave > kLdsPerCu)
-                throw std::runtime_error("limit: the model tables do not fit in LDS");
-            pl.table_bytes = 0;
-            pl.group_waves = 1;
+        int best = 0;
+        // (as many on each of a CU's four SIMDs)
+        for (int g = 1; g <= SMC_MAX_GROUP_WAVES; g *= 2) {
+            const size_t lds = m->table_bytes + (size_t)g * wave + kLdsStatic;
+            if (lds > kLdsPerCu) break;
+            const int n = std::min((int)(kLdsPerCu / lds), std::max(per_cu / g, 1)) * g;
+            if (n >= best) { best = n; pl.group_waves = g; }
+        }
+        pl.tab = best > 0;
+        if (pl.tab) {
+            pl.table_bytes = m->table_bytes;
+            per_cu = best;
+        } else if (want.tables == 1 && !trace && (size_t)m->dm.n_locs * 48 + 4 * wave > kLdsPerCu) {
+            throw std::runtime_error("limit: the model tables do not fit in LDS");
+        } else {
+            // tables that fit beside four waves at 48 bytes a location are
+            // accepted all the same, and read from global memory
+            per_cu = register_waves(pl.C, trace, pl.occ, false);
         }
     }
+    if (!pl.tab) per_cu = std::max(1, std::min(per_cu, (int)(kLdsPerCu / (wave + kLdsStatic))));
+    if (want.waves_per_cu > 0 && want.waves_per_cu < per_cu) per_cu = want.waves_per_cu;
+    pl.per_cu = per_cu;
+    int waves = want.waves > 0 ? want.waves : m->cu_count * per_cu;
+    // chunks: a wave takes as many as it has segments to start, and sixteen
+    // times that on its way; what is left of a chunk waits in the wave, so
+    // the waves end together only with small ones
+    pl.chunk_runs = (uint32_t)std::min<uint64_t>(total_runs / (16ull * (uint64_t)waves * (uint64_t)pl.R) + 1, 256);
+    // with fewer runs than one wave on every SIMD can hold, spread over the
+    // SIMDs instead, segments left idle: a lone wave's step takes the longer
+    // the more runs differ in it
+    const uint64_t spread = (total_runs + 4ull * m->cu_count - 1) / (4ull * m->cu_count);
+    pl.segments = (int)std::min<uint64_t>(spread, (uint64_t)pl.R);
+    waves = (int)std::min<uint64_t>((uint64_t)waves, (total_runs + pl.segments - 1) / pl.segments);
+    // few waves: no more of them in a workgroup than it takes to use every CU
+    pl.group_waves = std::min(pl.group_waves, std::max(1, (waves + m->cu_count - 1) / m->cu_count));
     pl.lds = pl.table_bytes + (size_t)pl.group_waves * wave;
-    int waves = want.waves;
-    if (waves <= 0) {
-        int blocks = 0;
-        hip_check(smc::sim_occupancy(pl.C, trace, pl.occ, pl.tab, pl.group_waves, pl.lds, &blocks), "occupancy query");
-        int per_cu = blocks * pl.group_waves;
-        if (want.waves_per_cu > 0 && want.waves_per_cu < per_cu) per_cu = want.waves_per_cu;
-        if (per_cu <= 0) {
-            if (pl.tab) throw std::runtime_error("limit: the model tables do not fit in LDS");
-            per_cu = 1;
-        }
-        waves = m->cu_count * per_cu;
-    }
-    waves = (waves + pl.group_waves - 1) / pl.group_waves * pl.group_waves;
-    // chunks: enough per wave to balance uneven run lengths, at most 64 rounds of the wave's segments
-    uint64_t per_wave = (total_runs + (uint64_t)waves - 1) / (uint64_t)waves;
-    uint64_t k = (per_wave + 4ull * pl.R - 1) / (4ull * pl.R);
-    if (k < 1) k = 1;
-    if (k > 64) k = 64;
-    uint64_t chunk = k * pl.R;
-    if (chunk > total_runs) chunk = total_runs;
-    if (chunk < 1) chunk = 1;
-    pl.chunk_runs = (uint32_t)chunk;
-    pl.waves = waves;
+    pl.waves = (waves + pl.group_waves - 1) / pl.group_waves * pl.group_waves;
     return pl;
 }
 
@@ -345,21 +369,19 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         hip_check(hipSetDevice(m->device), "hipSetDevice");
         Plan pl = plan_launch(m, use, n_runs, trace);
         m->runs.ensure(n_runs);
-        pl.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
-        int waves = pl.waves;
-        if ((uint64_t)waves > pl.total_chunks)
-            waves = (int)((pl.total_chunks + pl.group_waves - 1) / pl.group_waves * pl.group_waves);
+        const int waves = pl.waves;
 
         m->h_inst.m = m->dm;
         m->h_inst.p = make_params(q, m->img, seed, run_begin, n_runs, m->runs, outputs && outputs->time, trace);
         m->h_inst.chunk_first = 0;
-        m->h_inst.lanes = pl.S;
         m->h_inst.chunk_runs = pl.chunk_runs;
+        m->h_inst.lanes = pl.S;
         LaunchParams lp{};
         lp.inst = m->d_inst;
         lp.n_inst = 1;
         lp.var_stride = pl.stride;
-        lp.total_chunks = pl.total_chunks;
+        lp.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
+        lp.segments = pl.segments;
         lp.counter = m->d_counter;
         lp.round = nullptr;
         lp.tables = pl.tab ? (decltype(lp.tables))m->arena : nullptr;
@@ -418,10 +440,7 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         hip_check(smc::noalloc_scratch(m->device, &scr), "scratch address");
         uint8_t *base = (uint8_t *)scr;
         Plan pl = plan_launch(m, use, n_runs, false);
-        pl.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
-        int waves = pl.waves;
-        if ((uint64_t)waves > pl.total_chunks)
-            waves = (int)((pl.total_chunks + pl.group_waves - 1) / pl.group_waves * pl.group_waves);
+        const int waves = pl.waves;
 
         // the per-run buffers are the scratch's (the whole run range of
         // this call is written by the run kernel before the reduction reads)
@@ -440,13 +459,14 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         m->h_inst.m = m->dm;
         m->h_inst.p = make_params(q, m->img, seed, run_begin, n_runs, b, false, false);
         m->h_inst.chunk_first = 0;
-        m->h_inst.lanes = pl.S;
         m->h_inst.chunk_runs = pl.chunk_runs;
+        m->h_inst.lanes = pl.S;
         LaunchParams lp{};
         lp.inst = d_inst;
         lp.n_inst = 1;
         lp.var_stride = pl.stride;
-        lp.total_chunks = pl.total_chunks;
+        lp.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
+        lp.segments = pl.segments;
         lp.counter = d_counter;
         lp.round = nullptr;
         lp.tables = pl.tab ? (decltype(lp.tables))m->arena : nullptr;
@@ -577,13 +597,9 @@ int smc_autotune(smc_model *m, const smc_query *q, uint64_t seed, uint64_t sampl
             for (int occ : {0, 3})
                 for (int tab : {0, 1}) {
                     cands.push_back(smc_launch{S, 0, 0, occ, tab});
-                    int blocks = 0;
                     try {
-                        Plan pl = plan_launch(m, &cands.back(), sample_runs, false);
-                        hip_check(smc::sim_occupancy(pl.C, false, pl.occ, pl.tab, pl.group_waves, pl.lds, &blocks),
-                                  "occupancy query");
-                        const int per_cu = blocks * pl.group_waves;
-                        if (per_cu >= 2 * pl.group_waves) cands.push_back(smc_launch{S, 0, per_cu / 2, occ, tab});
+                        const int per_cu = plan_launch(m, &cands.back(), sample_runs, false).per_cu;
+                        if (per_cu >= 2) cands.push_back(smc_launch{S, 0, per_cu / 2, occ, tab});
                     } catch (const std::exception &) {
                     }
                 }
@@ -596,7 +612,7 @@ int smc_autotune(smc_model *m, const smc_query *q, uint64_t seed, uint64_t sampl
             uint64_t n = sample_runs;
             try {
                 Plan pl = plan_launch(m, &c, sample_runs, false);
-                n = std::max<uint64_t>(n, 2ull * (uint64_t)pl.waves * (uint64_t)pl.R);
+                n = std::max<uint64_t>(n, 2ull * (uint64_t)(pl.per_cu * m->cu_count) * (uint64_t)pl.R);
             } catch (const std::exception &) {
                 continue;  // e.g. LDS budget exceeded at this packing
             }
@@ -652,25 +668,20 @@ struct smc_batch {
 namespace {
 
 // The instance records of one batch launch with C slots per lane: lanes per
-// run S_i = next_pow2(components_i) / C (at least 1), chunks of k R_i runs
-// (R_i = 64 / S_i runs per wave) sized so the queue holds several chunks per
-// wave; returns the LDS bytes one wave needs (the largest instance) and the
-// total chunk count.  `runs` overrides every instance's n_runs (tuning
-// samples).
+// run S_i = next_pow2(components_i) / C (at least 1), R_i = 64 / S_i runs per
+// wave and as many per chunk; returns the LDS bytes one wave needs (the
+// largest instance) and the total of the chunks.  `runs_override` overrides every instance's n_runs
+// (tuning samples).
 struct BatchShape {
     std::vector<InstDesc> inst;
     size_t wave_lds = 0;
-    int levels = 0;
     uint64_t chunks = 0;
 };
 
-BatchShape batch_shape(smc_batch *b, int C, int waves, uint64_t runs_override) {
+BatchShape batch_shape(smc_batch *b, int C, uint64_t runs_override) {
     BatchShape sh;
     bool fits = true;
     int max_R = 1;
-    uint64_t total = 0;
-    for (auto &it : b->items) total += runs_override ? std::min<uint64_t>(runs_override, it.n_runs) : it.n_runs;
-    const uint64_t per_wave = (total + (uint64_t)waves - 1) / (uint64_t)waves;
     for (size_t i = 0; i < b->items.size(); ++i) {
         const smc_batch_item &it = b->items[i];
         const int P = it.model->img.n_leaves;
@@ -681,16 +692,13 @@ BatchShape batch_shape(smc_batch *b, int C, int waves, uint64_t runs_override) {
         fits = fits && vars_fit(R, b->max_vars, levels);
         max_R = std::max(max_R, R);
         const uint64_t n = runs_override ? std::min<uint64_t>(runs_override, it.n_runs) : it.n_runs;
-        uint64_t k = (per_wave + 4ull * R - 1) / (4ull * R);
-        k = std::max<uint64_t>(1, std::min<uint64_t>(k, 64));
-        const uint64_t chunk = std::max<uint64_t>(1, std::min<uint64_t>(k * R, n));
         InstDesc d{};
         d.m = it.model->dm;
         d.p = make_params(&it.query, it.model->img, it.seed, it.run_begin, n, b->bufs[i], false, false);
         d.chunk_first = sh.chunks;
         d.lanes = S;
-        d.chunk_runs = (uint32_t)chunk;
-        sh.chunks += (n + chunk - 1) / chunk;
+        d.chunk_runs = (uint32_t)R;
+        sh.chunks += (n + R - 1) / R;
         sh.inst.push_back(d);
     }
     if (!fits) throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
@@ -766,6 +774,7 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
             b->lp.n_inst = n_items;
             b->lp.var_stride = b->stride;
             b->lp.total_chunks = sh.chunks;
+            b->lp.segments = 64;
             b->lp.counter = b->d_counter;
             b->lp.round = b->d_round;
             b->lp.tables = nullptr;
@@ -781,9 +790,8 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
             for (auto &it : b->items) sample = std::max<uint64_t>(sample, std::min<uint64_t>(it.n_runs, 2048));
             for (int C = Cmin; C <= 16; C <<= 1)
                 for (int occ : {0, 3}) {
-                    BatchShape probe = batch_shape(b.get(), C, 1, sample);
-                    const int waves = batch_waves(C, occ, probe.wave_lds, 0, cu);
-                    BatchShape sh = batch_shape(b.get(), C, waves, sample);
+                    BatchShape sh = batch_shape(b.get(), C, sample);
+                    const int waves = batch_waves(C, occ, sh.wave_lds, 0, cu);
                     set_launch(sh, C, occ, waves);
                     float ms = 0.f;
                     for (int rep = 0; rep < 2; ++rep) {  // the first launch warms the code
@@ -798,9 +806,8 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
                 }
         }
         {
-            BatchShape probe = batch_shape(b.get(), bestC, 1, 0);
-            const int waves = batch_waves(bestC, best_occ, probe.wave_lds, 0, cu);
-            BatchShape sh = batch_shape(b.get(), bestC, waves, 0);
+            BatchShape sh = batch_shape(b.get(), bestC, 0);
+            const int waves = batch_waves(bestC, best_occ, sh.wave_lds, 0, cu);
             set_launch(sh, bestC, best_occ, waves);
         }
         hip_check(hipDeviceSynchronize(), "batch setup");

@@ -42,6 +42,7 @@ struct LaunchParams {
     int32_t var_stride;         // doubles of LDS per segment (> every n_vars)
     uint64_t total_chunks;
     unsigned long long *counter;  // chunks handed out (cleared by launch_prep)
+    int32_t segments;           // segments of a wave that take runs, at most
     const uint64_t *round;      // optional: runs of round r start at run_begin + r * n_runs
     const SMC_GLOBAL uint8_t *tables;  // tables staged in LDS (one instance): first staged byte
     uint32_t table_bytes;       // bytes staged (multiple of 16), 0 without staging
@@ -49,7 +50,7 @@ struct LaunchParams {
 };
 
 // Waves per workgroup of the run kernel, at most.
-#define SMC_MAX_GROUP_WAVES 4
+#define SMC_MAX_GROUP_WAVES 8
 
 struct ReducePartial {
     double sum, sumsq, vmin, vmax;

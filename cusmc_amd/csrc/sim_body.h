@@ -53,17 +53,67 @@ namespace {
 
 // ------------------------------------------------------------ run kernel
 
+// A value that is the same on every lane, as a scalar.
+__device__ __forceinline__ unsigned long long first_lane(unsigned long long v) {
+    return ((unsigned long long)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) |
+           (unsigned long long)__builtin_amdgcn_readfirstlane((uint32_t)v);
+}
+
+// The launch's next n chunks, for the whole wave: the first of them.
+__device__ __forceinline__ unsigned long long take_chunks(unsigned long long *counter, uint32_t n, int lane) {
+    unsigned long long g = 0;
+    if (lane == 0) g = atomicAdd(counter, (unsigned long long)n);
+    return first_lane(g);
+}
+
+// A run's first state; the reads of several variables and of all state words
+// are under way together.
+template <int C, bool TRACE>
+__device__ __forceinline__ void start_state(const SMC_CONSTANT DevModel &m, double *vars, uint32_t *words,
+                                            int32_t *locs, int sl, int S) {
+    const int n_vars = m.n_vars, n_comp = m.n_comp;
+    const auto *init = m.var_init;
+    const auto *word = m.comp_word;
+    uint32_t w[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) w[j] = sl * C + j < n_comp ? word[sl * C + j] : 0u;
+    int v = sl;
+#pragma clang loop unroll(disable)
+    for (; v + 3 * S < n_vars; v += 4 * S) {
+        const double a = init[v], b = init[v + S], c = init[v + 2 * S], d = init[v + 3 * S];
+        vars[v] = a;
+        vars[v + S] = b;
+        vars[v + 2 * S] = c;
+        vars[v + 3 * S] = d;
+    }
+#pragma clang loop unroll(disable)
+    for (; v < n_vars; v += S) vars[v] = init[v];
+    if (sl == 0) vars[n_vars] = 0.0;
+#pragma unroll
+    for (int j = 0; j < C; ++j) words[64 * j] = w[j];
+    if (TRACE) {
+#pragma clang loop unroll(disable)
+        for (int j = 0; j < C; ++j) locs[64 * j] = sl * C + j < n_comp ? m.comp_init_loc[sl * C + j] : -1;
+    }
+}
+
+// A wave starts new runs when its idle lanes have cost it this part of its
+// time since the last start.  Times at 1/4, 1/8, 1/16 and 1/32: Fischer-32,
+// 1e6 runs, 31.7, 30.9, 30.1 and 31.2 ms; SIR-77, 5e4 runs, 2.39, 2.22, 2.18
+// and 2.65 ms.
+constexpr uint32_t kWaitShare = 16;
+
 // The same pointer, as far as the optimiser knows another one.
 __device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTANT InstDesc *p) {
     asm volatile("" : "+s"(p));
     return p;
 }
 
-// One wave at a time takes a chunk of runs of one instance from the launch's
-// queue, so the instance (its tables, query and outputs) is uniform across
-// the wave and lives in scalar registers; the wave's segments then pull the
-// chunk's runs one by one from a counter in LDS.  A workgroup holds
-// blockDim/64 independent waves.  With TAB (single-instance launches) the
+// A wave takes chunks of runs from the launch's queue and hands the runs to
+// its segments; all its segments work on one instance, which (its tables,
+// query and outputs) is thereby uniform across the wave and lives in scalar
+// registers.  A chunk of another instance waits until this one's runs are
+// done.  A workgroup holds blockDim/64 independent waves.  With TAB (single-instance launches) the
 // workgroup first copies the model's tables into LDS and every wave reads
 // them there: the race and the transitions are chains of dependent table
 // reads, and LDS answers them several times sooner than the caches.
@@ -74,38 +124,39 @@ __device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTAN
 // different points of different runs, so whatever one of them needs, all
 // wait for, and a step's code has to stay in the 64 KB instruction cache
 // (with per-slot copies of the general code in every branch it was 320 KB).
-// Fischer-32, 1e6 runs at 4 lanes a run: 76.2 ms in that form, 51.0 ms with
-// record classes and rolled cold paths, 44.2 ms with the slot loop free of
-// branches and its invariants out of spilled registers, 40.7 ms with the
-// step's rare parts behind branches the whole wave takes or leaves, 36.3 ms
-// with the race's sums and windows kept out of LDS; SIR-350, 2e5 runs at 64
-// lanes: 355, 117, 97, 81.8 and 76.8 ms.
+// Fischer-32, 1e6 runs: 76.2 ms in that form, 51.0 ms with record classes
+// and rolled cold paths, 44.2 ms with the slot loop free of branches and its
+// invariants out of spilled registers, 40.7 ms with the step's rare parts
+// behind branches the whole wave takes or leaves, 36.3 ms with the race's sums
+// and windows kept out of LDS, 30.3 ms with runs handed out as below; SIR-350,
+// 2e5 runs: 355, 117, 97, 81.8, 76.7 and 74.6 ms.
 //
 // LDS: [tables: lp.table_bytes, TAB only] then per wave [variables of the
 // wave's 64/S runs and a constant 0: var_stride doubles each][state words: 4
 // bytes per slot and lane][TRACE: locations, the same]; lp.wave_lds covers
 // the largest of these over the launch's instances.
+//
+// When a segment's run ends, it waits: for the last of the wave's runs, or
+// until the waiting lanes have cost the wave 1/16 of its time.  Runs of equal
+// length then start together and take the same parts of a step in the same
+// steps; a Fischer run ends when its goal is reached, and waiting for the
+// longest of a chunk left half of the lanes idle.
 template <int C, bool TRACE, bool TAB>
 __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     extern __shared__ __attribute__((aligned(16))) double lds[];
-    __shared__ unsigned int chunk_next_of[SMC_MAX_GROUP_WAVES];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    unsigned int &chunk_next = chunk_next_of[wv];
     double *wbase = lds + (TAB ? lp.table_bytes / 8 : 0) + (size_t)wv * (lp.wave_lds / 8);
     const double INF = __builtin_huge_val();
     const uint64_t round = lp.round ? *lp.round : 0;
     using Tables = typename std::conditional<TAB, SmcLdsTables, SmcGlobalTables>::type;
     if (TAB) stage_tables(lp.tables, lp.table_bytes, lds);
 
+  unsigned long long g = 0, g_end = 0;  // chunks the wave has taken and not begun
   for (;;) {
-    unsigned long long g = 0;
-    if (lane == 0) g = atomicAdd(lp.counter, 1ull);
-    g = __shfl(g, 0);
-    // the same on every lane: make it a scalar, so the instance lookup and
-    // its tables and parameters live in scalar registers
-    g = ((unsigned long long)__builtin_amdgcn_readfirstlane((uint32_t)(g >> 32)) << 32) |
-        (unsigned long long)__builtin_amdgcn_readfirstlane((uint32_t)g);
+    g = first_lane(g);
+    g_end = first_lane(g_end);
+    if (g == g_end) g_end = (g = take_chunks(lp.counter, 1, lane)) + 1;
     if (g >= lp.total_chunks) break;
     int lo = 0, hi = lp.n_inst - 1;
     while (lo < hi) {
@@ -158,15 +209,12 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     uint32_t *words_of = (uint32_t *)(wbase + (size_t)(64 / S0) * lp.var_stride);
     uint32_t *words = words_of + lane;
     int32_t *locs = (int32_t *)words_of + 64 * C + lane;  // TRACE only
-    const uint32_t chunk_runs = inst->chunk_runs;
-    const uint64_t chunk = g - inst->chunk_first;
-    const uint32_t r_first = (uint32_t)(chunk * chunk_runs);
-    const uint32_t r_end = (uint32_t)((uint64_t)r_first + chunk_runs < inst->p.n_runs ? r_first + chunk_runs
-                                                                               : inst->p.n_runs);
-    if (lane == 0) chunk_next = r_first;
-    wave_sync();
+    // since runs were started: turns of the loop, lanes without a run summed
+    // over them
+    uint32_t turns = 0, waited = 0;
+    uint32_t r_next = 0, r_end = 0;  // runs of chunks begun, not started yet
 
-    bool active = false, done = false;
+    bool active = false, done = lane / S0 >= lp.segments;
     uint64_t run = 0;
     uint32_t ridx = 0;
     double t = 0.0;
@@ -187,6 +235,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
         const bool in_time = t < bound;
         const bool at_goal = reach & goal & in_time & !over;
         const bool end = active & (!in_time | over | at_goal | (step >= max_steps));
+        ++turns;
         if (unlikely(any_lane(end | (!active & !done)))) {
             const SMC_CONSTANT InstDesc *I = opaque(inst);
             if (end) {
@@ -224,33 +273,54 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                 wave_sync();
                 active = false;
             }
-            if (!active && !done) {
-                unsigned int r = 0;
-                if (sl == 0) r = atomicAdd(&chunk_next, 1u);
-                r = __shfl(r, seg_base);
-                if (r >= r_end) {
-                    done = true;
-                } else {
-                    ridx = r;
-                    run = I->p.run_begin + round * I->p.n_runs + r;
-                    active = true;
-                    t = 0.0; step = 0; trans = 0; chan = 0; sender = -1;
-                    goal = false; over = false; changed = true;
-                    q.qmax = I->p.qinit; q.qmin = I->p.qinit;
-                    digest = TRACE ? smc_mix(0, run) : 0;
-                    for (int v = sl; v < I->m.n_vars; v += S) vars[v] = I->m.var_init[v];
-                    if (sl == 0) vars[I->m.n_vars] = 0.0;
-#pragma clang loop unroll(disable)
-                    for (int j = 0; j < C; ++j) {
-                        const int c = sl * C + j;
-                        words[64 * j] = c < I->m.n_comp ? I->m.comp_word[c] : 0u;
-                        if (TRACE) locs[64 * j] = c < I->m.n_comp ? I->m.comp_init_loc[c] : -1;
+            // new runs once none is left, or once the waiting lanes have
+            // stood still for a share of the wave's time
+            const bool want = !active & !done;
+            waited += (uint32_t)__popcll(__ballot(want));
+            if (!any_lane(active) || kWaitShare * waited > 64 * turns) {
+                waited = turns = 0;
+                const uint64_t heads = __ballot(want & (sl == 0));
+                const int need = __popcll(heads), rank = __popcll(heads & ((1ull << seg_base) - 1));
+                const uint32_t chunk = I->chunk_runs, n_runs = (uint32_t)I->p.n_runs;
+                const uint64_t c0 = I->chunk_first, c1 = c0 + (n_runs + (uint64_t)chunk - 1) / chunk;
+                uint32_t r = 0xFFFFFFFFu;
+                for (int given = 0; given < need;) {
+                    if (r_next == r_end) {
+                        if (g == g_end) {
+                            // (of several instances one at a time: it may be another's)
+                            const uint32_t n = lp.n_inst == 1 ? ((uint32_t)(need - given) + chunk - 1) / chunk : 1u;
+                            g = take_chunks(lp.counter, n, lane);
+                            g_end = g + n;
+                        }
+                        if (g >= c1) break;
+                        const uint64_t stop = g_end < c1 ? g_end : c1, r1 = (stop - c0) * chunk;
+                        r_next = (uint32_t)((g - c0) * chunk);
+                        r_end = r1 < n_runs ? (uint32_t)r1 : n_runs;
+                        g = stop;
                     }
-                    wave_sync();
+                    const int left = (int)(r_end - r_next), n = left < need - given ? left : need - given;
+                    if ((rank >= given) & (rank < given + n)) r = r_next + (uint32_t)(rank - given);
+                    r_next += (uint32_t)n;
+                    given += n;
                 }
+                if (want) {
+                    if (r == 0xFFFFFFFFu) {
+                        done = true;
+                    } else {
+                        ridx = r;
+                        run = I->p.run_begin + round * I->p.n_runs + r;
+                        active = true;
+                        t = 0.0; step = 0; trans = 0; chan = 0; sender = -1;
+                        goal = false; over = false; changed = true;
+                        q.qmax = I->p.qinit; q.qmin = I->p.qinit;
+                        digest = TRACE ? smc_mix(0, run) : 0;
+                        start_state<C, TRACE>(I->m, vars, words, locs, sl, S);
+                        wave_sync();
+                    }
+                }
+                if (!any_lane(active)) break;
+                continue;  // a new run passes the loop test first
             }
-            if (!any_lane(active)) break;
-            continue;  // a new run passes the loop test first
         }
         if (!active) continue;
 
