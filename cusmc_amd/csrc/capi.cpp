@@ -84,10 +84,41 @@ int register_waves(int C, bool trace, int occ, bool tab) {
     return v;
 }
 
+// The launch of a call that asks for none on a model without a tuned one:
+// the fewest lanes per run at which two waves per SIMD have their runs and
+// their LDS, tables staged, and three waves per SIMD where sixteen slots a
+// lane leave registers for two and there are runs for more.  A step costs a wave much the same whether it
+// advances one run or many, so many runs are packed; few runs are spread, for
+// the shortest steps.  Against one run per 64 lanes and tables in global
+// memory (ms): covid-350, 16384 runs, 32 lanes 19.1 for 35.2; SIR-77, 5e4
+// runs, 8 lanes 1.73 for 4.69; Fischer-32, 2e5 runs, 2 lanes 6.68 for 25.2;
+// at 2000 runs Fischer-32 takes 0.85 at 32 lanes, 0.95 at 16 and 2.0 at 2.
+// Where slots are tested one after another (invariants and blocking tests of
+// several records) a lane gets as few as there are: csma-100, 16384 runs, 5.5
+// at 64 lanes and 11.0 at 32.
+smc_launch default_launch(const smc_model *m, uint64_t total_runs, bool trace) {
+    const int P = m->img.n_leaves, stride = (m->img.n_vars + 1) | 1;
+    const uint64_t simds = 4ull * (uint64_t)m->cu_count;
+    smc_launch d{};
+    int S = std::min(P, 64);
+    if (!(m->img.tests & (SMC_HF_XINV | SMC_HF_XBLK)))
+        while (S > 1 && P / (S / 2) <= 16) {
+            const int s = S / 2, R = 64 / s;
+            if (total_runs / (uint64_t)R < 2 * simds) break;
+            if (!vars_fit(R, m->img.n_vars, tree_levels(s))) break;
+            if (8 * (wave_lds_bytes(R, stride, P / s, trace) + kLdsStatic) > kLdsPerCu) break;
+            S = s;
+        }
+    d.lanes_per_run = S;
+    d.occupancy = P / S == 16 && total_runs / (uint64_t)(64 / S) > 2 * simds ? 3 : 0;
+    d.tables = 2;  // staged if they fit
+    return d;
+}
+
 Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs, bool trace) {
     Plan pl;
     const int P = m->img.n_leaves;
-    const smc_launch want = use ? *use : smc_launch{};
+    const smc_launch want = use ? *use : default_launch(m, total_runs, trace);
     if (want.occupancy != 0 && want.occupancy != 3) throw std::runtime_error("occupancy must be 0 or 3");
     if (want.tables < 0 || want.tables > 2) throw std::runtime_error("tables must be 0, 1 or 2");
     pl.occ = want.occupancy;
@@ -104,22 +135,37 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
         throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
     const size_t wave = wave_lds_bytes(pl.R, pl.stride, pl.C, trace);
     pl.wave_lds = (uint32_t)wave;
-    // what the registers allow per CU, and for staged tables the waves per
-    // workgroup (one copy of the tables each) that put most waves on a CU
+    // with fewer runs than one wave on every SIMD can hold, spread over the
+    // SIMDs instead, segments left idle: a lone wave's step takes the longer
+    // the more runs differ in it
+    const uint64_t spread = (total_runs + 4ull * m->cu_count - 1) / (4ull * m->cu_count);
+    pl.segments = (int)std::min<uint64_t>(spread, (uint64_t)pl.R);
+    const uint64_t most_waves = (total_runs + pl.segments - 1) / pl.segments;
+    // Waves a CU holds: what the registers allow, and with staged tables
+    // (one copy per workgroup) the LDS, for g waves per workgroup, as many on
+    // each of the CU's four SIMDs.
     int per_cu = register_waves(pl.C, trace, pl.occ, want.tables != 0);
+    const auto staged = [&](int g) {
+        const size_t lds = m->table_bytes + (size_t)g * wave + kLdsStatic;
+        return std::min((int)(kLdsPerCu / lds), std::max(per_cu / g, 1)) * g;
+    };
     if (want.tables) {
         int best = 0;
-        // (as many on each of a CU's four SIMDs)
-        for (int g = 1; g <= SMC_MAX_GROUP_WAVES; g *= 2) {
-            const size_t lds = m->table_bytes + (size_t)g * wave + kLdsStatic;
-            if (lds > kLdsPerCu) break;
-            const int n = std::min((int)(kLdsPerCu / lds), std::max(per_cu / g, 1)) * g;
-            if (n >= best) { best = n; pl.group_waves = g; }
-        }
+        for (int g = 1; g <= SMC_MAX_GROUP_WAVES; g *= 2) best = std::max(best, staged(g));
         pl.tab = best > 0;
+        // (left to choose: where they cost no waves)
+        if (!use && best < std::min(per_cu, (int)(kLdsPerCu / (wave + kLdsStatic)))) pl.tab = false;
         if (pl.tab) {
+            // the smallest workgroups that hold what the runs ask for: few
+            // runs then spread over the CUs evenly
+            int need = best;
+            if (want.waves > 0) need = (want.waves + m->cu_count - 1) / m->cu_count;
+            else if (want.waves_per_cu > 0) need = want.waves_per_cu;
+            need = (int)std::min<uint64_t>((uint64_t)std::min(need, best), (most_waves + m->cu_count - 1) / m->cu_count);
+            pl.group_waves = 1;
+            while (staged(pl.group_waves) < need) pl.group_waves *= 2;
             pl.table_bytes = m->table_bytes;
-            per_cu = best;
+            per_cu = staged(pl.group_waves);
         } else if (want.tables == 1 && !trace && (size_t)m->dm.n_locs * 48 + 4 * wave > kLdsPerCu) {
             throw std::runtime_error("limit: the model tables do not fit in LDS");
         } else {
@@ -136,14 +182,7 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
     // times that on its way; what is left of a chunk waits in the wave, so
     // the waves end together only with small ones
     pl.chunk_runs = (uint32_t)std::min<uint64_t>(total_runs / (16ull * (uint64_t)waves * (uint64_t)pl.R) + 1, 256);
-    // with fewer runs than one wave on every SIMD can hold, spread over the
-    // SIMDs instead, segments left idle: a lone wave's step takes the longer
-    // the more runs differ in it
-    const uint64_t spread = (total_runs + 4ull * m->cu_count - 1) / (4ull * m->cu_count);
-    pl.segments = (int)std::min<uint64_t>(spread, (uint64_t)pl.R);
-    waves = (int)std::min<uint64_t>((uint64_t)waves, (total_runs + pl.segments - 1) / pl.segments);
-    // few waves: no more of them in a workgroup than it takes to use every CU
-    pl.group_waves = std::min(pl.group_waves, std::max(1, (waves + m->cu_count - 1) / m->cu_count));
+    waves = (int)std::min<uint64_t>((uint64_t)waves, most_waves);
     pl.lds = pl.table_bytes + (size_t)pl.group_waves * wave;
     pl.waves = (waves + pl.group_waves - 1) / pl.group_waves * pl.group_waves;
     return pl;
