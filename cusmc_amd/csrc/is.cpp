@@ -138,11 +138,17 @@ struct smc_is {
     smc_model *m = nullptr;
     smc_query q{};
     smc_is_config cfg{};
-    int S = 1, C = 1, R = 64, stride = 1;
-    size_t lds = 0;
-    uint32_t wave_lds = 0;
-    bool tab = false;            // advance kernel stages the model tables in LDS
-    int max_groups = 0;          // its persistent workgroups when it does
+    // launch shapes of the advance kernel, the widest packing first
+    struct Shape {
+        int S = 1, C = 1, R = 64;    // lanes per run, slots per lane, runs per wave
+        size_t lds = 0;
+        uint32_t wave_lds = 0;
+        bool tab = false;            // stages the model tables in LDS
+        int max_groups = 0;          // its persistent workgroups when it does
+        bool rec = true;             // two waves per SIMD when recording, too
+    };
+    std::vector<Shape> shapes;
+    int stride = 1;
     int n_locs = 0, n_vars = 0, n_comp = 0, F = 0, fpad = 0, H = 128, Lpad = 0;
     int n_groups = 0, Gpad = 0;  // tilt groups: the MLP's outputs
     int G16 = 0;                 // groups rounded up to 16: the outputs the fused forward pass computes
@@ -223,12 +229,23 @@ struct smc_is {
         work.ensure(std::max<size_t>((size_t)2048 * 4096, (size_t)1024 * std::max(Gpad, H)), "hipMalloc workspace");
     }
 
+    // The shape for a launch over `rows` rows: the narrowest that gives every
+    // other SIMD a wave.  A step costs a wave much the same whether it
+    // advances one row or several; few rows take shorter steps at one row a
+    // wave.  SIR-100 under a proposal network, the whole call at 64, 32 and 16
+    // lanes a row: 5e4 rows 58.4, 39.6 and 28.7 ms, 4000 rows 9.7, 8.0 and
+    // 7.5, 2000 rows 6.9, 6.6 and 6.7, 1000 rows 5.8, 5.9 and 6.2.
+    const Shape &shape_for(int rows, bool record) const {
+        size_t k = 0;
+        while (k + 1 < shapes.size() && rows / shapes[k + 1].R >= 2 * m->cu_count && (!record || shapes[k + 1].rec)) ++k;
+        return shapes[k];
+    }
+
     IsParams params(int rows, uint64_t seed) const {
         IsParams P{};
         P.m = m->dm;
         P.st = rows_a.view();
         P.n_rows = rows;
-        P.lanes = S;
         P.var_stride = stride;
         P.lpad = Lpad;
         P.fpad = fpad;
@@ -242,9 +259,6 @@ struct smc_is {
         P.max_steps = q.max_steps ? q.max_steps : SMC_DEFAULT_MAX_STEPS;
         P.tiltable = tiltable.p;
         P.tilt_index = tix_loc.p;
-        P.tables = tab ? (decltype(P.tables))m->arena : nullptr;
-        P.table_bytes = tab ? m->table_bytes : 0;
-        P.wave_lds = wave_lds;
         P.theta_cap = Gpad;
         P.theta_len = 0;
         P.var_scale = var_scale.p;
@@ -373,16 +387,9 @@ struct smc_is {
             P.theta_len = Lpad;
             P.tilt_index = tix_loc.p;
         }
-        size_t lds_use = lds;
         if (b.record) {
             P.rec_X = rX.p; P.rec_A = rA.p; P.rec_B = rB.p; P.rec_w = rw.p;
             hip_check(hipMemsetAsync(counters.p + 1, 0, sizeof(unsigned int), s), "clear record count");
-            // the recording build reads the tables from global memory and
-            // keeps its per-slot statistics in LDS (16 C bytes per lane)
-            P.tables = nullptr;
-            P.table_bytes = 0;
-            P.wave_lds = wave_lds + (uint32_t)(16 * C * 64);
-            lds_use = (size_t)Lpad * 12 + P.wave_lds;
         }
         // Lock-step macro-steps.  The host never waits for the step it just
         // launched: after launching step k it reads the active count of step
@@ -408,7 +415,21 @@ struct smc_is {
             unsigned int *cnt = counters.p + 3 + (k & 1);
             hip_check(hipMemsetAsync(cnt, 0, sizeof(unsigned int), s), "clear active count");
             P.active_count = cnt;
-            hip_check(smc::is_launch_advance(P, C, lds_use, max_groups, s), "advance kernel launch");
+            const Shape &sh = shape_for(rows, b.record);
+            P.lanes = sh.S;
+            P.tables = sh.tab ? (decltype(P.tables))m->arena : nullptr;
+            P.table_bytes = sh.tab ? m->table_bytes : 0;
+            P.wave_lds = sh.wave_lds;
+            size_t lds_use = sh.lds;
+            if (b.record) {
+                // the recording build reads the tables from global memory and
+                // keeps its per-slot statistics in LDS (16 C bytes per lane)
+                P.tables = nullptr;
+                P.table_bytes = 0;
+                P.wave_lds = sh.wave_lds + (uint32_t)(16 * sh.C * 64);
+                lds_use = (size_t)Lpad * 12 + P.wave_lds;
+            }
+            hip_check(smc::is_launch_advance(P, sh.C, lds_use, sh.max_groups, s), "advance kernel launch");
             ++launches;
             if (!b.lockstep) break;
             hip_check(hipMemcpyAsync(h_counters + 2 + (k & 1), cnt, sizeof(unsigned int), hipMemcpyDeviceToHost, s),
@@ -548,25 +569,25 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         s->cfg = c;
         hip_check(hipSetDevice(m->device), "hipSetDevice");
 
-        // launch shape of the advance kernel
+        // launch shapes of the advance kernel
         // lanes per run: the model's tuned packing (smc_autotune) when there
-        // is one, else the widest
+        // is one, else the widest, and narrower ones for many rows
         const int P = img.n_leaves;
         if (P > 512) throw std::runtime_error("limit: importance sampling takes networks of at most 512 components");
-        s->S = P < 64 ? P : 64;
-        if (m->has_tuned && m->tuned.lanes_per_run > 0 && m->tuned.lanes_per_run <= s->S &&
+        int lanes = P < 64 ? P : 64, fewest = lanes;
+        if (m->has_tuned && m->tuned.lanes_per_run > 0 && m->tuned.lanes_per_run <= lanes &&
             P / m->tuned.lanes_per_run <= 8) {
-            s->S = m->tuned.lanes_per_run;
+            fewest = lanes = m->tuned.lanes_per_run;
+        } else if (!m->has_tuned && !(img.tests & (SMC_HF_XINV | SMC_HF_XBLK))) {
+            while (fewest > 1 && P / (fewest / 2) <= 8) fewest /= 2;
         }
         // SMC_IS_LANES=<power of two> overrides the lanes per run (diagnosis:
         // the sampler's best packing may differ from the plain simulator's)
         if (const char *lv = std::getenv("SMC_IS_LANES")) {
             const int L = std::atoi(lv);
-            if (L >= 1 && L <= 64 && (L & (L - 1)) == 0 && L <= P && P / L <= 8) s->S = L;
+            if (L >= 1 && L <= 64 && (L & (L - 1)) == 0 && L <= P && P / L <= 8) fewest = lanes = L;
         }
-        s->C = P / s->S;
-        if (s->C > 8) throw std::runtime_error("internal: more than 8 slots per lane");
-        s->R = 64 / s->S;
+        if (P / lanes > 8) throw std::runtime_error("internal: more than 8 slots per lane");
         s->stride = (img.n_vars + 1) | 1;  // the variables and a constant 0
 
         s->n_locs = (int)img.info.size();
@@ -619,29 +640,38 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         // tilt tables (theta and 2^theta, up to Gpad entries), slot scratch,
         // state words and locations (is_advance.h), after a shared part (tilt
         // index and a shared 2^theta vector, Lpad each)
-        int levels = 0;
-        while ((1 << levels) < s->S) ++levels;
-        const size_t tilts = (size_t)s->R * s->Gpad * 12;
-        // the most variables and tilts a packing may hold: with a clock time
-        // per row and two doubles per lane and level, 60,000 bytes
-        if ((size_t)s->R * ((img.n_vars + 1) | 1) * 8 + tilts + (size_t)levels * 1024 > 60000)
-            throw std::runtime_error("limit: variables exceed the LDS budget");
-        s->wave_lds = (uint32_t)rup((size_t)s->R * s->stride * sizeof(double) + tilts +
-                                        (size_t)s->C * 64 * sizeof(double) + (size_t)s->C * 512, 16);
-        {
-            const size_t shared = (size_t)s->Lpad * 12;
+        for (int S = lanes; S >= fewest; S /= 2) {
+            smc_is::Shape sh;
+            sh.S = S;
+            sh.C = P / S;
+            sh.R = 64 / S;
+            int levels = 0;
+            while ((1 << levels) < S) ++levels;
+            const size_t tilts = (size_t)sh.R * s->Gpad * 12, shared = (size_t)s->Lpad * 12;
+            sh.wave_lds = (uint32_t)rup((size_t)sh.R * s->stride * sizeof(double) + tilts +
+                                            (size_t)sh.C * 64 * sizeof(double) + (size_t)sh.C * 512, 16);
             // hot tables staged in LDS when the model's tuned launch does so
             // (or SMC_IS_TABLES=1/0 says) and four waves fit beside them
             const char *tv = std::getenv("SMC_IS_TABLES");
             bool want = m->has_tuned && m->tuned.tables == 1;
             if (tv) want = std::string(tv) == "1";
-            const size_t need = (size_t)m->table_bytes + shared + 4 * (size_t)s->wave_lds;
-            s->tab = want && m->table_bytes > 0 && need <= 160 * 1024;
-            s->lds = s->tab ? need : shared + s->wave_lds;
-            if (s->lds > 160 * 1024) throw std::runtime_error("limit: the advance kernel's LDS exceeds the budget");
+            const size_t need = (size_t)m->table_bytes + shared + 4 * (size_t)sh.wave_lds;
+            sh.tab = want && m->table_bytes > 0 && need <= 160 * 1024;
+            sh.lds = sh.tab ? need : shared + sh.wave_lds;
+            // the most variables and tilts a packing may hold: with a clock
+            // time per row and two doubles per lane and level, 60,000 bytes
+            const bool vars = (size_t)sh.R * ((img.n_vars + 1) | 1) * 8 + tilts + (size_t)levels * 1024 <= 60000;
+            if (S == lanes) {
+                if (!vars) throw std::runtime_error("limit: variables exceed the LDS budget");
+                if (sh.lds > 160 * 1024) throw std::runtime_error("limit: the advance kernel's LDS exceeds the budget");
+            } else if (!vars || 8 * (shared + sh.wave_lds) > 160 * 1024) {
+                break;  // not two waves per SIMD
+            }
+            sh.rec = 8 * (shared + sh.wave_lds + (size_t)16 * sh.C * 64) <= 160 * 1024;
             // two waves per SIMD: two workgroups of four waves per CU
-            const int per_cu = s->tab ? std::max(1, std::min(2, (int)((160 * 1024) / need))) : 0;
-            s->max_groups = per_cu * m->cu_count;
+            const int per_cu = sh.tab ? std::max(1, std::min(2, (int)((160 * 1024) / need))) : 0;
+            sh.max_groups = per_cu * m->cu_count;
+            s->shapes.push_back(sh);
         }
         // the fused forward pass when its weights fit in LDS;
         // SMC_IS_FORWARD=gemm forces the three-GEMM path (the two agree bit
