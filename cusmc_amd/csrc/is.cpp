@@ -638,7 +638,7 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         s->G16 = (int)rup((size_t)std::max(s->n_groups, 1), 16);
         // advance kernel LDS: per wave the variables of its 64/S rows, their
         // tilt tables (theta and 2^theta, up to Gpad entries), slot scratch,
-        // state words and locations (is_advance.h), after a shared part (tilt
+        // state words, locations and their bitmap (is_advance.h), after a shared part (tilt
         // index and a shared 2^theta vector, Lpad each)
         for (int S = lanes; S >= fewest; S /= 2) {
             smc_is::Shape sh;
@@ -649,7 +649,8 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
             while ((1 << levels) < S) ++levels;
             const size_t tilts = (size_t)sh.R * s->Gpad * 12, shared = (size_t)s->Lpad * 12;
             sh.wave_lds = (uint32_t)rup((size_t)sh.R * s->stride * sizeof(double) + tilts +
-                                            (size_t)sh.C * 64 * sizeof(double) + (size_t)sh.C * 512, 16);
+                                            (size_t)sh.C * 64 * sizeof(double) + (size_t)sh.C * 512 +
+                                            (size_t)sh.R * (s->Lpad / 8), 16);
             // hot tables staged in LDS when the model's tuned launch does so
             // (or SMC_IS_TABLES=1/0 says) and four waves fit beside them
             const char *tv = std::getenv("SMC_IS_TABLES");

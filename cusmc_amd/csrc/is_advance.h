@@ -54,25 +54,31 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_floa
 // variables, time / bound.  Each entry is written by exactly one lane.
 template <int C>
 __device__ __forceinline__ void write_features(const IsParams &P, uint16_t *f, const int32_t *locs, const double *vars,
-                                               double t, int sl, int S, int n) {
-#pragma clang loop unroll(disable)
-    for (int j = 0; j < C; ++j) {
-        const int c = sl * C + j;
-        if (c < n) {
+                                               uint32_t *bits, double t, int sl, int S, int n) {
+    const int base = P.m.n_locs, n_vars = P.m.n_vars;
+    // the locations held as a bitmap, then eight features a lane and store:
+    // written by component they were scattered 2-byte stores, three for each
+    for (int k = sl; k < P.lpad / 32; k += S) bits[k] = 0;
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+        if (sl * C + j < n) {
             const int at = locs[64 * j];
-            for (int l = P.m.comp_first_loc[c]; l < P.m.comp_first_loc[c + 1]; ++l)
-                f[l] = at == l ? (uint16_t)0x3F80 : (uint16_t)0;
+            atomicOr(&bits[at >> 5], 1u << (at & 31));
         }
+    wave_sync();
+    const auto two = [](uint32_t b) { return ((b & 1u) | ((b & 2u) << 15)) * 0x3F80u; };
+    for (int k = sl; k < base / 8; k += S) {
+        const uint32_t b = bits[k >> 2] >> (8 * (k & 3));
+        ((uint4 *)f)[k] = uint4{two(b), two(b >> 2), two(b >> 4), two(b >> 6)};
     }
-    const int base = P.m.n_locs;
-    for (int v = sl; v < P.m.n_vars; v += S) {
+    for (int l = (base & ~7) + sl; l < base; l += S) f[l] = (bits[l >> 5] >> (l & 31)) & 1u ? (uint16_t)0x3F80 : (uint16_t)0;
+    for (int v = sl; v < n_vars; v += S) {
         const double x = P.m.var_clock[v] ? t - vars[v] : vars[v];
         f[base + v] = f32_to_bf16((float)(x * P.var_scale[v]));
     }
-    if (sl == 0) {
-        f[base + P.m.n_vars] = f32_to_bf16((float)(t / P.bound));
-        for (int k = base + P.m.n_vars + 1; k < P.fpad; ++k) f[k] = 0;
-    }
+    if (sl == 0) f[base + n_vars] = f32_to_bf16((float)(t / P.bound));
+    for (int k = base + n_vars + 1 + sl; k < P.fpad; k += S) f[k] = 0;
 }
 
 // Whether a var-probability query is already decided: the segment-wide
@@ -99,6 +105,7 @@ struct TiltLds {
     double *scr;          // the wave's slot scratch [C][64] (windows of bounded slots)
     uint32_t *words;      // state words [C][64]
     int32_t *locs;        // locations [C][64]
+    uint32_t *bits;       // the wave's rows: locations held, [64/S][lpad / 32]
     double *rec;          // recording build: [C][64] rates, [C][64] int32 locations, [C][64] uint32 wins
 };
 
@@ -119,6 +126,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
     double *scr = tl.scr + lane;
     uint32_t *words = tl.words + lane;
     int32_t *locs = tl.locs + lane;
+    uint32_t *bits = tl.bits + (lane / S) * (P.lpad / 32);
     const IsRows &st = P.st;
     const int n = m.n_comp;
     const double INF = __builtin_huge_val();
@@ -143,20 +151,22 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
     double *hz = tl.rec + lane;
     int32_t *loc0 = (int32_t *)(tl.rec + 64 * C) + lane;
     uint32_t *wins = (uint32_t *)(tl.rec + 64 * C) + 64 * C + lane;
-#pragma clang loop unroll(disable)
+    // (the reads of all slots under way together: one after another, two
+    // dependent reads each, they were most of a short step)
+    int at[C];
+    uint32_t rec_of[C], base_of[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) at[j] = sl * C + j < n ? (int)st.loc[(size_t)row * n + sl * C + j] : -1;
+#pragma unroll
+    for (int j = 0; j < C; ++j) base_of[j] = sl * C + j < n ? m.comp_word[sl * C + j] & m.base_mask : 0u;
+#pragma unroll
+    for (int j = 0; j < C; ++j) rec_of[j] = at[j] >= 0 ? m.loc_rec[at[j]] : 0u;
+#pragma unroll
     for (int j = 0; j < C; ++j) {
-        const int c = sl * C + j;
-        int at = -1;
-        uint32_t w = 0;
-        if (c < n) {
-            // the private variables' base stays with the component
-            at = (int)st.loc[(size_t)row * n + c];
-            w = (m.loc_rec[at] << m.rec_shift) | (m.comp_word[c] & m.base_mask);
-        }
-        locs[64 * j] = at;
-        words[64 * j] = w;
+        locs[64 * j] = at[j];
+        words[64 * j] = (rec_of[j] << m.rec_shift) | base_of[j];
         if (REC) {
-            loc0[64 * j] = at;
+            loc0[64 * j] = at[j];
             hz[64 * j] = 0.0;
             wins[64 * j] = 0;
         }
@@ -185,7 +195,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
     }
     const int rec = (REC && P.rec_pos) ? P.rec_pos[row] : -1;
     if (rec >= 0) {
-        write_features<C>(P, P.rec_X + (size_t)rec * P.fpad, locs, vars, t, sl, S, n);
+        write_features<C>(P, P.rec_X + (size_t)rec * P.fpad, locs, vars, bits, t, sl, S, n);
         if (sl == 0) P.rec_w[rec] = P.weight[st.job[row]];
     }
     bool hit = false, end = false, fired_any = false;
@@ -417,11 +427,9 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                 digest = smc_mix(digest, (uint64_t)(uint32_t)tl.locs[(c % C) * 64 + seg_base + c / C]);
         }
     }
-#pragma clang loop unroll(disable)
-    for (int j = 0; j < C; ++j) {
-        const int c = sl * C + j;
-        if (c < n) st.loc[(size_t)row * n + c] = (uint16_t)locs[64 * j];
-    }
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+        if (sl * C + j < n) st.loc[(size_t)row * n + sl * C + j] = (uint16_t)locs[64 * j];
     for (int v = sl; v < m.n_vars; v += S) st.vars[(size_t)row * m.n_vars + v] = vars[v];
     if (sl == 0) {
         st.t[row] = t;
@@ -437,7 +445,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                                    (still && mid ? IS_MID : 0));
         if (still && P.active_count) atomicAdd(P.active_count, 1u);
     }
-    if (P.feat) write_features<C>(P, P.feat + (size_t)row * P.fpad, locs, vars, t, sl, S, n);
+    if (P.feat) write_features<C>(P, P.feat + (size_t)row * P.fpad, locs, vars, bits, t, sl, S, n);
     if (rec >= 0) {
         // statistics of the macro-step for the locations its components
         // started in (a component changes location only at the macro-step's
@@ -489,7 +497,9 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     tl.scr = (double *)(tl.row_th + (size_t)R * P.theta_cap);
     tl.words = (uint32_t *)(tl.scr + 64 * C);
     tl.locs = (int32_t *)tl.words + 64 * C;
-    tl.rec = (double *)(tl.locs + 64 * C);
+    tl.bits = (uint32_t *)(tl.locs + 64 * C);
+    tl.rec = (double *)(tl.bits + R * (P.lpad / 32));
+#pragma unroll 4
     for (int i = threadIdx.x; i < P.lpad; i += blockDim.x) tix[i] = P.tilt_index[i];
     if (P.theta && P.theta_stride == 0)
         for (int i = threadIdx.x; i < P.theta_len; i += blockDim.x) ex[i] = smc_exp2((double)P.theta[i]);
