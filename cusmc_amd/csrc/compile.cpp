@@ -594,7 +594,8 @@ ModelImage lower(const smc_network &n, bool use_locals) {
             // receive edges
             bool fast = true, plain_recv = true;
             int chan = 0, n_recv = 0;
-            int64_t weight = 0;
+            int64_t weight = 0, low = 0;
+            bool idle[2] = {true, true};
             for (int k = 0; k < L.edge_count; ++k) {
                 const smc_edge &E = n.edges[L.edge_first + k];
                 if (E.channel >= 0) continue;
@@ -614,20 +615,32 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                 if ((re.e.flags & SMC_EF_NEVER) || !re.guards.empty() || (chan && chan != -E.channel)) plain_recv = false;
                 chan = -E.channel;
                 if (k < 32) d.recv_mask |= 1u << k;
-                if (n_recv++ == 0) d.recv_low = re.e.weight;
+                idle[n_recv != 0] = re.e.dst == 0 && E.upd_count == 0 && !(re.e.flags & SMC_EF_GOAL);
+                if (n_recv++ == 0) low = re.e.weight;
             }
             if (weight >= 2147483648ll) fast = false;
             if (fast) d.flags |= SMC_LF_RECV_FAST;
             if (n_recv == 0) d.recv_chan = 0;
             else if (fast && plain_recv) {
                 d.recv_chan = chan;
-                d.recv_weight = (uint32_t)weight;
-                if (n_recv == 2) d.flags |= SMC_LF_RECV_TWO;
+                d.recv_flags = (n_recv == 2 ? SMC_RF_TWO : n_recv > 2 ? SMC_RF_MORE : 0u) |
+                               (idle[0] ? SMC_RF_LOW_IDLE : 0u) | (idle[1] ? SMC_RF_HIGH_IDLE : 0u);
+                if (n_recv == 2) {
+                    // the higher edge is picked unless the draw, of the sum of
+                    // the weights, falls below the lower one's: monotone in
+                    // the draw's 32 bits, and true of the largest
+                    uint32_t from = 0, to = 0xFFFFFFFFu;
+                    while (from < to) {
+                        const uint32_t mid = from + (to - from) / 2;
+                        if (low <= (int64_t)((double)weight * smc_u01_32(mid))) to = mid;
+                        else from = mid + 1;
+                    }
+                    d.recv_split = to;
+                }
             } else {
                 d.recv_chan = -1;
                 d.recv_mask = 0;
             }
-            if (!(d.flags & SMC_LF_RECV_TWO)) d.recv_low = 0xFFFFFFFFu;
 
             // spontaneous edges with constant weights
             int64_t pick_sum = 0;

@@ -1114,41 +1114,110 @@ __device__ __forceinline__ int race_pick(const double (&leaf)[C], const double (
 
 // ------------------------------------------------------------ receivers
 
-// Receivers of the broadcast `chan` sent by component `sender`
-// (SyncInSerial simulation.cu:357-407): the enabled receive edges of every
-// other component, then one edge fired per component that has any.
-//
-// Nearly always every receive edge commutes (SMC_LF_RECV_FAST): constant
-// weights make each receiver's pick independent of the others' updates, and
-// integer additions and private constants give the same variables in any
-// order, so all fire at once.  The query variable's running max/min needs
-// the values in component order: they are v0 plus the prefix sums of the
-// additions, an exclusive scan over the segment (blocked layout: lane order
-// then slot order is component order).  Otherwise they fire one at a time in
-// component order, the enabled sets computed before any of them fires.
-// TRACE mixes the fired edges into the digest in component order; LOCS keeps
-// the network's locations beside the state words; `trans` counts this
-// lane's.
+// Word of the receivers' draw that component c uses.
+__device__ __forceinline__ uint32_t receiver_word(const smc_u32x4 &w, uint32_t c) {
+    const uint32_t a = (c & 1u) ? w.v[1] : w.v[0], b = (c & 1u) ? w.v[3] : w.v[2];
+    return (c & 2u) ? b : a;
+}
+
+// A lane's additions to the query variable by receivers that fire at once:
+// their sum, and the extremes of its prefixes.
+struct ReceiverSums {
+    double sum = 0.0, hi = -DBL_MAX, lo = DBL_MAX;
+    bool any = false;
+};
+
+// The updates (additions and constants) of a receiver's edge record e, whose
+// third quarter is `tail`, on the lanes where `on`.
+template <class M>
+__device__ __forceinline__ void receiver_updates(bool on, uint32_t e, const uint4 &tail, const Ctx &x, const M &m,
+                                                 LaneQuery &q, ReceiverSums &sum) {
+    auto update = [&](double value, double *at, bool add, bool clock) {
+        if (add) {
+            if (at == x.vars + q.qvar) {
+                sum.sum += value;
+                sum.hi = fmax(sum.hi, sum.sum);
+                sum.lo = fmin(sum.lo, sum.sum);
+                sum.any = true;
+            }
+            atomicAdd(at, value);
+        } else {
+            if (at == x.vars + q.qvar) {
+                q.qmax = fmax(q.qmax, value);
+                q.qmin = fmin(q.qmin, value);
+            }
+            *at = clock ? x.now - value : value;
+        }
+    };
+    const uint4 u0 = load_quad(rec_at(m.edges, e), 3);
+    if (any_lane(on && (u0.z >> 16) >= SMC_EU_ADD)) {
+        const uint4 u1 = load_quad(rec_at(m.edges, e), 4);
+        if (on && (u0.z >> 16) >= SMC_EU_ADD)
+            update(quad_f64(u0), var_ptr(x, u0.z & 0xFFFFu, u0.z >> 16), (u0.z & (SMC_EU_ADD << 16)) != 0,
+                   (u0.z & (SMC_EU_CLOCK << 16)) != 0);
+        if (on && (u1.z >> 16) >= SMC_EU_ADD)
+            update(quad_f64(u1), var_ptr(x, u1.z & 0xFFFFu, u1.z >> 16), (u1.z & (SMC_EU_ADD << 16)) != 0,
+                   (u1.z & (SMC_EU_CLOCK << 16)) != 0);
+        const int n = on ? (int)(tail.z >> 16) : 0;
+        if (any_lane(n != 0)) {
+            for (int k = 0; k < n; ++k) {
+                const DevUpd U = load_rec(m.upds + tail.w + k);
+                update(U.value, x.vars + var_at(U.var, x.base), U.kind == SMC_U_ADD, U.clock != 0);
+            }
+        }
+    }
+}
+
+// The query variable's extremes over them, in component order.
+__device__ __forceinline__ void receiver_query(const ReceiverSums &sum, double v0, LaneQuery &q, int sl, int S) {
+    if (q.qvar >= 0 && any_lane(sum.any)) {
+        double incl = sum.sum;
+        for (int k = 1; k < S; k <<= 1) {
+            const double y = __shfl_up(incl, k, S);
+            if (sl >= k) incl += y;
+        }
+        const double at = v0 + (incl - sum.sum);  // value before this lane's additions
+        if (sum.any) {
+            q.qmax = fmax(q.qmax, at + sum.hi);
+            q.qmin = fmin(q.qmin, at + sum.lo);
+        }
+    }
+}
+
+// Their edges into the digest, in component order.
+template <int C>
+__device__ __forceinline__ void digest_receivers(const int (&fired)[C], bool any, uint64_t &digest, uint32_t step,
+                                                 int seg_base, uint64_t seg_mask) {
+    for (uint64_t lanes_with = __ballot(any) & seg_mask; lanes_with; lanes_with &= lanes_with - 1) {
+        const int L = lowest_lane(lanes_with);
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            const int e = __shfl(fired[j], L);
+            if (e >= 0)
+                digest = smc_mix(digest, ((uint64_t)step << 40) | ((uint64_t)((L - seg_base) * C + j) << 20) |
+                                             (uint64_t)e);
+        }
+    }
+}
+
+// Receivers with guards, on several channels, or with three edges or more.
 template <int C, bool TRACE, bool LOCS, class M>
-__device__ __forceinline__ void fire_receivers(uint32_t *words, int32_t *locs, Ctx x, const M &m, int chan,
-                                               int sender, LaneQuery &q, bool &goal, uint64_t seed, uint64_t run,
-                                               uint32_t step, int lane, int sl, int S, int seg_base, uint64_t seg_mask,
-                                               uint32_t &trans, uint64_t &digest) {
+__device__ __forceinline__ void fire_receivers_general(uint32_t *words, int32_t *locs, Ctx x, const M &m, int chan,
+                                                       int sender, LaneQuery &q, bool &goal, uint64_t seed,
+                                                       uint64_t run, uint32_t step, int lane, int sl, int S,
+                                                       int seg_base, uint64_t seg_mask, uint32_t &trans,
+                                                       uint64_t &digest) {
     // the enabled receive edges of every slot but the sender's: one bit set
     // each, from its location's record where they are all unguarded on one
     // channel
     uint32_t mk[C];
     uint32_t other = 0;
-    {
-        uint4 rv[C];  // recv_chan, recv_mask, ...
 #pragma unroll
-        for (int j = 0; j < C; ++j) rv[j] = load_quad(m.locs + word_rec(words[64 * j], m), 0);
-#pragma unroll
-        for (int j = 0; j < C; ++j) {
-            const bool me = sl * C + j == sender;
-            mk[j] = (((int)rv[j].x == chan) & !me) ? rv[j].y : 0u;
-            other |= (((int)rv[j].x == -1) & !me) ? 1u << j : 0u;
-        }
+    for (int j = 0; j < C; ++j) {
+        const uint4 rv = load_quad(m.locs + word_rec(words[64 * j], m), 0);
+        const bool me = sl * C + j == sender;
+        mk[j] = (((int)rv.x == chan) & !me) ? rv.y : 0u;
+        other |= (((int)rv.x == -1) & !me) ? 1u << j : 0u;
     }
     uint64_t slow = 0;
     uint32_t mk_hi[C];  // edges past the 32nd (only where receivers fire one at a time)
@@ -1175,8 +1244,7 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, int32_t *locs, C
     if (!slow) {
         int fired[TRACE ? C : 1];  // the network's index of each slot's edge (digests)
         bool any = false;
-        double qsum = 0.0, qhi = -DBL_MAX, qlo = DBL_MAX;  // prefix sums of this lane's query additions
-        bool qany = false;
+        ReceiverSums sum;
         const double v0 = q.qvar >= 0 ? x.vars[q.qvar] : 0.0;
         wave_sync();  // read before any receiver's additions
         // Receivers 4g .. 4g+3 share draw g: the lane's slots of one draw are
@@ -1201,15 +1269,13 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, int32_t *locs, C
                 int i = on ? __ffs(mk[j]) - 1 : 0;
                 if (any_lane(choice)) {
                     // weighted choice; weights are constants summing below
-                    // 2^31.  Two edges: the higher one unless the draw falls
-                    // below the lower one's weight.
-                    const double u = smc_receiver_u(rw, c);
-                    const bool two = choice & (rv.w != 0xFFFFFFFFu) & (mk[j] == rv.y);
-                    const int rnd2 = (int)((double)rv.z * u);
-                    if (two & ((int)rv.w <= rnd2)) i = 31 - __clz((int)mk[j]);
+                    // 2^31
+                    const bool two = choice & ((rv.w & SMC_RF_TWO) != 0) & (mk[j] == rv.y);
+                    if (two & (receiver_word(rw, c) >= rv.z)) i = 31 - __clz((int)mk[j]);
                     const bool several = choice & !two;
                     if (unlikely(any_lane(several))) {
                         if (several) {
+                            const double u = smc_receiver_u(rw, c);
                             int W = 0;
                             for (uint32_t r = mk[j]; r; r &= r - 1) W += (int)rec_at(m.edges, ef + __ffs(r) - 1)->weight;
                             const int rnd = (int)((double)W * u);
@@ -1231,68 +1297,12 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, int32_t *locs, C
                 if (on) words[64 * j] = (head.x << m.rec_shift) | base;
                 if (TRACE) fired[j] = on ? m.loc_edge0[on ? locs[64 * j] : 0] + i : -1;
                 if (LOCS && on) locs[64 * j] += rec_at(m.edges, e)->dst;
-                // updates: additions and constants
-                auto update = [&](double value, double *at, bool add, bool clock) {
-                    if (add) {
-                        if (at == x.vars + q.qvar) {
-                            qsum += value;
-                            qhi = fmax(qhi, qsum);
-                            qlo = fmin(qlo, qsum);
-                            qany = true;
-                        }
-                        atomicAdd(at, value);
-                    } else {
-                        if (at == x.vars + q.qvar) {
-                            q.qmax = fmax(q.qmax, value);
-                            q.qmin = fmin(q.qmin, value);
-                        }
-                        *at = clock ? x.now - value : value;
-                    }
-                };
                 x.base = base;
-                const uint4 u0 = load_quad(rec_at(m.edges, e), 3);
-                if (any_lane(on && (u0.z >> 16) >= SMC_EU_ADD)) {
-                    const uint4 u1 = load_quad(rec_at(m.edges, e), 4);
-                    if (on && (u0.z >> 16) >= SMC_EU_ADD)
-                        update(quad_f64(u0), var_ptr(x, u0.z & 0xFFFFu, u0.z >> 16), (u0.z & (SMC_EU_ADD << 16)) != 0,
-                               (u0.z & (SMC_EU_CLOCK << 16)) != 0);
-                    if (on && (u1.z >> 16) >= SMC_EU_ADD)
-                        update(quad_f64(u1), var_ptr(x, u1.z & 0xFFFFu, u1.z >> 16), (u1.z & (SMC_EU_ADD << 16)) != 0,
-                               (u1.z & (SMC_EU_CLOCK << 16)) != 0);
-                    const int n = on ? (int)(tail.z >> 16) : 0;
-                    if (any_lane(n != 0)) {
-                        for (int k = 0; k < n; ++k) {
-                            const DevUpd U = load_rec(m.upds + tail.w + k);
-                            update(U.value, x.vars + var_at(U.var, base), U.kind == SMC_U_ADD, U.clock != 0);
-                        }
-                    }
-                }
+                receiver_updates(on, e, tail, x, m, q, sum);
             } else if (TRACE) fired[j] = -1;
         }
-        if (q.qvar >= 0 && any_lane(qany)) {
-            double incl = qsum;
-            for (int k = 1; k < S; k <<= 1) {
-                const double y = __shfl_up(incl, k, S);
-                if (sl >= k) incl += y;
-            }
-            const double at = v0 + (incl - qsum);  // value before this lane's additions
-            if (qany) {
-                q.qmax = fmax(q.qmax, at + qhi);
-                q.qmin = fmin(q.qmin, at + qlo);
-            }
-        }
-        if (TRACE) {
-            for (uint64_t lanes_with = __ballot(any) & seg_mask; lanes_with; lanes_with &= lanes_with - 1) {
-                const int L = lowest_lane(lanes_with);
-#pragma unroll
-                for (int j = 0; j < C; ++j) {
-                    const int e = __shfl(fired[j], L);
-                    if (e >= 0)
-                        digest = smc_mix(digest, ((uint64_t)step << 40) |
-                                                     ((uint64_t)((L - seg_base) * C + j) << 20) | (uint64_t)e);
-                }
-            }
-        }
+        receiver_query(sum, v0, q, sl, S);
+        if constexpr (TRACE) digest_receivers<C>(fired, any, digest, step, seg_base, seg_mask);
     } else {
         // one at a time: the lanes holding enabled receivers in lane order,
         // their slots in slot order; each picks with its own stream
@@ -1330,6 +1340,105 @@ __device__ __forceinline__ void fire_receivers(uint32_t *words, int32_t *locs, C
             }
         }
     }
+    wave_sync();
+}
+
+// Receivers of the broadcast `chan` sent by component `sender`
+// (SyncInSerial simulation.cu:357-407): the enabled receive edges of every
+// other component, then one edge fired per component that has any.
+//
+// Nearly always every receive edge commutes (SMC_LF_RECV_FAST): constant
+// weights make each receiver's pick independent of the others' updates, and
+// integer additions and private constants give the same variables in any
+// order, so all fire at once.  The query variable's running max/min needs
+// the values in component order: they are v0 plus the prefix sums of the
+// additions, an exclusive scan over the segment (blocked layout: lane order
+// then slot order is component order).  Otherwise they fire one at a time in
+// component order, the enabled sets computed before any of them fires.
+// TRACE mixes the fired edges into the digest in component order; LOCS keeps
+// the network's locations beside the state words; `trans` counts this
+// lane's.
+template <int C, bool TRACE, bool LOCS, class M>
+__device__ __forceinline__ void fire_receivers(uint32_t *words, int32_t *locs, Ctx x, const M &m, int chan,
+                                               int sender, LaneQuery &q, bool &goal, uint64_t seed, uint64_t run,
+                                               uint32_t step, int lane, int sl, int S, int seg_base, uint64_t seg_mask,
+                                               uint32_t &trans, uint64_t &digest) {
+    uint32_t on = 0, two = 0, low_idle = 0, high_idle = 0, general = 0;
+    uint32_t split[C];
+    constexpr int G = C < 8 ? C : 8;  // records read at a time
+#pragma unroll
+    for (int j0 = C - G; j0 >= 0; j0 -= G) {
+        uint4 rv[G];  // recv_chan, recv_mask, recv_split, recv_flags
+#pragma unroll
+        for (int j = 0; j < G; ++j) rv[j] = load_quad(m.locs + word_rec(words[64 * (j0 + j)], m), 0);
+#pragma unroll
+        for (int j = G - 1; j >= 0; --j) {
+            const bool here = (int)rv[j].x == chan;
+            on = shift_in(on, here);
+            general = shift_in(general, ((int)rv[j].x == -1) | (here & ((rv[j].w & SMC_RF_MORE) != 0)));
+            two = shift_in_sign(two, rv[j].w);
+            low_idle = shift_in_sign(low_idle, rv[j].w << 2);
+            high_idle = shift_in_sign(high_idle, rv[j].w << 3);
+            split[j0 + j] = rv[j].z;
+        }
+    }
+    const uint32_t others = sl == sender / C ? ~(1u << (sender % C)) : ~0u;
+    on &= others;
+    general &= others;
+    if (any_lane(general != 0)) {
+        fire_receivers_general<C, TRACE, LOCS>(words, locs, x, m, chan, sender, q, goal, seed, run, step, lane, sl, S,
+                                               seg_base, seg_mask, trans, digest);
+        return;
+    }
+    // the picks: receivers 4g .. 4g+3 share draw g, made when any of the
+    // lane's slots of it has a choice
+    const uint32_t choice = on & two;
+    uint32_t high = 0;
+    constexpr int D = C < 4 ? C : 4;
+#pragma unroll
+    for (int j0 = C - D; j0 >= 0; j0 -= D) {
+        const uint32_t c0 = (uint32_t)(sl * C + j0);
+        if (any_lane(((choice >> j0) & ((1u << D) - 1u)) != 0)) {
+            const smc_u32x4 rw = draw(seed, run, step, SMC_P_RECEIVER, smc_receiver_draw(c0));
+#pragma unroll
+            for (int j = D - 1; j >= 0; --j)
+                high = shift_in(high, (D == 4 ? rw.v[j] : receiver_word(rw, c0 + j)) >= split[j0 + j]);
+        } else {
+            high <<= D;
+        }
+    }
+    high &= choice;
+    trans += (uint32_t)__popc(on);
+    int fired[TRACE ? C : 1];  // the network's index of each slot's edge (digests)
+    if (TRACE) {
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            const uint32_t mask = load_quad(m.locs + word_rec(words[64 * j], m), 0).y;
+            const int i = (high >> j) & 1u ? 31 - __clz((int)mask) : __ffs(mask) - 1;
+            fired[j] = (on >> j) & 1u ? m.loc_edge0[locs[64 * j]] + i : -1;
+        }
+    }
+    const double v0 = q.qvar >= 0 ? x.vars[q.qvar] : 0.0;
+    wave_sync();  // read before any receiver's additions
+    ReceiverSums sum;
+#pragma clang loop unroll(disable)
+    for (uint32_t act = on & ~((high & high_idle) | (~high & low_idle)); any_lane(act != 0); act &= act - 1) {
+        const bool go = act != 0;
+        const int j = go ? __ffs(act) - 1 : 0;
+        const uint32_t w = words[64 * j];
+        const auto L = m.locs + word_rec(w, m);
+        const uint32_t mask = load_quad(L, 0).y;
+        const int i = (high >> j) & 1u ? 31 - __clz((int)mask) : __ffs(mask) - 1;
+        const uint32_t e = go ? L->edge_first + i : 0u;
+        const uint4 head = load_quad(rec_at(m.edges, e), 0), tail = load_quad(rec_at(m.edges, e), 2);
+        goal |= go & ((head.y & SMC_EF_GOAL) != 0);
+        x.base = word_base(w, m);
+        if (go) words[64 * j] = (head.x << m.rec_shift) | x.base;
+        if (LOCS && go) locs[64 * j] += rec_at(m.edges, e)->dst;
+        receiver_updates(go, e, tail, x, m, q, sum);
+    }
+    receiver_query(sum, v0, q, sl, S);
+    if constexpr (TRACE) digest_receivers<C>(fired, on != 0, digest, step, seg_base, seg_mask);
     wave_sync();
 }
 

@@ -76,8 +76,15 @@ enum {
                             // there is none): always blocked
     SMC_LF_GUARDED = 4,     // blocked or not by the variables: every spontaneous edge without
                             // `!=` has a conjunct that reads no clock (DevLoc.block_first)
-    SMC_LF_RECV_FAST = 8,   // every receive edge commutes (see DevUpd), constant weights below 2^31 in all
-    SMC_LF_RECV_TWO = 16    // recv_chan > 0 and exactly two receive edges
+    SMC_LF_RECV_FAST = 8    // every receive edge commutes (see DevUpd), constant weights below 2^31 in all
+};
+
+// DevLoc.recv_flags (recv_chan > 0).
+enum : uint32_t {
+    SMC_RF_TWO = 0x80000000u,     // exactly two receive edges
+    SMC_RF_MORE = 0x40000000u,    // three or more
+    SMC_RF_LOW_IDLE = 0x20000000u,   // the lower one (or the only one) changes nothing
+    SMC_RF_HIGH_IDLE = 0x10000000u   // the higher one of two changes nothing
 };
 
 // What a race step has to look at in a location (high half of DevHot.what).
@@ -117,8 +124,8 @@ struct DevHot {
 struct DevLoc {
     int32_t recv_chan;      // every receive edge is unguarded, on this channel; 0 none; -1 other
     uint32_t recv_mask;     // the receive edges, as bits of the edge list
-    uint32_t recv_weight;   // sum of their weights
-    uint32_t recv_low;      // of two receive edges, the lower one's weight; else 0xFFFFFFFF
+    uint32_t recv_split;    // of two: the least draw that picks the higher one
+    uint32_t recv_flags;    // SMC_RF_*
     uint32_t edge_first;    // edges [edge_first, edge_first + edge_n)
     uint16_t edge_n;
     uint8_t klass;
