@@ -129,6 +129,7 @@ struct OutSet {
 
 constexpr uint64_t kTrainRunBase = 1ull << 48;  // run indices of training rounds
 constexpr int kMaxBatchRows = 1 << 18;
+constexpr int kActiveWords = SMC_IS_COUNTS * SMC_IS_COUNT_STRIDE;
 constexpr int kTrainChunk = 1 << 21;  // pairs per training pass (all of a round's, usually)
 constexpr double kZ95 = 1.959963984540054;
 
@@ -141,13 +142,9 @@ struct smc_is {
     // launch shapes of the advance kernel, the widest packing first
     struct Shape {
         int S = 1, C = 1, R = 64;    // lanes per run, slots per lane, runs per wave
-        size_t lds = 0;
-        uint32_t wave_lds = 0;
-        bool tab = false;            // stages the model tables in LDS
-        int max_groups = 0;          // its persistent workgroups when it does
-        bool rec = true;             // two waves per SIMD when recording, too
     };
     std::vector<Shape> shapes;
+    bool stage = false;  // model tables staged in LDS
     int stride = 1;
     int n_locs = 0, n_vars = 0, n_comp = 0, F = 0, fpad = 0, H = 128, Lpad = 0;
     int n_groups = 0, Gpad = 0;  // tilt groups: the MLP's outputs
@@ -182,8 +179,8 @@ struct smc_is {
     // training activations of one chunk of pairs
     DevBuf<uint16_t> th1, th2, Gb, dh2b, dh1b, xin;
     DevBuf<float> tth, tthg, dh2, dh1, work, xf;
-    DevBuf<unsigned int> counters;  // [0] active rows, [1] record slots used, [2] compaction count
-    unsigned int *h_counters = nullptr;  // [0..1] copies of counters[0..1]; [2..3] active counts of alternate macro-steps
+    DevBuf<unsigned int> counters, active;  // [0] active rows, [1] record slots used, [2] compaction count
+    unsigned int *h_counters = nullptr;  // [0..1] copies of counters[0..1]; then the active counts of alternate macro-steps
     hipEvent_t step_done[2] = {nullptr, nullptr};
     int adam_t = 0;
     bool zero_output = true;  // output layer all zero: theta == 0 exactly
@@ -235,10 +232,21 @@ struct smc_is {
     // wave.  SIR-100 under a proposal network, the whole call at 64, 32 and 16
     // lanes a row: 5e4 rows 58.4, 39.6 and 28.7 ms, 4000 rows 9.7, 8.0 and
     // 7.5, 2000 rows 6.9, 6.6 and 6.7, 1000 rows 5.8, 5.9 and 6.2.
-    const Shape &shape_for(int rows, bool record) const {
+    const Shape &shape_for(int rows, const IsParams &P, bool record) const {
         size_t k = 0;
-        while (k + 1 < shapes.size() && rows / shapes[k + 1].R >= 2 * m->cu_count && (!record || shapes[k + 1].rec)) ++k;
+        while (k + 1 < shapes.size() && rows / shapes[k + 1].R >= 2 * m->cu_count &&
+               8 * (shared_lds(P) + wave_lds(shapes[k + 1], P, record)) <= kLdsPerCu)
+            ++k;
         return shapes[k];
+    }
+
+    // LDS of the advance kernel (is_advance.h): the workgroup's, and a wave's.
+    static constexpr size_t kLdsPerCu = 160 * 1024;
+    size_t shared_lds(const IsParams &P) const { return (size_t)Lpad * 4 + (size_t)P.theta_shared * 8; }
+    size_t wave_lds(const Shape &sh, const IsParams &P, bool record) const {
+        return rup((size_t)sh.R * stride * sizeof(double) + (size_t)sh.R * P.theta_cap * 12 +
+                       (size_t)sh.C * (P.windows ? 1024 : 512) + (size_t)sh.R * (Lpad / 8), 16) +
+               (record ? (size_t)16 * sh.C * 64 : 0);
     }
 
     IsParams params(int rows, uint64_t seed) const {
@@ -259,11 +267,9 @@ struct smc_is {
         P.max_steps = q.max_steps ? q.max_steps : SMC_DEFAULT_MAX_STEPS;
         P.tiltable = tiltable.p;
         P.tilt_index = tix_loc.p;
-        P.theta_cap = Gpad;
-        P.theta_len = 0;
+        P.windows = (m->img.tests & (SMC_HF_INV | SMC_HF_XINV)) ? 1 : 0;
         P.var_scale = var_scale.p;
         P.weight = weight.p;
-        P.active_count = counters.p;
         return P;
     }
 
@@ -384,7 +390,7 @@ struct smc_is {
         if (b.tilt == Tilt::FIXED) {
             P.theta = theta_fixed.p;
             P.theta_stride = 0;
-            P.theta_len = Lpad;
+            P.theta_len = P.theta_shared = Lpad;
             P.tilt_index = tix_loc.p;
         }
         if (b.record) {
@@ -398,12 +404,13 @@ struct smc_is {
         // (step k then found no live row); compaction sizes the new row set
         // from the same bound.
         int launches = 0;
+        hip_check(hipMemsetAsync(active.p, 0, kActiveWords * sizeof(unsigned int), s), "clear active count");
         for (int k = 0;; ++k) {
             if (feats) {
                 // the tilts from the features of the rows' states (the
                 // advance kernel then overwrites the features, in order)
                 P.theta_stride = forward(A->X.p, rows, nullptr, nullptr, thg.p, true, nullptr);
-                P.theta_len = P.theta_stride;
+                P.theta_len = P.theta_cap = P.theta_stride;
                 P.theta = thg.p;
                 P.tilt_index = tix_group.p;
             }
@@ -412,41 +419,41 @@ struct smc_is {
                           "record slots");
                 P.rec_pos = pos.p;
             }
-            unsigned int *cnt = counters.p + 3 + (k & 1);
-            hip_check(hipMemsetAsync(cnt, 0, sizeof(unsigned int), s), "clear active count");
+            unsigned int *cnt = active.p + (k & 1) * kActiveWords, *h_cnt = h_counters + 2 + (k & 1) * kActiveWords;
             P.active_count = cnt;
-            const Shape &sh = shape_for(rows, b.record);
+            P.next_count = active.p + ((k + 1) & 1) * kActiveWords;  // (its copy to the host is ahead in the stream)
+            const Shape &sh = shape_for(rows, P, b.record);
             P.lanes = sh.S;
-            P.tables = sh.tab ? (decltype(P.tables))m->arena : nullptr;
-            P.table_bytes = sh.tab ? m->table_bytes : 0;
-            P.wave_lds = sh.wave_lds;
-            size_t lds_use = sh.lds;
-            if (b.record) {
-                // the recording build reads the tables from global memory and
-                // keeps its per-slot statistics in LDS (16 C bytes per lane)
-                P.tables = nullptr;
-                P.table_bytes = 0;
-                P.wave_lds = sh.wave_lds + (uint32_t)(16 * sh.C * 64);
-                lds_use = (size_t)Lpad * 12 + P.wave_lds;
-            }
-            hip_check(smc::is_launch_advance(P, sh.C, lds_use, sh.max_groups, s), "advance kernel launch");
+            P.wave_lds = (uint32_t)wave_lds(sh, P, b.record);
+            // staged tables: workgroups of four waves, as many as the LDS
+            // holds, at most four a CU (four waves per SIMD); the recording
+            // build reads the tables from global memory
+            size_t lds = m->table_bytes + shared_lds(P) + 4 * (size_t)P.wave_lds;
+            const bool tab = stage && !b.record && m->table_bytes > 0 && lds <= kLdsPerCu;
+            P.tables = tab ? (decltype(P.tables))m->arena : nullptr;
+            P.table_bytes = tab ? m->table_bytes : 0;
+            if (!tab) lds = shared_lds(P) + P.wave_lds;
+            const int max_groups = tab ? std::min(4, (int)(kLdsPerCu / lds)) * m->cu_count : 0;
+            hip_check(smc::is_launch_advance(P, sh.C, lds, max_groups, s), "advance kernel launch");
             ++launches;
             if (!b.lockstep) break;
-            hip_check(hipMemcpyAsync(h_counters + 2 + (k & 1), cnt, sizeof(unsigned int), hipMemcpyDeviceToHost, s),
+            hip_check(hipMemcpyAsync(h_cnt, cnt, kActiveWords * sizeof(unsigned int), hipMemcpyDeviceToHost, s),
                       "copy active count");
             hip_check(hipEventRecord(step_done[k & 1], s), "event");
             if (k == 0) continue;
             hip_check(hipEventSynchronize(step_done[(k - 1) & 1]), "advance");
-            const int active = (int)h_counters[2 + ((k - 1) & 1)];
-            if (active == 0) break;
-            if (active * 2 <= rows && rows > 1024) {
+            int live = 0;
+            for (int i = 0; i < SMC_IS_COUNTS; ++i)
+                live += (int)h_counters[2 + ((k - 1) & 1) * kActiveWords + i * SMC_IS_COUNT_STRIDE];
+            if (live == 0) break;
+            if (live * 2 <= rows && rows > 1024) {
                 // compaction: results of the finished rows out, live rows
                 // to the front of the other set, in row order
                 hip_check(smc::is_collect(P, out.view(), s), "collect results");
                 hip_check(hipMemsetAsync(counters.p + 2, 0, sizeof(unsigned int), s), "clear compaction count");
                 hip_check(smc::is_record_slots(A->status.p, rows, cpos.p, counters.p + 2, 0xFFFFFFFFu, s),
                           "compaction slots");
-                const int nrows = (int)rup((size_t)active, 64);
+                const int nrows = (int)rup((size_t)live, 64);
                 B->ensure((size_t)nrows, n_comp, n_vars, fpad, feats);
                 hip_check(hipMemsetAsync(B->status.p, 0, (size_t)nrows, s), "clear rows");
                 hip_check(hipMemsetAsync(B->job.p, 0xFF, (size_t)nrows * 4, s), "clear rows");
@@ -636,10 +643,6 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         }
         s->Gpad = (int)rup((size_t)std::max(s->n_groups, 1), 64);
         s->G16 = (int)rup((size_t)std::max(s->n_groups, 1), 16);
-        // advance kernel LDS: per wave the variables of its 64/S rows, their
-        // tilt tables (theta and 2^theta, up to Gpad entries), slot scratch,
-        // state words, locations and their bitmap (is_advance.h), after a shared part (tilt
-        // index and a shared 2^theta vector, Lpad each)
         for (int S = lanes; S >= fewest; S /= 2) {
             smc_is::Shape sh;
             sh.S = S;
@@ -647,32 +650,28 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
             sh.R = 64 / S;
             int levels = 0;
             while ((1 << levels) < S) ++levels;
-            const size_t tilts = (size_t)sh.R * s->Gpad * 12, shared = (size_t)s->Lpad * 12;
-            sh.wave_lds = (uint32_t)rup((size_t)sh.R * s->stride * sizeof(double) + tilts +
-                                            (size_t)sh.C * 64 * sizeof(double) + (size_t)sh.C * 512 +
-                                            (size_t)sh.R * (s->Lpad / 8), 16);
-            // hot tables staged in LDS when the model's tuned launch does so
-            // (or SMC_IS_TABLES=1/0 says) and four waves fit beside them
-            const char *tv = std::getenv("SMC_IS_TABLES");
-            bool want = m->has_tuned && m->tuned.tables == 1;
-            if (tv) want = std::string(tv) == "1";
-            const size_t need = (size_t)m->table_bytes + shared + 4 * (size_t)sh.wave_lds;
-            sh.tab = want && m->table_bytes > 0 && need <= 160 * 1024;
-            sh.lds = sh.tab ? need : shared + sh.wave_lds;
             // the most variables and tilts a packing may hold: with a clock
             // time per row and two doubles per lane and level, 60,000 bytes
-            const bool vars = (size_t)sh.R * ((img.n_vars + 1) | 1) * 8 + tilts + (size_t)levels * 1024 <= 60000;
-            if (S == lanes) {
-                if (!vars) throw std::runtime_error("limit: variables exceed the LDS budget");
-                if (sh.lds > 160 * 1024) throw std::runtime_error("limit: the advance kernel's LDS exceeds the budget");
-            } else if (!vars || 8 * (shared + sh.wave_lds) > 160 * 1024) {
-                break;  // not two waves per SIMD
+            const size_t tilts = (size_t)sh.R * s->Gpad * 12;
+            if ((size_t)sh.R * ((img.n_vars + 1) | 1) * 8 + tilts + (size_t)levels * 1024 > 60000) {
+                if (S == lanes) throw std::runtime_error("limit: variables exceed the LDS budget");
+                break;
             }
-            sh.rec = 8 * (shared + sh.wave_lds + (size_t)16 * sh.C * 64) <= 160 * 1024;
-            // two waves per SIMD: two workgroups of four waves per CU
-            const int per_cu = sh.tab ? std::max(1, std::min(2, (int)((160 * 1024) / need))) : 0;
-            sh.max_groups = per_cu * m->cu_count;
             s->shapes.push_back(sh);
+        }
+        {
+            // the advance kernel's LDS at its largest: tilts per location
+            IsParams big{};
+            big.theta_cap = s->Gpad;
+            big.theta_shared = s->Lpad;
+            big.windows = 1;
+            if (s->shared_lds(big) + s->wave_lds(s->shapes[0], big, false) > 160 * 1024)
+                throw std::runtime_error("limit: the advance kernel's LDS exceeds the budget");
+            // hot tables staged in LDS (where they fit beside four waves)
+            // unless the model's tuned launch does not, or SMC_IS_TABLES=1/0
+            // says
+            s->stage = !m->has_tuned || m->tuned.tables != 0;
+            if (const char *tv = std::getenv("SMC_IS_TABLES")) s->stage = std::string(tv) == "1";
         }
         // the fused forward pass when its weights fit in LDS;
         // SMC_IS_FORWARD=gemm forces the three-GEMM path (the two agree bit
@@ -743,10 +742,11 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         s->var_scale.ensure(scale.size(), "hipMalloc scales");
         s->theta_fixed.ensure(L, "hipMalloc tilts");
         s->feat0.ensure(fp, "hipMalloc features");
-        // counters: [0] active rows, [1] recorded pairs, [2] compaction slots,
-        // [3..4] active rows after alternate macro-steps
-        s->counters.ensure(5, "hipMalloc counters");
-        hip_check(hipHostMalloc((void **)&s->h_counters, 4 * sizeof(unsigned int), hipHostMallocDefault), "hipHostMalloc");
+        // counters: [1] recorded pairs, [2] compaction slots; active: the
+        // active rows after alternate macro-steps
+        s->counters.ensure(3, "hipMalloc counters");
+        s->active.ensure(2 * kActiveWords, "hipMalloc counters");
+        hip_check(hipHostMalloc((void **)&s->h_counters, (2 + 2 * kActiveWords) * sizeof(unsigned int), hipHostMallocDefault), "hipHostMalloc");
         for (hipEvent_t &e : s->step_done)
             hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
         hip_check(hipMemcpyAsync(s->tiltable.p, s->h_tiltable.data(), L, hipMemcpyHostToDevice, st), "upload");

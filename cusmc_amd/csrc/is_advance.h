@@ -443,8 +443,10 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
         st.digest[row] = digest;
         st.status[row] = (uint8_t)((still ? IS_ACTIVE : 0) | (hit ? IS_HIT : 0) | (goal ? IS_GOAL : 0) |
                                    (still && mid ? IS_MID : 0));
-        if (still && P.active_count) atomicAdd(P.active_count, 1u);
     }
+    const uint64_t rows_on = __ballot(still && sl == 0);
+    if (P.active_count && rows_on && lane == lowest_lane(rows_on))
+        atomicAdd(P.active_count + (blockIdx.x % SMC_IS_COUNTS) * SMC_IS_COUNT_STRIDE, (unsigned int)__popcll(rows_on));
     if (P.feat) write_features<C>(P, P.feat + (size_t)row * P.fpad, locs, vars, bits, t, sl, S, n);
     if (rec >= 0) {
         // statistics of the macro-step for the locations its components
@@ -480,14 +482,15 @@ template <int C, bool TAB, bool REC>
 __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     extern __shared__ __attribute__((aligned(16))) double lds[];
     const int wv = threadIdx.x >> 6, W = blockDim.x >> 6;
-    // LDS: [tables: TAB only][tilt index: lpad int32][2^theta: lpad doubles]
-    //      then per wave [variables][rows' 2^theta][rows' theta][scratch: C
-    //      doubles per lane][state words, locations: 4 C bytes per lane each][recording
-    //      build: 16 C bytes per lane]
+    // LDS: [tables: TAB only][tilt index: lpad int32][2^theta: theta_shared
+    //      doubles] then per wave [variables][rows' 2^theta][rows' theta]
+    //      [windows: C doubles per lane, if any location has an invariant]
+    //      [state words, locations: 4 C bytes per lane each][locations held:
+    //      lpad bits per row][recording build: 16 C bytes per lane]
     double *shared = lds + (TAB ? P.table_bytes / 8 : 0);
     int32_t *tix = (int32_t *)shared;
     double *ex = shared + P.lpad / 2;
-    double *wlds = shared + (size_t)P.lpad * 3 / 2 + (size_t)wv * (P.wave_lds / 8);
+    double *wlds = shared + P.lpad / 2 + P.theta_shared + (size_t)wv * (P.wave_lds / 8);
     const int R = 64 / P.lanes;
     TiltLds tl;
     tl.tix = tix;
@@ -495,7 +498,7 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     tl.row_ex = wlds + (size_t)R * P.var_stride;
     tl.row_th = (float *)(tl.row_ex + (size_t)R * P.theta_cap);
     tl.scr = (double *)(tl.row_th + (size_t)R * P.theta_cap);
-    tl.words = (uint32_t *)(tl.scr + 64 * C);
+    tl.words = (uint32_t *)(tl.scr + (P.windows ? 64 * C : 0));
     tl.locs = (int32_t *)tl.words + 64 * C;
     tl.bits = (uint32_t *)(tl.locs + 64 * C);
     tl.rec = (double *)(tl.bits + R * (P.lpad / 32));
@@ -503,6 +506,8 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     for (int i = threadIdx.x; i < P.lpad; i += blockDim.x) tix[i] = P.tilt_index[i];
     if (P.theta && P.theta_stride == 0)
         for (int i = threadIdx.x; i < P.theta_len; i += blockDim.x) ex[i] = smc_exp2((double)P.theta[i]);
+    if (blockIdx.x == 0 && threadIdx.x < SMC_IS_COUNTS && P.next_count)
+        P.next_count[threadIdx.x * SMC_IS_COUNT_STRIDE] = 0;
     const int groups = (P.n_rows + R - 1) / R;
     if constexpr (TAB) {
         stage_tables(P.tables, P.table_bytes, lds);  // ends with the workgroup barrier

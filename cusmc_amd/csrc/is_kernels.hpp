@@ -53,7 +53,9 @@ struct IsParams {
     uint32_t table_bytes;       // bytes staged (multiple of 16)
     uint32_t wave_lds;          // LDS bytes of one wave after the shared part (multiple of 16)
     int32_t theta_len;          // entries of a theta row (<= lpad when theta_stride == 0, else <= theta_cap)
-    int32_t theta_cap;          // per-row tilt entries each wave's LDS holds room for
+    int32_t theta_cap;          // per-row tilt entries each wave's LDS holds room for (0 or a multiple of 16)
+    int32_t theta_shared;       // entries of 2^theta the workgroup's LDS holds room for
+    int32_t windows;            // each wave's LDS holds a window per slot
     uint16_t *feat;             // [rows][fpad] bf16 features of the end state, or null
     const float *var_scale;     // [n_vars]
     // recording of cross-entropy statistics (replay of elite runs)
@@ -63,8 +65,15 @@ struct IsParams {
     float *rec_B;               // [slots][lpad] ln2 * dt * base rate per location
     float *rec_w;               // [slots] weight of the row
     const float *weight;        // [jobs]
-    unsigned int *active_count; // rows still active after the launch
+    unsigned int *active_count; // rows still active after the launch: SMC_IS_COUNTS parts
+    unsigned int *next_count;   // the next launch's, cleared by this one
 };
+
+// The active rows are counted in parts, a cache line each, one atomic per
+// wave: with an atomic per row on one word, 5e4 rows took 181 us a launch,
+// which is the rate of that word's atomics.
+#define SMC_IS_COUNTS 16
+#define SMC_IS_COUNT_STRIDE 32
 
 // The proposal network's forward pass in one launch: theta_g =
 // clamp(W3^T relu(W2^T relu(W1^T x + b1) + b2) + b3), zero at untiltable
