@@ -816,6 +816,37 @@ __device__ __forceinline__ double slot_window(const uint32_t *words, int j, Ctx 
     return left;
 }
 
+// The delay windows of slots j and j + 1, read side by side: one after the
+// other, three dependent LDS reads each, they were a tenth of a Fischer-32
+// step.  Meaningless for a slot that is not bounded.
+template <class M>
+__device__ __forceinline__ void slot_windows(double (&left)[2], const uint32_t *words, int j, Ctx x, const M &m) {
+    uint32_t w[2];
+    DevHot h[2];
+    double v[2];
+    bool other = false;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) w[k] = words[64 * (j + k)];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) h[k] = load_rec(m.hots + word_rec(w[k], m));
+#pragma unroll
+    for (int k = 0; k < 2; ++k) v[k] = hot_value(h[k], w[k], x.vars);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        left[k] = h[k].a - (x.now - v[k]) - h[k].b;
+        other |= (h[k].what & (SMC_HF_XINV << 16)) != 0;
+    }
+    if (unlikely(any_lane(other))) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (h[k].what & (SMC_HF_XINV << 16)) {
+                x.base = word_base(w[k], m);
+                left[k] = window_of(load_rec(m.locs + word_rec(w[k], m)), x, m);
+            }
+        }
+    }
+}
+
 // Classify the lane's slots: one straight line over them, each reading its
 // class's 32-byte record and its variable.  No branch depends on a lane or a
 // slot: the lanes of a wave hold components in every kind of location, so

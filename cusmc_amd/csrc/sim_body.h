@@ -382,26 +382,25 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
 #pragma clang loop unroll(disable)
                 do {
                     const bool delay = b != 0;
-                    const int j = delay ? __ffs(b) - 1 : 0;
+                    const int j = C > 1 && delay ? (__ffs(b) - 1) & ~1 : 0;
                     const uint32_t c = (uint32_t)(sl * C + j);
                     const smc_u32x4 rw = draw_at(seed, run, step,
                                                  delay ? ((uint32_t)SMC_P_UNIFORM << 24) | smc_uniform_draw(c)
                                                        : (uint32_t)SMC_P_RACE << 24);
-                    const double M0 = C > 2 ? slot_window(words, j, Ctx{vars, t, 0}, m)
-                                            : (C == 2 && j ? rs.left[C - 1] : rs.left[0]);
-                    const double du = M0 * smc_uniform_u(rw, c);
-                    if (delay && du < umin) { umin = du; unif_j = j; }
-                    b &= b - 1;
-                    if (C > 1) {
-                        const int j1 = j + 1 < C ? j + 1 : j;
-                        const bool pair = !(c & 1u) && ((b >> j1) & 1u);
-                        if (any_lane(pair)) {
-                            const double M1 = C > 2 ? slot_window(words, j1, Ctx{vars, t, 0}, m) : rs.left[C - 1];
-                            const double du1 = M1 * smc_uniform_u(rw, c + 1);
-                            if (pair && du1 < umin) { umin = du1; unif_j = j1; }
-                            b = pair ? b & (b - 1) : b;
-                        }
+                    double left[2];
+                    if constexpr (C > 2) {
+                        slot_windows(left, words, j, Ctx{vars, t, 0}, m);
+                    } else {
+                        left[0] = rs.left[0];
+                        left[1] = rs.left[C - 1];
                     }
+                    const double du = left[0] * smc_uniform_u(rw, c);
+                    if (((b >> j) & 1u) && du < umin) { umin = du; unif_j = j; }
+                    if (C > 1) {
+                        const double du1 = left[1] * smc_uniform_u(rw, c + 1);
+                        if (((b >> j) & 2u) && du1 < umin) { umin = du1; unif_j = j + 1; }
+                    }
+                    b &= ~(3u << j);
                     // every draw of the race is the same: keep the last
                     race.v[0] = delay ? race.v[0] : rw.v[0];
                     race.v[1] = delay ? race.v[1] : rw.v[1];
