@@ -382,7 +382,8 @@ int smc_model_create(const smc_network *net, int device, smc_model **out) {
         hip_check(hipMalloc(&m->d_inst, sizeof(InstDesc)), "hipMalloc instance");
         hip_check(hipMalloc(&m->d_counter, sizeof(unsigned long long)), "hipMalloc counter");
         hip_check(hipMalloc(&m->d_partials, 1024 * sizeof(ReducePartial)), "hipMalloc partials");
-        hip_check(hipMalloc(&m->d_acc, sizeof(ReducePartial)), "hipMalloc totals");
+        // the totals are written straight to host memory
+        hip_check(hipHostMalloc((void **)&m->totals, sizeof(ReducePartial), hipHostMallocDefault), "hipHostMalloc totals");
         *out = m.release();
         return SMC_OK;
     });
@@ -428,14 +429,12 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         lp.wave_lds = pl.wave_lds;
         const uint32_t blocks = reduce_blocks(n_runs);
 
-        hip_check(hipMemcpyAsync(m->d_inst, &m->h_inst, sizeof(InstDesc), hipMemcpyHostToDevice, m->stream), "upload instance");
-        hip_check(smc::launch_prep(m->d_counter, nullptr, 0, m->stream), "prep kernel launch");
+        hip_check(smc::launch_setup(m->h_inst, m->d_inst, m->d_counter, m->stream), "setup kernel launch");
         hip_check(hipEventRecord(m->ev[0], m->stream), "event");
         hip_check(smc::launch_sim(lp, pl.C, trace, pl.occ, waves, pl.group_waves, pl.lds, m->stream), "run kernel launch");
         hip_check(hipEventRecord(m->ev[1], m->stream), "event");
-        hip_check(smc::launch_reduce(m->d_inst, 1, blocks, m->d_partials, m->d_acc, 0, m->stream), "reduce kernel launch");
+        hip_check(smc::launch_reduce(m->d_inst, 1, blocks, m->d_partials, m->totals, 0, m->stream), "reduce kernel launch");
         hip_check(hipEventRecord(m->ev[2], m->stream), "event");
-        hip_check(hipMemcpyAsync(&m->h_acc, m->d_acc, sizeof(ReducePartial), hipMemcpyDeviceToHost, m->stream), "copy totals");
         if (outputs) {
             const RunBuffers &b = m->runs;
             if (outputs->flag) hip_check(hipMemcpyAsync(outputs->flag, b.flag, n_runs, hipMemcpyDeviceToHost, m->stream), "copy flags");
@@ -449,7 +448,7 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         float k_ms = 0.f, r_ms = 0.f;
         hip_check(hipEventElapsedTime(&k_ms, m->ev[0], m->ev[1]), "event time");
         hip_check(hipEventElapsedTime(&r_ms, m->ev[1], m->ev[2]), "event time");
-        fill_result(q, m->h_acc, n_runs, out);
+        fill_result(q, *m->totals, n_runs, out);
         out->kernel_ms = k_ms;
         out->reduce_ms = r_ms;
         out->lanes_per_run = pl.S;
@@ -512,8 +511,7 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         lp.table_bytes = pl.table_bytes;
         lp.wave_lds = pl.wave_lds;
 
-        hip_check(hipMemcpyAsync(d_inst, &m->h_inst, sizeof(InstDesc), hipMemcpyHostToDevice, m->stream), "upload instance");
-        hip_check(smc::launch_prep(d_counter, nullptr, 0, m->stream), "prep kernel launch");
+        hip_check(smc::launch_setup(m->h_inst, d_inst, d_counter, m->stream), "setup kernel launch");
         hip_check(hipEventRecord(m->ev[0], m->stream), "event");
         hip_check(smc::launch_sim(lp, pl.C, false, pl.occ, waves, pl.group_waves, pl.lds, m->stream), "run kernel launch");
         hip_check(hipEventRecord(m->ev[1], m->stream), "event");

@@ -88,7 +88,8 @@ struct smc_model {
     InstDesc h_inst{};
     InstDesc *d_inst = nullptr;
     unsigned long long *d_counter = nullptr;
-    ReducePartial *d_partials = nullptr, *d_acc = nullptr;
+    ReducePartial *d_partials = nullptr;
+    ReducePartial *totals = nullptr;  // pinned
     ReducePartial h_acc{};
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     smc_launch tuned{};
@@ -97,8 +98,9 @@ struct smc_model {
     ~smc_model() {
         if (device >= 0) hipSetDevice(device);
         runs.release();
-        for (void *p : {(void *)d_inst, (void *)d_counter, (void *)d_partials, (void *)d_acc, arena})
+        for (void *p : {(void *)d_inst, (void *)d_counter, (void *)d_partials, arena})
             if (p) hipFree(p);
+        if (totals) hipHostFree(totals);
         for (auto &e : ev) if (e) hipEventDestroy(e);
         if (stream) hipStreamDestroy(stream);
     }

@@ -87,5 +87,7 @@ hipError_t sim_occupancy(int slots, bool trace, int occ, bool tab, int group_wav
 hipError_t launch_reduce(const InstDesc *inst, int n_inst, uint32_t blocks_per_inst, ReducePartial *partials,
                          ReducePartial *acc, int accumulate, hipStream_t s);
 hipError_t launch_prep(unsigned long long *counter, uint64_t *round, int advance, hipStream_t s);
+// the start of a launch of one instance: its record written, the counter cleared
+hipError_t launch_setup(const InstDesc &inst, InstDesc *dst, unsigned long long *counter, hipStream_t s);
 
 }  // namespace smc

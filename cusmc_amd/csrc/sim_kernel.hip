@@ -26,6 +26,9 @@ __global__ __launch_bounds__(256) void reduce_kernel(const InstDesc *inst, uint3
     const uint64_t b1 = b0 + per_block < n ? b0 + per_block : n;
     double sum = 0.0, sq = 0.0, mn = __builtin_huge_val(), mx = -__builtin_huge_val();
     unsigned long long hits = 0, st = 0, tr = 0, tc = 0;
+    // (several runs' reads under way together: one after another they were
+    // the kernel's time, 16 trips to memory a thread)
+#pragma unroll 8
     for (uint64_t i = b0 + threadIdx.x; i < b1; i += 256) {
         const double v = p.value[i];
         sum += v;
@@ -72,6 +75,7 @@ __global__ void finalize_kernel(const ReducePartial *partials, int n_inst, uint3
     if (accumulate) t = acc[i];
     else { t.sum = 0; t.sumsq = 0; t.vmin = __builtin_huge_val(); t.vmax = -__builtin_huge_val();
            t.hits = 0; t.steps = 0; t.trans = 0; t.truncated = 0; }
+#pragma unroll 8
     for (uint32_t b = 0; b < blocks_per_inst; ++b) {
         const ReducePartial r = partials[(size_t)i * blocks_per_inst + b];
         t.sum += r.sum; t.sumsq += r.sumsq;
@@ -89,6 +93,15 @@ __global__ void prep_kernel(unsigned long long *counter, uint64_t *round, int ad
         *counter = 0;
         if (round && advance) *round += 1;
     }
+}
+
+// The same for a launch of one instance, whose record comes in the kernel's
+// arguments: no copy ahead of it.
+__global__ void setup_kernel(InstDesc inst, InstDesc *dst, unsigned long long *counter) {
+    static_assert(sizeof(InstDesc) % 8 == 0, "record size");
+    const uint64_t *from = (const uint64_t *)&inst;
+    for (int i = threadIdx.x; i < (int)(sizeof(InstDesc) / 8); i += 64) ((uint64_t *)dst)[i] = from[i];
+    if (threadIdx.x == 0) *counter = 0;
 }
 
 }  // namespace
@@ -126,6 +139,10 @@ hipError_t sim_occupancy(int slots, bool trace, int occ, bool tab, int group_wav
 
 hipError_t launch_reduce(const InstDesc *inst, int n_inst, uint32_t blocks_per_inst, ReducePartial *partials,
                          ReducePartial *acc, int accumulate, hipStream_t s) {
+    if (blocks_per_inst == 1 && n_inst == 1 && !accumulate) {  // the one partial is the total
+        hipLaunchKernelGGL(reduce_kernel, dim3(1), dim3(256), 0, s, inst, 1u, acc);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(reduce_kernel, dim3(blocks_per_inst, n_inst), dim3(256), 0, s, inst, blocks_per_inst, partials);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -136,6 +153,11 @@ hipError_t launch_reduce(const InstDesc *inst, int n_inst, uint32_t blocks_per_i
 
 hipError_t launch_prep(unsigned long long *counter, uint64_t *round, int advance, hipStream_t s) {
     hipLaunchKernelGGL(prep_kernel, dim3(1), dim3(64), 0, s, counter, round, advance);
+    return hipGetLastError();
+}
+
+hipError_t launch_setup(const InstDesc &inst, InstDesc *dst, unsigned long long *counter, hipStream_t s) {
+    hipLaunchKernelGGL(setup_kernel, dim3(1), dim3(64), 0, s, inst, dst, counter);
     return hipGetLastError();
 }
 
