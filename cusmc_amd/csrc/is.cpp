@@ -826,29 +826,24 @@ int smc_is_mlp_eval(smc_is *s, const float *x, int rows, const float *gout, floa
         s->ensure_train(rp, true);
         s->xf.ensure(std::max(nx, nt), "hipMalloc inputs");
         s->xin.ensure(nx, "hipMalloc inputs");
-        hip_check(hipMemsetAsync(s->xf.p, 0, nx * 4, st), "clear inputs");
-        hip_check(hipMemcpyAsync(s->xf.p, x, (size_t)rows * s->fpad * 4, hipMemcpyHostToDevice, st), "upload inputs");
+        const size_t mx = (size_t)rows * s->fpad, mt = (size_t)rows * s->Lpad;
+        if (nx > mx) hip_check(hipMemsetAsync(s->xf.p + mx, 0, (nx - mx) * 4, st), "clear inputs");
+        hip_check(hipMemcpyAsync(s->xf.p, x, mx * 4, hipMemcpyHostToDevice, st), "upload inputs");
         hip_check(smc::to_bf16(s->xf.p, s->xin.p, nx, st), "inputs to bf16");
         s->forward(s->xin.p, rp, s->th1.p, s->th2.p, s->tthg.p, false, s->tth.p);
-        std::vector<float> th((size_t)rows * s->Lpad);
-        hip_check(hipMemcpyAsync(th.data(), s->tth.p, th.size() * 4, hipMemcpyDeviceToHost, st), "copy tilts");
-        hip_check(hipStreamSynchronize(st), "MLP forward");
-        if (theta_out) memcpy(theta_out, th.data(), th.size() * 4);
+        if (theta_out)
+            hip_check(hipMemcpyAsync(theta_out, s->tth.p, mt * 4, hipMemcpyDeviceToHost, st), "copy tilts");
         if (gout) {
             // the output gradient, zero where the output is clamped or untiltable
-            std::vector<float> gm((size_t)rp * s->Lpad, 0.f);
-            for (int r = 0; r < rows; ++r)
-                for (int l = 0; l < s->Lpad; ++l) {
-                    const size_t i = (size_t)r * s->Lpad + l;
-                    if (s->h_tiltable[l] && std::fabs(th[i]) < s->cfg.tilt_max) gm[i] = gout[i];
-                }
-            hip_check(hipMemcpyAsync(s->tth.p, gm.data(), nt * 4, hipMemcpyHostToDevice, st), "upload output gradient");
+            hip_check(hipMemcpyAsync(s->xf.p, gout, mt * 4, hipMemcpyHostToDevice, st), "upload output gradient");
+            hip_check(smc::mask_gradient(s->xf.p, s->tiltable.p, s->cfg.tilt_max, s->Lpad, mt, nt, s->tth.p, st),
+                      "mask output gradient");
             hip_check(hipMemsetAsync(s->g.p, 0, s->n_params * 4, st), "clear gradient");
             s->backward(s->xin.p, rp);
             if (grad_out)
                 hip_check(hipMemcpyAsync(grad_out, s->g.p, s->n_params * 4, hipMemcpyDeviceToHost, st), "copy gradient");
-            hip_check(hipStreamSynchronize(st), "MLP backward");
         }
+        hip_check(hipStreamSynchronize(st), "MLP pass");
         return SMC_OK;
     });
 }

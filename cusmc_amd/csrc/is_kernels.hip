@@ -301,6 +301,16 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
             }
 }
 
+// theta = the gradient g where the output theta moves with the parameters
+// (tiltable, not clamped), else 0; rows past the last (i >= valid) too.
+__global__ __launch_bounds__(256) void mask_gradient_kernel(const float *g, const uint8_t *tiltable, float tilt_max,
+                                                            int lpad, size_t valid, size_t n, float *theta) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const bool on = i < valid && tiltable[i % (size_t)lpad] && fabsf(theta[i]) < tilt_max;
+    theta[i] = on ? g[i] : 0.f;
+}
+
 __global__ void to_bf16_kernel(const float *x, uint16_t *y, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) y[i] = f32_to_bf16(x[i]);
@@ -668,6 +678,13 @@ hipError_t is_ce_grad(const float *theta, const float *A, const float *B, const 
     if (!n) return hipSuccess;
     hipLaunchKernelGGL(ce_grad_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, theta, A, B, w, tiltable,
                        tilt_max, lpad, n, G);
+    return hipGetLastError();
+}
+
+hipError_t mask_gradient(const float *g, const uint8_t *tiltable, float tilt_max, int lpad, size_t valid, size_t n,
+                         float *theta, hipStream_t s) {
+    hipLaunchKernelGGL(mask_gradient_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, tiltable, tilt_max,
+                       lpad, valid, n, theta);
     return hipGetLastError();
 }
 

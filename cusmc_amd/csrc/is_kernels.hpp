@@ -157,6 +157,8 @@ hipError_t mlp_forward(const MlpFwdArgs &a, hipStream_t s);
 hipError_t gemm_splitk(const GemmArgs &g, bool ta, bool tb, int splits, float *work, hipStream_t s);
 // dst[N] (+)= column sums of X[rows][ld] (first N columns), split over rows.
 hipError_t colsum(const float *X, int rows, int ld, int N, float *dst, int splits, float *work, hipStream_t s);
+hipError_t mask_gradient(const float *g, const uint8_t *tiltable, float tilt_max, int lpad, size_t valid, size_t n,
+                         float *theta, hipStream_t s);
 hipError_t to_bf16(const float *x, uint16_t *y, size_t n, hipStream_t s);
 hipError_t adam_step(float *w, const float *g, float *m1, float *m2, size_t n, float lr, int t, uint16_t *wb,
                      hipStream_t s);
