@@ -435,16 +435,44 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         hip_check(hipEventRecord(m->ev[1], m->stream), "event");
         hip_check(smc::launch_reduce(m->d_inst, 1, blocks, m->d_partials, m->totals, 0, m->stream), "reduce kernel launch");
         hip_check(hipEventRecord(m->ev[2], m->stream), "event");
+        // per-run outputs: small ones through pinned memory (a copy to memory
+        // that is not waits for the device, each one some 25 us)
+        struct Output { void *to; const void *from; size_t bytes; const char *what; };
+        std::vector<Output> outs;
+        size_t staged = 0;
         if (outputs) {
             const RunBuffers &b = m->runs;
-            if (outputs->flag) hip_check(hipMemcpyAsync(outputs->flag, b.flag, n_runs, hipMemcpyDeviceToHost, m->stream), "copy flags");
-            if (outputs->value) hip_check(hipMemcpyAsync(outputs->value, b.value, n_runs * 8, hipMemcpyDeviceToHost, m->stream), "copy values");
-            if (outputs->steps) hip_check(hipMemcpyAsync(outputs->steps, b.steps, n_runs * 4, hipMemcpyDeviceToHost, m->stream), "copy steps");
-            if (outputs->transitions) hip_check(hipMemcpyAsync(outputs->transitions, b.trans, n_runs * 4, hipMemcpyDeviceToHost, m->stream), "copy transitions");
-            if (outputs->digest) hip_check(hipMemcpyAsync(outputs->digest, b.digest, n_runs * 8, hipMemcpyDeviceToHost, m->stream), "copy digests");
-            if (outputs->time) hip_check(hipMemcpyAsync(outputs->time, b.time, n_runs * 8, hipMemcpyDeviceToHost, m->stream), "copy times");
+            const Output all[] = {{outputs->flag, b.flag, n_runs, "copy flags"},
+                                  {outputs->value, b.value, n_runs * 8, "copy values"},
+                                  {outputs->steps, b.steps, n_runs * 4, "copy steps"},
+                                  {outputs->transitions, b.trans, n_runs * 4, "copy transitions"},
+                                  {outputs->digest, b.digest, n_runs * 8, "copy digests"},
+                                  {outputs->time, b.time, n_runs * 8, "copy times"}};
+            for (const Output &o : all)
+                if (o.to) {
+                    outs.push_back(o);
+                    staged += align_up(o.bytes, 64);
+                }
+        }
+        uint8_t *stage = nullptr;
+        if (staged && staged <= smc_model::kStageBytes) {
+            if (!m->stage && hipHostMalloc((void **)&m->stage, smc_model::kStageBytes, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();  // without it the copies go straight to the caller's arrays
+                m->stage = nullptr;
+            }
+            stage = m->stage;
+        }
+        size_t at = 0;
+        for (const Output &o : outs) {
+            hip_check(hipMemcpyAsync(stage ? stage + at : o.to, o.from, o.bytes, hipMemcpyDeviceToHost, m->stream), o.what);
+            at += align_up(o.bytes, 64);
         }
         hip_check(hipStreamSynchronize(m->stream), "run");
+        at = 0;
+        for (const Output &o : outs) {
+            if (stage) memcpy(o.to, stage + at, o.bytes);
+            at += align_up(o.bytes, 64);
+        }
         float k_ms = 0.f, r_ms = 0.f;
         hip_check(hipEventElapsedTime(&k_ms, m->ev[0], m->ev[1]), "event time");
         hip_check(hipEventElapsedTime(&r_ms, m->ev[1], m->ev[2]), "event time");

@@ -90,6 +90,8 @@ struct smc_model {
     unsigned long long *d_counter = nullptr;
     ReducePartial *d_partials = nullptr;
     ReducePartial *totals = nullptr;  // pinned
+    static constexpr size_t kStageBytes = 1 << 20;
+    uint8_t *stage = nullptr;         // pinned, kStageBytes, from the first call with per-run outputs on
     ReducePartial h_acc{};
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     smc_launch tuned{};
@@ -101,6 +103,7 @@ struct smc_model {
         for (void *p : {(void *)d_inst, (void *)d_counter, (void *)d_partials, arena})
             if (p) hipFree(p);
         if (totals) hipHostFree(totals);
+        if (stage) hipHostFree(stage);
         for (auto &e : ev) if (e) hipEventDestroy(e);
         if (stream) hipStreamDestroy(stream);
     }
