@@ -419,7 +419,6 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         LaunchParams lp{};
         lp.inst = m->d_inst;
         lp.n_inst = 1;
-        lp.var_stride = pl.stride;
         lp.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
         lp.segments = pl.segments;
         lp.counter = m->d_counter;
@@ -530,7 +529,6 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         LaunchParams lp{};
         lp.inst = d_inst;
         lp.n_inst = 1;
-        lp.var_stride = pl.stride;
         lp.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
         lp.segments = pl.segments;
         lp.counter = d_counter;
@@ -707,7 +705,7 @@ struct smc_batch {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<smc_batch_item> items;
     std::vector<RunBuffers> bufs;
-    int C = 8, occ = 0, waves = 1, stride = 1, max_vars = 1;  // the one launch: slots per lane, register policy
+    int C = 8, occ = 0, waves = 1, max_vars = 1;  // the one launch: slots per lane, register policy
     size_t lds = 0;
     InstDesc *d_all = nullptr;
     unsigned long long *d_counter = nullptr;
@@ -743,19 +741,34 @@ struct BatchShape {
     uint64_t chunks = 0;
 };
 
+// Lanes per run of an instance at C slots per lane.
+int batch_lanes(const smc_batch_item &it, int C) { return std::max(it.model->img.n_leaves / C, 1); }
+
+bool batch_fits(const smc_batch &b, int C) {
+    for (const smc_batch_item &it : b.items) {
+        const int S = batch_lanes(it, C);
+        if (!vars_fit(64 / S, b.max_vars, tree_levels(S))) return false;
+    }
+    return true;
+}
+
+// Waves that the runs fill at C slots per lane.
+uint64_t batch_chunks(const smc_batch &b, int C) {
+    uint64_t n = 0;
+    for (const smc_batch_item &it : b.items) n += it.n_runs * (uint64_t)batch_lanes(it, C) / 64;
+    return n;
+}
+
 BatchShape batch_shape(smc_batch *b, int C, uint64_t runs_override) {
     BatchShape sh;
-    bool fits = true;
-    int max_R = 1;
+    if (!batch_fits(*b, C)) throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
     for (size_t i = 0; i < b->items.size(); ++i) {
         const smc_batch_item &it = b->items[i];
         const int P = it.model->img.n_leaves;
         if (P > 64 * C) throw std::runtime_error("internal: instance wider than the launch's packing");
-        const int S = P / C >= 1 ? P / C : 1;
+        const int S = batch_lanes(it, C);
         const int R = 64 / S;
-        const int levels = tree_levels(S);
-        fits = fits && vars_fit(R, b->max_vars, levels);
-        max_R = std::max(max_R, R);
+        sh.wave_lds = std::max(sh.wave_lds, wave_lds_bytes(R, (it.model->img.n_vars + 1) | 1, C, false));
         const uint64_t n = runs_override ? std::min<uint64_t>(runs_override, it.n_runs) : it.n_runs;
         InstDesc d{};
         d.m = it.model->dm;
@@ -766,8 +779,6 @@ BatchShape batch_shape(smc_batch *b, int C, uint64_t runs_override) {
         sh.chunks += (n + R - 1) / R;
         sh.inst.push_back(d);
     }
-    if (!fits) throw std::runtime_error("limit: variables of the packed runs exceed the LDS budget");
-    sh.wave_lds = wave_lds_bytes(max_R, b->stride, C, false);
     return sh;
 }
 
@@ -807,7 +818,6 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
         for (hipEvent_t *e : {&b->ev0, &b->ev1}) hip_check(hipEventCreate(e), "hipEventCreate");
         const int cu = items[0].model->cu_count;
         b->max_vars = max_vars;
-        b->stride = (max_vars + 1) | 1;  // the variables and a constant 0
         b->bufs.resize(n_items);
         uint64_t maxr = 0;
         for (int i = 0; i < n_items; ++i) {
@@ -822,10 +832,10 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
         hip_check(hipMalloc(&b->d_round, sizeof(uint64_t)), "hipMalloc round");
         hip_check(hipMemset(b->d_round, 0, sizeof(uint64_t)), "clear round");
 
-        // the launch's slots per lane: the smallest that holds the widest
-        // instance in 64 lanes, or (tune) the fastest of that and wider
-        // packings under both register policies on a sample of every
-        // instance's runs
+        // the launch's slots per lane: left to choose (below), or (tune) the
+        // fastest of the smallest that holds the widest instance in 64 lanes
+        // and wider packings under both register policies on a sample of
+        // every instance's runs
         int Cmin = 1;
         while (64 * Cmin < maxP) Cmin <<= 1;
         if (Cmin > 16) throw std::runtime_error("limit: more than 1024 components per network");
@@ -837,7 +847,6 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
             b->lp = LaunchParams{};
             b->lp.inst = b->d_all;
             b->lp.n_inst = n_items;
-            b->lp.var_stride = b->stride;
             b->lp.total_chunks = sh.chunks;
             b->lp.segments = 64;
             b->lp.counter = b->d_counter;
@@ -848,7 +857,14 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
             hip_check(hipMemcpy(b->d_all, sh.inst.data(), n_items * sizeof(InstDesc), hipMemcpyHostToDevice),
                       "upload instances");
         };
+        // (a batch that does not fit at eight slots is refused)
         int bestC = std::max(Cmin, 8), best_occ = 0;
+        batch_shape(b.get(), bestC, 0);
+        // eight slots per lane where that leaves every SIMD two waves' runs,
+        // else the fewest that hold the widest instance, for shorter steps: 34
+        // instances of 1000 runs take 3.7 ms at 8 slots, 4.0 at 4, 4.9 at 2
+        // and 4.7 at 16, 16 of 600 runs 2.7 ms at 8 and 1.8 at 4
+        if (!tune && batch_fits(*b, Cmin) && batch_chunks(*b, bestC) < 8ull * (uint64_t)cu) bestC = Cmin;
         if (tune) {
             double best_ms = 1e300;
             uint64_t sample = 0;

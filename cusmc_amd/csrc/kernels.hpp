@@ -39,7 +39,6 @@ struct InstDesc {
 struct LaunchParams {
     const InstDesc *inst;       // sorted by chunk_first
     int32_t n_inst;
-    int32_t var_stride;         // doubles of LDS per segment (> every n_vars)
     uint64_t total_chunks;
     unsigned long long *counter;  // chunks handed out (cleared by launch_prep)
     int32_t segments;           // segments of a wave that take runs, at most

@@ -132,7 +132,7 @@ __device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTAN
 // 2e5 runs: 355, 117, 97, 81.8, 76.7 and 74.6 ms.
 //
 // LDS: [tables: lp.table_bytes, TAB only] then per wave [variables of the
-// wave's 64/S runs and a constant 0: var_stride doubles each][state words: 4
+// wave's 64/S runs and a constant 0, an odd number of doubles each][state words: 4
 // bytes per slot and lane][TRACE: locations, the same]; lp.wave_lds covers
 // the largest of these over the launch's instances.
 //
@@ -205,8 +205,9 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     const int seg_base = lane - sl;
     const uint64_t seg_ones = (S0 == 64) ? ~0ull : ((1ull << S0) - 1ull);
     const uint64_t seg_mask = seg_ones << seg_base;
-    double *vars = wbase + (size_t)(lane / S0) * lp.var_stride;
-    uint32_t *words_of = (uint32_t *)(wbase + (size_t)(64 / S0) * lp.var_stride);
+    const int stride = (inst->m.n_vars + 1) | 1;
+    double *vars = wbase + (lane / S0) * stride;
+    uint32_t *words_of = (uint32_t *)(wbase + (64 / S0) * stride);
     uint32_t *words = words_of + lane;
     int32_t *locs = (int32_t *)words_of + 64 * C + lane;  // TRACE only
     // since runs were started: turns of the loop, lanes without a run summed
