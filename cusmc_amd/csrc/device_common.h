@@ -1070,19 +1070,23 @@ __device__ __forceinline__ void race_frozen(RaceSlots<C> &rs, const uint32_t *wo
     }
 }
 
-// The exponential race over the segment: a fixed pairwise tree over the
-// leaves (in-lane levels, then a butterfly).  `level` keeps each level's own
-// partial sum from the sum to the descent (12 registers; in LDS, read back
-// and exchanged through it again, the two took 40 instructions and several
-// hundred cycles more on a full segment).  Returns the total.
+// The exponential race over the segment is a fixed pairwise tree over the
+// leaves.  Its levels within the lane:
 template <int C>
-__device__ __forceinline__ double race_total(const double (&leaf)[C], double (&level)[6], int S) {
+__device__ __forceinline__ double lane_total(const double (&leaf)[C]) {
     double tr[2 * C];
 #pragma unroll
     for (int j = 0; j < C; ++j) tr[C + j] = leaf[j];
 #pragma unroll
     for (int i = C - 1; i >= 1; --i) tr[i] = tr[2 * i] + tr[2 * i + 1];
-    double s = (C == 1) ? leaf[0] : tr[1];
+    return (C == 1) ? leaf[0] : tr[1];
+}
+
+// The levels above, a butterfly, from the lanes' sums s.  `level` keeps each
+// level's own partial sum from the sum to the descent (12 registers; in LDS,
+// read back and exchanged through it again, the two took 40 instructions and
+// several hundred cycles more on a full segment).  Returns the total.
+__device__ __forceinline__ double race_total(double s, double (&level)[6], int S) {
     // one way out of the levels, taken once
 #pragma unroll
     for (int k = 0; k < 6; ++k) {

@@ -298,7 +298,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
             }
             // tilted race: the run kernel's tree over the tilted rates
             double lvl[6] = {};
-            const double Rt = race_total<C>(leaft, lvl, S);
+            const double Rt = race_total(lane_total<C>(leaft), lvl, S);
             const double R = theta ? tree_total<C>(rs.leaf, S) : Rt;
             double dexp = INF;
             int wexp = 0x7FFFFFFF;
@@ -525,7 +525,11 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     }
 }
 
-// Registers unrestricted: 190-250 VGPRs, two waves per SIMD.
+// What bounds it: the latency of a row's loads and of its step, and of the
+// slowest row of a launch (a row may race several times before an edge
+// fires).  Registers unrestricted: 171-243 VGPRs, two waves per SIMD.  Held to
+// 168 it spills 43-71 of them at eight slots a lane: SIR-100, 5e4 rows, 24.1
+// ms for 22.2.
 template <int C, bool TAB, bool REC>
 __global__ __launch_bounds__(256) void is_advance_kernel(IsParams P) {
     is_advance_body<C, TAB, REC>(P);

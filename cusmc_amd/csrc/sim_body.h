@@ -113,10 +113,11 @@ __device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTAN
 // its segments; all its segments work on one instance, which (its tables,
 // query and outputs) is thereby uniform across the wave and lives in scalar
 // registers.  A chunk of another instance waits until this one's runs are
-// done.  A workgroup holds blockDim/64 independent waves.  With TAB (single-instance launches) the
-// workgroup first copies the model's tables into LDS and every wave reads
-// them there: the race and the transitions are chains of dependent table
-// reads, and LDS answers them several times sooner than the caches.
+// done.  A workgroup holds blockDim/64 independent waves.  With TAB
+// (single-instance launches) the workgroup first copies the model's tables
+// into LDS and every wave reads them there: the race and the transitions are
+// chains of dependent table reads, and LDS answers them several times sooner
+// than the caches.
 //
 // What bounds it: VALU issue while the chip is full, the latency of the
 // step's chain of dependent reads when it is not.  Both ask for few
@@ -128,13 +129,17 @@ __device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTAN
 // and rolled cold paths, 44.2 ms with the slot loop free of branches and its
 // invariants out of spilled registers, 40.7 ms with the step's rare parts
 // behind branches the whole wave takes or leaves, 36.3 ms with the race's sums
-// and windows kept out of LDS, 30.3 ms with runs handed out as below; SIR-350,
-// 2e5 runs: 355, 117, 97, 81.8, 76.7 and 74.6 ms.
+// and windows kept out of LDS, 30.3 ms with runs handed out as below, 29.5 ms
+// with the windows of a pair read side by side; SIR-350, 2e5 runs: 355, 117,
+// 97, 81.8, 76.7 and 74.6 ms, 66.4 ms with the receivers' picks reduced to a
+// comparison.  Now a SIMD's three waves of SIR-350 issue a VALU instruction in
+// 88 % of its cycles; Fischer-32 at 32 runs a wave, two waves per SIMD, issues
+// instructions of all kinds in 52 % of each wave's.
 //
 // LDS: [tables: lp.table_bytes, TAB only] then per wave [variables of the
-// wave's 64/S runs and a constant 0, an odd number of doubles each][state words: 4
-// bytes per slot and lane][TRACE: locations, the same]; lp.wave_lds covers
-// the largest of these over the launch's instances.
+// wave's 64/S runs and a constant 0, an odd number of doubles each][state
+// words: 4 bytes per slot and lane][TRACE: locations, the same]; lp.wave_lds
+// covers the largest of these over the launch's instances.
 //
 // When a segment's run ends, it waits: for the last of the wave's runs, or
 // until the waiting lanes have cost the wave 1/16 of its time.  Runs of equal
@@ -376,6 +381,9 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
             // first on ties).  The lanes of a run make them side by side: a
             // lane without delays left to draw makes the race's, and its
             // words are handed to the others afterwards.
+            // A run without exponential racers needs none for the race.
+            const double own = lane_total<C>(rs.leaf);
+            const uint64_t racers = __ballot(own > 0.0) & seg_mask;
             smc_u32x4 race{};
             uint64_t got = 0;  // lanes of the run that made the race's draw
             {
@@ -408,16 +416,22 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                     race.v[2] = delay ? race.v[2] : rw.v[2];
                     race.v[3] = delay ? race.v[3] : rw.v[3];
                     got |= __ballot(!delay) & seg_mask;
-                } while (any_lane(b != 0 || got == 0));
-                const int from = lowest_lane(got);
+                } while (any_lane(b != 0 || (got == 0 && racers != 0)));
+                const int from = got ? lowest_lane(got) : lane;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) race.v[k] = (uint32_t)__shfl((int)race.v[k], from);
             }
-            double level[6] = {};
-            const double R = race_total<C>(rs.leaf, level, S);
-            const double e = -device_log2(smc_u01(race.v[0], race.v[1])) / R;
-            w = race_pick<C>(rs.leaf, level, smc_u01(race.v[2], race.v[3]) * R, S, seg_base, seg_mask);
-            const double dexp = R > 0.0 ? e : INF;
+            // the exponential race, if any run has racers (slotted Aloha,
+            // every delay under a clock bound, one run a wave: 61.8 ms with
+            // it in every step, 42.7 ms without)
+            double dexp = INF;
+            if (any_lane(racers != 0)) {
+                double level[6] = {};
+                const double R = race_total(own, level, S);
+                const double e = -device_log2(smc_u01(race.v[0], race.v[1])) / R;
+                w = race_pick<C>(rs.leaf, level, smc_u01(race.v[2], race.v[3]) * R, S, seg_base, seg_mask);
+                dexp = R > 0.0 ? e : INF;
+            }
             d = dexp;
             if (any_lane(unif_j >= 0)) {
                 double gu = umin;
@@ -494,10 +508,13 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
   }
 }
 
-// Two register policies of the run kernel: unrestricted (two waves per SIMD
-// for every slot count: 150-256 VGPRs), and at most 168 (three waves per
-// SIMD; up to four slots per lane fit, more spill).  Which is faster depends
-// on the packing; the autotuner measures both.
+// Two register policies of the run kernel: unrestricted (100-119 VGPRs and
+// four waves per SIMD up to two slots per lane, 119-132 and three or four at
+// four, 145-158 and three at eight, 195-207 and two at sixteen), and at most
+// 168 (three waves per SIMD), which only sixteen slots spill to keep (some
+// thirty registers).  At sixteen it depends on the packing: SIR-350, 2e4 runs,
+// 8.1 ms with three waves and 10.5 with two, Fischer-32, 2e5 runs, whose LDS
+// holds two, 6.8 and 6.7; the autotuner measures both.
 template <int C, bool TRACE, bool TAB>
 __global__ __launch_bounds__(64 * SMC_MAX_GROUP_WAVES) void sim_kernel(LaunchParams lp) {
     sim_body<C, TRACE, TAB>(lp);
