@@ -426,8 +426,9 @@ struct smc_is {
             P.lanes = sh.S;
             P.wave_lds = (uint32_t)wave_lds(sh, P, b.record);
             // staged tables: workgroups of four waves, as many as the LDS
-            // holds, at most four a CU (four waves per SIMD); the recording
-            // build reads the tables from global memory
+            // holds, at most four a CU (the registers hold two at a time; the
+            // others even out the end); the recording build reads the tables
+            // from global memory
             size_t lds = m->table_bytes + shared_lds(P) + 4 * (size_t)P.wave_lds;
             const bool tab = stage && !b.record && m->table_bytes > 0 && lds <= kLdsPerCu;
             P.tables = tab ? (decltype(P.tables))m->arena : nullptr;
@@ -473,23 +474,28 @@ struct smc_is {
 
     size_t rec_pairs = 0;  // recorded pairs (padded to 64 with zero pairs)
 
-    void ensure_records() {
-        if (rec_cap) return;
-        // pairs of (features, wins, ln2 dt r) within 8 GiB
+    // Room for `need` pairs of (features, wins, ln2 dt r), at most 8 GiB of
+    // them.  (Memory that is freed is cleared by the driver before it is given
+    // out again, 8 GiB in some 200 ms: more than the study takes.)
+    void ensure_records(size_t need) {
         const size_t per_pair = (size_t)fpad * 2 + (size_t)Lpad * 8 + (size_t)Gpad * 8 + 4;
-        rec_cap = std::min<size_t>(((size_t)8 << 30) / per_pair, (size_t)1 << 23) / 64 * 64;
-        rX.ensure(rec_cap * fpad, "hipMalloc records");
-        rA.ensure(rec_cap * Lpad, "hipMalloc records");
-        rB.ensure(rec_cap * Lpad, "hipMalloc records");
-        rw.ensure(rec_cap, "hipMalloc records");
-        rAg.ensure(rec_cap * Gpad, "hipMalloc records");
-        rBg.ensure(rec_cap * Gpad, "hipMalloc records");
+        const size_t most = std::min<size_t>(((size_t)8 << 30) / per_pair, (size_t)1 << 23) / 64 * 64;
+        const size_t want = need < most ? rup(std::max<size_t>(need, 64), 64) : most;
+        if (want <= rec_cap) return;
+        rec_cap = rec_pairs = 0;
+        rX.ensure(want * fpad, "hipMalloc records");
+        rA.ensure(want * Lpad, "hipMalloc records");
+        rB.ensure(want * Lpad, "hipMalloc records");
+        rw.ensure(want, "hipMalloc records");
+        rAg.ensure(want * Gpad, "hipMalloc records");
+        rBg.ensure(want * Gpad, "hipMalloc records");
+        rec_cap = want;
     }
 
     // Replay runs (device array runs_in, weights in `weight`) under the
     // batch's proposal and record their macro-steps; returns the pair count.
-    size_t record(Batch b) {
-        ensure_records();
+    size_t record(Batch b, size_t need = SIZE_MAX) {
+        ensure_records(need);
         b.record = true;
         b.d_runs = runs_in.p;
         run_rows(b);
@@ -578,14 +584,15 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
 
         // launch shapes of the advance kernel
         // lanes per run: the model's tuned packing (smc_autotune) when there
-        // is one, else the widest, and narrower ones for many rows
+        // is one of at most eight slots per lane, else the widest, and
+        // narrower ones for many rows
         const int P = img.n_leaves;
         if (P > 512) throw std::runtime_error("limit: importance sampling takes networks of at most 512 components");
         int lanes = P < 64 ? P : 64, fewest = lanes;
         if (m->has_tuned && m->tuned.lanes_per_run > 0 && m->tuned.lanes_per_run <= lanes &&
             P / m->tuned.lanes_per_run <= 8) {
             fewest = lanes = m->tuned.lanes_per_run;
-        } else if (!m->has_tuned && !(img.tests & (SMC_HF_XINV | SMC_HF_XBLK))) {
+        } else if (!(img.tests & (SMC_HF_XINV | SMC_HF_XBLK))) {
             while (fewest > 1 && P / (fewest / 2) <= 8) fewest /= 2;
         }
         // SMC_IS_LANES=<power of two> overrides the lanes per run (diagnosis:
@@ -942,7 +949,6 @@ int smc_is_train(smc_is *s, smc_is_round *rounds) {
         const smc_is_config &c = s->cfg;
         const int N = (int)c.runs_per_round;
         const bool reach = s->q.kind == SMC_QUERY_REACH;
-        s->ensure_records();
 
         std::vector<uint8_t> stat;
         std::vector<double> lr, qm;
@@ -961,6 +967,7 @@ int smc_is_train(smc_is *s, smc_is_round *rounds) {
             std::vector<double> score;
             std::vector<uint8_t> hit;
             std::vector<double> l2;
+            std::vector<uint32_t> taken;
             double sw = 0, sw2 = 0;
             uint64_t hits = 0, steps = 0, trans = 0;
             for (int done = 0; done < N;) {
@@ -980,6 +987,7 @@ int smc_is_train(smc_is *s, smc_is_round *rounds) {
                     run_of.push_back(b.run_begin + (uint64_t)i);
                     hit.push_back(h);
                     l2.push_back(lr[i]);
+                    taken.push_back(stp[i]);
                     // larger is closer to the event
                     score.push_back(reach ? (h ? 1.0 : 0.0) : (s->q.is_max ? qm[i] : -qm[i]));
                 }
@@ -1038,7 +1046,10 @@ int smc_is_train(smc_is *s, smc_is_round *rounds) {
                 rb.tilt = s->zero_output ? Tilt::NONE : Tilt::MLP;
                 rb.seed = c.seed;
                 rb.n_valid = ne;
-                info.pairs = s->record(rb);
+                // (a launch that finds a row live races it or ends it)
+                size_t need = 0;
+                for (int i : elite) need += (size_t)taken[i] + 2;
+                info.pairs = s->record(rb, need);
                 // 5. epochs over the recorded pairs
                 for (int e = 0; e < c.epochs && s->rec_pairs > 0; ++e) {
                     s->ce_gradient();
@@ -1096,7 +1107,7 @@ int smc_is_ce_gradient(smc_is *s, float *grad_out) {
     if (!s || !grad_out) return fail(SMC_E_INVALID, "null argument");
     return guarded([&]() -> int {
         hip_check(hipSetDevice(s->m->device), "hipSetDevice");
-        s->ensure_records();
+        s->ensure_records(64);
         s->ce_gradient();
         hip_check(hipMemcpyAsync(grad_out, s->g.p, s->n_params * 4, hipMemcpyDeviceToHost, s->stream()), "copy gradient");
         hip_check(hipStreamSynchronize(s->stream()), "gradient");
