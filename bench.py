@@ -52,9 +52,9 @@ SEED = 20261202
 # what they read for a 1 GiB device copy).  valu: SQ_INSTS_VALU (wave64 VALU
 # instructions) per race step.
 PROFILED = {
-    "fischer32": {"shape": (4, 3, 1), "traffic_per_run": 23.1, "valu_per_step": 113.9,
+    "fischer32": {"shape": (2, 0, 1), "traffic_per_run": 40.1, "valu_per_step": 48.5,
                   "source": "profiles/sim_kernel_fischer32.md"},
-    "sir350": {"shape": (64, 3, 2), "traffic_per_run": 25.9, "valu_per_step": 1543.6,
+    "sir350": {"shape": (32, 3, 1), "traffic_per_run": 90.7, "valu_per_step": 449.7,
                "source": "profiles/sim_kernel_sir350.md"},
 }
 
@@ -359,7 +359,7 @@ def main() -> int:
                     help="with --lanes: register policy (0 unrestricted, 3 three waves per SIMD)")
     ap.add_argument("--tables", type=int, default=0, choices=[0, 1, 2],
                     help="with --lanes: model tables in global memory (0), staged in LDS (1), or staged "
-                         "but for the location records (2)")
+                         "if they fit (2)")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-is", action="store_true", help="fischer32: skip the learned-IS leg")
     args = ap.parse_args()

@@ -69,21 +69,25 @@ typedef struct smc_model smc_model;
 int smc_model_create(const smc_network *net, int device, smc_model **out);
 void smc_model_destroy(smc_model *m);
 
-/* Launch shape.  Zero fields mean "choose": lanes_per_run = next power of two
- * of the component count capped at 64; waves = enough to fill the GPU. */
+/* Launch shape.  All fields zero mean "choose": the tuned launch if there is
+ * one (smc_autotune), else by the number of runs: the fewest lanes per run
+ * that give every SIMD two waves, tables in LDS where they fit.  With some
+ * field named, zero lanes_per_run means the next power of two of the component
+ * count capped at 64, zero waves enough to fill the GPU.  Results do not depend
+ * on the shape. */
 typedef struct smc_launch {
     int32_t lanes_per_run;     /* S: power of two <= 64                    */
     int32_t waves;             /* persistent waves in the grid              */
     int32_t waves_per_cu;      /* occupancy target used when waves == 0     */
     int32_t occupancy;         /* 0: registers unrestricted (two waves per
-                                  SIMD); 3: at most 168 registers, three
-                                  waves per SIMD                           */
+                                  SIMD at sixteen slots per lane, three at
+                                  eight, four below); 3: at most 168
+                                  registers, three waves per SIMD          */
     int32_t tables;            /* 0: model tables read from global memory;
-                                  1: staged in LDS, one copy per workgroup
-                                  of four waves; 2: staged in LDS but for the
-                                  location records, read from global memory
-                                  (smc_run only; batches read the tables
-                                  from global memory)                      */
+                                  1: staged in LDS, one copy per workgroup;
+                                  2: staged if they fit, else read from
+                                  global memory (smc_run only; batches read
+                                  the tables from global memory)           */
 } smc_launch;
 
 /* Per-run outputs, all optional (NULL = not wanted), each n_runs long. */
