@@ -696,7 +696,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                 }
             }
             h.what = (uint32_t)hot_at | (hf << 16);
-            h.base = hot_local ? 0x1FFFu : 0u;
+            h.base = (hot_local ? 0x1FFFu : 0u) | (hf & SMC_HF_EXPR ? SMC_HB_EXPR : 0u);
             for (RawEdge &re : R.edges) inline_edge(re);
             img.tests |= hf;
         }

@@ -853,8 +853,10 @@ __device__ __forceinline__ void slot_windows(double (&left)[2], const uint32_t *
 // branches would run every kind's code for every slot, and they would keep
 // the slots' reads, a chain of three each, from overlapping.  What only some
 // slots of a step need (the length of a bounded delay, rates that are
-// expressions) is left to later passes over those.  17 vector instructions a
-// slot; with delays, expressions and zero tests in line it was 40.
+// expressions) is left to later passes over those.  About 17 vector
+// instructions a slot with tests; with delays, expressions and zero tests in
+// line it was 40.  Without tests half of the record is enough: SIR-350, 2e5
+// runs, 65.3 ms for 66.4 with all of it.
 // TESTS: some location has an invariant or a guard; RATE: 0 all rates are
 // constant, 1 one expression of the value `shared`, 2 several (bits expr).
 //
@@ -884,7 +886,16 @@ __device__ __forceinline__ void classify(RaceSlots<C> &rs, const uint32_t *words
 #pragma unroll
         for (int j = 0; j < G; ++j) w[j] = words[64 * (j0 + j)];
 #pragma unroll
-        for (int j = 0; j < G; ++j) h[j] = load_rec(m.hots + word_rec(w[j], m));
+        for (int j = 0; j < G; ++j) {
+            if (TESTS) {
+                h[j] = load_rec(m.hots + word_rec(w[j], m));
+            } else {
+                const uint4 half = load_quad(m.hots + word_rec(w[j], m), 0);
+                h[j].rate = quad_f64(half);
+                h[j].what = half.z;
+                h[j].base = half.w;
+            }
+        }
         if (TESTS) {
 #pragma unroll
             for (int j = 0; j < G; ++j) v[j] = hot_value(h[j], w[j], x.vars);
@@ -894,7 +905,7 @@ __device__ __forceinline__ void classify(RaceSlots<C> &rs, const uint32_t *words
             const uint32_t bit = 1u << (j0 + j), d = h[j].what;
             double rate = h[j].rate;
             zero = shift_in_sign(zero, (uint32_t)__double2hiint(rate));
-            if (RATE == 1) rate = (d & (SMC_HF_EXPR << 16)) ? shared : rate;
+            if (RATE == 1) rate = (int32_t)h[j].base < 0 ? shared : rate;
             bool in = true;
             if (TESTS) {
                 // an invariant x <= a holds the delay to a - x - b while that

@@ -99,6 +99,8 @@ enum {
     SMC_HF_INV = 0x8000     // one invariant with a constant bound: a = bound, b = 1e-6 if strict
 };
 
+#define SMC_HB_EXPR 0x80000000u  // DevHot.base: the rate is an expression
+
 struct DevInsn {
     uint8_t op;
     uint8_t dst;
@@ -112,11 +114,14 @@ struct DevInsn {
 // positive).  A location with neither
 // invariant nor guard tests a constant 0 (kept behind the run's variables)
 // against [-inf, inf], so that all take the same steps.
+// The first half is all that a model without invariants and blocking tests
+// reads.
 struct DevHot {
     double rate;
-    double a, b;
     uint32_t what;          // low half: the variable's byte offset; high half: SMC_HF_*
-    uint32_t base;          // mask of the state word's base: all ones if the variable is private, else 0
+    uint32_t base;          // mask of the state word's base: all ones if the variable is private, else 0;
+                            // SMC_HB_EXPR, a bit that no state word has
+    double a, b;
 };
 
 // The rest, 64 bytes: receive edges; spontaneous edges; invariants, blocking

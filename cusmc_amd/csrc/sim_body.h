@@ -132,9 +132,10 @@ __device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTAN
 // and windows kept out of LDS, 30.3 ms with runs handed out as below, 29.5 ms
 // with the windows of a pair read side by side; SIR-350, 2e5 runs: 355, 117,
 // 97, 81.8, 76.7 and 74.6 ms, 66.4 ms with the receivers' picks reduced to a
-// comparison.  Now a SIMD's three waves of SIR-350 issue a VALU instruction in
-// 88 % of its cycles; Fischer-32 at 32 runs a wave, two waves per SIMD, issues
-// instructions of all kinds in 52 % of each wave's.
+// comparison, 65.3 ms with half records where nothing is tested.  Now the
+// three waves of a SIMD issue a VALU instruction in 88 % of its cycles with
+// SIR-350; a wave of Fischer-32, 32 runs and two waves per SIMD, issues
+// instructions of all kinds in 52 % of its own.
 //
 // LDS: [tables: lp.table_bytes, TAB only] then per wave [variables of the
 // wave's 64/S runs and a constant 0, an odd number of doubles each][state
