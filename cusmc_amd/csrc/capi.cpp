@@ -382,8 +382,6 @@ int smc_model_create(const smc_network *net, int device, smc_model **out) {
         hip_check(hipMalloc(&m->d_inst, sizeof(InstDesc)), "hipMalloc instance");
         hip_check(hipMalloc(&m->d_counter, sizeof(unsigned long long)), "hipMalloc counter");
         hip_check(hipMalloc(&m->d_partials, 1024 * sizeof(ReducePartial)), "hipMalloc partials");
-        // the totals are written straight to host memory
-        hip_check(hipHostMalloc((void **)&m->totals, sizeof(ReducePartial), hipHostMallocDefault), "hipHostMalloc totals");
         *out = m.release();
         return SMC_OK;
     });
@@ -409,6 +407,9 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         hip_check(hipSetDevice(m->device), "hipSetDevice");
         Plan pl = plan_launch(m, use, n_runs, trace);
         m->runs.ensure(n_runs);
+        // the totals are written straight to host memory
+        if (!m->totals)
+            hip_check(hipHostMalloc((void **)&m->totals, sizeof(ReducePartial), hipHostMallocDefault), "hipHostMalloc totals");
         const int waves = pl.waves;
 
         m->h_inst.m = m->dm;

@@ -89,7 +89,7 @@ struct smc_model {
     InstDesc *d_inst = nullptr;
     unsigned long long *d_counter = nullptr;
     ReducePartial *d_partials = nullptr;
-    ReducePartial *totals = nullptr;  // pinned
+    ReducePartial *totals = nullptr;  // pinned, from the first call on
     static constexpr size_t kStageBytes = 1 << 20;
     uint8_t *stage = nullptr;         // pinned, kStageBytes, from the first call with per-run outputs on
     ReducePartial h_acc{};
