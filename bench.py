@@ -54,7 +54,7 @@ SEED = 20261202
 PROFILED = {
     "fischer32": {"shape": (2, 0, 1), "traffic_per_run": 40.1, "valu_per_step": 48.5,
                   "source": "profiles/sim_kernel_fischer32.md"},
-    "sir350": {"shape": (32, 3, 1), "traffic_per_run": 90.7, "valu_per_step": 449.7,
+    "sir350": {"shape": (32, 3, 1), "traffic_per_run": 54.7, "valu_per_step": 439.7,
                "source": "profiles/sim_kernel_sir350.md"},
 }
 
