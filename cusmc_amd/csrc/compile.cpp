@@ -442,6 +442,16 @@ ModelImage lower(const smc_network &n, bool use_locals) {
         return vu.set == 0 || (vu.add == 0 && vu.one_value);
     };
 
+    // Clocks whose values are constants far inside the doubles, plus time: a
+    // window under such a bound is finite.
+    auto moderate = [](double v) { return std::fabs(v) <= 1e300; };
+    std::vector<uint8_t> clock_moderate(n.n_vars);
+    for (int v = 0; v < n.n_vars; ++v) clock_moderate[v] = moderate(n.var_init[v]);
+    for (int u = 0; u < n.n_updates; ++u) {
+        double c;
+        if (!literal(n.updates[u].expr, &c) || !moderate(c)) clock_moderate[n.updates[u].var] = 0;
+    }
+
     // Null racers leave an all-exponential race only while every rate is
     // constant between transitions (a rate reading a clock changes at each
     // null step of the reference's race).
@@ -463,6 +473,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
             LocInfo &info = img.info[l];
             d.type = (uint8_t)L.type;
             d.rate = lw.ref(L.rate, 1.0);
+            int inv_clock = -1;
             for (int k = 0; k < L.inv_count; ++k) {
                 const smc_constraint &C = n.constraints[L.inv_first + k];
                 if (!C.uses_variable) continue;
@@ -470,6 +481,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                 if (C.op != SMC_C_LE && C.op != SMC_C_LT) continue;
                 DevInv iv{};
                 iv.var = lw.field(C.var);
+                inv_clock = C.var;
                 iv.strict = C.op == SMC_C_LT;
                 iv.bound = lw.ref(C.rhs, 0.0);
                 if (SMC_REF_KIND(iv.bound) == SMC_REF_CONST) {
@@ -681,6 +693,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                     inline_var(R.invs[0].var, &hot_at, &hot_local);
                     h.a = R.invs[0].bound_value;
                     h.b = R.invs[0].strict ? 1e-6 : 0.0;
+                    if (!moderate(h.a) || !clock_moderate[inv_clock]) hf |= SMC_HF_OPEN;
                 } else if (d.n_inv) {
                     hf |= SMC_HF_XINV;
                 }
