@@ -229,7 +229,9 @@ void range_of(int op, double r, double *lo, double *hi) {
     if (std::fabs(r) == INF) return;
     auto end = [&](double outside) {
         int64_t in = order_of(r), out = order_of(outside);  // the test holds at `in`, fails at `out`
-        while (in - out > 1 || out - in > 1) {
+        // (the two may lie further apart than a signed difference holds)
+        const auto apart = [&] { return in > out ? (uint64_t)in - (uint64_t)out : (uint64_t)out - (uint64_t)in; };
+        while (apart() > 1) {
             const int64_t mid = in / 2 + out / 2 + (in % 2 + out % 2) / 2;
             if (std::fabs(double_of(mid) - r) <= SMC_TOL) in = mid;
             else out = mid;
