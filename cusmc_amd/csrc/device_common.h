@@ -275,12 +275,11 @@ __device__ __forceinline__ DevRange load_range(const SMC_LDS DevEdge *p) {
     return load_rec((const SMC_LDS DevRange *)p + 1);
 }
 #endif
-// Record i of a table.  24-bit products: a full-rate instruction, where the
-// 32-bit multiply of an index is a quarter-rate one.
+// Record i of a table.  In LDS, which holds fewer than 2^24 records, a 24-bit
+// product: a full-rate instruction, where the 32-bit multiply of an index is a
+// quarter-rate one.  A table in global memory may be longer.
 template <class T>
-__device__ __forceinline__ const SMC_GLOBAL T *rec_at(const SMC_GLOBAL T *p, uint32_t i) {
-    return (const SMC_GLOBAL T *)((const SMC_GLOBAL char *)p + __umul24(i, (uint32_t)sizeof(T)));
-}
+__device__ __forceinline__ const SMC_GLOBAL T *rec_at(const SMC_GLOBAL T *p, uint32_t i) { return p + i; }
 #if defined(__HIP_DEVICE_COMPILE__)
 template <class T>
 __device__ __forceinline__ const SMC_LDS T *rec_at(const SMC_LDS T *p, uint32_t i) {
