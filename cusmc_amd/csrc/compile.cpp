@@ -307,9 +307,11 @@ void inline_edge(RawEdge &re) {
 
 // Partition of the locations into classes of equal records: first by their
 // own content, then, until nothing splits, by the classes their edges lead
-// to.  Networks whose classes take long to separate (chains of equal
-// locations) keep one class per location.
-std::vector<uint32_t> classes_of(const std::vector<RawLoc> &raw, uint32_t *count) {
+// to.  The model fixtures are stable after one to three passes; a chain of equal
+// locations separates by one link a pass.  Where 64 passes do not do, the
+// locations at the same place of equal components are a class: instances of a
+// template still share their records.
+std::vector<uint32_t> classes_of(const smc_network &net, const std::vector<RawLoc> &raw, uint32_t *count) {
     const size_t n = raw.size();
     std::vector<uint32_t> cls(n), next(n);
     auto put = [](std::string &k, const auto &v) {
@@ -331,6 +333,7 @@ std::vector<uint32_t> classes_of(const std::vector<RawLoc> &raw, uint32_t *count
         cls[l] = ids.emplace(std::move(k), (uint32_t)ids.size()).first->second;
     }
     *count = (uint32_t)ids.size();
+    const std::vector<uint32_t> own = cls;  // by their own content, destinations relative to the location
     for (int pass = 0; pass < 64; ++pass) {
         ids.clear();
         for (size_t l = 0; l < n; ++l) {
@@ -342,8 +345,15 @@ std::vector<uint32_t> classes_of(const std::vector<RawLoc> &raw, uint32_t *count
         if (ids.size() == *count) return cls;
         *count = (uint32_t)ids.size();
     }
-    for (size_t l = 0; l < n; ++l) cls[l] = (uint32_t)l;
-    *count = (uint32_t)n;
+    ids.clear();
+    *count = 0;
+    for (int c = 0; c < net.n_components; ++c) {
+        const int l0 = net.comp_first_loc[c], locs = net.comp_first_loc[c + 1] - l0;
+        std::string k((const char *)&own[l0], (size_t)locs * 4);
+        const auto at = ids.emplace(std::move(k), *count);  // the component's first class
+        if (at.second) *count += (uint32_t)locs;
+        for (int l = 0; l < locs; ++l) cls[l0 + l] = at.first->second + (uint32_t)l;
+    }
     return cls;
 }
 
@@ -722,7 +732,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
     // classes of equal locations, and their records; record 0 is a slot
     // without a component (no edge, rate 0)
     uint32_t n_cls = 0;
-    const std::vector<uint32_t> cls = classes_of(raw, &n_cls);
+    const std::vector<uint32_t> cls = classes_of(n, raw, &n_cls);
     // a state word holds the class and the base; with more classes than fit
     // beside a base, the class alone
     if (use_locals && n_cls >= (1u << 18)) return lower(n, false);

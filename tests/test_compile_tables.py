@@ -72,3 +72,31 @@ def test_models_lower_without_undefined_behaviour(check):
     texts += [G.race_network(8)[0], G.fischer_network(32)[0], G.sir_network(77, 0.3, 0.1)[0]]
     for lines in check(*texts):
         assert int(lines[0][2]) > 0
+
+
+def _chains(components, length, last=""):
+    """Instances of a template whose locations are a chain of equal ones; `last`:
+    a guard on the final edge of the first component alone."""
+    tpls, names = [], []
+    for c in range(components):
+        loc = "".join(f'<location id="id{c * 1000 + k}"><name>l{c}_{k}</name></location>' for k in range(length))
+        tr = "".join(f"""<transition><source ref="id{c * 1000 + k}"/><target ref="id{c * 1000 + k + 1}"/>"""
+                     + (f'<label kind="guard">{last}</label>' if last and c == 0 and k == length - 2 else "")
+                     + "</transition>" for k in range(length - 1))
+        tpls.append(f"""<template><name>T{c}</name><declaration></declaration>{loc}<init ref="id{c * 1000}"/>{tr}
+</template>""")
+        names.append(f"T{c}")
+    return f"""<?xml version="1.0" encoding="utf-8"?>
+<nta><declaration>int v = 0;</declaration>{"".join(tpls)}<system>system {", ".join(names)};</system></nta>"""
+
+
+@pytest.mark.parametrize("length", [63, 64, 65, 66, 67, 100, 300])
+def test_chains_of_equal_locations_share_records(check, length):
+    """Equal locations of a chain differ by how far they are from its end, which
+    takes a pass a link to find out; instances share their records whatever the
+    length (record 0 stands for no component)."""
+    one, eight, odd = check(_chains(1, length), _chains(8, length), _chains(8, length, last="v == 0"))
+    assert int(one[0][4]) == length + 1
+    assert int(eight[0][2]) == 8 * length and int(eight[0][4]) == length + 1
+    # one instance leads to another guard: its records are its own, but for those past the guard
+    assert length + 2 < int(odd[0][4]) <= 2 * length + 1

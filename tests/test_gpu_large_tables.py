@@ -98,3 +98,60 @@ def test_guard_records_past_24_bits():
                        updates=np.array([(0, 1), (0, 2)], UPDATE), exprs=exprs)
     ro = _runs_equal(net, cs.var_query(0, 50.0, estimate=True, max_steps=40), 24, [1])
     assert set(ro["value"]) == {2.0} and set(ro["transitions"]) == {1}
+
+
+def test_more_record_classes_than_a_state_word_holds_beside_a_base():
+    """Two components of 131,100 locations, all different: variables keep their
+    own indices and a state word holds the class alone."""
+    n_comp, L, rates = 2, 131100, 256
+    n = n_comp * L
+    l = np.arange(n) % L
+    c = np.arange(n) // L
+    # expressions: 0 the first update, 1 the second, then rates, then guard bounds
+    head = [(ADD, 2, 3, -1, 0.0), (ADD, 2, 4, -1, 0.0), (VAR, -1, -1, 0, 0.0), (LIT, -1, -1, 0, 1.0),
+            (LIT, -1, -1, 0, -1.0)]
+    bounds = -(-L // rates)
+    ex = np.zeros(rates + n_comp * bounds, EXPR)
+    ex["op"] = LIT
+    ex["value"][:rates] = 0.5 + np.arange(rates) / 64.0
+    ex["value"][rates:] = np.arange(n_comp * bounds) - 3.0
+    locations = np.zeros(n, LOCATION)
+    locations["rate"] = len(head) + l % rates
+    locations["edge_first"], locations["edge_count"] = 2 * np.arange(n), 2
+    edges = np.zeros(2 * n, EDGE)
+    edges["src"] = np.repeat(np.arange(n), 2)
+    edges["weight"] = -1
+    edges["dst"][0::2] = c * L + (5 * l + 1) % L
+    edges["dst"][1::2] = c * L + (l + 12345) % L
+    edges["guard_first"][0::2], edges["guard_count"][0::2] = np.arange(n), 1   # v <= a bound of its own
+    edges["upd_first"], edges["upd_count"] = np.tile([0, 1], n), 1
+    g = np.zeros(n, CONSTRAINT)
+    g["op"], g["uses_variable"], g["var"], g["lhs"] = LE, 1, 0, -1
+    g["rhs"] = len(head) + rates + c * bounds + l // rates
+    net = ArrayNetwork(var_init=[0.0], first_loc=[0, L, n], init_loc=[0, L + 7], locations=locations, edges=edges,
+                       constraints=g, updates=np.array([(0, 0), (0, 1)], UPDATE), exprs=np.concatenate([_expr(head), ex]))
+    ro = _runs_equal(net, cs.var_query(0, 30.0, estimate=True), 200, [1, 2])
+    assert len(set(ro["value"])) > 3
+
+
+@pytest.mark.parametrize("n_comp,length", [(3, 65), (7, 100), (40, 90)])
+def test_chains_of_equal_locations(n_comp, length):
+    """Instances of a chain of equal locations, each adding to one variable, the
+    last link back to the first: classes by place."""
+    n = n_comp * length
+    k = np.arange(n) % length
+    c = np.arange(n) // length
+    ex = _expr([(ADD, 1, 2, -1, 0.0), (VAR, -1, -1, 0, 0.0), (LIT, -1, -1, 0, 1.0), (LIT, -1, -1, 0, 2.0)])
+    locations = np.zeros(n, LOCATION)
+    locations["rate"] = np.where(k == length - 1, 3, -1)
+    locations["edge_first"], locations["edge_count"] = np.arange(n), 1
+    edges = np.zeros(n, EDGE)
+    edges["src"], edges["dst"] = np.arange(n), c * length + (k + 1) % length
+    edges["weight"], edges["upd_first"], edges["upd_count"] = -1, 0, 1
+    net = ArrayNetwork(var_init=[0.0], first_loc=np.arange(n_comp + 1) * length, init_loc=np.arange(n_comp) * length,
+                       locations=locations, edges=edges, constraints=np.zeros(0, CONSTRAINT),
+                       updates=np.array([(0, 0)], UPDATE), exprs=ex)
+    P = 1 << (n_comp - 1).bit_length()
+    for tables in (0, 1):
+        ro = _runs_equal(net, cs.var_query(0, 120.0, estimate=True), 64, sorted({P, max(1, P // 8)}), tables=tables)
+    assert ro["value"].min() > n_comp * length / 2
