@@ -158,10 +158,11 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
         if (pl.tab) {
             // the smallest workgroups that hold what the runs ask for: few
             // runs then spread over the CUs evenly
-            int need = best;
-            if (want.waves > 0) need = (want.waves + m->cu_count - 1) / m->cu_count;
-            else if (want.waves_per_cu > 0) need = want.waves_per_cu;
-            need = (int)std::min<uint64_t>((uint64_t)std::min(need, best), (most_waves + m->cu_count - 1) / m->cu_count);
+            const int64_t cus = m->cu_count;
+            int64_t need = best;
+            if (want.waves > 0) need = std::min(need, (want.waves + cus - 1) / cus);
+            else if (want.waves_per_cu > 0) need = std::min<int64_t>(need, want.waves_per_cu);
+            need = std::min(need, (int64_t)((most_waves + (uint64_t)cus - 1) / (uint64_t)cus));
             pl.group_waves = 1;
             while (staged(pl.group_waves) < need) pl.group_waves *= 2;
             pl.table_bytes = m->table_bytes;
@@ -184,7 +185,7 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
     pl.chunk_runs = (uint32_t)std::min<uint64_t>(total_runs / (16ull * (uint64_t)waves * (uint64_t)pl.R) + 1, 256);
     waves = (int)std::min<uint64_t>((uint64_t)waves, most_waves);
     pl.lds = pl.table_bytes + (size_t)pl.group_waves * wave;
-    pl.waves = (waves + pl.group_waves - 1) / pl.group_waves * pl.group_waves;
+    pl.waves = (int)(((int64_t)waves + pl.group_waves - 1) / pl.group_waves * pl.group_waves);
     return pl;
 }
 
