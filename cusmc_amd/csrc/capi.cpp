@@ -14,6 +14,7 @@
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <unordered_set>
 #include <tuple>
 #include <vector>
 
@@ -65,6 +66,46 @@ size_t wave_lds_bytes(int R, int stride, int C, bool trace) {
 // time each and two doubles per lane and race-tree level, in 60,000 bytes.
 bool vars_fit(int R, int n_vars, int levels) {
     return (size_t)R * ((n_vars + 1) | 1) * 8 + (size_t)levels * 1024 <= 60000;
+}
+
+// What a launch that names table staging is held to where the tables do not
+// fit: with a record per location, 48 bytes each, and edges, guards and updates in
+// their shortest form, 32, 8 and 16 bytes, equal runs of them shared (also by
+// edges that only lead to different classes), they have to fit beside four
+// waves.  Such tables were always accepted, though they may take several times
+// as much; they are read from global memory then.
+size_t named_tables_bytes(const smc_model *m, bool locations) {
+    const smc::ModelImage &im = m->img;
+    std::unordered_set<std::string> seen;
+    const auto fresh = [&](char kind, const void *p, size_t n) {
+        return seen.insert(kind + std::string((const char *)p, n)).second;
+    };
+    size_t edges = 0, guards = 0, upds = 0;
+    for (const DevLoc &L : im.locs) {
+        std::vector<DevEdge> run(im.edges.begin() + L.edge_first, im.edges.begin() + L.edge_first + L.edge_n);
+        for (DevEdge &e : run) {
+            e.dst_rec = 0;
+            DevEdge g{}, u{};  // its guards, and its updates
+            g.lo = e.lo, g.hi = e.hi, g.g_var = e.g_var, g.g_flags = e.g_flags;
+            g.guard_first = e.guard_first, g.guard_n = e.guard_n, g.flags = e.flags & SMC_EF_NO_GUARD;
+            u.u0_value = e.u0_value, u.u0_var = e.u0_var, u.u0_flags = e.u0_flags;
+            u.u1_value = e.u1_value, u.u1_var = e.u1_var, u.u1_flags = e.u1_flags;
+            u.upd_first = e.upd_first, u.upd_n = e.upd_n;
+            if (fresh('g', &g, sizeof g)) guards += e.guard_n + ((e.flags & SMC_EF_NO_GUARD) ? 0 : 1);
+            if (fresh('u', &u, sizeof u)) upds += e.upd_n + (e.u0_flags >= SMC_EU_ADD) + (e.u1_flags >= SMC_EU_ADD);
+        }
+        if (fresh('e', run.data(), run.size() * sizeof(DevEdge))) edges += run.size();
+        if ((L.flags & SMC_LF_GUARDED) && fresh('b', &L.block_first, sizeof L.block_first)) {
+            size_t k = L.block_first;
+            while (!(im.guards[k].flags & SMC_GF_END_LOC)) ++k;
+            guards += k + 1 - L.block_first;
+        }
+    }
+    size_t total = 0;
+    for (size_t part : {locations ? im.loc_rec.size() * 48 : 0, im.invs.size() * 16, edges * 32, guards * 8, upds * 16,
+                        im.consts.size() * 8, im.code.size() * 8})
+        total += align_up(part, 256);
+    return total;
 }
 
 // Waves per CU that the registers of a run-kernel build allow (a property of
@@ -167,11 +208,12 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
             while (staged(pl.group_waves) < need) pl.group_waves *= 2;
             pl.table_bytes = m->table_bytes;
             per_cu = staged(pl.group_waves);
-        } else if (want.tables == 1 && !trace && (size_t)m->dm.n_locs * 48 + 4 * wave > kLdsPerCu) {
-            throw std::runtime_error("limit: the model tables do not fit in LDS");
         } else {
-            // tables that fit beside four waves at 48 bytes a location are
-            // accepted all the same, and read from global memory
+            // a launch that names them is refused, but for what never was:
+            // with digests, and tables that take little by the record
+            if (use && !trace && named_tables_bytes(m, want.tables == 1) +
+                                         4 * align_up((size_t)pl.R * pl.stride * 8 + (size_t)levels * 1024, 16) > kLdsPerCu)
+                throw std::runtime_error("limit: the model tables do not fit in LDS");
             per_cu = register_waves(pl.C, trace, pl.occ, false);
         }
     }
@@ -661,26 +703,25 @@ int smc_autotune(smc_model *m, const smc_query *q, uint64_t seed, uint64_t sampl
             if (P / S > 16) break;
             for (int occ : {0, 3})
                 for (int tab : {0, 1}) {
-                    cands.push_back(smc_launch{S, 0, 0, occ, tab});
+                    const smc_launch c{S, 0, 0, occ, tab};
                     try {
-                        const int per_cu = plan_launch(m, &cands.back(), sample_runs, false).per_cu;
-                        if (per_cu >= 2) cands.push_back(smc_launch{S, 0, per_cu / 2, occ, tab});
-                    } catch (const std::exception &) {
+                        const Plan pl = plan_launch(m, &c, sample_runs, false);
+                        if (pl.tab != (tab == 1)) continue;  // the same as without
+                        cands.push_back(c);
+                        if (pl.per_cu >= 2) cands.push_back(smc_launch{S, 0, pl.per_cu / 2, occ, tab});
+                    } catch (const std::exception &) {  // e.g. LDS budget exceeded at this packing
                     }
                 }
         }
+        if (cands.empty()) throw std::runtime_error("no launch shape could run this model");
         // each candidate runs at least twice the runs its grid holds at once,
         // so the sample measures the steady state rather than the tail
         double best_cost = 1e300;
         smc_launch pick = cands.front();
         for (const smc_launch &c : cands) {
             uint64_t n = sample_runs;
-            try {
-                Plan pl = plan_launch(m, &c, sample_runs, false);
-                n = std::max<uint64_t>(n, 2ull * (uint64_t)(pl.per_cu * m->cu_count) * (uint64_t)pl.R);
-            } catch (const std::exception &) {
-                continue;  // e.g. LDS budget exceeded at this packing
-            }
+            const Plan pl = plan_launch(m, &c, sample_runs, false);
+            n = std::max<uint64_t>(n, 2ull * (uint64_t)(pl.per_cu * m->cu_count) * (uint64_t)pl.R);
             smc_result r;
             int rc = smc_run(m, q, seed, 0, std::min<uint64_t>(n, 4096), &c, nullptr, &r);  // warm
             if (rc != SMC_OK) continue;

@@ -85,9 +85,14 @@ typedef struct smc_launch {
                                   registers, three waves per SIMD          */
     int32_t tables;            /* 0: model tables read from global memory;
                                   1: staged in LDS, one copy per workgroup;
-                                  2: staged if they fit, else read from
-                                  global memory (smc_run only; batches read
-                                  the tables from global memory)           */
+                                  refused where they do not fit, unless they
+                                  would beside four waves at 48 bytes a
+                                  location and 32, 8 and 16 an edge, guard
+                                  and update (equal ones shared): those, and
+                                  digest runs', are read from global memory;
+                                  2: the same without the locations in that
+                                  count (smc_run only; batches read the
+                                  tables from global memory)              */
 } smc_launch;
 
 /* Per-run outputs, all optional (NULL = not wanted), each n_runs long. */

@@ -6,7 +6,10 @@ import numpy as np
 import pytest
 
 import cusmc_amd as cs
+from cusmc_amd import _capi as A
 from cusmc_amd import generators as G
+
+from _models import E_ADD, RawNetwork
 
 pytestmark = pytest.mark.gpu
 
@@ -14,6 +17,7 @@ PER_RUN = ("flag", "value", "steps", "transitions", "time")
 
 
 def _same(a, b, what):
+    assert a.keys() == b.keys()
     for k in a:
         assert a[k].tobytes() == b[k].tobytes(), (what, k)
 
@@ -36,3 +40,56 @@ def test_any_number_of_waves(waves):
                 assert r.waves <= max(8, -(-n // (64 // lanes)) + 8)
     finally:
         sim.close()
+
+
+def _distinct(n_locs):
+    """One component of n_locs locations that share no record: a ring with a
+    rate of its own each, and constants of its own in every edge."""
+    net = RawNetwork()
+    v = net.var(0.0)
+    first = net.component([dict(type=0, rate=net.lit(1.0 + l / 4096.0)) for l in range(n_locs)])
+    for l in range(n_locs):
+        net.edge(first + l, first + (l + 1) % n_locs, upds=[(v, net.expr(E_ADD, net.ref(v), net.lit(float(1 + l))))])
+    return net.build()
+
+
+# locations, and whether tables = 1 and tables = 2 are accepted: staged; within
+# the counted bytes but not in LDS; the locations past them; the edges past them
+@pytest.mark.parametrize("n_locs,one,two", [(500, True, True), (1200, True, True), (1900, False, True),
+                                            (5000, False, False)])
+def test_named_tables_are_staged_or_refused(n_locs, one, two):
+    net = _distinct(n_locs)
+    q = cs.var_query(0, 20.0, estimate=True)
+    sim = cs.GpuSimulator(net)
+    try:
+        n = 500
+        with_digest = PER_RUN + ("digest",)
+        ref = sim.run(q, seed=2, n_runs=n, lanes_per_run=1, per_run=with_digest)
+        for tables, accepted in ((1, one), (2, two)):
+            print(f"[gpu requests] locations={n_locs} tables={tables}", flush=True)
+            if accepted:
+                r = sim.run(q, seed=2, n_runs=n, lanes_per_run=1, tables=tables, per_run=PER_RUN)
+                _same(r.per_run, {k: ref.per_run[k] for k in PER_RUN}, (n_locs, tables))
+            else:
+                with pytest.raises(A.SmcError) as e:
+                    sim.run(q, seed=2, n_runs=n, lanes_per_run=1, tables=tables, per_run=PER_RUN)
+                assert e.value.code == A.SMC_E_LIMIT
+            # digest runs take tables from anywhere
+            r = sim.run(q, seed=2, n_runs=n, lanes_per_run=1, tables=tables, per_run=with_digest)
+            _same(r.per_run, ref.per_run, (n_locs, tables, "digest"))
+    finally:
+        sim.close()
+
+
+def test_autotuner_names_only_what_a_launch_does(monkeypatch):
+    """Tables that do not fit in LDS are not a choice of the autotuner's."""
+    monkeypatch.setenv("SMC_TUNE_CACHE", "off")
+    for n_locs, staged in ((4, None), (1200, 0), (5000, 0)):
+        net = _distinct(n_locs)
+        sim = cs.GpuSimulator(net)
+        try:
+            print(f"[gpu requests] autotune locations={n_locs}", flush=True)
+            best = sim.autotune(cs.var_query(0, 20.0, estimate=True), sample_runs=4096)
+            assert best.tables in (0, 1) if staged is None else best.tables == staged
+        finally:
+            sim.close()
