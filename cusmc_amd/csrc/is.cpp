@@ -144,6 +144,7 @@ struct smc_is {
         int S = 1, C = 1, R = 64;    // lanes per run, slots per lane, runs per wave
     };
     std::vector<Shape> shapes;
+    Shape widest;
     bool stage = false;  // model tables staged in LDS
     int stride = 1;
     int n_locs = 0, n_vars = 0, n_comp = 0, F = 0, fpad = 0, H = 128, Lpad = 0;
@@ -240,12 +241,26 @@ struct smc_is {
         return shapes[k];
     }
 
+    // The launch's shape, within what LDS holds.  A sampler is accepted by the
+    // LDS of its tilts, variables and race sums (smc_is_create); what the kernel
+    // keeps for slots and features may take more than the latter with some
+    // 12,000 locations, under one tilt vector for all rows.  The widest packing
+    // holds one row's, and with more than 256 components the windows are left
+    // out: computed where they are used.
+    Shape fit_shape(int rows, IsParams &P, bool record) const {
+        P.windows = (m->img.tests & (SMC_HF_INV | SMC_HF_XINV)) ? 1 : 0;
+        Shape sh = shape_for(rows, P, record);
+        if (shared_lds(P) + wave_lds(sh, P, record) > kLdsPerCu) sh = widest;
+        if (P.windows && shared_lds(P) + wave_lds(sh, P, record) > kLdsPerCu) P.windows = -1;
+        return sh;
+    }
+
     // LDS of the advance kernel (is_advance.h): the workgroup's, and a wave's.
     static constexpr size_t kLdsPerCu = 160 * 1024;
     size_t shared_lds(const IsParams &P) const { return (size_t)Lpad * 4 + (size_t)P.theta_shared * 8; }
     size_t wave_lds(const Shape &sh, const IsParams &P, bool record) const {
         return rup((size_t)sh.R * stride * sizeof(double) + (size_t)sh.R * P.theta_cap * 12 +
-                       (size_t)sh.C * (P.windows ? 1024 : 512) + (size_t)sh.R * (Lpad / 8), 16) +
+                       (size_t)sh.C * (P.windows > 0 ? 1024 : 512) + (size_t)sh.R * (Lpad / 8), 16) +
                (record ? (size_t)16 * sh.C * 64 : 0);
     }
 
@@ -267,7 +282,6 @@ struct smc_is {
         P.max_steps = q.max_steps ? q.max_steps : SMC_DEFAULT_MAX_STEPS;
         P.tiltable = tiltable.p;
         P.tilt_index = tix_loc.p;
-        P.windows = (m->img.tests & (SMC_HF_INV | SMC_HF_XINV)) ? 1 : 0;
         P.var_scale = var_scale.p;
         P.weight = weight.p;
         return P;
@@ -422,7 +436,7 @@ struct smc_is {
             unsigned int *cnt = active.p + (k & 1) * kActiveWords, *h_cnt = h_counters + 2 + (k & 1) * kActiveWords;
             P.active_count = cnt;
             P.next_count = active.p + ((k + 1) & 1) * kActiveWords;  // (its copy to the host is ahead in the stream)
-            const Shape &sh = shape_for(rows, P, b.record);
+            const Shape sh = fit_shape(rows, P, b.record);
             P.lanes = sh.S;
             P.wave_lds = (uint32_t)wave_lds(sh, P, b.record);
             // staged tables: workgroups of four waves, as many as the LDS
@@ -430,7 +444,7 @@ struct smc_is {
             // others even out the end); the recording build reads the tables
             // from global memory
             size_t lds = m->table_bytes + shared_lds(P) + 4 * (size_t)P.wave_lds;
-            const bool tab = stage && !b.record && m->table_bytes > 0 && lds <= kLdsPerCu;
+            const bool tab = stage && !b.record && P.windows >= 0 && m->table_bytes > 0 && lds <= kLdsPerCu;
             P.tables = tab ? (decltype(P.tables))m->arena : nullptr;
             P.table_bytes = tab ? m->table_bytes : 0;
             if (!tab) lds = shared_lds(P) + P.wave_lds;
@@ -667,13 +681,17 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
             s->shapes.push_back(sh);
         }
         {
-            // the advance kernel's LDS at its largest: tilts per location
-            IsParams big{};
-            big.theta_cap = s->Gpad;
-            big.theta_shared = s->Lpad;
-            big.windows = 1;
-            if (s->shared_lds(big) + s->wave_lds(s->shapes[0], big, false) > 160 * 1024)
+            // tilt index and 2^theta per location, variables and tilts of a
+            // wave's rows, two doubles per lane and level
+            const smc_is::Shape &sh = s->shapes[0];
+            int levels = 0;
+            while ((1 << levels) < sh.S) ++levels;
+            if ((size_t)s->Lpad * 12 + rup((size_t)sh.R * s->stride * 8 + (size_t)sh.R * s->Gpad * 12 +
+                                               (size_t)levels * 1024, 16) > smc_is::kLdsPerCu)
                 throw std::runtime_error("limit: the advance kernel's LDS exceeds the budget");
+            s->widest.S = P < 64 ? P : 64;
+            s->widest.C = P / s->widest.S;
+            s->widest.R = 64 / s->widest.S;
             // hot tables staged in LDS (where they fit beside four waves)
             // unless the model's tuned launch does not, or SMC_IS_TABLES=1/0
             // says

@@ -110,8 +110,9 @@ struct TiltLds {
 };
 
 // REC: the build that records macro-step statistics (elite replays); the
-// sampling build leaves the recording state out of its registers.
-template <int C, bool REC, class MT>
+// sampling build leaves the recording state out of its registers.  KEEP: the
+// bounded slots' windows are kept in LDS; else they are computed at each use.
+template <int C, bool REC, bool KEEP, class MT>
 __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, double *wlds, const TiltLds &tl,
                                                 int group) {
     const int lane = threadIdx.x & 63;
@@ -251,10 +252,13 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
         RaceSlots<C> rs;
         race_slots<C>(rs, words, Ctx{vars, t, 0}, m, changed, xblk);
         // windows of the bounded slots
-        for (uint32_t b = rs.bounded; b; b &= b - 1) {
-            const int j = __ffs(b) - 1;
-            scr[64 * j] = slot_window(words, j, Ctx{vars, t, 0}, m);
+        if (KEEP) {
+            for (uint32_t b = rs.bounded; b; b &= b - 1) {
+                const int j = __ffs(b) - 1;
+                scr[64 * j] = slot_window(words, j, Ctx{vars, t, 0}, m);
+            }
         }
+        const auto window = [&](int j) { return KEEP ? scr[64 * j] : slot_window(words, j, Ctx{vars, t, 0}, m); };
         if (!full) changed = false;
         // frozen components race only in a full race (as in the run kernel)
         if (m.freeze && full) race_frozen<C>(rs, words, Ctx{vars, t, 0}, m);
@@ -288,7 +292,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                 for (int k = 0; k < nj; ++k) {
                     const int jk = j + k;
                     const double u = smc_uniform_u(rw, c + (uint32_t)k);
-                    const double M = scr[64 * jk];
+                    const double M = window(jk);
                     const int ti = theta ? tl.tix[locs[64 * jk]] : -1;
                     const bool tilted = ti >= 0 && theta[ti] != 0.0f;
                     const double du = tilted ? M * (1.0 - smc_exp2(device_log2(1.0 - u) / tex[ti])) : M * u;
@@ -350,7 +354,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
                         if ((rs.bounded >> j) & 1u) {
                             const int ti = tl.tix[locs[64 * j]];
                             if (ti >= 0 && theta[ti] != 0.0f)
-                                ut[j] = (1.0 - tex[ti]) * device_log2(1.0 - d / scr[64 * j]);
+                                ut[j] = (1.0 - tex[ti]) * device_log2(1.0 - d / window(j));
                         }
                     }
                     log2lr = log2lr + tree_total<C>(ut, S);
@@ -365,7 +369,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
 #pragma unroll
                 for (int j = 0; j < C; ++j) {
                     if (rs.leaf[j] > 0.0) hz[64 * j] = hz[64 * j] + LN2 * rs.leaf[j] * d;
-                    else if ((rs.bounded >> j) & 1u) hz[64 * j] = hz[64 * j] + -LN2 * device_log2(1.0 - d / scr[64 * j]);
+                    else if ((rs.bounded >> j) & 1u) hz[64 * j] = hz[64 * j] + -LN2 * device_log2(1.0 - d / window(j));
                 }
             }
         }
@@ -478,7 +482,7 @@ __device__ __forceinline__ void is_advance_rows(const IsParams &P, const MT &m, 
 // (blockIdx.x * waves + wave, then strided by the grid).  With TAB the
 // workgroup first stages the model's hot tables in LDS (as the run kernel).
 // LDS: [tables: TAB only][per wave: variables of its rows].
-template <int C, bool TAB, bool REC>
+template <int C, bool TAB, bool REC, bool KEEP>
 __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     extern __shared__ __attribute__((aligned(16))) double lds[];
     const int wv = threadIdx.x >> 6, W = blockDim.x >> 6;
@@ -498,7 +502,7 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
     tl.row_ex = wlds + (size_t)R * P.var_stride;
     tl.row_th = (float *)(tl.row_ex + (size_t)R * P.theta_cap);
     tl.scr = (double *)(tl.row_th + (size_t)R * P.theta_cap);
-    tl.words = (uint32_t *)(tl.scr + (P.windows ? 64 * C : 0));
+    tl.words = (uint32_t *)(tl.scr + (P.windows > 0 ? 64 * C : 0));
     tl.locs = (int32_t *)tl.words + 64 * C;
     tl.bits = (uint32_t *)(tl.locs + 64 * C);
     tl.rec = (double *)(tl.bits + R * (P.lpad / 32));
@@ -513,13 +517,13 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
         stage_tables(P.tables, P.table_bytes, lds);  // ends with the workgroup barrier
         const DevModelT<SmcLdsTables> m = lds_model(P.m, P.tables, lds);
         for (int g = blockIdx.x * W + wv; g < groups; g += gridDim.x * W) {
-            is_advance_rows<C, REC>(P, m, wlds, tl, g);
+            is_advance_rows<C, REC, KEEP>(P, m, wlds, tl, g);
             wave_sync();
         }
     } else {
         __syncthreads();
         for (int g = blockIdx.x * W + wv; g < groups; g += gridDim.x * W) {
-            is_advance_rows<C, REC>(P, P.m, wlds, tl, g);
+            is_advance_rows<C, REC, KEEP>(P, P.m, wlds, tl, g);
             wave_sync();
         }
     }
@@ -530,9 +534,9 @@ __device__ __forceinline__ void is_advance_body(const IsParams &P) {
 // fires).  Registers unrestricted: 171-243 VGPRs, two waves per SIMD.  Held to
 // 168 it spills 43-71 of them at eight slots a lane: SIR-100, 5e4 rows, 24.1
 // ms for 22.2.
-template <int C, bool TAB, bool REC>
+template <int C, bool TAB, bool REC, bool KEEP = true>
 __global__ __launch_bounds__(256) void is_advance_kernel(IsParams P) {
-    is_advance_body<C, TAB, REC>(P);
+    is_advance_body<C, TAB, REC, KEEP>(P);
 }
 
 }  // namespace

@@ -55,7 +55,8 @@ struct IsParams {
     int32_t theta_len;          // entries of a theta row (<= lpad when theta_stride == 0, else <= theta_cap)
     int32_t theta_cap;          // per-row tilt entries each wave's LDS holds room for (0 or a multiple of 16)
     int32_t theta_shared;       // entries of 2^theta the workgroup's LDS holds room for
-    int32_t windows;            // each wave's LDS holds a window per slot
+    int32_t windows;            // > 0: each wave's LDS holds a window per slot; < 0: there is no room for them
+                                // (eight slots per lane only)
     uint16_t *feat;             // [rows][fpad] bf16 features of the end state, or null
     const float *var_scale;     // [n_vars]
     // recording of cross-entropy statistics (replay of elite runs)

@@ -16,9 +16,16 @@ namespace {
 hipError_t launch(const IsParams &p, int grid, int group_waves, size_t lds, hipStream_t s) {
     const dim3 g(grid), b(64 * group_waves);
     // builds: staged tables (sampling), global tables (sampling), global
-    // tables with recording
+    // tables with recording; at eight slots the latter two without the windows'
+    // LDS too
     if (p.rec_pos && p.table_bytes) return hipErrorInvalidValue;
-    if (p.rec_pos) hipLaunchKernelGGL((is_advance_kernel<SMC_C, false, true>), g, b, lds, s, p);
+    if (p.windows < 0) {
+        if (SMC_C != 8 || p.table_bytes) return hipErrorInvalidValue;
+        if constexpr (SMC_C == 8) {
+            if (p.rec_pos) hipLaunchKernelGGL((is_advance_kernel<SMC_C, false, true, false>), g, b, lds, s, p);
+            else hipLaunchKernelGGL((is_advance_kernel<SMC_C, false, false, false>), g, b, lds, s, p);
+        }
+    } else if (p.rec_pos) hipLaunchKernelGGL((is_advance_kernel<SMC_C, false, true>), g, b, lds, s, p);
     else if (p.table_bytes) hipLaunchKernelGGL((is_advance_kernel<SMC_C, true, false>), g, b, lds, s, p);
     else hipLaunchKernelGGL((is_advance_kernel<SMC_C, false, false>), g, b, lds, s, p);
     return hipGetLastError();
