@@ -9,6 +9,8 @@ import cusmc_amd as cs
 from cusmc_amd import _capi as A
 from cusmc_amd import generators as G
 
+import oracle
+
 from _models import E_ADD, RawNetwork
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +95,41 @@ def test_autotuner_names_only_what_a_launch_does(monkeypatch):
             assert best.tables in (0, 1) if staged is None else best.tables == staged
         finally:
             sim.close()
+
+
+@pytest.mark.parametrize("n_comp,lanes,n_vars", [(16, 1, 116), (16, 16, 1746), (2, 1, 116), (40, 4, 450)])
+def test_as_many_variables_as_a_packing_holds(n_comp, lanes, n_vars):
+    """Variables of the packed runs up to the limit of 60,000 bytes: with the
+    state words, and a digest run's locations, a wave takes more than 64 KB of
+    LDS.  One variable more is refused."""
+    def network(n):
+        net = RawNetwork()
+        vs = [net.var(float(k % 7)) for k in range(n)]
+        for c in range(n_comp):
+            first = net.component([dict(type=0, rate=net.lit(1.0 + c)), dict(type=0, rate=net.lit(2.0))])
+            a, b = vs[(37 * c + 5) % n], vs[n - 1 - c % 2]
+            net.edge(first, first + 1, upds=[(a, net.expr(E_ADD, net.ref(a), net.ref(b)))])
+            net.edge(first + 1, first, upds=[(b, net.expr(E_ADD, net.ref(b), net.lit(1.0)))])
+        return net.build()
+
+    n = 300
+    with_digest = PER_RUN + ("digest",)
+    net = network(n_vars)
+    q = cs.var_query(n_vars - 1, 3.0, estimate=True)
+    _, want = oracle.run(net, q, seed=6, n_runs=n, threads=8, per_run=with_digest)
+    sim = cs.GpuSimulator(net)
+    try:
+        for tables in (0, 1):
+            print(f"[gpu requests] components={n_comp} lanes={lanes} variables={n_vars} tables={tables}", flush=True)
+            r = sim.run(q, seed=6, n_runs=n, lanes_per_run=lanes, tables=tables, per_run=with_digest)
+            _same(r.per_run, want, (n_comp, lanes, tables))
+    finally:
+        sim.close()
+    more = network(n_vars + 2)
+    sim = cs.GpuSimulator(more)
+    try:
+        with pytest.raises(A.SmcError) as e:
+            sim.run(q, seed=6, n_runs=n, lanes_per_run=lanes)
+        assert e.value.code == A.SMC_E_LIMIT
+    finally:
+        sim.close()
