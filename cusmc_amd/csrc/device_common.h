@@ -634,13 +634,13 @@ __device__ __forceinline__ int pick_edge(uint64_t mask, uint32_t edge_first, uin
         const double u = smc_u01(w.v[0], w.v[1]);
         const bool quick = choice & (mask == (uint64_t)full);
         if (any_lane(quick)) {
-            const int rnd = (int)((double)total * u);
+            const uint32_t rnd = (uint32_t)((double)total * u);
             uint32_t r = quick ? full : 0u;
-            int below = 0;
+            uint32_t below = 0;  // (a lane that is done may wrap it)
 #pragma clang loop unroll(disable)
             do {
                 const int k = r ? __ffs(r) - 1 : 0;
-                const int wk = (int)rec_at(m.edges, edge_first + k)->weight;
+                const uint32_t wk = rec_at(m.edges, edge_first + k)->weight;
                 i = (r && below <= rnd) ? k : i;
                 below += wk;
                 r &= r - 1;
