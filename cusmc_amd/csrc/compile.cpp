@@ -686,7 +686,6 @@ ModelImage lower(const smc_network &n, bool use_locals) {
             h.a = -HUGE_VAL;
             h.b = HUGE_VAL;
             if (d.klass == SMC_K_ZERO) {
-                hf = SMC_HF_ZERO;
                 h.rate = -0.0;
             } else {
                 if (img.freeze && kind == 1) {

@@ -33,10 +33,6 @@ __device__ __forceinline__ uint64_t scalar_here(uint64_t v) {
     asm volatile("" : "+s"(v));
     return v;
 }
-__device__ __forceinline__ int lane_here(int v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
 
 // Whether any active lane has c: a wave-uniform condition, so what it guards
 // is branched around as a whole, and with `unlikely` laid out away from the

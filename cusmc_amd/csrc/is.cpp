@@ -180,8 +180,9 @@ struct smc_is {
     // training activations of one chunk of pairs
     DevBuf<uint16_t> th1, th2, Gb, dh2b, dh1b, xin;
     DevBuf<float> tth, tthg, dh2, dh1, work, xf;
-    DevBuf<unsigned int> counters, active;  // [0] active rows, [1] record slots used, [2] compaction count
-    unsigned int *h_counters = nullptr;  // [0..1] copies of counters[0..1]; then the active counts of alternate macro-steps
+    DevBuf<unsigned int> counters;  // [0] record slots used, [1] compaction count
+    DevBuf<unsigned int> active;    // active rows after alternate macro-steps, in parts
+    unsigned int *h_counters = nullptr;  // [0] copy of counters[0]; from kActiveWords on copies of active
     hipEvent_t step_done[2] = {nullptr, nullptr};
     int adam_t = 0;
     bool zero_output = true;  // output layer all zero: theta == 0 exactly
@@ -409,7 +410,7 @@ struct smc_is {
         }
         if (b.record) {
             P.rec_X = rX.p; P.rec_A = rA.p; P.rec_B = rB.p; P.rec_w = rw.p;
-            hip_check(hipMemsetAsync(counters.p + 1, 0, sizeof(unsigned int), s), "clear record count");
+            hip_check(hipMemsetAsync(counters.p, 0, sizeof(unsigned int), s), "clear record count");
         }
         // Lock-step macro-steps.  The host never waits for the step it just
         // launched: after launching step k it reads the active count of step
@@ -429,11 +430,11 @@ struct smc_is {
                 P.tilt_index = tix_group.p;
             }
             if (b.record) {
-                hip_check(smc::is_record_slots(A->status.p, rows, pos.p, counters.p + 1, (unsigned int)rec_cap, s),
+                hip_check(smc::is_record_slots(A->status.p, rows, pos.p, counters.p, (unsigned int)rec_cap, s),
                           "record slots");
                 P.rec_pos = pos.p;
             }
-            unsigned int *cnt = active.p + (k & 1) * kActiveWords, *h_cnt = h_counters + 2 + (k & 1) * kActiveWords;
+            unsigned int *cnt = active.p + (k & 1) * kActiveWords, *h_cnt = h_counters + (1 + (k & 1)) * kActiveWords;
             P.active_count = cnt;
             P.next_count = active.p + ((k + 1) & 1) * kActiveWords;  // (its copy to the host is ahead in the stream)
             const Shape sh = fit_shape(rows, P, b.record);
@@ -459,14 +460,14 @@ struct smc_is {
             hip_check(hipEventSynchronize(step_done[(k - 1) & 1]), "advance");
             int live = 0;
             for (int i = 0; i < SMC_IS_COUNTS; ++i)
-                live += (int)h_counters[2 + ((k - 1) & 1) * kActiveWords + i * SMC_IS_COUNT_STRIDE];
+                live += (int)h_counters[(1 + ((k - 1) & 1)) * kActiveWords + i * SMC_IS_COUNT_STRIDE];
             if (live == 0) break;
             if (live * 2 <= rows && rows > 1024) {
                 // compaction: results of the finished rows out, live rows
                 // to the front of the other set, in row order
                 hip_check(smc::is_collect(P, out.view(), s), "collect results");
-                hip_check(hipMemsetAsync(counters.p + 2, 0, sizeof(unsigned int), s), "clear compaction count");
-                hip_check(smc::is_record_slots(A->status.p, rows, cpos.p, counters.p + 2, 0xFFFFFFFFu, s),
+                hip_check(hipMemsetAsync(counters.p + 1, 0, sizeof(unsigned int), s), "clear compaction count");
+                hip_check(smc::is_record_slots(A->status.p, rows, cpos.p, counters.p + 1, 0xFFFFFFFFu, s),
                           "compaction slots");
                 const int nrows = (int)rup((size_t)live, 64);
                 B->ensure((size_t)nrows, n_comp, n_vars, fpad, feats);
@@ -514,9 +515,9 @@ struct smc_is {
         b.d_runs = runs_in.p;
         run_rows(b);
         hipStream_t st = stream();
-        hip_check(hipMemcpyAsync(h_counters, counters.p, 2 * sizeof(unsigned int), hipMemcpyDeviceToHost, st), "copy count");
+        hip_check(hipMemcpyAsync(h_counters, counters.p, sizeof(unsigned int), hipMemcpyDeviceToHost, st), "copy count");
         hip_check(hipStreamSynchronize(st), "record");
-        const size_t pairs = std::min<size_t>(h_counters[1], rec_cap);
+        const size_t pairs = std::min<size_t>(h_counters[0], rec_cap);
         const size_t padded = rup(pairs, 64);
         if (padded > pairs) {
             const size_t z = padded - pairs;
@@ -767,11 +768,9 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         s->var_scale.ensure(scale.size(), "hipMalloc scales");
         s->theta_fixed.ensure(L, "hipMalloc tilts");
         s->feat0.ensure(fp, "hipMalloc features");
-        // counters: [1] recorded pairs, [2] compaction slots; active: the
-        // active rows after alternate macro-steps
-        s->counters.ensure(3, "hipMalloc counters");
+        s->counters.ensure(2, "hipMalloc counters");
         s->active.ensure(2 * kActiveWords, "hipMalloc counters");
-        hip_check(hipHostMalloc((void **)&s->h_counters, (2 + 2 * kActiveWords) * sizeof(unsigned int), hipHostMallocDefault), "hipHostMalloc");
+        hip_check(hipHostMalloc((void **)&s->h_counters, 3 * kActiveWords * sizeof(unsigned int), hipHostMallocDefault), "hipHostMalloc");
         for (hipEvent_t &e : s->step_done)
             hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
         hip_check(hipMemcpyAsync(s->tiltable.p, s->h_tiltable.data(), L, hipMemcpyHostToDevice, st), "upload");
