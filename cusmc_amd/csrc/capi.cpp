@@ -156,6 +156,13 @@ smc_launch default_launch(const smc_model *m, uint64_t total_runs, bool trace) {
     return d;
 }
 
+// Half of a wave's even share of what is left, as a power of two.
+int share_shift(int waves) {
+    int s = 1;
+    while (s < 62 && (1ll << (s - 1)) < waves) ++s;
+    return s;
+}
+
 Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs, bool trace) {
     Plan pl;
     const int P = m->img.n_leaves;
@@ -465,6 +472,9 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         lp.n_inst = 1;
         lp.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
         lp.segments = pl.segments;
+        lp.share_shift = share_shift(waves);
+        lp.first = ((uint32_t)pl.segments + pl.chunk_runs - 1) / pl.chunk_runs;
+        lp.handed = (uint64_t)lp.first * (uint64_t)waves;
         lp.counter = m->d_counter;
         lp.round = nullptr;
         lp.tables = pl.tab ? (decltype(lp.tables))m->arena : nullptr;
@@ -575,6 +585,9 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         lp.n_inst = 1;
         lp.total_chunks = (n_runs + pl.chunk_runs - 1) / pl.chunk_runs;
         lp.segments = pl.segments;
+        lp.share_shift = share_shift(waves);
+        lp.first = ((uint32_t)pl.segments + pl.chunk_runs - 1) / pl.chunk_runs;
+        lp.handed = (uint64_t)lp.first * (uint64_t)waves;
         lp.counter = d_counter;
         lp.round = nullptr;
         lp.tables = pl.tab ? (decltype(lp.tables))m->arena : nullptr;
@@ -892,6 +905,9 @@ int smc_batch_create(const smc_batch_item *items, int n_items, int tune, smc_bat
             b->lp.n_inst = n_items;
             b->lp.total_chunks = sh.chunks;
             b->lp.segments = 64;
+            b->lp.share_shift = share_shift(b->waves);
+            b->lp.first = 1;
+            b->lp.handed = (uint64_t)b->waves;
             b->lp.counter = b->d_counter;
             b->lp.round = b->d_round;
             b->lp.tables = nullptr;

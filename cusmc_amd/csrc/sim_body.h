@@ -103,14 +103,27 @@ __device__ __forceinline__ void start_state(const SMC_CONSTANT DevModel &m, doub
 // and 2.65 ms.
 constexpr uint32_t kWaitShare = 16;
 
+// The launch's counter gives some 80 takes a microsecond, whatever their size:
+// thousands of waves that come for the next runs every few turns wait longer for
+// it than for their runs.  So a wave begins with runs of its own, and one
+// whose last runs took fewer turns than this takes as many more at a time, up to
+// sixteen times its need and half its even share of what is left.  One step a run,
+// 1e7 runs: 0.37 ms for 1.98 with a take by need, 2e4 runs 10.4 us for 40.9;
+// UppaalWeightTest, 25 steps a run, 1e7 runs 4.4 ms for 12.0.  At 16 turns the
+// first and third are 0.69 and 6.2 ms; at 64 they are the same, but Fischer-32, 1e6
+// runs, takes 29.9 ms for 29.7.  (Runs of several instances differ too much: a
+// chunk at a time.)
+constexpr uint32_t kShortRuns = 32;
+
 // The same pointer, as far as the optimiser knows another one.
-__device__ __forceinline__ const SMC_CONSTANT InstDesc *opaque(const SMC_CONSTANT InstDesc *p) {
+template <class T>
+__device__ __forceinline__ const SMC_CONSTANT T *opaque(const SMC_CONSTANT T *p) {
     asm volatile("" : "+s"(p));
     return p;
 }
 
-// A wave takes chunks of runs from the launch's queue and hands the runs to
-// its segments; all its segments work on one instance, which (its tables,
+// A wave begins with runs of its own, then takes chunks of runs from the
+// launch's queue, and hands the runs to its segments; all its segments work on one instance, which (its tables,
 // query and outputs) is thereby uniform across the wave and lives in scalar
 // registers.  A chunk of another instance waits until this one's runs are
 // done.  A workgroup holds blockDim/64 independent waves.  With TAB
@@ -154,37 +167,50 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     const int wv = threadIdx.x >> 6;
     double *wbase = lds + (TAB ? lp.table_bytes / 8 : 0) + (size_t)wv * (lp.wave_lds / 8);
     const double INF = __builtin_huge_val();
-    const uint64_t round = lp.round ? *lp.round : 0;
     using Tables = typename std::conditional<TAB, SmcLdsTables, SmcGlobalTables>::type;
     if (TAB) stage_tables(lp.tables, lp.table_bytes, lds);
 
-  unsigned long long g = 0, g_end = 0;  // chunks the wave has taken and not begun
+  const SMC_CONSTANT LaunchParams *args = (const SMC_CONSTANT LaunchParams *)__builtin_amdgcn_kernarg_segment_ptr();
+  // chunks the wave has taken and not begun, the first of them without the queue
+  unsigned long long g = (unsigned long long)(blockIdx.x * (blockDim.x >> 6) + wv) * lp.first, g_end = g + lp.first;
+  // n more, where any are left
+  const auto take = [&](uint32_t n, const SMC_CONSTANT LaunchParams *L) {
+      const uint64_t total = L->total_chunks, handed = L->handed;
+      if (handed >= total || g_end >= total) {
+          g = g_end = total;
+      } else {
+          g = handed + take_chunks(L->counter, n, lane);
+          g_end = g + n;
+      }
+  };
   for (;;) {
     g = first_lane(g);
     g_end = first_lane(g_end);
-    if (g == g_end) g_end = (g = take_chunks(lp.counter, 1, lane)) + 1;
-    if (g >= lp.total_chunks) break;
-    int lo = 0, hi = lp.n_inst - 1;
+    const SMC_CONSTANT LaunchParams *launch = opaque(args);
+    if (g == g_end) take(1, launch);
+    if (g >= launch->total_chunks) break;
+    int lo = 0, hi = launch->n_inst - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (lp.inst[mid].chunk_first <= g) lo = mid;
+        if (launch->inst[mid].chunk_first <= g) lo = mid;
         else hi = mid - 1;
     }
     // What every step needs of the instance stays in registers; what only a
     // run's start or end needs is read again there (through `inst` made
     // opaque, or it would be loaded here and spilled).
-    const SMC_CONSTANT InstDesc *inst = (const SMC_CONSTANT InstDesc *)(uintptr_t)lp.inst + lo;
+    const SMC_CONSTANT InstDesc *inst = (const SMC_CONSTANT InstDesc *)(uintptr_t)launch->inst + lo;
     DevModelT<Tables> m;
     if constexpr (TAB) {
+        const SMC_GLOBAL uint8_t *tables = launch->tables;
         const SMC_LDS uint8_t *copy = (const SMC_LDS uint8_t *)(SMC_LDS double *)lds;
-        m.hots = in_lds(inst->m.hots, lp.tables, copy);
-        m.locs = in_lds(inst->m.locs, lp.tables, copy);
-        m.invs = in_lds(inst->m.invs, lp.tables, copy);
-        m.edges = in_lds(inst->m.edges, lp.tables, copy);
-        m.guards = in_lds(inst->m.guards, lp.tables, copy);
-        m.upds = in_lds(inst->m.upds, lp.tables, copy);
-        m.consts = in_lds(inst->m.consts, lp.tables, copy);
-        m.code = in_lds(inst->m.code, lp.tables, copy);
+        m.hots = in_lds(inst->m.hots, tables, copy);
+        m.locs = in_lds(inst->m.locs, tables, copy);
+        m.invs = in_lds(inst->m.invs, tables, copy);
+        m.edges = in_lds(inst->m.edges, tables, copy);
+        m.guards = in_lds(inst->m.guards, tables, copy);
+        m.upds = in_lds(inst->m.upds, tables, copy);
+        m.consts = in_lds(inst->m.consts, tables, copy);
+        m.code = in_lds(inst->m.code, tables, copy);
     } else {
         m.hots = inst->m.hots;
         m.locs = inst->m.locs;
@@ -218,10 +244,10 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     int32_t *locs = (int32_t *)words_of + 64 * C + lane;  // TRACE only
     // since runs were started: turns of the loop, lanes without a run summed
     // over them
-    uint32_t turns = 0, waited = 0;
+    uint32_t turns = kShortRuns, waited = 0;
     uint32_t r_next = 0, r_end = 0;  // runs of chunks begun, not started yet
 
-    bool active = false, done = lane / S0 >= lp.segments;
+    bool active = false, done = lane / S0 >= launch->segments;
     uint64_t run = 0;
     uint32_t ridx = 0;
     double t = 0.0;
@@ -285,6 +311,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
             const bool want = !active & !done;
             waited += (uint32_t)__popcll(__ballot(want));
             if (!any_lane(active) || kWaitShare * waited > 64 * turns) {
+                const uint32_t more = turns < kShortRuns ? min(kShortRuns / max(turns, 1u), 16u) : 1u;
                 waited = turns = 0;
                 const uint64_t heads = __ballot(want & (sl == 0));
                 const int need = __popcll(heads), rank = __popcll(heads & ((1ull << seg_base) - 1));
@@ -294,10 +321,14 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                 for (int given = 0; given < need;) {
                     if (r_next == r_end) {
                         if (g == g_end) {
-                            // (of several instances one at a time: it may be another's)
-                            const uint32_t n = lp.n_inst == 1 ? ((uint32_t)(need - given) + chunk - 1) / chunk : 1u;
-                            g = take_chunks(lp.counter, n, lane);
-                            g_end = g + n;
+                            const SMC_CONSTANT LaunchParams *L = opaque(args);
+                            uint32_t n = 1;
+                            if (L->n_inst == 1) {
+                                const uint64_t total = L->total_chunks, left = g < total ? total - g : 0;
+                                n = ((uint32_t)(need - given) + chunk - 1) / chunk;
+                                n = max(n, (uint32_t)min((uint64_t)(n * more), left >> L->share_shift));
+                            }
+                            take(n, L);
                         }
                         if (g >= c1) break;
                         const uint64_t stop = g_end < c1 ? g_end : c1, r1 = (stop - c0) * chunk;
@@ -315,7 +346,8 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                         done = true;
                     } else {
                         ridx = r;
-                        run = I->p.run_begin + round * I->p.n_runs + r;
+                        const SMC_CONSTANT uint64_t *round = (const SMC_CONSTANT uint64_t *)(uintptr_t)opaque(args)->round;
+                        run = I->p.run_begin + (round ? *round : 0) * I->p.n_runs + r;
                         active = true;
                         t = 0.0; step = 0; trans = 0; chan = 0; sender = -1;
                         goal = false; over = false; changed = true;
