@@ -704,9 +704,9 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                     inline_var(R.invs[0].var, &hot_at, &hot_local);
                     h.a = R.invs[0].bound_value;
                     h.b = R.invs[0].strict ? 1e-6 : 0.0;
-                    if (!moderate(h.a) || !clock_moderate[inv_clock]) hf |= SMC_HF_OPEN;
+                    if (!moderate(h.a) || !clock_moderate[inv_clock]) hf |= SMC_HF_WINDOW;
                 } else if (d.n_inv) {
-                    hf |= SMC_HF_XINV;
+                    hf |= SMC_HF_XINV | SMC_HF_WINDOW;
                 }
                 if (img.freeze && kind == 2) {
                     if (R.block.size() == 1 && (R.block[0].flags & SMC_GF_RANGE) && !(hf & SMC_HF_INV)) {

@@ -795,18 +795,14 @@ __device__ __forceinline__ double hot_value(const DevHot &h, uint32_t word, cons
     return *(const double *)((const char *)vars + ((word & h.base) << 3) + (h.what & 0xFFFFu));
 }
 
-// Records whose delay window is not their own invariant's remaining time: other
-// invariants, or one whose window may have no end (window_of then gives the
-// largest double).
-constexpr uint32_t kWindowOther = SMC_HF_XINV | SMC_HF_OPEN;
-
-// The delay window of slot j, which is bounded.
+// The delay window of slot j, which is bounded.  (One without an end is
+// window_of's largest double.)
 template <class M>
 __device__ __forceinline__ double slot_window(const uint32_t *words, int j, Ctx x, const M &m) {
     const uint32_t w = words[64 * j];
     const DevHot h = load_rec(m.hots + word_rec(w, m));
     double left = h.a - (x.now - hot_value(h, w, x.vars)) - h.b;
-    const bool other = (h.what & (kWindowOther << 16)) != 0;
+    const bool other = (h.what & (SMC_HF_WINDOW << 16)) != 0;
     if (unlikely(any_lane(other))) {
         if (other) {
             x.base = word_base(w, m);
@@ -834,12 +830,12 @@ __device__ __forceinline__ void slot_windows(double (&left)[2], const uint32_t *
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         left[k] = h[k].a - (x.now - v[k]) - h[k].b;
-        other |= (h[k].what & (kWindowOther << 16)) != 0;
+        other |= (h[k].what & (SMC_HF_WINDOW << 16)) != 0;
     }
     if (unlikely(any_lane(other))) {
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            if (h[k].what & (kWindowOther << 16)) {
+            if (h[k].what & (SMC_HF_WINDOW << 16)) {
                 x.base = word_base(w[k], m);
                 left[k] = window_of(load_rec(m.locs + word_rec(w[k], m)), x, m);
             }
@@ -954,7 +950,7 @@ __device__ __forceinline__ void race_slots(RaceSlots<C> &rs, const uint32_t *wor
         classify<C, true, 2>(rs, words, x, m, 0.0, expr, own);
     }
     // (up to two slots' windows are kept, so one without an end is set here)
-    constexpr uint32_t kWindow = C <= 2 ? kWindowOther : (uint32_t)SMC_HF_XINV;
+    constexpr uint32_t kWindow = C <= 2 ? SMC_HF_WINDOW : SMC_HF_XINV;
     if (tests & (kWindow | SMC_HF_XBLK)) {
         if (changed) xblk = 0;
         uint32_t out = 0;

@@ -89,7 +89,8 @@ enum : uint32_t {
 
 // What a race step has to look at in a location (high half of DevHot.what).
 enum {
-    SMC_HF_OPEN = 0x80,     // with INV: the window may have no end (an infinite or very large bound or clock)
+    SMC_HF_WINDOW = 0x80,   // the delay window is not what the record's invariant leaves: XINV, or with INV one
+                            // that may have no end (an infinite or very large bound or clock)
     SMC_HF_EXPR = 0x200,    // the rate is an expression (DevLoc.rate)
     SMC_HF_EXPR_LOCAL = 0x400,  // ... which reads private variables
     SMC_HF_XINV = 0x800,    // other invariants: DevInv records
