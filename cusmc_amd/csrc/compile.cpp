@@ -642,7 +642,6 @@ ModelImage lower(const smc_network &n, bool use_locals) {
                 idle[n_recv != 0] = re.e.dst == 0 && E.upd_count == 0 && !(re.e.flags & SMC_EF_GOAL);
                 if (n_recv++ == 0) low = re.e.weight;
             }
-            if (weight >= 2147483648ll) fast = false;
             if (fast) d.flags |= SMC_LF_RECV_FAST;
             if (n_recv == 0) d.recv_chan = 0;
             else if (fast && plain_recv) {

@@ -1312,21 +1312,20 @@ __device__ __forceinline__ void fire_receivers_general(uint32_t *words, int32_t 
                 const uint32_t ef = m.locs[word_rec(w, m)].edge_first;
                 int i = on ? __ffs(mk[j]) - 1 : 0;
                 if (any_lane(choice)) {
-                    // weighted choice; weights are constants summing below
-                    // 2^31
+                    // weighted choice; weights are constants
                     const bool two = choice & ((rv.w & SMC_RF_TWO) != 0) & (mk[j] == rv.y);
                     if (two & (receiver_word(rw, c) >= rv.z)) i = 31 - __clz((int)mk[j]);
                     const bool several = choice & !two;
                     if (unlikely(any_lane(several))) {
                         if (several) {
                             const double u = smc_receiver_u(rw, c);
-                            int W = 0;
-                            for (uint32_t r = mk[j]; r; r &= r - 1) W += (int)rec_at(m.edges, ef + __ffs(r) - 1)->weight;
-                            const int rnd = (int)((double)W * u);
+                            int64_t W = 0;
+                            for (uint32_t r = mk[j]; r; r &= r - 1) W += rec_at(m.edges, ef + __ffs(r) - 1)->weight;
+                            const int64_t rnd = (int64_t)((double)W * u);
                             for (uint32_t r = mk[j]; r;) {
                                 const int k = 31 - __clz((int)r);
                                 r &= ~(1u << k);
-                                W -= (int)rec_at(m.edges, ef + k)->weight;
+                                W -= rec_at(m.edges, ef + k)->weight;
                                 if (W <= rnd) { i = k; break; }
                             }
                         }

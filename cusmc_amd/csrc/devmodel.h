@@ -76,7 +76,7 @@ enum {
                             // there is none): always blocked
     SMC_LF_GUARDED = 4,     // blocked or not by the variables: every spontaneous edge without
                             // `!=` has a conjunct that reads no clock (DevLoc.block_first)
-    SMC_LF_RECV_FAST = 8    // every receive edge commutes (see DevUpd), constant weights below 2^31 in all
+    SMC_LF_RECV_FAST = 8    // every receive edge commutes (see DevUpd), constant weights
 };
 
 // DevLoc.recv_flags (recv_chan > 0).
@@ -128,7 +128,8 @@ struct DevHot {
 // The rest, 64 bytes: receive edges; spontaneous edges; invariants, blocking
 // test and rate.
 struct DevLoc {
-    int32_t recv_chan;      // every receive edge is unguarded, on this channel; 0 none; -1 other
+    int32_t recv_chan;      // every receive edge is unguarded, on this channel, among the first 32 edges, and
+                            // they commute; 0 none; -1 other
     uint32_t recv_mask;     // the receive edges, as bits of the edge list
     uint32_t recv_split;    // of two: the least draw that picks the higher one
     uint32_t recv_flags;    // SMC_RF_*

@@ -100,3 +100,27 @@ def test_chains_of_equal_locations_share_records(check, length):
     assert int(eight[0][2]) == 8 * length and int(eight[0][4]) == length + 1
     # one instance leads to another guard: its records are its own, but for those past the guard
     assert length + 2 < int(odd[0][4]) <= 2 * length + 1
+
+
+def _receivers(edges):
+    """A sender and two components that receive on the given (channel, weight) edges."""
+    tpls = ["""<template><name>S</name><declaration></declaration><location id="id0"><name>s</name></location>
+<init ref="id0"/><transition><source ref="id0"/><target ref="id0"/><label kind="synchronisation">a!</label></transition>
+<transition><source ref="id0"/><target ref="id0"/><label kind="synchronisation">b!</label></transition></template>"""]
+    for c in (1, 2):
+        tr = "".join(f"""<transition><source ref="id{c}0"/><target ref="id{c}0"/><label kind="synchronisation">{ch}?</label>
+<label kind="assignment">n = n + {k % 3}</label>{f'<label kind="probability">{w}</label>' if w else ""}</transition>"""
+                     for k, (ch, w) in enumerate(edges))
+        tpls.append(f"""<template><name>R{c}</name><declaration></declaration><location id="id{c}0"><name>r</name></location>
+<init ref="id{c}0"/>{tr}</template>""")
+    return f"""<?xml version="1.0" encoding="utf-8"?>
+<nta><declaration>broadcast chan a, b; int n = 0;</declaration>{"".join(tpls)}<system>system S, R1, R2;</system></nta>"""
+
+
+def test_commuting_receivers_fire_together(check):
+    """Receivers whose edges add integers fire all at once, with up to 32 edges
+    and whatever their constant weights sum to."""
+    cases = [[("a", 1), ("a", 3)], [("a", 2147483647)] * 2, [("a", 1)] * 32, [("a", 1)] * 3, [("a", 2), ("b", 2147483647)] * 16]
+    for case, lines in zip(cases, check(*map(_receivers, cases))):
+        kinds = [l[1] for l in lines if l[0] == "receives"]
+        assert kinds == ["together"], case

@@ -153,3 +153,36 @@ def test_template_networks_bit_exact_vs_oracle(n_comp, clock_rate):
                         assert np.array_equal(a, b), (n_comp, seed, S, occ, tab, k)
         finally:
             sim.close()
+
+
+@pytest.mark.parametrize("edges", [
+    [(1, 2147483647)] * 2, [(1, 2147483647), (1, 1), (1, 2147483647)], [(1, 2147483647), (2, 1), (1, 2147483647)],
+    [(1, 2147483647)] * 32, [(1, 3), (2, 2147483647)] * 16, [(1, 2147483647)] * 33])
+@pytest.mark.parametrize("guarded", [False, True])
+def test_heavy_receivers_bit_exact_vs_oracle(edges, guarded):
+    """Weights that sum past 31 and 32 bits, on one channel and on two, with as
+    many edges as are tested together and one more."""
+    net = RawNetwork()
+    v = [net.var(0.0) for _ in range(4)]
+    up = lambda k: [(v[k], net.expr(E_ADD, net.ref(v[k]), net.lit(1.0)))]  # noqa: E731
+    first = net.component([dict(type=0, rate=net.lit(2.0))])
+    for channel in (1, 2):
+        net.edge(first, first, channel=channel)
+    for c in range(20):
+        first = net.component([dict(type=0), dict(type=0)])
+        for l in range(2):
+            for k, (channel, weight) in enumerate(edges):
+                net.edge(first + l, first + (k + l) % 2, channel=-channel, weight=net.lit(float(weight)), upds=up(k % 4),
+                         guards=[(LE, v[0], net.lit(150.0))] if guarded and k == 1 else [])
+    net = net.build()
+    q = cs.var_query(1, 100.0, estimate=True, max_steps=100)
+    _, ro = oracle.run(net, q, seed=3, n_runs=200, threads=8, per_run=PER_RUN)
+    sim = cs.GpuSimulator(net)
+    try:
+        for S in (2, 8, 32):
+            print(f"[gpu records] edges={len(edges)} guarded={guarded} lanes={S}", flush=True)
+            r = sim.run(q, seed=3, n_runs=200, lanes_per_run=S, per_run=PER_RUN)
+            for k in PER_RUN:
+                assert np.array_equal(r.per_run[k].view(np.uint8), ro[k].view(np.uint8)), (S, k)
+    finally:
+        sim.close()
