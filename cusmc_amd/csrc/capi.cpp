@@ -136,14 +136,18 @@ int register_waves(int C, bool trace, int occ, bool tab) {
 // at 2000 runs Fischer-32 takes 0.85 at 32 lanes, 0.95 at 16 and 2.0 at 2.
 // Where slots are tested one after another (invariants and blocking tests of
 // several records) a lane gets as few as there are: csma-100, 16384 runs, 5.5
-// at 64 lanes and 11.0 at 32.
+// at 64 lanes and 11.0 at 32.  Receivers tested edge by edge have at most four to
+// a lane where the lists are longer than that (5, 20 and 34 edges on two channels, 70
+// components, 2e4 runs: 1.25, 2.58 and 3.72 ms; at sixteen 1.86, 4.13 and 6.56); with
+// two edges on 300 components sixteen are better, 2.1 ms for 2.9.
 smc_launch default_launch(const smc_model *m, uint64_t total_runs, bool trace) {
     const int P = m->img.n_leaves, stride = (m->img.n_vars + 1) | 1;
     const uint64_t simds = 4ull * (uint64_t)m->cu_count;
     smc_launch d{};
     int S = std::min(P, 64);
+    const int most = m->img.recv_tested > 4 ? 4 : 16;
     if (!(m->img.tests & (SMC_HF_XINV | SMC_HF_XBLK)))
-        while (S > 1 && P / (S / 2) <= 16) {
+        while (S > 1 && P / (S / 2) <= most) {
             const int s = S / 2, R = 64 / s;
             if (total_runs / (uint64_t)R < 2 * simds) break;
             if (!vars_fit(R, m->img.n_vars, tree_levels(s))) break;

@@ -663,6 +663,7 @@ ModelImage lower(const smc_network &n, bool use_locals) {
             } else {
                 d.recv_chan = -1;
                 d.recv_mask = 0;
+                img.recv_tested = std::max(img.recv_tested, L.edge_count);
             }
 
             // spontaneous edges with constant weights

@@ -40,6 +40,7 @@ struct ModelImage {
     uint32_t tests = 0;   // every SMC_HF_* flag in use
     uint32_t one_rate = SMC_NO_REF;  // the one rate expression, if there is just one
     bool freeze = true;   // no location's rate reads a clock
+    int recv_tested = 0;  // most edges of a location whose receive edges are tested one by one (DevLoc.recv_chan -1)
 };
 
 // Throws std::runtime_error (message prefixed "limit:" for size limits).

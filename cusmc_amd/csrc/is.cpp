@@ -600,14 +600,16 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
         // launch shapes of the advance kernel
         // lanes per run: the model's tuned packing (smc_autotune) when there
         // is one of at most eight slots per lane, else the widest, and
-        // narrower ones for many rows
+        // narrower ones for many rows.  Not where slots are tested one after
+        // another for long (20 and 34 receive edges on two channels, 200
+        // components, 1000 rows: 1.15 and 1.29 ms at 64 lanes, 1.89 and 2.15 at 32)
         const int P = img.n_leaves;
         if (P > 512) throw std::runtime_error("limit: importance sampling takes networks of at most 512 components");
         int lanes = P < 64 ? P : 64, fewest = lanes;
         if (m->has_tuned && m->tuned.lanes_per_run > 0 && m->tuned.lanes_per_run <= lanes &&
             P / m->tuned.lanes_per_run <= 8) {
             fewest = lanes = m->tuned.lanes_per_run;
-        } else if (!(img.tests & (SMC_HF_XINV | SMC_HF_XBLK))) {
+        } else if (!(img.tests & (SMC_HF_XINV | SMC_HF_XBLK)) && img.recv_tested <= 4) {
             while (fewest > 1 && P / (fewest / 2) <= 8) fewest /= 2;
         }
         // SMC_IS_LANES=<power of two> overrides the lanes per run (diagnosis:
