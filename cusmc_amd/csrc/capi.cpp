@@ -47,7 +47,6 @@ struct Plan {
     int segments = 64;  // segments of a wave that take runs
 };
 
-constexpr size_t kLdsPerCu = 160 * 1024;
 constexpr size_t kLdsStatic = 64;  // the run kernel's own
 
 int tree_levels(int S) {
@@ -198,15 +197,14 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
     // each of the CU's four SIMDs.
     int per_cu = register_waves(pl.C, trace, pl.occ, want.tables != 0);
     const auto staged = [&](int g) {
-        const size_t lds = m->table_bytes + (size_t)g * wave + kLdsStatic;
-        return std::min((int)(kLdsPerCu / lds), std::max(per_cu / g, 1)) * g;
+        return std::min(groups_per_cu(m->table_bytes + (size_t)g * wave + kLdsStatic), std::max(per_cu / g, 1)) * g;
     };
     if (want.tables) {
         int best = 0;
         for (int g = 1; g <= SMC_MAX_GROUP_WAVES; g *= 2) best = std::max(best, staged(g));
         pl.tab = best > 0;
         // (left to choose: where they cost no waves)
-        if (!use && best < std::min(per_cu, (int)(kLdsPerCu / (wave + kLdsStatic)))) pl.tab = false;
+        if (!use && best < std::min(per_cu, groups_per_cu(wave + kLdsStatic))) pl.tab = false;
         if (pl.tab) {
             // the smallest workgroups that hold what the runs ask for: few
             // runs then spread over the CUs evenly
@@ -228,7 +226,7 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
             per_cu = register_waves(pl.C, trace, pl.occ, false);
         }
     }
-    if (!pl.tab) per_cu = std::max(1, std::min(per_cu, (int)(kLdsPerCu / (wave + kLdsStatic))));
+    if (!pl.tab) per_cu = std::max(1, std::min(per_cu, groups_per_cu(wave + kLdsStatic)));
     if (want.waves_per_cu > 0 && want.waves_per_cu < per_cu) per_cu = want.waves_per_cu;
     pl.per_cu = per_cu;
     int waves = want.waves > 0 ? want.waves : m->cu_count * per_cu;
@@ -847,7 +845,7 @@ BatchShape batch_shape(smc_batch *b, int C, uint64_t runs_override) {
 int batch_waves(int C, int occ, size_t wave_lds, int waves_per_cu, int cu_count) {
     int blocks = 0;
     hip_check(smc::sim_occupancy(C, false, occ, false, 1, wave_lds, &blocks), "occupancy query");
-    int per_cu = blocks;
+    int per_cu = std::min(blocks, groups_per_cu(wave_lds + kLdsStatic));
     if (waves_per_cu > 0 && waves_per_cu < per_cu) per_cu = waves_per_cu;
     return std::max(1, per_cu) * cu_count;
 }

@@ -45,6 +45,13 @@ int guarded(F &&f) {
 
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// LDS of a compute unit, and workgroups of `lds` bytes that it holds: LDS is
+// handed out in 128 parts.  (The runtime's occupancy query rounds to less.  Twelve
+// waves a CU that it held to fit, two in 26.9 to 27.3 KB, were ten: a run of 98,304
+// started the last of them when the first ended, 4.9 ms for 3.1.)
+constexpr size_t kLdsPerCu = 160 * 1024;
+inline int groups_per_cu(size_t lds) { return (int)(kLdsPerCu / align_up(std::max<size_t>(lds, 1), kLdsPerCu / 128)); }
+
 // Per-run device outputs of one instance, grown on demand.
 struct RunBuffers {
     size_t cap = 0;

@@ -257,7 +257,6 @@ struct smc_is {
     }
 
     // LDS of the advance kernel (is_advance.h): the workgroup's, and a wave's.
-    static constexpr size_t kLdsPerCu = 160 * 1024;
     size_t shared_lds(const IsParams &P) const { return (size_t)Lpad * 4 + (size_t)P.theta_shared * 8; }
     size_t wave_lds(const Shape &sh, const IsParams &P, bool record) const {
         return rup((size_t)sh.R * stride * sizeof(double) + (size_t)sh.R * P.theta_cap * 12 +
@@ -449,7 +448,7 @@ struct smc_is {
             P.tables = tab ? (decltype(P.tables))m->arena : nullptr;
             P.table_bytes = tab ? m->table_bytes : 0;
             if (!tab) lds = shared_lds(P) + P.wave_lds;
-            const int max_groups = tab ? std::min(4, (int)(kLdsPerCu / lds)) * m->cu_count : 0;
+            const int max_groups = tab ? std::min(4, groups_per_cu(lds)) * m->cu_count : 0;
             hip_check(smc::is_launch_advance(P, sh.C, lds, max_groups, s), "advance kernel launch");
             ++launches;
             if (!b.lockstep) break;
@@ -690,7 +689,7 @@ int smc_is_create(smc_model *m, const smc_query *q, const smc_is_config *cfg_in,
             int levels = 0;
             while ((1 << levels) < sh.S) ++levels;
             if ((size_t)s->Lpad * 12 + rup((size_t)sh.R * s->stride * 8 + (size_t)sh.R * s->Gpad * 12 +
-                                               (size_t)levels * 1024, 16) > smc_is::kLdsPerCu)
+                                               (size_t)levels * 1024, 16) > kLdsPerCu)
                 throw std::runtime_error("limit: the advance kernel's LDS exceeds the budget");
             s->widest.S = P < 64 ? P : 64;
             s->widest.C = P / s->widest.S;

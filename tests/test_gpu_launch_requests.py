@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 import cusmc_amd as cs
 from cusmc_amd import _capi as A
@@ -131,5 +132,28 @@ def test_as_many_variables_as_a_packing_holds(n_comp, lanes, n_vars):
         with pytest.raises(A.SmcError) as e:
             sim.run(q, seed=6, n_runs=n, lanes_per_run=lanes)
         assert e.value.code == A.SMC_E_LIMIT
+    finally:
+        sim.close()
+
+
+@pytest.mark.parametrize("n_vars,stays", [(145, 7), (147, 6)])
+def test_waves_left_to_choose_are_resident(n_vars, stays):
+    """A wave whose LDS, handed out in parts of 1280 bytes, fits a compute unit
+    one time less than its bytes do: sixteen runs of 145 and of 147 variables
+    take 18 and 19 parts of 128."""
+    net = RawNetwork()
+    vs = [net.var(0.0) for _ in range(n_vars)]
+    for c in range(64):
+        first = net.component([dict(type=0, rate=net.lit(1.0 + c))])
+        net.edge(first, first, upds=[(vs[c], net.expr(E_ADD, net.ref(vs[c]), net.lit(1.0)))])
+    net = net.build()
+    q = cs.var_query(63, 3.0, estimate=True)
+    n = 60_000
+    sim = cs.GpuSimulator(net)
+    try:
+        print(f"[gpu requests] variables={n_vars}", flush=True)
+        r = sim.run(q, seed=8, n_runs=n, lanes_per_run=4, tables=0, per_run=PER_RUN)
+        assert r.waves == stays * torch.cuda.get_device_properties(0).multi_processor_count
+        _same(r.per_run, sim.run(q, seed=8, n_runs=n, lanes_per_run=64, per_run=PER_RUN).per_run, n_vars)
     finally:
         sim.close()
