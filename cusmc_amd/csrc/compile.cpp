@@ -454,15 +454,57 @@ ModelImage lower(const smc_network &n, bool use_locals) {
         return vu.set == 0 || (vu.add == 0 && vu.one_value);
     };
 
-    // Clocks whose values are constants far inside the doubles, plus time: a
-    // window under such a bound is finite.
+    // Clocks set to values far inside the doubles: a window under such a bound
+    // is finite.  `most` bounds what a variable that is no clock holds; what a
+    // run adds up, at most 1e20 terms, counts with the term.
     auto moderate = [](double v) { return std::fabs(v) <= 1e300; };
-    std::vector<uint8_t> clock_moderate(n.n_vars);
-    for (int v = 0; v < n.n_vars; ++v) clock_moderate[v] = moderate(n.var_init[v]);
+    std::vector<double> most(n.n_vars);
+    std::function<double(int)> reach = [&](int x) -> double {
+        if (x < 0) return HUGE_VAL;
+        const smc_expr_node &e = n.exprs[x];
+        double v = HUGE_VAL;
+        switch (e.op) {
+        case SMC_E_LIT: v = std::fabs(e.value); break;
+        case SMC_E_VAR: v = n.var_kind[e.var] == SMC_VAR_CLOCK ? HUGE_VAL : most[e.var]; break;
+        case SMC_E_ADD: case SMC_E_SUB: v = reach(e.a) + reach(e.b); break;
+        case SMC_E_MUL: v = reach(e.a) * reach(e.b); break;
+        case SMC_E_NEG: v = reach(e.a); break;
+        case SMC_E_COND: v = std::max(reach(e.b), reach(e.c)); break;
+        case SMC_E_RANDOM: case SMC_E_NOT: case SMC_E_AND: case SMC_E_OR: case SMC_E_LE: case SMC_E_GE:
+        case SMC_E_LT: case SMC_E_GT: case SMC_E_EQ: case SMC_E_NE: v = 1.0; break;
+        default: break;
+        }
+        return moderate(v) ? v : HUGE_VAL;
+    };
+    for (int v = 0; v < n.n_vars; ++v) most[v] = std::fabs(n.var_init[v]);
+    bool grows = false;  // (needed for clocks set to expressions only)
     for (int u = 0; u < n.n_updates; ++u) {
         double c;
-        if (!literal(n.updates[u].expr, &c) || !moderate(c)) clock_moderate[n.updates[u].var] = 0;
+        grows |= n.var_kind[n.updates[u].var] == SMC_VAR_CLOCK && !literal(n.updates[u].expr, &c);
     }
+    for (int round = 0; grows; ++round) {
+        std::vector<double> set(n.n_vars), sum(n.n_vars, 0.0);
+        for (int v = 0; v < n.n_vars; ++v) set[v] = std::fabs(n.var_init[v]);
+        for (int u = 0; u < n.n_updates; ++u) {
+            const int v = n.updates[u].var, x = n.updates[u].expr;
+            const smc_expr_node *e = x >= 0 ? &n.exprs[x] : nullptr;
+            if (n.var_kind[v] == SMC_VAR_CLOCK) continue;
+            if (e && (e->op == SMC_E_ADD || e->op == SMC_E_SUB) && is_var(e->a, v)) sum[v] = std::max(sum[v], reach(e->b));
+            else if (e && e->op == SMC_E_ADD && is_var(e->b, v)) sum[v] = std::max(sum[v], reach(e->a));
+            else set[v] = std::max(set[v], reach(x));
+        }
+        grows = false;
+        for (int v = 0; v < n.n_vars; ++v) {
+            const double now = set[v] + 1e20 * sum[v];
+            if (!(now > most[v])) continue;
+            most[v] = round < 8 ? now : HUGE_VAL;
+            grows = true;
+        }
+    }
+    std::vector<uint8_t> clock_moderate(n.n_vars);
+    for (int v = 0; v < n.n_vars; ++v) clock_moderate[v] = moderate(n.var_init[v]);
+    for (int u = 0; u < n.n_updates; ++u)
+        if (!moderate(reach(n.updates[u].expr))) clock_moderate[n.updates[u].var] = 0;
 
     // Null racers leave an all-exponential race only while every rate is
     // constant between transitions (a rate reading a clock changes at each

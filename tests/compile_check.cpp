@@ -14,6 +14,8 @@ int main(int argc, char **argv) {
         std::printf("model locations %zu classes %zu edges %zu\n", im.loc_rec.size(), im.locs.size(), im.edges.size());
         for (const DevLoc &L : im.locs)
             if (L.recv_chan) std::printf("receives %s chan %d\n", L.flags & SMC_LF_RECV_FAST ? "together" : "in turn", L.recv_chan);
+        for (const DevHot &h : im.hots)
+            if ((h.what >> 16) & SMC_HF_INV) std::printf("window %s\n", (h.what >> 16) & SMC_HF_WINDOW ? "general" : "inline");
         for (const DevEdge &e : im.edges)
             if (!(e.flags & SMC_EF_NO_GUARD)) std::printf("interval %a %a\n", e.lo, e.hi);
     }

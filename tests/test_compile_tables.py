@@ -124,3 +124,20 @@ def test_commuting_receivers_fire_together(check):
     for case, lines in zip(cases, check(*map(_receivers, cases))):
         kinds = [l[1] for l in lines if l[0] == "receives"]
         assert kinds == ["together"], case
+
+
+@pytest.mark.parametrize("declared,updates,window", [
+    ("", "x = 0", "inline"), ("int v = 7;", "x = v", "inline"), ("int v = 7;", "x = v - 2 * v", "inline"),
+    ("int v = 7; int w = 1;", "v = v + 3, w = v * v, x = w", "inline"), ("int v; int w;", "v = w, w = v, x = w", "inline"),
+    ("int v; int w;", "v = w + 1, w = v, x = w", "general"), ("int v = 2;", "v = v * v, x = v", "general"),
+    ("int v = 2;", "v = v + v, x = v", "general"), ("int v = 2;", "x = v / 2", "general"),
+    ("clock y;", "x = y", "general"), ("", "x = x + 1", "general"), ("int v = 2;", "v = x, x = v", "general")])
+def test_windows_known_to_end(check, declared, updates, window):
+    """A window under one constant bound is read off its record where the values
+    that its clock is set to are known to be moderate."""
+    model = f"""<?xml version="1.0" encoding="utf-8"?>
+<nta><declaration>clock x; {declared}</declaration><template><name>T</name><declaration></declaration>
+<location id="id0"><name>l</name><label kind="invariant">x &lt;= 3</label></location><init ref="id0"/>
+<transition><source ref="id0"/><target ref="id0"/><label kind="assignment">{updates.replace(">", "&gt;")}</label></transition>
+</template><system>system T;</system></nta>"""
+    assert [l[1] for l in check(model)[0] if l[0] == "window"] == [window]

@@ -17,7 +17,7 @@ import cusmc_amd as cs
 
 import oracle
 
-from _models import E_ADD, E_DIV, RawNetwork
+from _models import E_ADD, E_DIV, E_MUL, E_SUB, RawNetwork
 
 pytestmark = pytest.mark.gpu
 
@@ -84,5 +84,33 @@ def test_windows_without_an_end_match_oracle(n_comp, live):
                     _equal(r.per_run[k], o[k], (n_comp, "sampler", lock, k))
         finally:
             s.close()
+    finally:
+        sim.close()
+
+
+@pytest.mark.parametrize("n_comp", [1, 2, 5, 40])
+def test_clocks_set_from_growing_variables_match_oracle(n_comp):
+    """A clock set to minus a variable that squares itself, which reaches
+    infinity, under a finite bound; the other components' to a counter's value."""
+    net = RawNetwork()
+    g = net.var(0.0)
+    for c in range(n_comp):
+        x, v = net.var(0.0, clock=True), net.var(2.0)
+        first = net.component([dict(type=0, invs=[(LE, x, net.lit(3.0))])])
+        grow = net.expr(E_MUL, net.ref(v), net.ref(v)) if c % 2 == 0 else net.expr(E_ADD, net.ref(v), net.lit(0.25))
+        net.edge(first, first, upds=[(g, net.expr(E_ADD, net.ref(g), net.lit(1.0))), (v, grow),
+                                     (x, net.expr(E_SUB, net.lit(0.0), net.ref(v)))])
+    net = net.build()
+    q = cs.var_query(0, 60.0, estimate=True, max_steps=60 * n_comp)
+    n_runs = 200
+    _, ro = oracle.run(net, q, seed=3, n_runs=n_runs, threads=8, per_run=PER_RUN)
+    sim = cs.GpuSimulator(net)
+    try:
+        P = 1 << (n_comp - 1).bit_length()
+        for S in sorted({min(P, 64), max(1, P // 2), max(1, P // 4), max(1, P // 16)}):
+            print(f"[gpu windows] growing n={n_comp} lanes={S}", flush=True)
+            r = sim.run(q, seed=3, n_runs=n_runs, lanes_per_run=S, per_run=PER_RUN)
+            for k in PER_RUN:
+                _equal(r.per_run[k], ro[k], (n_comp, S, k))
     finally:
         sim.close()
