@@ -138,13 +138,15 @@ int register_waves(int C, bool trace, int occ, bool tab) {
 // at 64 lanes and 11.0 at 32.  Receivers tested edge by edge have at most four to
 // a lane where the lists are longer than that (5, 20 and 34 edges on two channels, 70
 // components, 2e4 runs: 1.25, 2.58 and 3.72 ms; at sixteen 1.86, 4.13 and 6.56); with
-// two edges on 300 components sixteen are better, 2.1 ms for 2.9.
+// two edges on 300 components sixteen are better, 2.1 ms for 2.9, and where the
+// choice is eight or sixteen, 400 components: 6, 10 and 20 edges 5.26, 6.06 and 7.6 ms,
+// at eight 6.30, 6.71 and 7.5.
 smc_launch default_launch(const smc_model *m, uint64_t total_runs, bool trace) {
     const int P = m->img.n_leaves, stride = (m->img.n_vars + 1) | 1;
     const uint64_t simds = 4ull * (uint64_t)m->cu_count;
     smc_launch d{};
     int S = std::min(P, 64);
-    const int most = m->img.recv_tested > 4 ? 4 : 16;
+    const int most = m->img.recv_tested > 4 && P <= 256 ? 4 : 16;
     if (!(m->img.tests & (SMC_HF_XINV | SMC_HF_XBLK)))
         while (S > 1 && P / (S / 2) <= most) {
             const int s = S / 2, R = 64 / s;
