@@ -201,12 +201,18 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
     const auto staged = [&](int g) {
         return std::min(groups_per_cu(m->table_bytes + (size_t)g * wave + kLdsStatic), std::max(per_cu / g, 1)) * g;
     };
+    const int unstaged = std::min(per_cu, (int)(kLdsPerCu / (wave + kLdsStatic)));
     if (want.tables) {
-        int best = 0;
-        for (int g = 1; g <= SMC_MAX_GROUP_WAVES; g *= 2) best = std::max(best, staged(g));
-        pl.tab = best > 0;
-        // (left to choose: where they cost no waves)
-        if (!use && best < std::min(per_cu, groups_per_cu(wave + kLdsStatic))) pl.tab = false;
+        // (left to choose: where their bytes cost no waves.  What LDS rounds up may
+        // cost one of ten; 150 components with a clock each, 5e4 runs: eleven waves a
+        // CU 22.0 ms, ten that stage 19.4)
+        int best = 0, by_bytes = 0;
+        for (int g = 1; g <= SMC_MAX_GROUP_WAVES; g *= 2) {
+            best = std::max(best, staged(g));
+            by_bytes = std::max(by_bytes, std::min((int)(kLdsPerCu / (m->table_bytes + (size_t)g * wave + kLdsStatic)),
+                                                   std::max(per_cu / g, 1)) * g);
+        }
+        pl.tab = best > 0 && (use || by_bytes >= unstaged);
         if (pl.tab) {
             // the smallest workgroups that hold what the runs ask for: few
             // runs then spread over the CUs evenly
