@@ -105,15 +105,17 @@ constexpr uint32_t kWaitShare = 16;
 
 // The launch's counter gives some 80 takes a microsecond, whatever their size:
 // thousands of waves that come for the next runs every few turns wait longer for
-// it than for their runs.  So a wave begins with runs of its own, and one
-// whose last runs took fewer turns than this takes as many more at a time, up to
-// sixteen times its need and half its even share of what is left.  One step a run,
-// 1e7 runs: 0.37 ms for 1.98 with a take by need, 2e4 runs 10.4 us for 40.9;
-// UppaalWeightTest, 25 steps a run, 1e7 runs 4.4 ms for 12.0.  At 16 turns the
-// first and third are 0.69 and 6.2 ms; at 64 they are the same, but Fischer-32, 1e6
-// runs, takes 29.9 ms for 29.7.  (Runs of several instances differ too much: a
-// chunk at a time.)
+// it than for their runs.  So a wave begins with runs of its own, and where its runs
+// so far took fewer than 64 turns on average, one that comes again within this many
+// takes as many more at a time, up to sixteen times its need and half its even share
+// of what is left.  One step a run, 1e7 runs: 0.38 ms for 1.98 with a take by need, 2e4
+// runs 10.5 us for 40.9; UppaalWeightTest, 25 steps a run, 1e7 runs 4.6 ms for 12.0.
+// At 16 turns the first and third are 0.69 and 6.2 ms; at 64 they are the same, but
+// Fischer-32, 1e6 runs, takes 29.9 ms for 29.7.  Longer runs wait in a wave while
+// others stand idle: race-8, 1e6 runs, 11.8 ms with the length looked at, 13.0 without.
+// (Runs of several instances differ too much: a chunk at a time.)
 constexpr uint32_t kShortRuns = 32;
+constexpr int kLengthMost = 1 << 20;
 
 // The same pointer, as far as the optimiser knows another one.
 template <class T>
@@ -245,6 +247,7 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
     // since runs were started: turns of the loop, lanes without a run summed
     // over them
     uint32_t turns = kShortRuns, waited = 0;
+    int length = 64;  // turns less what as many runs of 64 turns would have taken, from the first refill on
     uint32_t r_next = 0, r_end = 0;  // runs of chunks begun, not started yet
 
     bool active = false, done = lane / S0 >= launch->segments;
@@ -311,7 +314,9 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
             const bool want = !active & !done;
             waited += (uint32_t)__popcll(__ballot(want));
             if (!any_lane(active) || kWaitShare * waited > 64 * turns) {
-                const uint32_t more = turns < kShortRuns ? min(kShortRuns / max(turns, 1u), 16u) : 1u;
+                length += (int)min(turns, 65536u) - (int)__popcll(__ballot(want));
+                length = min(max(length, -kLengthMost), kLengthMost);
+                const uint32_t more = length < 0 && turns < kShortRuns ? min(kShortRuns / max(turns, 1u), 16u) : 1u;
                 waited = turns = 0;
                 const uint64_t heads = __ballot(want & (sl == 0));
                 const int need = __popcll(heads), rank = __popcll(heads & ((1ull << seg_base) - 1));
@@ -324,7 +329,8 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                             const SMC_CONSTANT LaunchParams *L = opaque(args);
                             uint32_t n = 1;
                             if (L->n_inst == 1) {
-                                const uint64_t total = L->total_chunks, left = g < total ? total - g : 0;
+                                const uint64_t total = L->total_chunks, at = max((uint64_t)g, L->handed);
+                                const uint64_t left = at < total ? total - at : 0;
                                 n = ((uint32_t)(need - given) + chunk - 1) / chunk;
                                 n = max(n, (uint32_t)min((uint64_t)(n * more), left >> L->share_shift));
                             }
