@@ -43,6 +43,7 @@ struct Plan {
     uint32_t table_bytes = 0, wave_lds = 0;
     size_t lds = 0;
     int waves = 1, per_cu = 1;
+    int64_t resident = 1;  // waves that run side by side
     uint32_t chunk_runs = 1;
     int segments = 64;  // segments of a wave that take runs
 };
@@ -235,6 +236,7 @@ Plan plan_launch(const smc_model *m, const smc_launch *use, uint64_t total_runs,
         }
     }
     if (!pl.tab) per_cu = std::max(1, std::min(per_cu, groups_per_cu(wave + kLdsStatic)));
+    pl.resident = (int64_t)m->cu_count * per_cu;
     if (want.waves_per_cu > 0 && want.waves_per_cu < per_cu) per_cu = want.waves_per_cu;
     pl.per_cu = per_cu;
     int waves = want.waves > 0 ? want.waves : m->cu_count * per_cu;
@@ -484,7 +486,7 @@ int smc_run(smc_model *m, const smc_query *q, uint64_t seed, uint64_t run_begin,
         lp.segments = pl.segments;
         lp.share_shift = share_shift(waves);
         lp.first = ((uint32_t)pl.segments + pl.chunk_runs - 1) / pl.chunk_runs;
-        lp.handed = (uint64_t)lp.first * (uint64_t)waves;
+        lp.handed = (uint64_t)lp.first * (uint64_t)std::min<int64_t>(waves, pl.resident);
         lp.counter = m->d_counter;
         lp.round = nullptr;
         lp.tables = pl.tab ? (decltype(lp.tables))m->arena : nullptr;
@@ -597,7 +599,7 @@ int smc_run_noalloc(smc_model *m, const smc_query *q, uint64_t seed, uint64_t ru
         lp.segments = pl.segments;
         lp.share_shift = share_shift(waves);
         lp.first = ((uint32_t)pl.segments + pl.chunk_runs - 1) / pl.chunk_runs;
-        lp.handed = (uint64_t)lp.first * (uint64_t)waves;
+        lp.handed = (uint64_t)lp.first * (uint64_t)std::min<int64_t>(waves, pl.resident);
         lp.counter = d_counter;
         lp.round = nullptr;
         lp.tables = pl.tab ? (decltype(lp.tables))m->arena : nullptr;

@@ -41,8 +41,8 @@ struct LaunchParams {
     int32_t n_inst;
     uint64_t total_chunks;
     unsigned long long *counter;  // chunks handed out beyond those (cleared by launch_prep)
-    uint64_t handed;            // chunks that the waves begin with, in all
-    uint32_t first;             // ... and each
+    uint64_t handed;            // chunks that waves begin with, in all: those that run side by side
+    uint32_t first;             // ... and each of these
     int32_t segments;           // segments of a wave that take runs, at most
     int32_t share_shift;        // beyond its need a wave takes at most a 2^share_shift-th of what is left
     const uint64_t *round;      // optional: runs of round r start at run_begin + r * n_runs
