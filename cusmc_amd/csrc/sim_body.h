@@ -108,12 +108,13 @@ constexpr uint32_t kWaitShare = 16;
 // it than for their runs.  So a wave begins with runs of its own, and where its runs
 // so far took fewer than 64 turns on average, one that comes again within this many
 // takes as many more at a time, up to sixteen times its need and half its even share
-// of what is left.  One step a run, 1e7 runs: 0.38 ms for 1.98 with a take by need, 2e4
-// runs 10.5 us for 40.9; UppaalWeightTest, 25 steps a run, 1e7 runs 4.6 ms for 12.0.
-// At 16 turns the first and third are 0.69 and 6.2 ms; at 64 they are the same, but
-// Fischer-32, 1e6 runs, takes 29.9 ms for 29.7.  Longer runs wait in a wave while
-// others stand idle: race-8, 1e6 runs, 11.8 ms with the length looked at, 13.0 without.
-// (Runs of several instances differ too much: a chunk at a time.)
+// of what is left, less one for each of its segments unless the last took under eight
+// turns.  One step a run, 1e7 runs: 0.38 ms for 1.98 with a take by need, 2e4 runs
+// 10.5 us for 40.9; UppaalWeightTest, 25 steps a run, 1e7 runs 5.9 ms for 12.0.  Longer
+// runs wait in a wave while others stand idle: race-8, 1e6 runs, 11.8 ms with the length
+// looked at and 13.0 without; SIR-60, 1e5 runs, 1.17 ms with the segments' share left
+// and 1.30 without (UppaalWeightTest 4.6).  (Runs of several instances differ too much:
+// a chunk at a time.)
 constexpr uint32_t kShortRuns = 32;
 constexpr int kLengthMost = 1 << 20;
 
@@ -317,8 +318,9 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
             const bool want = !active & !done;
             waited += (uint32_t)__popcll(__ballot(want));
             if (!any_lane(active) || kWaitShare * waited > 64 * turns) {
-                length += (int)min(turns, 65536u) - (int)__popcll(__ballot(want));
-                length = min(max(length, -kLengthMost), kLengthMost);
+                const uint32_t idle = (uint32_t)__popcll(__ballot(want));
+                const bool brief = 8 * turns < idle;
+                length = min(max(length + (int)min(turns, 65536u) - (int)idle, -kLengthMost), kLengthMost);
                 const uint32_t more = length < 0 && turns < kShortRuns ? min(kShortRuns / max(turns, 1u), 16u) : 1u;
                 waited = turns = 0;
                 const uint64_t heads = __ballot(want & (sl == 0));
@@ -335,7 +337,8 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
                                 const uint64_t total = L->total_chunks, at = max((uint64_t)g, L->handed);
                                 const uint64_t left = at < total ? total - at : 0;
                                 n = ((uint32_t)(need - given) + chunk - 1) / chunk;
-                                n = max(n, (uint32_t)min((uint64_t)(n * more), left >> L->share_shift));
+                                const uint64_t half = left >> L->share_shift, keep = brief ? 0u : (uint32_t)L->segments;
+                                n = max(n, (uint32_t)min((uint64_t)(n * more), half > keep ? half - keep : 0));
                             }
                             take(n, L);
                         }
