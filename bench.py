@@ -52,9 +52,9 @@ SEED = 20261202
 # what they read for a 1 GiB device copy).  valu: SQ_INSTS_VALU (wave64 VALU
 # instructions) per race step.
 PROFILED = {
-    "fischer32": {"shape": (2, 0, 1), "traffic_per_run": 40.1, "valu_per_step": 48.5,
+    "fischer32": {"shape": (2, 0, 1), "traffic_per_run": 39.7, "valu_per_step": 48.4,
                   "source": "profiles/sim_kernel_fischer32.md"},
-    "sir350": {"shape": (32, 3, 1), "traffic_per_run": 54.7, "valu_per_step": 439.7,
+    "sir350": {"shape": (32, 3, 1), "traffic_per_run": 46.2, "valu_per_step": 438.2,
                "source": "profiles/sim_kernel_sir350.md"},
 }
 
@@ -358,8 +358,8 @@ def main() -> int:
     ap.add_argument("--occupancy", type=int, default=0, choices=[0, 3],
                     help="with --lanes: register policy (0 unrestricted, 3 three waves per SIMD)")
     ap.add_argument("--tables", type=int, default=0, choices=[0, 1, 2],
-                    help="with --lanes: model tables in global memory (0), staged in LDS (1), or staged "
-                         "if they fit (2)")
+                    help="with --lanes: model tables in global memory (0) or staged in LDS (1 or 2; refused "
+                         "where they do not fit)")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-is", action="store_true", help="fischer32: skip the learned-IS leg")
     args = ap.parse_args()

@@ -128,15 +128,15 @@ int register_waves(int C, bool trace, int occ, bool tab) {
 // The launch of a call that asks for none on a model without a tuned one:
 // the fewest lanes per run at which two waves per SIMD have their runs and
 // their LDS, tables staged, and three waves per SIMD where sixteen slots a
-// lane leave registers for two and there are runs for more.  A step costs a wave much the same whether it
-// advances one run or many, so many runs are packed; few runs are spread, for
-// the shortest steps.  Against one run per 64 lanes and tables in global
-// memory (ms): covid-350, 16384 runs, 32 lanes 19.1 for 35.2; SIR-77, 5e4
-// runs, 8 lanes 1.73 for 4.69; Fischer-32, 2e5 runs, 2 lanes 6.68 for 25.2;
-// at 2000 runs Fischer-32 takes 0.85 at 32 lanes, 0.95 at 16 and 2.0 at 2.
+// lane leave registers for two and there are runs for more.  A step costs a wave
+// much the same whether it advances one run or many, so many runs are packed; few
+// runs are spread, for the shortest steps.  Against the widest packing and tables in
+// global memory (kernel ms): covid-350, 16384 runs, 32 lanes 17.6 for 34.4; SIR-77,
+// 5e4 runs, 8 lanes 1.52 for 5.06; Fischer-32, 2e5 runs, 2 lanes 7.2 for 25.1;
+// at 2000 runs Fischer-32 takes 0.82 at 32 lanes, 0.88 at 16 and 1.64 at 2.
 // Where slots are tested one after another (invariants and blocking tests of
-// several records) a lane gets as few as there are: csma-100, 16384 runs, 5.5
-// at 64 lanes and 11.0 at 32.  Receivers tested edge by edge have at most four to
+// several records) a lane gets as few as there are: csma-100, 16384 runs, 4.8
+// at 64 lanes and 10.7 at 32.  Receivers tested edge by edge have at most four to
 // a lane where the lists are longer than that (5, 20 and 34 edges on two channels, 70
 // components, 2e4 runs: 1.25, 2.58 and 3.72 ms; at sixteen 1.86, 4.13 and 6.56); with
 // two edges on 300 components sixteen are better, 2.1 ms for 2.9, and where the

@@ -37,8 +37,8 @@
 //     order (SyncInSerial), each lane executing its own component's
 //     transition.  The winner's edges are tested side by side, one per lane
 //     of the segment.
-//   * Runs are handed out by an atomic counter, so a segment that finishes a
-//     short run immediately starts the next one.
+//   * Beyond a wave's first, runs are handed out by an atomic counter, so a
+//     segment that finishes a short run soon starts the next one.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -126,9 +126,9 @@ __device__ __forceinline__ const SMC_CONSTANT T *opaque(const SMC_CONSTANT T *p)
 }
 
 // A wave begins with runs of its own, then takes chunks of runs from the
-// launch's queue, and hands the runs to its segments; all its segments work on one instance, which (its tables,
-// query and outputs) is thereby uniform across the wave and lives in scalar
-// registers.  A chunk of another instance waits until this one's runs are
+// launch's queue, and hands the runs to its segments; all its segments work on
+// one instance, which (its tables, query and outputs) is thereby uniform across
+// the wave and lives in scalar registers.  A chunk of another instance waits until this one's runs are
 // done.  A workgroup holds blockDim/64 independent waves.  With TAB
 // (single-instance launches) the workgroup first copies the model's tables
 // into LDS and every wave reads them there: the race and the transitions are
@@ -553,13 +553,13 @@ __device__ __forceinline__ void sim_body(const LaunchParams &lp) {
   }
 }
 
-// Two register policies of the run kernel: unrestricted (100-119 VGPRs and
-// four waves per SIMD up to two slots per lane, 119-132 and three or four at
-// four, 145-158 and three at eight, 195-207 and two at sixteen), and at most
-// 168 (three waves per SIMD), which only sixteen slots spill to keep (some
-// thirty registers).  At sixteen it depends on the packing: SIR-350, 2e4 runs,
-// 8.1 ms with three waves and 10.5 with two, Fischer-32, 2e5 runs, whose LDS
-// holds two, 6.8 and 6.7; the autotuner measures both.
+// Two register policies of the run kernel: unrestricted (99-123 VGPRs and
+// four waves per SIMD up to two slots per lane, 118 and four at four, with
+// digests 131 and three, 143-156 and three at eight, 193-206 and two at
+// sixteen), and at most 168 (three waves per SIMD), which only sixteen slots
+// spill to keep (some thirty registers).  At sixteen it depends on the packing:
+// SIR-350, 2e4 runs, 7.2 ms with three waves and 9.5 with two, Fischer-32, 2e5
+// runs, whose LDS holds two, 6.6 both; the autotuner measures both.
 template <int C, bool TRACE, bool TAB>
 __global__ __launch_bounds__(64 * SMC_MAX_GROUP_WAVES) void sim_kernel(LaunchParams lp) {
     sim_body<C, TRACE, TAB>(lp);

@@ -81,8 +81,9 @@ typedef struct smc_launch {
     int32_t waves_per_cu;      /* occupancy target used when waves == 0     */
     int32_t occupancy;         /* 0: registers unrestricted (two waves per
                                   SIMD at sixteen slots per lane, three at
-                                  eight, four below); 3: at most 168
-                                  registers, three waves per SIMD          */
+                                  eight and with digests at four, four
+                                  below); 3: at most 168 registers, three
+                                  waves per SIMD                           */
     int32_t tables;            /* 0: model tables read from global memory;
                                   1: staged in LDS, one copy per workgroup;
                                   refused where they do not fit, unless they
