@@ -500,6 +500,13 @@ ModelImage lower(const smc_network &n, bool use_locals) {
             most[v] = round < 8 ? now : HUGE_VAL;
             grows = true;
         }
+        // (a long chain of variables: one link a round)
+        if (round < 64) continue;
+        for (int u = 0; u < n.n_updates; ++u) {
+            double c;
+            if (!literal(n.updates[u].expr, &c)) most[n.updates[u].var] = HUGE_VAL;
+        }
+        break;
     }
     std::vector<uint8_t> clock_moderate(n.n_vars);
     for (int v = 0; v < n.n_vars; ++v) clock_moderate[v] = moderate(n.var_init[v]);

@@ -131,7 +131,11 @@ def test_commuting_receivers_fire_together(check):
     ("int v = 7; int w = 1;", "v = v + 3, w = v * v, x = w", "inline"), ("int v; int w;", "v = w, w = v, x = w", "inline"),
     ("int v; int w;", "v = w + 1, w = v, x = w", "general"), ("int v = 2;", "v = v * v, x = v", "general"),
     ("int v = 2;", "v = v + v, x = v", "general"), ("int v = 2;", "x = v / 2", "general"),
-    ("clock y;", "x = y", "general"), ("", "x = x + 1", "general"), ("int v = 2;", "v = x, x = v", "general")])
+    ("clock y;", "x = y", "general"), ("", "x = x + 1", "general"), ("int v = 2;", "v = x, x = v", "general"),
+    ("int " + ", ".join(f"v{k}" for k in range(200)) + ";",
+     ", ".join(f"v{k + 1} = v{k} + 1" for k in range(199)) + ", x = v199", "general"),
+    ("int " + ", ".join(f"v{k}" for k in range(6)) + ";",
+     ", ".join(f"v{k + 1} = v{k} + 1" for k in range(5)) + ", x = v5", "inline")])
 def test_windows_known_to_end(check, declared, updates, window):
     """A window under one constant bound is read off its record where the values
     that its clock is set to are known to be moderate."""
